@@ -4,7 +4,7 @@
 //  engine/inference_executor.py:776-806).
 //
 // One 1024-thread workgroup per logits row; the row is only ever READ
-// (no sort, no [B,V] temporaries).  All three filters keep a "top set by
+// (no sort, no [B,V] temporaries), 16-bit rows that fit a CU from memory only once.  All three filters keep a "top set by
 // value", so each one reduces to a threshold on the order-preserving
 // integer key of the raw logit, found by radix select over LDS histograms:
 //   top-k : k-th largest key (count histogram) + how many ties of it to keep
@@ -12,7 +12,9 @@
 //   min-p : weight threshold  exp((x-max)/T) >= min_p
 // then a single multinomial draw (Philox4x32-10) over the surviving weights.
 // Math is fp32 throughout (the reference computes in the logits dtype).
-#include "common.h"
+#include <algorithm>
+
+#include "latent.h"
 
 namespace {
 
@@ -48,6 +50,7 @@ struct Shared {
   unsigned bcast_u[4];
   float bcast_f[4];
 };
+static_assert(sizeof(Shared) % 16 == 0, "the row lies behind it");
 
 // ---- Philox4x32-10 -----------------------------------------------------------
 __device__ __forceinline__ void philox_round(uint32_t (&c)[4], const uint32_t (&k)[2]) {
@@ -170,14 +173,14 @@ __device__ __forceinline__ unsigned block_exscan_u(unsigned x, unsigned &total, 
 // All threads run the same trip count and call f(index, raw, in_range) with
 // the wave fully converged (f may use cross-lane operations: DPP / bpermute
 // read stale registers from lanes that left a divergent loop).
-template <typename Tag, typename F>
+// U: vectors of a thread in flight (a pass is L2/MALL-latency bound otherwise)
+template <typename Tag, int U = 4, typename F>
 __device__ __forceinline__ void row_foreach(const typename elem<Tag>::T *row, int vocab, bool vec_ok, F &&f) {
   typedef typename elem<Tag>::T T;
   constexpr int VEC = elem<Tag>::VEC;
   int scalar_from = 0;
   if (vec_ok) {
     const int nvec = vocab / VEC;
-    constexpr int U = 4;  // loads in flight per thread: a pass is L2/MALL-latency bound otherwise
     for (int c0 = 0; c0 < nvec; c0 += kThreads * U) {
       u32x4 raw[U];
 #pragma unroll
@@ -222,29 +225,163 @@ __device__ __forceinline__ void hist_add(V *hist, bool active, unsigned bin, V v
   if (active) atomicAdd(&hist[bin], val);
 }
 
-template <typename Tag>
+typedef __attribute__((ext_vector_type(2))) short s16x2;
+
+// A row of 16-bit logits on its workgroup's CU: the first kLdsVectors vectors of a thread in LDS, NR more in registers.  Vector u of thread t is
+// vector t + 1024 u of the row, so a thread's elements and their order are those of row_foreach.
+constexpr int kLdsVectors = 9, kRegVectors = 10;
+template <typename Tag, int NR>
+struct RowOnChip {
+  const u32x4 *lds;   // [kLdsVectors][kThreads]
+  u32x4 r[NR ? NR : 1];
+  int nvec;
+  __device__ __forceinline__ void load_registers(const uint16_t *row) {
+#pragma unroll
+    for (int u = 0; u < NR; ++u)
+      r[u] = *reinterpret_cast<const u32x4 *>(row + (int64_t)min((u + kLdsVectors) * kThreads + (int)threadIdx.x, nvec - 1) * 8);
+  }
+  __device__ __forceinline__ void load(const uint16_t *row, int n, char *smem) {
+    nvec = n, lds = (const u32x4 *)smem;
+    load_registers(row);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int u = 0; u < kLdsVectors && u * kThreads < nvec; ++u)
+      __builtin_amdgcn_global_load_lds((const MV_AS1 void *)(row + (int64_t)min(u * kThreads + (int)threadIdx.x, nvec - 1) * 8),
+                                       (MV_AS3 void *)(smem + (u * kThreads + wave * 64) * 16), 16, 0, 0);
+  }
+  // largest element of this thread; the vectors in registers, asked for first, while those for the LDS are on their way
+  __device__ __forceinline__ float largest() const {
+    float best = -INFINITY;
+    auto take = [&](u32x4 v, bool in) {
+      float f[8];
+      unpack8<Tag>(v, f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) best = in && f[j] > best ? f[j] : best;
+    };
+    const int own = (nvec - (int)threadIdx.x + kThreads - 1) / kThreads, most = min(kLdsVectors, (nvec + kThreads - 1) / kThreads);
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      if ((u + kLdsVectors) * kThreads >= nvec) break;
+      take(r[u], u + kLdsVectors < own);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (a thread reads only what its own wave has brought)
+#pragma unroll 1
+    for (int u = 0; u < most; ++u) take(lds[u * kThreads + threadIdx.x], u < own);
+    return best;
+  }
+  // f(u, vector) of this thread's vectors, in order; `in`: there is such a vector (the wave stays together)
+  template <typename F>
+  __device__ __forceinline__ void vectors(F &&f) const {
+    int own = (nvec - (int)threadIdx.x + kThreads - 1) / kThreads;
+    const int most = min(kLdsVectors, (nvec + kThreads - 1) / kThreads);
+#pragma unroll 1
+    for (int u = 0; u < most; ++u) f(u, lds[u * kThreads + threadIdx.x], u < own);
+#pragma unroll
+    for (int u = 0; u < NR; ++u) {
+      if ((u + kLdsVectors) * kThreads >= nvec) break;
+      u32x4 v = r[u];
+      asm volatile("" : "+v"(v), "+v"(own));   // (what one pass unpacks is not kept for the next: it would take the row's registers)
+      f(u + kLdsVectors, v, u + kLdsVectors < own);
+    }
+  }
+  // f(raw) of every element
+  template <typename F>
+  __device__ __forceinline__ void foreach(F &&f) const {
+    vectors([&](int u, u32x4 v, bool in) {
+      if (in) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) f((uint16_t)(v[j] & 0xffffu)), f((uint16_t)(v[j] >> 16));
+      }
+    });
+  }
+  // f(index, raw) of every element whose bits, as a signed number, reach `least`: for a positive value all elements at least as large
+  // (and every NaN without a sign) qualify.  A wave takes as many turns over a vector as its busiest lane has such elements.
+  template <typename F>
+  __device__ __forceinline__ void foreach_from(short least, F &&f) const {
+    const s16x2 floor = {least, least};
+    vectors([&](int u, u32x4 v, bool in) {
+      uint32_t below = 0;   // signs of element - least (saturated): element 2 j in bit 2 j, element 2 j + 1 in bit 16 + 2 j
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t d = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(s16x2, (uint32_t)v[j]), floor));
+        below |= (d & 0x80008000u) >> (15 - 2 * j);
+      }
+      uint32_t todo = in ? ~((below & 0xffu) | below >> 15) & 0xffu : 0u;
+      while (todo) {
+        const int e = __builtin_ctz(todo);
+        todo &= todo - 1;
+        const uint32_t w = e < 4 ? (e < 2 ? v[0] : v[1]) : (e < 6 ? v[2] : v[3]);
+        f((u * kThreads + (int)threadIdx.x) * 8 + e, (uint16_t)(e & 1 ? w >> 16 : w & 0xffffu));
+      }
+    });
+  }
+  // f(top - bits) of every element, `top` the bits of a positive value: up to `top` the places of the values from `top` down to zero, more for
+  // negative values, larger ones and NaN
+  template <typename F>
+  __device__ __forceinline__ void foreach_place(uint32_t top, F &&f) const {
+    typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
+    const u16x2 t = {(unsigned short)top, (unsigned short)top};
+    vectors([&](int u, u32x4 v, bool in) {
+      if (in) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t d = __builtin_bit_cast(uint32_t, t - __builtin_bit_cast(u16x2, (uint32_t)v[j]));
+          f(d & 0xffffu), f(d >> 16);
+        }
+      }
+    });
+  }
+  static constexpr short kAll = -32768;
+  // the bound for elements with a key of at least `key` (make_key); none for keys of negative values
+  static __device__ __forceinline__ short least_of_key(uint32_t key) { return key >= 0x8000u ? (short)(key - 0x8000u) : kAll; }
+};
+
+// NR >= 0: the row stays on the CU (16-bit logits in whole, aligned vectors, no mask asked for; RowOnChip); -1: every pass reads memory.
+// A row is one pass for the maximum, one for the histogram of a filter, one for ties, one for the masses; 256 rows of 151 936 logits are one
+// workgroup a CU, 304 KB each: more than the LDS and, beside what the passes need, more than the registers, but not more than half in each.  Kept
+// there, the passes behind the first read no memory, and those behind a filter skip what cannot be kept.
+// 256 rows of 151 936 bf16 logits, us: greedy 19 -> 21, plain 59 -> 33, top-k 40 91 -> 41, top-p 0.9 83 -> 59, min-p 56 -> 30; one row 16 -> 12, 52 -> 22,
+// 81 -> 30, 73 -> 47, 49 -> 20.  What is left is vector arithmetic: an exponential and four instructions an element where every weight counts.
+template <typename Tag, int NR>
 __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   typedef typename elem<Tag>::T T;
   constexpr int KBITS = keyinfo<Tag>::BITS;
   constexpr int LEVELS = KBITS / 8;
-  __shared__ Shared sh;
+  constexpr bool CHIP = NR >= 0;
+  typedef RowOnChip<Tag, CHIP ? NR : 0> Row;
+  constexpr int U = CHIP ? 1 : 4;   // (beside a row in registers only rare passes read memory: little of it in flight)
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // Shared | the row's first vectors
+  Shared &sh = *(Shared *)smem;
+  char *row_lds = smem + sizeof(Shared);
 
   const int rowi = blockIdx.x;
   const int V = p.vocab;
   const T *row = (const T *)p.logits + (int64_t)rowi * p.ld;
   const bool vec_ok = ((reinterpret_cast<uintptr_t>(row) & 15u) == 0);
-  uint8_t *mask_row = p.keep_mask ? p.keep_mask + (int64_t)rowi * V : nullptr;
+  uint8_t *mask_row = !CHIP && p.keep_mask ? p.keep_mask + (int64_t)rowi * V : nullptr;
   const float temp = p.temperatures ? p.temperatures[rowi] : 1.0f;
 
   // ---- pass A: max (and argmax, lowest index on ties) ------------------------------
   float best = -INFINITY;
   int best_i = 0x7fffffff;
-  row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) {
-    const float x = elem<Tag>::ld(raw);
-    if (ok && (x > best || (x == best && i < best_i))) { best = x; best_i = i; }
-  });
+  Row chip;
+  if constexpr (CHIP) {
+    chip.load(row, V / 8, row_lds);
+    best = chip.largest();
+  } else {
+    row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) {
+      const float x = elem<Tag>::ld(raw);
+      if (ok && (x > best || (x == best && i < best_i))) { best = x; best_i = i; }
+    });
+  }
   const float xmax = block_max(best, sh);
   if (temp == 0.0f) {  // greedy (argmax, not multinomial over softmax(l/1e-8))
+    if constexpr (CHIP) {
+      const short least = xmax > 0.f ? Row::least_of_key(make_key<Tag>(elem<Tag>::st(xmax))) : Row::kAll;
+      if (best == xmax)
+        chip.foreach_from(least, [&](int i, T raw) {
+          if (elem<Tag>::ld(raw) == xmax) best_i = min(best_i, i);
+        });
+    }
     int cand = (best == xmax) ? best_i : 0x7fffffff;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) cand = min(cand, __shfl_xor(cand, off, 64));
@@ -282,6 +419,7 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   unsigned tie_before = 0;   // this thread's first tie rank (thread-major order)
   uint32_t key_p = 0;        // keep key >= key_p
   bool topk_done = false, topp_done = false;
+  unsigned kept_c = 0xffffffffu;   // elements with a key of at least key_p (top-k off; not counted by the radix select)
 
   // ---- 16-bit logits: ONE histogram pass resolves both thresholds.  Every bin of the window is
   //      exactly one representable value (bin = key(max) - key), so there is no second radix level;
@@ -290,98 +428,145 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   if constexpr (KBITS == 16) {
     if (topk_on || topp_on) {
       const uint32_t kmax = make_key<Tag>(elem<Tag>::st(xmax));
-      for (int i = threadIdx.x; i < kWin; i += kThreads) sh.wcnt[i] = 0u;
-      __syncthreads();
-      // only COUNTS are accumulated: all members of a bin are the same value, so its mass is
-      // count * weight(value).  Values below the window need their mass only when top-k is off.
-      unsigned under_c = 0;
-      float under_m = 0.f;
-      row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) {
-        const uint32_t bin = kmax - make_key<Tag>(raw);
-        if (ok) {
-          if (bin < (uint32_t)kWin) {
-            atomicAdd(&sh.wcnt[bin], 1u);
-          } else {
-            ++under_c;
-            if (!topk_on) under_m += weight(elem<Tag>::ld(raw));
-          }
-        }
-      });
-      __syncthreads();
       auto bin_weight = [&](uint32_t bin) -> float {  // weight of the value that owns `bin`
         const uint32_t key = kmax - bin;              // invert make_key: sortable key -> raw bits
         const uint32_t rawbits = (key & 0x8000u) ? (key & 0x7fffu) : (~key & 0xffffu);
         return weight(elem<Tag>::ld((T)rawbits));
       };
-      const unsigned c0 = sh.wcnt[2 * threadIdx.x], c1 = sh.wcnt[2 * threadIdx.x + 1];
-      const float m0 = c0 ? (float)c0 * bin_weight(2 * threadIdx.x) : 0.f;
-      const float m1 = c1 ? (float)c1 * bin_weight(2 * threadIdx.x + 1) : 0.f;
-      unsigned win_c;
-      float win_m;
-      const unsigned pc = block_exscan_u(c0 + c1, win_c, sh);   // elements in bins before mine
-      const float pm = block_exscan_f(m0 + m1, win_m, sh);      // their mass
-      const float under_mass = block_sum_f(under_m, sh);
-      unsigned under_cnt;
-      (void)block_exscan_u(under_c, under_cnt, sh);
-      __syncthreads();
-      if (threadIdx.x == 0) { sh.bcast_u[0] = 0xffffffffu; sh.bcast_u[3] = 0u; }
-      __syncthreads();
-      int limit = kWin - 1;       // last bin that still has top-k members
-      float z1 = win_m + under_mass;
-      bool ok_fast = true;
-      if (topk_on) {
-        if (win_c >= (unsigned)k_raw) {
-          const unsigned kk = (unsigned)k_raw;
-          if (pc < kk && kk <= pc + c0 + c1) {  // exactly one thread
-            const bool second = pc + c0 < kk;
-            const unsigned above = second ? pc + c0 : pc;
-            const unsigned bc = second ? c1 : c0;
-            const float bm = second ? m1 : m0;
-            const unsigned need = kk - above;
-            sh.bcast_u[0] = 2 * threadIdx.x + (second ? 1 : 0);
-            sh.bcast_u[1] = need;
-            sh.bcast_u[2] = bc;
-            sh.bcast_f[1] = (second ? pm + m0 : pm) + (float)need * (bm / (float)bc);  // mass of the top-k set
-          }
+      // this thread's two bins: counts, masses and what lies in the bins before them
+      unsigned c0, c1, win_c, pc;
+      float m0, m1, win_m, pm;
+      auto clear = [&]() {
+        for (int i = threadIdx.x; i < kWin; i += kThreads) sh.wcnt[i] = 0u;
+        if (threadIdx.x == 0) sh.bcast_u[0] = kWin - 1u, sh.bcast_u[3] = 0u;
+        __syncthreads();
+      };
+      auto scan = [&]() {
+        __syncthreads();
+        c0 = sh.wcnt[2 * threadIdx.x], c1 = sh.wcnt[2 * threadIdx.x + 1];
+        m0 = c0 ? (float)c0 * bin_weight(2 * threadIdx.x) : 0.f;
+        m1 = c1 ? (float)c1 * bin_weight(2 * threadIdx.x + 1) : 0.f;
+        pc = block_exscan_u(c0 + c1, win_c, sh);   // elements in bins before mine
+        pm = block_exscan_f(m0 + m1, win_m, sh);   // their mass
+      };
+      // only COUNTS are accumulated: all members of a bin are the same value, so its mass is count * weight(value).
+      auto count = [&](T raw, uint32_t bins) {
+        const uint32_t bin = kmax - make_key<Tag>(raw);
+        if (bin < bins) atomicAdd(&sh.wcnt[bin], 1u);
+        return bin < bins;
+      };
+      uint32_t win = kWin;    // bins counted
+      float all_m = 0.f;      // the row's mass (asked for when top-k is off)
+      if constexpr (CHIP) {
+        // What is asked of the whole row besides (top-p: its mass) is a pass without branches.  With top-k, at least k elements reach the k-th
+        // largest of the threads' maxima, so few elements are left to count; a bound that is no use (fewer maxima than k) is the whole window.
+        if (topk_on) {
+          clear();
+          if (best > -INFINITY) count(elem<Tag>::st(best), kWin);
+          scan();
+          const unsigned least_c = (unsigned)min(k_raw, (int64_t)kThreads + 1);
+          if (pc < least_c && least_c <= pc + c0 + c1) sh.bcast_u[0] = 2 * threadIdx.x + (pc + c0 < least_c ? 1 : 0);
           __syncthreads();
-          const unsigned bk = sh.bcast_u[0];
-          key_k = kmax - bk;
-          need_ties = sh.bcast_u[1];
-          ties_partial = need_ties < sh.bcast_u[2];
-          z1 = sh.bcast_f[1];
-          limit = (int)bk;
-          topk_done = true;
+          win = sh.bcast_u[0] + 1u;
         } else {
-          ok_fast = false;  // the k-th value lies below the window
+          float z = 0.f;
+          chip.foreach([&](T raw) { z += weight(elem<Tag>::ld(raw)); });
+          all_m = block_sum_f(z, sh);
         }
       }
-      if (ok_fast && topp_on) {
-        // largest bin index i <= limit whose strictly-larger mass E_i fits the budget (E_0 = 0 always does)
-        const float budget = top_p * z1;
-        unsigned cand = 0;
-        const int b0 = 2 * threadIdx.x, b1 = b0 + 1;
-        if (b0 <= limit && pm <= budget) cand = (unsigned)b0 + 1u;
-        if (b1 <= limit && pm + m0 <= budget) cand = (unsigned)b1 + 1u;
-        if (cand) atomicMax(&sh.bcast_u[3], cand);
+      bool ok_fast;
+      for (;; win = kWin) {
+        unsigned under_cnt = 0;
+        float z1;
+        ok_fast = true;
         __syncthreads();
-        const unsigned bp = sh.bcast_u[3] - 1u;  // >= 0: bin 0 always qualifies
-        // without top-k, "the whole window fits" means the nucleus edge is below the window
-        if (!topk_on && under_cnt > 0 && bp == (unsigned)(kWin - 1) && win_m <= budget) {
-          ok_fast = false;
-        } else {
-          key_p = kmax - bp;
-          topp_done = true;
+        clear();
+        if constexpr (CHIP) {
+          if (win < (uint32_t)kWin) chip.foreach_from(kmax >= win ? Row::least_of_key(kmax - win + 1) : Row::kAll, [&](int i, T raw) { count(raw, win); });
+          else if (kmax >= 0x8000u + kWin - 1u) chip.foreach_place(kmax - 0x8000u, [&](uint32_t bin) {   // (the window ends above zero)
+            if (bin < (uint32_t)kWin) atomicAdd(&sh.wcnt[bin], 1u);
+          });
+          else chip.foreach([&](T raw) { count(raw, kWin); });
+          scan();
+          under_cnt = (unsigned)V - win_c;
+          z1 = all_m;
+        } else {   // values below the window need their mass only when top-k is off
+          unsigned under_c = 0;
+          float under_m = 0.f;
+          row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) {
+            if (ok && !count(raw, kWin)) {
+              ++under_c;
+              if (!topk_on) under_m += weight(elem<Tag>::ld(raw));
+            }
+          });
+          scan();
+          z1 = win_m + block_sum_f(under_m, sh);
+          (void)block_exscan_u(under_c, under_cnt, sh);
         }
+        int limit = (int)win - 1;       // last bin that still has top-k members
+        if (topk_on) {
+          if (win_c >= (unsigned)k_raw) {
+            const unsigned kk = (unsigned)k_raw;
+            __syncthreads();
+            if (pc < kk && kk <= pc + c0 + c1) {  // exactly one thread
+              const bool second = pc + c0 < kk;
+              const unsigned above = second ? pc + c0 : pc;
+              const unsigned bc = second ? c1 : c0;
+              const float bm = second ? m1 : m0;
+              const unsigned need = kk - above;
+              sh.bcast_u[0] = 2 * threadIdx.x + (second ? 1 : 0);
+              sh.bcast_u[1] = need;
+              sh.bcast_u[2] = bc;
+              sh.bcast_f[1] = (second ? pm + m0 : pm) + (float)need * (bm / (float)bc);  // mass of the top-k set
+            }
+            __syncthreads();
+            const unsigned bk = sh.bcast_u[0];
+            key_k = kmax - bk;
+            need_ties = sh.bcast_u[1];
+            ties_partial = need_ties < sh.bcast_u[2];
+            z1 = sh.bcast_f[1];
+            limit = (int)bk;
+            topk_done = true;
+          } else {
+            ok_fast = false;  // the k-th value lies below the window
+          }
+        }
+        if (ok_fast && topp_on) {
+          // largest bin index i <= limit whose strictly-larger mass E_i fits the budget (E_0 = 0 always does)
+          const float budget = top_p * z1;
+          unsigned cand = 0;
+          const int b0 = 2 * threadIdx.x, b1 = b0 + 1;
+          if (b0 <= limit && pm <= budget) cand = (unsigned)b0 + 1u;
+          if (b1 <= limit && pm + m0 <= budget) cand = (unsigned)b1 + 1u;
+          if (cand) atomicMax(&sh.bcast_u[3], cand);
+          __syncthreads();
+          const unsigned bp = sh.bcast_u[3] - 1u;  // >= 0: bin 0 always qualifies
+          // without top-k, "the whole window fits" means the nucleus edge is below the window
+          if (!topk_on && under_cnt > 0 && bp == win - 1u && win_m <= budget) {
+            ok_fast = false;
+          } else {
+            key_p = kmax - bp;
+            topp_done = true;
+            if (bp >> 1 == threadIdx.x) sh.bcast_u[2] = pc + c0 + (bp & 1 ? c1 : 0);   // elements that are kept
+          }
+        }
+        if (ok_fast || win == (uint32_t)kWin) break;
+      }
+      if (topp_done && !topk_on) {
+        __syncthreads();
+        kept_c = sh.bcast_u[2];
       }
       if (ties_partial && topk_done) {
         unsigned mine_t = 0;
-        row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) { mine_t += ok && make_key<Tag>(raw) == key_k; });
+        if constexpr (CHIP) chip.foreach_from(Row::least_of_key(key_k), [&](int i, T raw) { mine_t += make_key<Tag>(raw) == key_k; });
+        else row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) { mine_t += ok && make_key<Tag>(raw) == key_k; });
         unsigned tot;
         tie_before = block_exscan_u(mine_t, tot, sh);
       }
     }
   }
 
+  const bool rare = (topk_on && !topk_done) || (topp_on && !topp_done);
   if (topk_on && !topk_done) {
     uint32_t prefix = 0;
     unsigned above = 0;      // elements with a strictly larger prefix
@@ -391,7 +576,7 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
       __syncthreads();
       if (threadIdx.x < 256) sh.ihist[threadIdx.x] = 0;
       __syncthreads();
-      row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) {
+      row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) {
         const uint32_t key = make_key<Tag>(raw);
         const bool in = ok && (lvl == 0 || (key >> (shift + 8)) == prefix);
         hist_add<unsigned>(sh.ihist, in, (key >> shift) & 0xffu, 1u);
@@ -418,7 +603,7 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
     ties_partial = need_ties < bin_count;
     if (ties_partial) {
       unsigned mine = 0;
-      row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) { mine += ok && make_key<Tag>(raw) == key_k; });
+      row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) { mine += ok && make_key<Tag>(raw) == key_k; });
       unsigned tot;
       tie_before = block_exscan_u(mine, tot, sh);
     }
@@ -437,7 +622,7 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   if (topp_on && !topp_done) {
     float z = 0.f;
     tie_seen = 0;
-    row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) {
+    row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) {
       if (ok && in_topk(make_key<Tag>(raw))) z += weight(elem<Tag>::ld(raw));
     });
     const float budget = top_p * block_sum_f(z, sh);
@@ -449,7 +634,7 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
       if (threadIdx.x < 256) sh.fhist[threadIdx.x] = 0.f;
       __syncthreads();
       tie_seen = 0;
-      row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) {
+      row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) {
         const uint32_t key = make_key<Tag>(raw);
         const bool member = ok && in_topk(key);
         const bool in = member && (lvl == 0 || (key >> (shift + 8)) == prefix);
@@ -474,6 +659,9 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
     }
     key_p = prefix;
   }
+  if constexpr (CHIP) {
+    if (rare) chip.load_registers(row);   // (the passes of the radix select read memory, and need the registers)
+  }
 
   // ---- min-p: prob < min_p * max_prob  <=>  weight < min_p  (the normaliser cancels) ----
   const float min_p = p.min_ps ? p.min_ps[rowi] : 0.0f;
@@ -489,12 +677,36 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   // ---- final: per-thread mass, exclusive scan in thread order, one draw -----------------
   float mine = 0.f;
   tie_seen = 0;
-  row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) {
-    const float w = weight(elem<Tag>::ld(raw));
-    const bool k = ok && kept(make_key<Tag>(raw), w);
-    if (ok && mask_row) mask_row[i] = k;
-    if (k) mine += w;
-  });
+  if constexpr (CHIP) {
+    if (topk_on || topp_on) {
+      const uint32_t floor_key = max(topk_on ? key_k : 0u, topp_on ? key_p : 0u);   // nothing with a smaller key is kept
+      if (topk_on || kept_c <= (unsigned)V / 128)
+        chip.foreach_from(Row::least_of_key(floor_key), [&](int i, T raw) {
+          const float w = weight(elem<Tag>::ld(raw));
+          if (kept(make_key<Tag>(raw), w)) mine += w;
+        });
+      else   // (many are kept: turns over a vector cost more than all of its elements)
+        chip.foreach([&](T raw) {
+          const float w = weight(elem<Tag>::ld(raw));
+          const bool out = make_key<Tag>(raw) < key_p || (minp_on && w < min_p);
+          mine += out ? 0.f : w;
+        });
+    } else if (minp_on) {
+      chip.foreach([&](T raw) {
+        const float w = weight(elem<Tag>::ld(raw));
+        mine += w < min_p ? 0.f : w;
+      });
+    } else {
+      chip.foreach([&](T raw) { mine += weight(elem<Tag>::ld(raw)); });
+    }
+  } else {
+    row_foreach<Tag>(row, V, vec_ok, [&](int i, T raw, bool ok) {
+      const float w = weight(elem<Tag>::ld(raw));
+      const bool k = ok && kept(make_key<Tag>(raw), w);
+      if (ok && mask_row) mask_row[i] = k;
+      if (k) mine += w;
+    });
+  }
   float total;
   const float before = block_exscan_f(mine, total, sh);
   const uint64_t off = p.offset + (p.offset_dev ? *p.offset_dev : 0ull);
@@ -603,7 +815,18 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
       ties_base += __shfl((int)tie_inc, 63, 64);
       if (pick >= 0) break;  // wave-uniform
     }
-    if (pick < 0) pick = last_kept >= 0 ? last_kept : best_i;  // rounding at the very end
+    if (pick < 0) {   // rounding at the very end
+      if constexpr (CHIP) {
+        if (last_kept < 0 && threadIdx.x == who) {   // (nothing was kept: a row with NaN) this thread's largest
+          for (int c = who; c < nvec; c += kThreads)
+            for (int i = c * 8; i < c * 8 + 8; ++i) {
+              const float x = elem<Tag>::ld(row[i]);
+              if (best_i == 0x7fffffff ? x >= -INFINITY : x > best) best = x, best_i = i;
+            }
+        }
+      }
+      pick = last_kept >= 0 ? last_kept : best_i;
+    }
     if (pick < 0 || pick >= V) pick = 0;
     if (threadIdx.x == who) p.out_tokens[rowi] = pick;
   }
@@ -1080,6 +1303,31 @@ extern "C" size_t mv_sample_workspace_bytes(int batch, int vocab) {
   return 256;  // the kernel keeps everything in LDS/registers; reserved for future use
 }
 
+namespace {
+// rows in whole, aligned 16-byte vectors that fit a CU stay there; a mask is written by the general form
+template <typename Tag>
+int launch_sample(const SampleParams &p, int batch, hipStream_t st) {
+  const dim3 grid(batch), block(kThreads);
+  if constexpr (keyinfo<Tag>::BITS == 16) {
+    const int nvec = p.vocab / 8, lds = sizeof(Shared) + std::min(kLdsVectors, (nvec + kThreads - 1) / kThreads) * kThreads * 16;
+    if (!p.keep_mask && p.vocab % 8 == 0 && p.ld % 8 == 0 && mv_aligned16(p.logits)) {
+      if (nvec <= kLdsVectors * kThreads) {
+        if (int rc = mv_allow_lds<sample_kernel<Tag, 0>>()) return rc;
+        hipLaunchKernelGGL((sample_kernel<Tag, 0>), grid, block, lds, st, p);
+        return MV_OK;
+      }
+      if (nvec <= (kLdsVectors + kRegVectors) * kThreads) {
+        if (int rc = mv_allow_lds<sample_kernel<Tag, kRegVectors>>()) return rc;
+        hipLaunchKernelGGL((sample_kernel<Tag, kRegVectors>), grid, block, lds, st, p);
+        return MV_OK;
+      }
+    }
+  }
+  hipLaunchKernelGGL((sample_kernel<Tag, -1>), grid, block, sizeof(Shared), st, p);
+  return MV_OK;
+}
+}  // namespace
+
 extern "C" int mv_sample(const void *logits, int64_t ld, const float *temperatures,
                          const int64_t *top_ks, const float *top_ps, const float *min_ps,
                          uint64_t seed, uint64_t offset, const uint64_t *offset_dev,
@@ -1096,8 +1344,9 @@ extern "C" int mv_sample(const void *logits, int64_t ld, const float *temperatur
   p.logits = logits; p.ld = ld; p.temperatures = temperatures; p.top_ks = top_ks;
   p.top_ps = top_ps; p.min_ps = min_ps; p.seed = seed; p.offset = offset;
   p.offset_dev = offset_dev; p.out_tokens = out_tokens; p.keep_mask = keep_mask; p.vocab = vocab;
-  MV_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((sample_kernel<Tag>), dim3(batch), dim3(kThreads), 0,
-                                              (hipStream_t)stream, p));
+  int rc = MV_OK;
+  MV_DISPATCH_DTYPE(dtype, rc = launch_sample<Tag>(p, batch, (hipStream_t)stream));
+  if (rc) return rc;
   MV_LAUNCH_CHECK();
   return MV_OK;
 }
