@@ -1,7 +1,7 @@
 // K2 — C-ABI entry of the packed varlen causal prefill attention
 // (reference call sites: minivllm/models/layers/attention.py:422-433 flash
-//  varlen, :467-504 fallback).  Dispatches to the MFMA flash kernel for
-// 16-bit tensors and to the vector-ALU kernel otherwise.
+//  varlen, :467-504 fallback).  Dispatches to the MFMA flash kernels of
+// 16-bit and fp32 tensors and to the vector-ALU kernel where they do not apply.
 #include "prefill.h"
 
 extern "C" int mv_prefill_varlen_ex(const void *q, int64_t q_stride_tok, const void *k, const void *v,
@@ -46,8 +46,8 @@ extern "C" int mv_prefill_varlen_ex(const void *q, int64_t q_stride_tok, const v
   p.out_stride = out_stride;
   hipStream_t st = (hipStream_t)stream;
   // MV_PREFILL_SIMPLE routes 16-bit tensors through the vector-ALU kernel (debug aid)
-  if (dtype != MV_F32 && !(flags & MV_PREFILL_SIMPLE)) {
-    const int rc = mv_prefill_mfma_launch(p, dtype, flags >> 4, st);
+  if (!(flags & MV_PREFILL_SIMPLE)) {
+    const int rc = dtype == MV_F32 ? mv_prefill_f32_launch(p, st) : mv_prefill_mfma_launch(p, dtype, flags >> 4, st);
     if (rc != MV_E_SHAPE) return rc;
   }
   return mv_prefill_simple_launch(p, (int64_t)n_seqs * max_seqlen_q, dtype, st);

@@ -1,0 +1,271 @@
+// K2 (fp32) — packed varlen causal prefill attention on the fp32 matrix cores (v_mfma_f32_32x32x2_f32: exact products, fp32 sums).
+//
+// Bound by the matrix cores: a flash tile of 32 keys x 32 queries is 64 of these products at head dim 64 (4096 cycles) beside some 800 of
+// vector arithmetic and 16 KiB of LDS reads.  One workgroup = 64 queries of one head, 32 to a wave, and two waves for the same queries that
+// take the tiles in turn and meet at the end: blocks of rows differ in length, and short chains of tiles even them out (128 queries a workgroup, four
+// waves, each over all tiles: 179 us where this takes 151).  S^T = K Q^T puts a query on a lane (and its partner 32 lanes on), so that the row maximum is one exchange and P, as it lies in the accumulators, is the
+// operand of O^T += V^T P^T: register r of lane half h holds key 8 (r / 4) + 4 h + r % 4, and V is read in that order.  Rows of O^T are
+// dealt so that D / 32 adjacent dims of a key are one read of V and one piece of an output row.
+// The vector kernel (prefill_simple.hip: a wave per query and head, every query reads its keys again) stays for head dim 256.
+// 6131 tokens in 8 prompts, 12 heads of 64: 801 -> 151 us (61 TFLOP/s of visible pairs; 4 x 2048: 89); 16 x 1024, 16 heads of 128: 75 TFLOP/s.
+// Relative error against 64 bits, this / the vector kernel: 50 tokens 1.1e-7 / 0.9e-7, 300 1.3e-7 / 1.3e-7, 1000 1.5e-7 / 1.7e-7, 3000 1.7e-7 / 2.4e-7.
+// Reference: minivllm/models/layers/attention.py:467-504,554-597.
+#include "prefill_row.h"
+
+namespace {
+
+constexpr int BN = 32, WAVES = 4, GROUPS = 2, TURNS = WAVES / GROUPS, BM = GROUPS * 32;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+// first key of its own that a position sees (chunk or window)
+__device__ __forceinline__ int first_key_of(const PrefillParams &p, int pos) {
+  return p.chunk > 0 ? max(pos, 0) / p.chunk * p.chunk : p.mask.window > 0 ? max(0, pos - p.mask.window + 1) : 0;
+}
+
+// GENERAL: paged keys, a window, chunks, capped scores; else whole prompts, keys side by side
+template <int D, bool GENERAL>
+__global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kernel(PrefillParams p) {
+  constexpr int CPR = D / 4, PER = TURNS * BN * CPR / (WAVES * 64), DT = D / 32;   // 16-byte pieces of a row, of a thread; tiles of 32 dims
+  constexpr bool QL = D == 64;   // queries in LDS (at head dim 128 they would halve the workgroups of a CU)
+  typedef __attribute__((ext_vector_type(DT))) float fdt;
+  __shared__ __attribute__((aligned(16))) f32x4 tiles_lds[2][TURNS * BN * CPR];   // K | V
+  __shared__ __attribute__((aligned(16))) int there[TURNS][BN];   // (paged) a key has a page
+  __shared__ __attribute__((aligned(16))) f32x4 qs[QL ? BM * CPR : 1];
+  __shared__ int wild[WAVES];                                     // a wave has put values of V that are not finite
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+  const int group = wave % GROUPS, turn = wave / GROUPS;
+  f32x4 *ks = tiles_lds[0], *vs = tiles_lds[1];
+  const int head = blockIdx.x, seq = blockIdx.y, hkv = head / (p.n_heads / p.n_kv_heads);
+  const int q0 = p.cu_q[seq], sq = p.cu_q[seq + 1] - q0, k0 = p.cu_k[seq], sk = p.cu_k[seq + 1] - k0;
+  const int qb = ((int)gridDim.z - 1 - (int)blockIdx.z) * BM;   // the longest rows first
+  if (qb >= sq) return;
+  const int keep = GENERAL ? p.mask.keep_first : 0;
+  const bool paged = GENERAL && p.block_tables != nullptr;
+  auto first_key = [&](int at) { return GENERAL ? first_key_of(p, at) : 0; };
+  // positions of the workgroup's, the wave's and the lane's queries (queries behind the end repeat the last one)
+  const int shift = sk - sq, last = min(qb + BM, sq) - 1;
+  const int wq = min(qb + group * 32, sq - 1), qi = min(qb + group * 32 + col, sq - 1), pos = qi + shift;
+  const int wave_lo = wq + shift, wave_hi = min(qb + group * 32 + 31, sq - 1) + shift;
+  const int first = first_key(pos);
+  // tiles [0, heads) hold the kept first keys, tiles [from, to) the rest
+  const int end = min(sk, last + shift + 1), to = end > 0 ? (end + BN - 1) / BN : 0;
+  const int from = min(first_key(qb + shift) / BN, to), heads = min((min(keep, sk) + BN - 1) / BN, from);
+  const int tiles = heads + to - from;
+  auto tile_at = [&](int i) { return i < heads ? i : from + i - heads; };
+
+  const float *qp = (const float *)p.q + (int64_t)(q0 + qi) * p.q_stride + (int64_t)head * D + half * (D / 2);
+  f32x4 q[QL ? 1 : CPR / 2];   // dims half * D / 2 .. of the lane's query
+  f32x4 *qt = qs + group * BM / GROUPS * CPR + col * CPR;
+#pragma unroll
+  for (int j = 0; j < CPR / 2; ++j) {
+    const f32x4 w = *(const f32x4 *)(qp + 4 * j);
+    if constexpr (QL) qt[(half * (CPR / 2) + j) ^ (col & 15)] = w;   // (the two waves of a group write the same; a wave reads what it wrote)
+    else q[j] = w;
+  }
+
+  f32x4 kr[PER], vr[PER];
+  int ok[PER];
+  // where piece n of this thread lies in K (V); false: no page
+  auto piece = [&](int i0, int n, const void *rows, const void *cache, int64_t stride, const float *&at) {
+    const int i = tid + n * WAVES * 64, row = i / CPR, c = i % CPR;
+    const int key = min(tile_at(min(i0 + row / BN, tiles - 1)) * BN + row % BN, sk - 1);   // (clamped rows are masked)
+    if (!paged) {
+      at = (const float *)rows + (int64_t)(k0 + key) * stride + (int64_t)hkv * D + 4 * c;
+      return true;
+    }
+    const int bi = key / p.block_size, blk = bi < p.table_width ? p.block_tables[(int64_t)seq * p.table_stride + bi] : -1;
+    const bool is = blk >= 0 && blk < p.num_blocks;
+    at = (const float *)cache + (((is ? (int64_t)blk * p.block_size : 0) + (key - bi * p.block_size)) * p.n_kv_heads + hkv) * D + 4 * c;
+    return is;
+  };
+  auto fetch_k = [&](int i0) {
+#pragma unroll
+    for (int n = 0; n < PER; ++n) {
+      const float *at;
+      ok[n] = piece(i0, n, p.k, p.k_cache, p.k_stride, at);
+      kr[n] = *(const f32x4 *)at;
+      if (paged && !ok[n]) kr[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  auto fetch_v = [&](int i0) {
+#pragma unroll
+    for (int n = 0; n < PER; ++n) {
+      const float *at;
+      const bool is = piece(i0, n, p.v, p.v_cache, p.v_stride, at);
+      vr[n] = *(const f32x4 *)at;
+      if (paged && !is) vr[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  auto put = [&]() {   // K's pieces in an order that spreads the rows over the banks
+#pragma unroll
+    for (int n = 0; n < PER; ++n) {
+      const int i = tid + n * WAVES * 64, row = i / CPR, c = i % CPR;
+      ks[row * CPR + (c ^ (row & 15))] = kr[n], vs[i] = vr[n];
+      if (paged && c == 0) there[row / BN][row % BN] = ok[n];
+    }
+    float z = 0.f;
+#pragma unroll
+    for (int n = 0; n < PER; ++n)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) z = fmaf(vr[n][e], 0.f, z);
+    const int any = __any(z != 0.f) ? 1 : 0;   // (NaN)
+    if (lane == 0) wild[wave] = any;
+  };
+
+  const float scale_log2 = p.scale * 1.4426950408889634f;
+  const float cap = GENERAL ? p.mask.softcap : 0.f, to_cap = cap > 0.f ? p.scale / cap : 0.f, cap_log2 = cap * 1.4426950408889634f;
+  float m = -1e30f, l = 0.f;
+  int apart = 0;   // a tile with masked keys holds values of V that are not finite
+  if (p.mask.sink) m = ((const float *)p.mask.sink)[head] * 1.4426950408889634f, l = half == 0 && turn == 0 ? 1.f : 0.f;
+  f32x16 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+
+  if (tiles > 0) {
+    fetch_k(0);
+    fetch_v(0);
+  }
+  for (int i0 = 0; i0 < tiles; i0 += TURNS) {
+    __syncthreads();   // every wave is done with the tiles before
+    put();
+    __syncthreads();
+    if (i0 + TURNS < tiles) fetch_k(i0 + TURNS);
+    const int tile = tile_at(min(i0 + turn, tiles - 1)), key0 = tile * BN;
+    const f32x4 *kt = ks + turn * BN * CPR, *vt = vs + turn * BN * CPR;
+    // of the wave's queries sees a key of it
+    const bool some = i0 + turn < tiles && key0 <= wave_hi && (key0 + BN > first_key(wave_lo) || key0 < keep);
+    f32x16 s;
+    if (some) {
+      // a score's D products in four chains: one alone has twice the rounding error of the vector kernel's, whose lanes meet in a tree
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        f32x16 chain = {};
+#pragma unroll
+        for (int j = c * CPR / 8; j < (c + 1) * CPR / 8; ++j) {
+          const int at = (half * (CPR / 2) + j) ^ (col & 15);
+          const f32x4 k = kt[col * CPR + at], w = QL ? qt[at] : q[QL ? 0 : j];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) chain = __builtin_amdgcn_mfma_f32_32x32x2f32(k[e], w[e], chain, 0, 0, 0);
+        }
+        if (c == 0) s = chain;
+        else s += chain;
+        __builtin_amdgcn_sched_barrier(0);   // (one chain's registers at a time)
+      }
+    }
+    if (i0 + TURNS < tiles) fetch_v(i0 + TURNS);   // (not before: the registers of a chain are free now)
+    if (some) {
+      if (cap > 0.f) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = capped_log2<f32_tag>(s[r], to_cap, cap_log2);
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] *= scale_log2;
+      }
+      if (paged || key0 + BN - 1 > wave_lo || key0 + BN > sk || key0 < first_key(wave_hi)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int j = 8 * (r >> 2) + 4 * half + (r & 3), key = key0 + j;
+          const bool seen = key <= pos && key < sk && (!GENERAL || key >= first || key < keep) && (!paged || there[turn][j]);
+          s[r] = seen ? s[r] : -INFINITY;
+        }
+        apart |= wild[0] | wild[1] | wild[2] | wild[3];
+      }
+      float mx = s[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));
+      if (__any(mx > m)) {
+        const float alpha = __builtin_amdgcn_exp2f(m - mx);
+        l *= alpha;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+        m = mx;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r] - m);
+      l += (((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))) + (((s[8] + s[9]) + (s[10] + s[11])) + ((s[12] + s[13]) + (s[14] + s[15])));
+      // Head dim 64: a tile's 32 keys in two chains, apart from the sums so far: fewer roundings on a path, as with the scores.  (At 128 the
+      // registers are not there; its rows have fewer roundings behind the scores than ahead of them.)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        f32x16 sums[DT];
+#pragma unroll
+        for (int t = 0; t < DT; ++t) sums[t] = D == 64 ? f32x16{} : o[t];
+#pragma unroll
+        for (int r = 8 * c; r < 8 * c + 8; ++r) {
+          const fdt v = ((const fdt *)vt)[(8 * (r >> 2) + 4 * half + (r & 3)) * 32 + col];
+#pragma unroll
+          for (int t = 0; t < DT; ++t) sums[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[t], s[r], sums[t], 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] = D == 64 ? o[t] + sums[t] : sums[t];
+        if constexpr (D == 64) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  // the second wave of each query group hands its part over
+  __syncthreads();
+  float *part = (float *)tiles_lds + group * 64 * (16 * DT + 2) + lane;
+  if (lane == 0) wild[wave] = apart;
+  if (turn > 0) {
+    part[0] = m, part[64] = l;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part[64 * (2 + 16 * t + r)] = o[t][r];
+  }
+  __syncthreads();
+  if (turn > 0) return;
+  if (wild[group] | wild[group + GROUPS]) {   // 0 x infinity of a masked key is in the sums: these rows again, key by key
+    for (int t = qb + group * 32; t < min(qb + group * 32 + 32, sq); ++t) prefill_row<f32_tag, D>(p, seq, q0 + t, head);
+    return;
+  }
+  {
+    const float m1 = part[0], mx = fmaxf(m, m1), f0 = __builtin_amdgcn_exp2f(m - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
+    l = l * f0 + part[64] * f1;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[t][r] = o[t][r] * f0 + part[64 * (2 + 16 * t + r)] * f1;
+  }
+  l += __shfl_xor(l, 32, 64);
+  // a lane's rows 8 a + 4 half + b of tile t are dims DT (8 a + 4 half + b) + t: 4 DT adjacent ones for each a
+  const bool mine = qb + group * 32 + col < sq;
+  const int64_t token = q0 + qi;
+  float *op = (float *)p.out + token * p.out_stride + (int64_t)head * D;
+  if (mine) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int c = 0; c < DT; ++c) {
+        const int dim = DT * (8 * a + 4 * half) + 4 * c;
+        f32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = o[(4 * c + e) % DT][4 * a + (4 * c + e) / DT];
+          w[e] = l > 0.f ? x / l * attn_factor<f32_tag>(p.mask, token, head * D + dim + e) : 0.f;
+        }
+        *(f32x4 *)(op + dim) = w;
+      }
+  }
+}
+
+}  // namespace
+
+int mv_prefill_f32_launch(const PrefillParams &p, hipStream_t stream) {
+  const dim3 grid(p.n_heads, p.n_seqs, (p.max_seqlen_q + BM - 1) / BM);
+  if (grid.y > 65535 || grid.z > 65535) return MV_E_SHAPE;
+  const bool general = p.block_tables || p.chunk > 0 || p.mask.window > 0 || p.mask.softcap > 0.f;
+  const dim3 block(WAVES * 64);
+  if (p.head_dim == 64 && general) hipLaunchKernelGGL((prefill_f32_kernel<64, true>), grid, block, 0, stream, p);
+  else if (p.head_dim == 64) hipLaunchKernelGGL((prefill_f32_kernel<64, false>), grid, block, 0, stream, p);
+  else if (p.head_dim == 128 && general) hipLaunchKernelGGL((prefill_f32_kernel<128, true>), grid, block, 0, stream, p);
+  else if (p.head_dim == 128) hipLaunchKernelGGL((prefill_f32_kernel<128, false>), grid, block, 0, stream, p);
+  else return MV_E_SHAPE;
+  MV_LAUNCH_CHECK();
+  return MV_OK;
+}

@@ -1,0 +1,109 @@
+"""fp32 prefill attention on the matrix cores (csrc/prefill_f32.hip) against 64 bits and the vector kernel: edges of its tiles of 32 keys and
+64 queries, every mask, pages with holes, values that are not finite."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def H():
+    from minivllm_amd import hip_ops
+
+    return hip_ops
+
+
+def _attend(q, k, v, scale, seen, cap=0.0, sink=None):
+    """q [nq, H, D], k / v [nk, Hkv, D], seen [nq, nk] in fp64."""
+    g = q.shape[1] // k.shape[1]
+    s = torch.einsum("qhd,khd->hqk", q.double(), k.double().repeat_interleave(g, 1)) * scale
+    if cap:
+        s = cap * torch.tanh(s / cap)
+    s = s.masked_fill(~seen, -float("inf"))
+    if sink is not None:
+        s = torch.cat([s, sink.double()[:, None, None].expand(-1, s.shape[1], 1)], -1)
+    p = s.softmax(-1).nan_to_num(0.0)[..., :k.shape[0]]      # (no key at all: zeros)
+    return torch.einsum("hqk,khd->qhd", p, v.double().repeat_interleave(g, 1))
+
+
+def _mask(nq, nk, window=0, keep=0, chunk=0):
+    pos, key = torch.arange(nq)[:, None] + nk - nq, torch.arange(nk)[None, :]
+    first = pos.clamp(min=0) // chunk * chunk if chunk else (pos - window + 1 if window else torch.zeros_like(pos))
+    return (key <= pos) & ((key >= first) | (key < (keep if window else 0)))
+
+
+def _check(H, monkeypatch, spans, heads, kv, d, seed, window=0, keep=0, chunk=0, cap=0.0, sink=False, gate=False, block=0, holes=False):
+    """spans: [(queries, keys)] of the sequences."""
+    g = torch.Generator().manual_seed(seed)
+    rand = lambda *s: torch.randn(*s, generator=g)
+    qs, ks, vs = ([rand(n, h, d) for n in ns] for ns, h in (([a for a, _ in spans], heads), ([b for _, b in spans], kv), ([b for _, b in spans], kv)))
+    sinks, gates = rand(heads) if sink else None, rand(sum(a for a, _ in spans), heads * d) if gate else None
+    cu = lambda ns: torch.tensor([0, *torch.tensor(ns).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    cq, ck, mq, mk = cu([a for a, _ in spans]), cu([b for _, b in spans]), max(a for a, _ in spans), max(b for _, b in spans)
+    mask = H.AttnMask(window, keep, cap, 0.7 if gate else 1.0, None if sinks is None else sinks.to(DEV), None if gates is None else gates.to(DEV))
+    kw, lost = {}, [torch.zeros(b, dtype=torch.bool) for _, b in spans]
+    k, v = torch.cat(ks).to(DEV), torch.cat(vs).to(DEV)
+    if block:
+        pages = [-(-b // block) for _, b in spans]
+        order, width = torch.randperm(sum(pages), generator=g).tolist(), max(pages)
+        kc, vc = (torch.full((sum(pages) + 1, block, kv, d), float("nan"), device=DEV) for _ in range(2))
+        table = torch.full((len(spans), width), -1, dtype=torch.int32)
+        for i, (_, b) in enumerate(spans):
+            for j in range(pages[i]):
+                at, lo = order.pop(), j * block
+                table[i, j] = at
+                kc[at, :min(block, b - lo)], vc[at, :min(block, b - lo)] = ks[i][lo:lo + block].to(DEV), vs[i][lo:lo + block].to(DEV)
+                if holes and j == 1:
+                    table[i, j], lost[i][lo:lo + block] = -1, True
+        kw, k, v = dict(k_cache=kc, v_cache=vc, block_tables=table.to(DEV)), None, None
+    call = lambda: H.prefill_varlen(torch.cat(qs).to(DEV), k, v, cq, ck, mq, mk, d ** -0.5, chunk=chunk, mask=mask, **kw).cpu()
+    got = call()
+    with monkeypatch.context() as m:
+        m.setattr(H, "PREFILL_FLAGS", H.MV_PREFILL_SIMPLE)
+        other = call()
+    want = torch.cat([_attend(a, b, c, d ** -0.5, _mask(a.shape[0], b.shape[0], window, keep, chunk) & ~l, cap, sinks)
+                      for a, b, c, l in zip(qs, ks, vs, lost)])
+    if gate:
+        want = want * 0.7 * torch.sigmoid(gates.double()).unflatten(1, (heads, d))
+    # sums of at most 300 products of 24 bits: a few 1e-6 of outputs of order one
+    torch.testing.assert_close(got.double(), want, rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(got, other, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("lens", [[1], [31, 32, 33], [63, 64, 65, 1], [128, 7, 200], [96, 97]], ids=str)
+def test_whole_prompts_at_the_edges_of_tiles(H, monkeypatch, lens, d):
+    _check(H, monkeypatch, [(n, n) for n in lens], 6, 2, d, sum(lens))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("kw", [dict(window=1), dict(window=40, keep=3), dict(window=33, keep=70), dict(chunk=32), dict(chunk=50), dict(cap=2.0),
+                                dict(sink=True), dict(gate=True), dict(window=64, keep=5, cap=3.0, sink=True, gate=True)], ids=str)
+def test_masks(H, monkeypatch, kw, d):
+    _check(H, monkeypatch, [(150, 150), (20, 20), (65, 65)], 4, 4, d, 3, **kw)
+
+
+@pytest.mark.parametrize("block", [1, 16, 24, 64])
+@pytest.mark.parametrize("kw", [{}, dict(window=30, keep=2), dict(chunk=40), dict(sink=True, holes=True)], ids=str)
+def test_portions_over_pages(H, monkeypatch, block, kw):
+    _check(H, monkeypatch, [(5, 130), (64, 64), (1, 33), (33, 97)], 4, 2, 64, 5, block=block, **kw)
+
+
+def test_more_queries_than_keys(H, monkeypatch):
+    _check(H, monkeypatch, [(70, 40), (3, 3)], 2, 1, 64, 9)      # the first queries see no key: zeros
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("d", [64, 128])
+def test_values_that_are_not_finite_reach_only_those_who_see_them(H, bad, d):
+    n, at = 100, 45
+    q, k, v = (torch.randn(n, 2, d, generator=torch.Generator().manual_seed(i)) for i in range(3))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    want = H.prefill_varlen(q.to(DEV), k.to(DEV), v.to(DEV), cu, cu, n, n, d ** -0.5)
+    v[at, 1, 3] = bad
+    got = H.prefill_varlen(q.to(DEV), k.to(DEV), v.to(DEV), cu, cu, n, n, d ** -0.5)
+    hit = torch.zeros(n, 2, d, dtype=torch.bool, device=DEV)
+    hit[at:, 1, 3] = True
+    assert not torch.isfinite(got[hit]).any()
+    torch.testing.assert_close(got[~hit], want[~hit], rtol=1e-5, atol=1e-5)
