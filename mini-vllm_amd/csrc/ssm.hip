@@ -352,14 +352,20 @@ extern "C" int mv_causal_conv(const MvSsmArgs *a, int dtype, void *stream) {
   return MV_OK;
 }
 
-extern "C" int mv_ssm_prefill(const MvSsmArgs *a, int dtype, int flags, void *stream) {
+extern "C" size_t mv_ssm_prefill_workspace_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int dtype) {
+  if (n_seqs <= 0 || total_q <= 0 || max_q <= 0 || heads <= 0 || p <= 0 || (p & 15) || n <= 0 || dtype == MV_F32) return 0;
+  return mv_ssm_chunk_workspace(n_seqs, total_q, max_q, heads, p, n);
+}
+
+extern "C" int mv_ssm_prefill_ws(const MvSsmArgs *a, void *workspace, size_t ws_bytes, int total_q, int dtype, int flags, void *stream) {
   if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
   if (int e = check_ssm(a, dtype)) return e;
   if (!a->dt || !a->dt_bias || !a->a_log || !a->d || !a->cu_q || !a->cu_k || (a->slots > 0 && !a->ssm_state)) return MV_E_NULLPTR;
   if (a->max_q < 0 || a->dt_stride < a->heads || a->out_stride < a->heads * a->p) return MV_E_SHAPE;
   if (a->ssm_state && !mv_aligned16(a->ssm_state)) return MV_E_ALIGN;
+  if (workspace && !mv_aligned16(workspace)) return MV_E_ALIGN;
   if (dtype != MV_F32 && !(flags & MV_SSM_SCAN)) {
-    const int rc = mv_ssm_chunk_launch(*a, dtype, (hipStream_t)stream);
+    const int rc = mv_ssm_chunk_launch(*a, workspace, ws_bytes, total_q, dtype, (hipStream_t)stream);
     if (rc != MV_E_SHAPE) return rc;
   }
   const size_t lds = (size_t)(2 * kScanRows * a->n + kScanRows * 16 + 2 * kScanRows) * 4;
@@ -367,6 +373,10 @@ extern "C" int mv_ssm_prefill(const MvSsmArgs *a, int dtype, int flags, void *st
   MV_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((ssm_scan_kernel<Tag>), grid, dim3(256), lds, (hipStream_t)stream, *a));
   MV_LAUNCH_CHECK();
   return MV_OK;
+}
+
+extern "C" int mv_ssm_prefill(const MvSsmArgs *a, int dtype, int flags, void *stream) {
+  return mv_ssm_prefill_ws(a, nullptr, 0, 0, dtype, flags, stream);
 }
 
 extern "C" int mv_ssm_step(const MvSsmArgs *a, int dtype, void *stream) {

@@ -14,6 +14,14 @@
 // one operand with k permuted (k = 8 g + e means key 16 (e >> 2) + 4 g + (e & 3)), and x is read in that order.  So S stays in
 // registers, and the scores go through LDS once (each wave computes some of the 4 token tiles, all waves read all).  The next
 // chunk's rows are requested before the current chunk's products.
+//
+// A chunk is some 550 vector instructions and 86 products of a wave between three barriers, one behind the other: 3.8 us where a workgroup has a CU
+// to itself, half of it in throughput.  Few long sequences are therefore cut into segments of whole chunks (pick_segment): a first launch
+// carries the state through every segment but the last from zeros (the recurrence is linear: b, x and step sizes only), the second starts a
+// segment from S = the sum of those before it, each decayed by the segments between.  64 heads of 64 x 128 with the convolution and the
+// norm: 4 sequences of up to 3900 tokens 315 -> 271 us (the recurrence 232 -> 139 + 69 under the profiler), 1 x 1900 127 -> 71; 32 heads, 1 x 3900 229 -> 83.
+#include <algorithm>
+
 #include "ssm.h"
 
 namespace {
@@ -45,25 +53,49 @@ __device__ __forceinline__ u32x2 read_tr(const char *p) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p));
 }
 
+// segments of `len` tokens: their states [slot][heads][n * p], what they decay by [slot][heads] (log2), the states that sequences of
+// several segments come with [sequence][heads][n * p]; a sequence's slots start at cu_q / len + its number
+struct Segments {
+  float *states, *decays, *first;
+  int len;
+};
+enum { WHOLE, STATES, SEGMENTS };   // workgroups are sequences, or segments; STATES: only the state a segment adds
+
 // NK: state rows / 32
-template <typename Tag, int NK, int PT>
-__global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvSsmArgs p) {
+template <typename Tag, int NK, int PT, int MODE>
+__global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvSsmArgs p, Segments sg) {
   typedef typename elem<Tag>::T T;
   constexpr int N = NK * 32, THREADS = PT * 64;
   // LDS rows: x an odd number of 16-byte pieces; b and c 2 (mod 4), so that the row reads stay apart over 8 rows and the
   // transposed reads, whose pieces lie 16 bytes apart, meet at most in pairs
   constexpr int RB = (N / 8 + 2) * 16, RX = (2 * PT + 1) * 16;
-  constexpr int CB = L * N / 8, CX = L * 2 * PT, PIECES = 2 * CB + CX;   // 16-byte pieces of b, c and x
+  constexpr bool OUT = MODE != STATES;
+  constexpr int CB = L * N / 8, CX = L * 2 * PT, BC = OUT ? 2 * CB : CB, PIECES = BC + CX;   // 16-byte pieces of b, c and x
   constexpr int PER = (PIECES + THREADS - 1) / THREADS, AHEAD = PER <= 20 ? PER : 20;
-  __shared__ __attribute__((aligned(16))) char bs[L * RB], cs[L * RB], xs[L * RX];
-  __shared__ u32x4 wf[2][4][2][64];            // weighted scores, high / remainder: [token tile][32 keys][lane]
+  __shared__ __attribute__((aligned(16))) char bs[L * RB], cs[OUT ? L * RB : 16], xs[L * RX];
+  __shared__ u32x4 wf[2][OUT ? 4 : 1][2][64];  // weighted scores, high / remainder: [token tile][32 keys][lane]
   __shared__ float steps[2][3][L];             // of this and the next chunk: r_i (log2), dt_i, exp(r_last - r_i) dt_i
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
-  const int slice = blockIdx.x, head = blockIdx.y, seq = blockIdx.z;
-  const int q0 = p.cu_q[seq], len = p.cu_q[seq + 1] - q0;
+  const int slice = blockIdx.x, head = blockIdx.y;
+  int seq = blockIdx.z, from = 0, q0 = p.cu_q[MODE == WHOLE ? seq : 0], len = 0, all = 0;
+  if constexpr (MODE == WHOLE) {
+    all = len = p.cu_q[seq + 1] - q0;
+  } else {
+    seq = 0;
+    for (int hi = p.n_seqs; hi - seq > 1;) {   // the sequence that the slot belongs to
+      const int mid = (seq + hi) >> 1;
+      if (p.cu_q[mid] / sg.len + mid <= (int)blockIdx.z) seq = mid;
+      else hi = mid;
+    }
+    q0 = p.cu_q[seq], all = p.cu_q[seq + 1] - q0;
+    from = ((int)blockIdx.z - q0 / sg.len - seq) * sg.len;
+    len = min(sg.len, all - from);
+    if (from < 0 || (MODE == STATES && from + sg.len >= all)) return;   // (nobody asks for the last one's)
+  }
   if (len <= 0) return;
-  const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq], grp = head / (p.heads / p.groups);
-  const bool keep = slot >= 0 && slot < p.slots;
+  const int before = p.cu_k[seq + 1] - p.cu_k[seq] - all, slot = p.state_slots[seq], grp = head / (p.heads / p.groups);
+  const bool keep = slot >= 0 && slot < p.slots, split = all > len;
+  q0 += from;
   const int64_t size = (int64_t)p.heads * p.n * p.p;
   const int64_t at = (int64_t)(keep ? slot : 0) * size + (int64_t)head * p.n * p.p + slice * 16 * PT + wave * 16 + r16;
   const T *x = (const T *)p.x + (int64_t)q0 * p.x_stride, *dt = (const T *)p.dt + (int64_t)q0 * p.dt_stride + head;
@@ -73,16 +105,36 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
 
   auto state_row = [&](int i, int e) { return (i >> 1) * 32 + g * 8 + (i & 1) * 4 + e; };
   f32x4 st[2 * NK];
+  // where this lane's elements lie in a state [n][p] of this head, and this segment's slot
+  const int64_t mine = (int64_t)slice * 16 * PT + wave * 16 + r16, hsize = (int64_t)p.n * p.p;
+  const int64_t here = MODE == WHOLE ? 0 : (int64_t)blockIdx.z * p.heads + head, own = (int64_t)seq * p.heads + head;
 #pragma unroll
   for (int i = 0; i < 2 * NK; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      st[i][e] = keep && before > 0 ? p.ssm_state[(before & 1) * p.slots * size + at + (int64_t)state_row(i, e) * p.p] : 0.f;
+    for (int e = 0; e < 4; ++e) {
+      const int64_t row = (int64_t)state_row(i, e) * p.p;
+      float v = 0.f;
+      // (the pool's state of a split sequence is read by the first launch alone: the second may write it)
+      if (from == 0 && keep && before > 0)
+        v = MODE == SEGMENTS && split ? sg.first[own * hsize + mine + row] : p.ssm_state[(before & 1) * p.slots * size + at + row];
+      if (MODE == STATES && from == 0 && before > 0) sg.first[own * hsize + mine + row] = v;
+      st[i][e] = v;
+    }
+  if constexpr (MODE == SEGMENTS) {
+    for (int64_t z = here - (int64_t)(from / sg.len) * p.heads; z < here; z += p.heads) {
+      const float decay = __builtin_amdgcn_exp2f(sg.decays[z]);
+#pragma unroll
+      for (int i = 0; i < 2 * NK; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) st[i][e] = fmaf(st[i][e], decay, sg.states[z * hsize + mine + (int64_t)state_row(i, e) * p.p]);
+    }
+  }
+  float decayed = 0.f;   // (STATES) log2 decay of the chunks so far
 
   // piece i of a chunk: its row, where it comes from (of row 0), where it goes
   auto piece = [&](int i, int &row, int &col) {
-    const bool isx = i >= 2 * CB;
-    const int j = isx ? i - 2 * CB : (i >= CB ? i - CB : i), c = isx ? j % (2 * PT) : j % (N / 8);
+    const bool isx = i >= BC;
+    const int j = isx ? i - BC : (i >= CB ? i - CB : i), c = isx ? j % (2 * PT) : j % (N / 8);
     row = isx ? j / (2 * PT) : j / (N / 8);
     col = (isx ? xcol : (i >= CB ? ccol : bcol)) + c * 8;
     return (isx ? xs + row * RX : (i >= CB ? cs : bs) + row * RB) + c * 16;
@@ -140,60 +192,63 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
     __syncthreads();
     if (t0 + L < len) request(t0 + L);
 
-    // ---- S^T c of all tokens (this wave's columns), scaled by exp(r_i)
     f32x4 y[4] = {};
+    if constexpr (OUT) {
+      // ---- S^T c of all tokens (this wave's columns), scaled by exp(r_i)
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      u32x2 h0, l0, h1, l1;
-      split4<Tag>(st[2 * s], h0, l0);
-      split4<Tag>(st[2 * s + 1], h1, l1);
-      const u32x4 hi = join(h0, h1), lo = join(l0, l1);
-      u32x4 c[4];
+      for (int s = 0; s < NK; ++s) {
+        u32x2 h0, l0, h1, l1;
+        split4<Tag>(st[2 * s], h0, l0);
+        split4<Tag>(st[2 * s + 1], h1, l1);
+        const u32x4 hi = join(h0, h1), lo = join(l0, l1);
+        u32x4 c[4];
 #pragma unroll
-      for (int it = 0; it < 4; ++it) c[it] = *(const u32x4 *)(cs + (it * 16 + r16) * RB + s * 64 + g * 16);
-      // (products of one accumulator never back to back: the second would wait for the first's whole latency)
+        for (int it = 0; it < 4; ++it) c[it] = *(const u32x4 *)(cs + (it * 16 + r16) * RB + s * 64 + g * 16);
+        // (products of one accumulator never back to back: the second would wait for the first's whole latency)
 #pragma unroll
-      for (int it = 0; it < 4; ++it) y[it] = mfma16x16x32<Tag>(hi, c[it], y[it]);
+        for (int it = 0; it < 4; ++it) y[it] = mfma16x16x32<Tag>(hi, c[it], y[it]);
 #pragma unroll
-      for (int it = 0; it < 4; ++it) y[it] = mfma16x16x32<Tag>(lo, c[it], y[it]);
-    }
-    float ri[4];
+        for (int it = 0; it < 4; ++it) y[it] = mfma16x16x32<Tag>(lo, c[it], y[it]);
+      }
+      float ri[4];
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      ri[it] = rs[it * 16 + r16];
-      y[it] *= __builtin_amdgcn_exp2f(ri[it]);
-    }
-    // ---- weighted scores of this wave's token tiles, [key][token]
-    for (int it = wave; it < 4; it += PT) {
-      u32x4 cf[NK];
+      for (int it = 0; it < 4; ++it) {
+        ri[it] = rs[it * 16 + r16];
+        y[it] *= __builtin_amdgcn_exp2f(ri[it]);
+      }
+      // ---- weighted scores of this wave's token tiles, [key][token]
+      for (int it = wave; it < 4; it += PT) {
+        u32x4 cf[NK];
 #pragma unroll
-      for (int s = 0; s < NK; ++s) cf[s] = *(const u32x4 *)(cs + (it * 16 + r16) * RB + s * 64 + g * 16);
-      const float r_tok = rs[it * 16 + r16];
-      f32x4 sc[4] = {};
+        for (int s = 0; s < NK; ++s) cf[s] = *(const u32x4 *)(cs + (it * 16 + r16) * RB + s * 64 + g * 16);
+        const float r_tok = rs[it * 16 + r16];
+        f32x4 sc[4] = {};
 #pragma unroll
-      for (int s = 0; s < NK; ++s)
+        for (int s = 0; s < NK; ++s)
 #pragma unroll
-        for (int jt = 0; jt < 4; ++jt)
-          if (jt <= it) sc[jt] = mfma16x16x32<Tag>(*(const u32x4 *)(bs + (jt * 16 + r16) * RB + s * 64 + g * 16), cf[s], sc[jt]);
+          for (int jt = 0; jt < 4; ++jt)
+            if (jt <= it) sc[jt] = mfma16x16x32<Tag>(*(const u32x4 *)(bs + (jt * 16 + r16) * RB + s * 64 + g * 16), cf[s], sc[jt]);
 #pragma unroll
-      for (int jt = 0; jt < 4; ++jt) {
-        u32x2 hi = {0u, 0u}, lo = {0u, 0u};
-        if (jt <= it) {
-          f32x4 a = sc[jt];
-          const f32x4 rk = *(const f32x4 *)(rs + jt * 16 + g * 4), dk = *(const f32x4 *)(dts + jt * 16 + g * 4);
+        for (int jt = 0; jt < 4; ++jt) {
+          u32x2 hi = {0u, 0u}, lo = {0u, 0u};
+          if (jt <= it) {
+            f32x4 a = sc[jt];
+            const f32x4 rk = *(const f32x4 *)(rs + jt * 16 + g * 4), dk = *(const f32x4 *)(dts + jt * 16 + g * 4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const bool seen = jt * 16 + g * 4 + e <= it * 16 + r16;
-            a[e] = seen ? a[e] * (__builtin_amdgcn_exp2f(seen ? r_tok - rk[e] : 0.f) * dk[e]) : 0.f;
+            for (int e = 0; e < 4; ++e) {
+              const bool seen = jt * 16 + g * 4 + e <= it * 16 + r16;
+              a[e] = seen ? a[e] * (__builtin_amdgcn_exp2f(seen ? r_tok - rk[e] : 0.f) * dk[e]) : 0.f;
+            }
+            split4<Tag>(a, hi, lo);
           }
-          split4<Tag>(a, hi, lo);
+          *((u32x2 *)&wf[0][it][jt >> 1][lane] + (jt & 1)) = hi;
+          *((u32x2 *)&wf[1][it][jt >> 1][lane] + (jt & 1)) = lo;
         }
-        *((u32x2 *)&wf[0][it][jt >> 1][lane] + (jt & 1)) = hi;
-        *((u32x2 *)&wf[1][it][jt >> 1][lane] + (jt & 1)) = lo;
       }
     }
     if (wave == 0 && t0 + L < len) scan(min(L, len - t0 - L), steps[cur ^ 1]);   // (wave 0 scored the fewest keys)
-    __syncthreads();
+    if constexpr (OUT) __syncthreads();
+    else decayed += rs[L - 1];
     // ---- sum over the chunk's keys; then the state moves on
     const float tail = __builtin_amdgcn_exp2f(rs[L - 1]);
 #pragma unroll
@@ -203,10 +258,12 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
       const char *xa = xs + (32 * s + 4 * g + (r16 >> 2)) * RX + wave * 32 + (r16 & 3) * 8;
       const u32x2 x0 = read_tr(xa), x1 = read_tr(xa + 16 * RX);
       const u32x4 xf = join(x0, x1);
+      if constexpr (OUT) {
 #pragma unroll
-      for (int part = 0; part < 2; ++part)
+        for (int part = 0; part < 2; ++part)
 #pragma unroll
-        for (int it = 2 * s; it < 4; ++it) y[it] = mfma16x16x32<Tag>(xf, wf[part][it][s][lane], y[it]);   // keys 32 s ..
+          for (int it = 2 * s; it < 4; ++it) y[it] = mfma16x16x32<Tag>(xf, wf[part][it][s][lane], y[it]);   // keys 32 s ..
+      }
       float f[8];
       unpack8<Tag>(xf, f);
       const f32x4 w0 = *(const f32x4 *)(ws + 32 * s + 4 * g), w1 = *(const f32x4 *)(ws + 32 * s + 16 + 4 * g);
@@ -232,7 +289,7 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
     }
     // ---- out: lane (token r16, columns 4 g ..)
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
+    for (int it = 0; it < (OUT ? 4 : 0); ++it) {
       const int t = it * 16 + r16;
       const u32x2 raw = *(const u32x2 *)(xs + t * RX + wave * 32 + g * 8);
       float o[4];
@@ -247,8 +304,14 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
     }
     __syncthreads();
   }
-  if (keep) {
-    float *ns = p.ssm_state + ((before + len) & 1) * p.slots * size + at;
+  if constexpr (MODE == STATES) {
+#pragma unroll
+    for (int i = 0; i < 2 * NK; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sg.states[here * hsize + mine + (int64_t)state_row(i, e) * p.p] = st[i][e];
+    if (slice == 0 && tid == 0) sg.decays[here] = decayed;
+  } else if (keep && from + len >= all) {
+    float *ns = p.ssm_state + ((before + all) & 1) * p.slots * size + at;
 #pragma unroll
     for (int i = 0; i < 2 * NK; ++i)
 #pragma unroll
@@ -256,27 +319,69 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
   }
 }
 
-template <typename Tag, int NK>
-int launch(const MvSsmArgs &a, hipStream_t stream) {
-  // column tiles per workgroup: as many as divide the head's.  They share the b / c rows and the scores; fewer per workgroup
-  // measured slower even where they fill an otherwise idle chip (a lone wave loads and scores everything by itself)
-  const int tiles = a.p / 16, pt = tiles % 4 == 0 ? 4 : tiles % 3 == 0 ? 3 : tiles % 2 == 0 ? 2 : 1;
-  const dim3 grid(tiles / pt, a.heads, a.n_seqs);
-#define MV_SC(PT_) hipLaunchKernelGGL((ssm_chunk_kernel<Tag, NK, PT_>), grid, dim3(PT_ * 64), 0, stream, a)
-  if (pt == 4) MV_SC(4);
-  else if (pt == 3) MV_SC(3);
-  else if (pt == 2) MV_SC(2);
-  else MV_SC(1);
-#undef MV_SC
+// column tiles per workgroup: as many as divide the head's.  They share the b / c rows and the scores; fewer per workgroup
+// measured slower even where they fill an otherwise idle chip (a lone wave loads and scores everything by itself)
+inline int column_tiles(int p) {
+  const int tiles = p / 16;
+  return tiles % 4 == 0 ? 4 : tiles % 3 == 0 ? 3 : tiles % 2 == 0 ? 2 : 1;
+}
+// chunks of a segment; 0: whole sequences.  Two workgroups fit a CU, so sequences that make 512 are left whole (8 x 1900 tokens, 64 heads: 262 us, in
+// segments 332); about four a CU even out; a segment is at least four chunks (its start is a load of the states before it) and a sequence at
+// most eight segments.
+inline int pick_segment(int n_seqs, int total_q, int max_q, int heads, int p) {
+  const int64_t per_chunk = (int64_t)heads * (p / 16 / column_tiles(p)), longest = (max_q + L - 1) / L;
+  if (per_chunk * n_seqs >= 512) return 0;
+  const int64_t chunks = (total_q + L - 1) / L, seg = std::max<int64_t>({4, (longest + 7) / 8, (chunks * per_chunk + 1023) / 1024});
+  return longest * 3 > seg * 4 ? (int)seg : 0;
+}
+
+template <typename Tag, int NK, int PT>
+int launch_tiles(const MvSsmArgs &a, int seg, void *workspace, int total_q, hipStream_t stream) {
+  const int slices = a.p / 16 / PT;
+  Segments sg{};
+  if (!seg) {
+    hipLaunchKernelGGL((ssm_chunk_kernel<Tag, NK, PT, WHOLE>), dim3(slices, a.heads, a.n_seqs), dim3(PT * 64), 0, stream, a, sg);
+    MV_LAUNCH_CHECK();
+    return MV_OK;
+  }
+  sg.len = seg * L;
+  const int64_t slots = total_q / sg.len + a.n_seqs, state = (int64_t)a.heads * a.n * a.p;
+  sg.states = (float *)workspace, sg.first = sg.states + slots * state, sg.decays = sg.first + a.n_seqs * state;
+  const dim3 grid(slices, a.heads, (unsigned)slots);
+  hipLaunchKernelGGL((ssm_chunk_kernel<Tag, NK, PT, STATES>), grid, dim3(PT * 64), 0, stream, a, sg);
+  MV_LAUNCH_CHECK();
+  hipLaunchKernelGGL((ssm_chunk_kernel<Tag, NK, PT, SEGMENTS>), grid, dim3(PT * 64), 0, stream, a, sg);
   MV_LAUNCH_CHECK();
   return MV_OK;
 }
 
+template <typename Tag, int NK>
+int launch(const MvSsmArgs &a, int seg, void *workspace, int total_q, hipStream_t stream) {
+  switch (column_tiles(a.p)) {
+    case 4: return launch_tiles<Tag, NK, 4>(a, seg, workspace, total_q, stream);
+    case 3: return launch_tiles<Tag, NK, 3>(a, seg, workspace, total_q, stream);
+    case 2: return launch_tiles<Tag, NK, 2>(a, seg, workspace, total_q, stream);
+  }
+  return launch_tiles<Tag, NK, 1>(a, seg, workspace, total_q, stream);
+}
+
 }  // namespace
 
-int mv_ssm_chunk_launch(const MvSsmArgs &a, int dtype, hipStream_t stream) {
+// states and decays of the segments, and the states that sequences come with
+size_t mv_ssm_chunk_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
+  const int seg = pick_segment(n_seqs, total_q, max_q, heads, p);
+  if (!seg) return 0;
+  const int64_t slots = total_q / (seg * L) + n_seqs;
+  if (slots > 65535) return 0;
+  return ((slots + n_seqs) * heads * n * p + slots * heads) * sizeof(float);
+}
+
+int mv_ssm_chunk_launch(const MvSsmArgs &a, void *workspace, size_t ws_bytes, int total_q, int dtype, hipStream_t stream) {
+  const size_t need = workspace ? mv_ssm_chunk_workspace(a.n_seqs, total_q, a.max_q, a.heads, a.p, a.n) : 0;
+  const int seg = need && ws_bytes >= need ? pick_segment(a.n_seqs, total_q, a.max_q, a.heads, a.p) : 0;
 #define MV_SN(N_) \
-  if (a.n == N_) return dtype == MV_BF16 ? launch<bf16_tag, N_ / 32>(a, stream) : launch<f16_tag, N_ / 32>(a, stream)
+  if (a.n == N_) return dtype == MV_BF16 ? launch<bf16_tag, N_ / 32>(a, seg, workspace, total_q, stream) \
+                                         : launch<f16_tag, N_ / 32>(a, seg, workspace, total_q, stream)
   MV_SN(32);
   MV_SN(64);
   MV_SN(96);

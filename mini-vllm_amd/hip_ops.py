@@ -87,6 +87,8 @@ _SIGNATURES = {
     "mv_latent_prefill": (c_int, [c_void_p, c_int, c_int, c_void_p]),
     "mv_causal_conv": (c_int, [c_void_p, c_int, c_void_p]),
     "mv_ssm_prefill": (c_int, [c_void_p, c_int, c_int, c_void_p]),
+    "mv_ssm_prefill_workspace_bytes": (c_size_t, [c_int] * 7),
+    "mv_ssm_prefill_ws": (c_int, [c_void_p, c_void_p, c_size_t, c_int, c_int, c_int, c_void_p]),
     "mv_ssm_step": (c_int, [c_void_p, c_int, c_void_p]),
     "mv_gated_group_norm": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int,
                                     c_int, c_float, c_int, c_void_p]),
@@ -1420,7 +1422,10 @@ def ssm_prefill(x, dt, dt_bias, a_log, d, shape, ssm_state, state_slots, cu_q, c
         out = torch.empty((x.shape[0], shape[0] * shape[2]), dtype=x.dtype, device=x.device)
     a = _ssm_args(shape, x, state_slots, out, ssm_state=ssm_state, dt=dt, dt_bias=dt_bias, a_log=a_log, d=d)
     a.cu_q, a.cu_k, a.max_q = cu_q.data_ptr(), cu_k.data_ptr(), int(max_q)
-    _check(_lib.mv_ssm_prefill(ctypes.byref(a), _dt(x), int(flags), _stream()), "mv_ssm_prefill")
+    rows = x.shape[0]
+    n = 0 if flags & MV_SSM_SCAN else int(_lib.mv_ssm_prefill_workspace_bytes(a.n_seqs, rows, a.max_q, a.heads, a.p, a.n, _dt(x)))
+    ws = torch.empty((n,), dtype=torch.uint8, device=x.device) if n else None
+    _check(_lib.mv_ssm_prefill_ws(ctypes.byref(a), _ptr(ws), n, rows, _dt(x), int(flags), _stream()), "mv_ssm_prefill")
     return out
 
 
