@@ -118,18 +118,29 @@ __device__ __forceinline__ float row16_max(float x) {
   x = fmaxf(x, row_ror<1>(x));
   return x;
 }
+// Exchanges between the rows of 16 lanes on the vector unit (a ds_bpermute is a trip to the LDS pipe of some hundred cycles): lane i gets x of lane i
+// and of lane i ^ 16 (^ 32), in an order that depends on the row.  As inline assembly: hipcc (ROCm 7.2) has taken the two results of the builtin on
+// one value for one result; s_nop 1: the wait between a vector instruction and v_permlane* on its result.
+__device__ __forceinline__ void swap16(float x, float &a, float &b) {
+  a = x, b = x;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ void swap32(float x, float &a, float &b) {
+  a = x, b = x;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
 // Full 64-lane reductions (every lane gets the result).
 __device__ __forceinline__ float wave_sum(float x) {
-  x = row16_sum(x);
-  x += __shfl_xor(x, 16, 64);
-  x += __shfl_xor(x, 32, 64);
-  return x;
+  float a, b;
+  swap16(row16_sum(x), a, b);
+  swap32(a + b, a, b);
+  return a + b;
 }
 __device__ __forceinline__ float wave_max(float x) {
-  x = row16_max(x);
-  x = fmaxf(x, __shfl_xor(x, 16, 64));
-  x = fmaxf(x, __shfl_xor(x, 32, 64));
-  return x;
+  float a, b;
+  swap16(row16_max(x), a, b);
+  swap32(fmaxf(a, b), a, b);
+  return fmaxf(a, b);
 }
 
 // tanh form of gelu: 0.5 z (1 + tanh(u)) = z / (1 + exp(-2 u)), u = sqrt(2/pi) (z + 0.044715 z^3)
