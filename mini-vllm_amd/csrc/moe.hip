@@ -446,93 +446,144 @@ __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
   }
 }
 
-// very many rows: 256 x 256 per workgroup of 2 x 4 waves, so that a row operand read from LDS serves four products and a weight operand
-// eight.  Two stages of 64 inputs; a stage is handed back half way through its products, when all of it is in registers.
+// Very many rows: 128 x 256 per workgroup of four waves side by side, two workgroups to a CU, so that one multiplies while the other starts or ends.
+// Bound by the matrix cores, if their operands are there in time: three stages of 32 inputs, of which two are under way, and the operands of a stage
+// are read one by one between the products of the stage before.  Results leave through LDS, 128 bytes of a row (gated: 64) to a store.
+// Workgroups are dealt to the XCDs in turn, and each XCD gets a run of an eighth of the work (eight tiles of rows and all their outputs at a time, the
+// rows first): its L2 holds what its workgroups share, and none has more than the others.
+// 36004 pairs of 32 experts, 2048 -> 2 x 768 gated and 768 -> 2048: 343 + 198 us (one workgroup of 256 x 256 to a CU, two stages of 64 inputs, four
+// tiles to an XCD in turn) -> 260 + 157.
+constexpr int kWideRows = 128, kWideStages = 3;
+template <typename Tag, bool GATED, int ACT>
+__device__ __forceinline__ float wide_result(float x, float up, MvGateAct act) {
+  if constexpr (!GATED) return x;
+  act.kind = ACT;   // (known at compile time: one branch per workgroup, not per output)
+  return gated_act<Tag>(x, up, act);
+}
+
 template <typename Tag, bool GATED>
-__global__ void __launch_bounds__(512, 1) moe_wide_kernel(MoeLinear p, int nx, int max_tiles) {
+__global__ void __launch_bounds__(256, 2) moe_wide_kernel(MoeLinear p, int nx, int max_tiles) {
   typedef typename elem<Tag>::T T;
-  constexpr int TILES = 16, WM = 8, WN = 4, PER = 4, STAGE = 4 * TILES * 1024;
-  extern __shared__ __attribute__((aligned(16))) char smem[];   // 2 stages of [rows: TILES][2] | [weights: TILES][2] fragments
-  // Workgroups are dealt to the XCDs in turn: four row tiles and all their outputs stay on one of them, the row tiles first.
-  const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3, group = turn / (4 * nx) * 8 + xcd, in = turn % (4 * nx);
-  const int ty = group * 4 + (in & 3), tx = in >> 2;
-  if (ty >= max_tiles) return;
-  const int32_t *tile = p.tiles + 3 * ty;
-  const int e = tile[0], m0 = tile[1], live = tile[2];
-  if (e < 0) return;
+  constexpr int TILES = 16, WM = 8, WN = 4, STAGE = (WM + TILES) * 1024, PER = 6;
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // stages of rows [WM] | weights [TILES] fragments
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  const int wm = wave & 1, wn = wave >> 1, ntiles = p.n / 16, steps = p.k / 32, nt0 = tx * (GATED ? TILES / 2 : TILES);
-  // this wave's fragments: one half of the 64 inputs of every fourth tile, of the rows and of the weights
-  const int half = wave & 1, first = wave >> 1;
-  const T *xs[PER], *ws[PER];
+  // the halves of a tile of 256 rows that are there
+  const unsigned long long below = (1ull << lane) - 1;
+  unsigned long long upper, lower;
+  auto halves = [&](int i0) {
+    const int i = min(i0 + lane, max_tiles - 1);
+    const bool there = i0 + lane < max_tiles && p.tiles[3 * i] >= 0;
+    upper = __ballot(there), lower = __ballot(there && p.tiles[3 * i + 2] > kWideRows);
+    return __popcll(upper) + __popcll(lower);
+  };
+  int total = 0;
+  for (int i0 = 0; i0 < max_tiles; i0 += 64) total += halves(i0);
+  const int per = (total * nx + 7) / 8, turn = blockIdx.x >> 3, index = (blockIdx.x & 7) * per + turn;
+  if (turn >= per || index >= total * nx) return;
+  const int group = index / (8 * nx), in = index - group * 8 * nx, high = min(8, total - group * 8), tx = in / high;
+  int nth = group * 8 + in % high, i0 = 0;
+  for (int n = halves(0); nth >= n; n = halves(i0)) nth -= n, i0 += 64;
+  const int ahead = __popcll(upper & below) + __popcll(lower & below);
+  const bool second = (lower >> lane & 1) && nth == ahead + 1;
+  const unsigned long long mine = __ballot((upper >> lane & 1) && (nth == ahead || second));
+  const int32_t *tile = p.tiles + 3 * (i0 + __ffsll(mine) - 1);
+  const int skip = __ballot(second) ? kWideRows : 0, e = tile[0], m0 = tile[1] + skip, live = tile[2] - skip;
+  const int ntiles = p.n / 16, steps = p.k / 32, nt0 = tx * (GATED ? TILES / 2 : TILES);
+  // this wave's fragments of a stage: two of the rows, four of the weights
+  const T *xs[2], *ws[4];
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int j = 4 * i + first, place = m0 + min(j * 16 + (lane >> 2), live - 1);
-    xs[i] = (const T *)p.x + (int64_t)(p.tokens ? p.tokens[place] : place) * p.x_stride + half * 32 + row_chunk(lane) * 8;
-    const int wt = min(nt0 + (GATED ? j >> 1 : j), ntiles - 1) + (GATED && (j & 1) ? ntiles : 0);
-    ws[i] = (const T *)p.w + e * p.w_expert + ((int64_t)wt * steps + half) * 512;
+  for (int i = 0; i < 4; ++i) {
+    const int j = 4 * i + wave, wt = min(nt0 + (GATED ? j >> 1 : j), ntiles - 1) + (GATED && (j & 1) ? ntiles : 0);
+    ws[i] = (const T *)p.w + e * p.w_expert + (int64_t)wt * steps * 512;
+    if (i < 2) {
+      const int place = m0 + min(j * 16 + (lane >> 2), live - 1);
+      xs[i] = (const T *)p.x + (int64_t)(p.tokens ? p.tokens[place] : place) * p.x_stride + row_chunk(lane) * 8;
+    }
   }
   const int lane8 = lane * 8;
-  auto fetch = [&](int t) {
-    char *to = smem + (t & 1) * STAGE + (first * 2 + half) * 1024;
-    const int64_t kx = (int64_t)t * 64, kw = (int64_t)t * 1024;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(xs[i] + kx),
-                                       (__attribute__((address_space(3))) void *)(to + i * 8192), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(ws[i] + kw + lane8),
-                                       (__attribute__((address_space(3))) void *)(to + (TILES * 2048) + i * 8192), 16, 0, 0);
-    }
+  auto transfer = [&](const T *from, char *to) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from, (__attribute__((address_space(3))) void *)to, 16, 0, 0);
   };
+  auto fetch = [&](int t, int slot) {
+    char *to = smem + slot * STAGE + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) transfer(xs[i] + (int64_t)t * 32, to + i * 4096);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) transfer(ws[i] + (int64_t)t * 512 + lane8, to + WM * 1024 + i * 4096);
+  };
+  for (int t = 0; t < min(kWideStages, steps); ++t) fetch(t, t);
   f32x4 acc[WN][WM] = {};
-  const uint32_t base = lds_address(smem) + lane * 16, rows = lds_address(smem) + row_place(r16, g) * 16;
-  const int trips = p.k / 64;
-  fetch(0);
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  const uint32_t rows = lds_address(smem) + row_place(r16, g) * 16, weights = lds_address(smem) + lane * 16 + (WM + wave * WN) * 1024;
+  u32x4 a[2][WN], b[2][WM];
+  auto landed = [&](auto H) __attribute__((always_inline)) {
+    constexpr int h = decltype(H)::value;
+    static_for<WN>([&](auto I) { lds_wait<0>(a[h][decltype(I)::value]); });
+    static_for<WM>([&](auto I) { lds_wait<0>(b[h][decltype(I)::value]); });
+  };
+  int slot = 0;
+  auto step = [&](auto H, int t) __attribute__((always_inline)) {
+    constexpr int h = decltype(H)::value;
+    // stage t + 1 is there, and every wave has stage t in registers, whose place the stage three ahead takes
+    if (t + kWideStages - 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * (kWideStages - 2)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+    if (t + kWideStages < steps) fetch(t + kWideStages, slot);
+    slot = slot == kWideStages - 1 ? 0 : slot + 1;
+    const uint32_t xa = rows + slot * STAGE, wa = weights + slot * STAGE;   // (behind the last stage: an old one, for nobody)
+    static_for<WM>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i < WN) lds_read128<i * 1024>(a[1 - h][i], wa);
+      lds_read128<i * 1024>(b[1 - h][i], xa);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < WN; ++j) acc[j][i] = mfma16x16x32<Tag>(a[h][j], b[h][i], acc[j][i]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    landed(std::integral_constant<int, 1 - h>{});
+  };
+  if (steps >= kWideStages) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * (kWideStages - 1)) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   lds_barrier();
-  if (trips > 1) fetch(1);
-  for (int t = 0; t < trips; ++t) {
-    const uint32_t at = (t & 1) * STAGE, xa = rows + at + wm * WM * 2048, wa = base + at + (TILES + wn * WN) * 2048;
-    u32x4 a[2][WN], b[2][WM];
-    static_for<2>([&](auto H) {
-      constexpr int h = decltype(H)::value;
-      static_for<WN>([&](auto I) { lds_read128<decltype(I)::value * 2048 + h * 1024>(a[h][decltype(I)::value], wa); });
-      static_for<WM>([&](auto I) { lds_read128<decltype(I)::value * 2048 + h * 1024>(b[h][decltype(I)::value], xa); });
-    });
-    static_for<2>([&](auto H) {
-      constexpr int h = decltype(H)::value;
-      static_for<WN>([&](auto I) { lds_wait<h == 0 ? WM + WN : 0>(a[h][decltype(I)::value]); });
-      static_for<WM>([&](auto I) { lds_wait<h == 0 ? WM + WN : 0>(b[h][decltype(I)::value]); });
-      if (h == 1 && t + 1 < trips) {   // every wave has read this stage; the next has landed
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        lds_barrier();
-        if (t + 2 < trips) fetch(t + 2);
-      }
-#pragma unroll
-      for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) acc[j][i] = mfma16x16x32<Tag>(a[h][j], b[h][i], acc[j][i]);
-    });
+  static_for<WN>([&](auto I) { lds_read128<decltype(I)::value * 1024>(a[0][decltype(I)::value], weights); });
+  static_for<WM>([&](auto I) { lds_read128<decltype(I)::value * 1024>(b[0][decltype(I)::value], rows); });
+  landed(std::integral_constant<int, 0>{});
+  for (int t = 0; t < steps; t += 2) {   // (an even number of them)
+    step(std::integral_constant<int, 0>{}, t);
+    step(std::integral_constant<int, 1>{}, t + 1);
   }
+  // (every wave has its last stage in registers, and no transfer is under way: LDS is free)
+  float sc[WM];
 #pragma unroll
-  for (int i = 0; i < WM; ++i) {
-    const int row = (wm * WM + i) * 16 + r16;
-    if (row >= live) continue;
-    const float sc = in_scale_of(p, m0 + row);
-    T *out = (T *)p.out + (int64_t)(m0 + row) * p.out_stride + g * 4;
+  for (int i = 0; i < WM; ++i) sc[i] = in_scale_of(p, m0 + min(i * 16 + r16, live - 1));
+  constexpr int COLS = GATED ? WN * 8 : WN * 16, ROW = COLS * 2 + 16, PIECES = COLS / 8;   // outputs of a wave; bytes of a row of them, 16-byte pieces
+  char *const mine_at = smem + wave * (kWideRows * ROW);
+  const int first = nt0 * 16 + wave * COLS;
+  auto results = [&](auto A) {
+    constexpr int ACT = decltype(A)::value;
 #pragma unroll
-    for (int j = 0; j < (GATED ? WN / 2 : WN); ++j) {
-      const int nt = nt0 + (GATED ? wn * (WN / 2) + j : wn * WN + j);
-      if (nt >= ntiles) continue;
-      f32x4 o;
-      if constexpr (GATED) {
+    for (int i = 0; i < WM; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) o[q] = gated_act<Tag>(acc[2 * j][i][q] * sc, acc[2 * j + 1][i][q] * sc, p.act);
-      } else {
-        o = acc[j][i] * sc;
+      for (int j = 0; j < COLS / 16; ++j) {
+        f32x4 o;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          o[q] = GATED ? wide_result<Tag, true, ACT>(acc[GATED ? 2 * j : j][i][q] * sc[i], acc[GATED ? 2 * j + 1 : j][i][q] * sc[i], p.act)
+                       : acc[j][i][q] * sc[i];
+        *(u32x2 *)(mine_at + (i * 16 + r16) * ROW + j * 32 + g * 8) = pack_quad<Tag>(o);
       }
-      *(u32x2 *)(out + nt * 16) = pack_quad<Tag>(o);
-    }
+  };
+  if (!GATED) results(std::integral_constant<int, 0>{});
+  else if (p.act.kind == MV_ACT_GELU) results(std::integral_constant<int, MV_ACT_GELU>{});
+  else if (p.act.kind == MV_ACT_CLAMPED) results(std::integral_constant<int, MV_ACT_CLAMPED>{});
+  else if (p.act.kind == MV_ACT_RELU) results(std::integral_constant<int, MV_ACT_RELU>{});
+  else results(std::integral_constant<int, MV_ACT_SILU>{});
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  const int piece = lane % PIECES, col = first + piece * 8;
+#pragma unroll
+  for (int n = 0; n < kWideRows * PIECES / 64; ++n) {
+    const int row = n * (64 / PIECES) + lane / PIECES;
+    const u32x4 v = *(const u32x4 *)(mine_at + row * ROW + piece * 16);
+    if (row < live && col < p.n) *(u32x4 *)((T *)p.out + (int64_t)(m0 + row) * p.out_stride + col) = v;
   }
 }
 
@@ -586,9 +637,10 @@ int launch_linear(const MoeLinear &p, int tile_m, int max_tiles, hipStream_t st)
     if (tile_m == 64) hipLaunchKernelGGL((moe_tile_kernel<Tag, 64, BN, GATED>), grid, dim3(256), (64 + BN) * 256, st, p);
     else hipLaunchKernelGGL((moe_tile_kernel<Tag, 128, BN, GATED>), grid, dim3(256), (128 + BN) * 256, st, p);
   } else if (tile_m == 256) {
-    const int nx = (nt * (GATED ? 2 : 1) + 15) / 16, groups = (max_tiles + 3) / 4;
+    const int nx = (nt * (GATED ? 2 : 1) + 15) / 16;
     if (int rc = mv_allow_lds<moe_wide_kernel<Tag, GATED>>()) return rc;
-    hipLaunchKernelGGL((moe_wide_kernel<Tag, GATED>), dim3((unsigned)((groups + 7) / 8 * 8) * 4u * nx), dim3(512), 128 * 1024, st, p, nx, max_tiles);
+    hipLaunchKernelGGL((moe_wide_kernel<Tag, GATED>), dim3((unsigned)(((int64_t)max_tiles * 2 * nx + 7) / 8 * 8)), dim3(256),
+                       kWideStages * 24 * 1024, st, p, nx, max_tiles);
   } else {
     return MV_E_SHAPE;
   }
