@@ -7,7 +7,7 @@
 //     S <- e^{r_last} S + sum_j k_j (e^{r_last - r_j} f_j u_j)^T
 // so k and q enter every product as they are in memory (exact in bf16) and only T, B, S and U are sums of two bf16 numbers.  Two launches:
 //   prepare: T, B and three factors per token, one workgroup per (chunk, head), 25 KiB of workspace;
-//   walk:    chunks one behind the other, one workgroup per (sequence, head, columns); rows of k and q come from the inputs, transposed out of
+//   walk:    chunks one behind the other, one workgroup per (sequence, head, columns); rows of k, q and v come from the inputs, transposed out of
 //            LDS where the state takes them in; the next chunk lands while this one is multiplied.
 #include "delta_chunk.h"
 
@@ -137,16 +137,28 @@ __global__ void __launch_bounds__(256, NK < 5 ? 4 : 3) delta_scalar_prepare_kern
   }
 }
 
-// Workgroup = 4 waves x CW tiles of 16 columns of one head of one sequence; a wave keeps S of its columns in accumulators, whose rows are
-// dealt so that tiles 2 s and 2 s + 1 together hold n = 32 s + 8 g .. + 7 in lane group g: operands of the next product as they are.
-template <int NK, int CW>
-__global__ void __launch_bounds__(256, 1) delta_scalar_walk_kernel(DeltaPrep q) {
+// Workgroup = W waves = W tiles of 16 columns of one head of one sequence; a wave keeps S of its columns in accumulators, whose rows are
+// dealt so that tiles 2 s and 2 s + 1 together hold n = 32 s + 8 g .. + 7 in lane group g: operands of the next product as they are.  o is
+// computed transposed (columns by tokens), so that a lane holds four columns of a token; the rows of v land in LDS like those of k and q and are
+// read transposed, and o leaves by way of their place as whole lines.
+// Bound by the chain of a chunk (132 products and some 500 vector instructions of a wave, each part waiting for the one before) and by the way of its
+// 75 KB through the memory pipeline.  16 heads of 128 x 128, 16 sequences of 745 .. 1490 tokens: 198 us with four waves of two tiles, v and o by
+// elements; 158 with eight waves of one tile, two on a SIMD, that fill each other's gaps, and v by LDS; 144 with transfers asked for between the
+// products (all at once they held a wave up for 3000 of 12000 cycles) and k, q on one XCD; 135 with o by lines (by 32 bytes its stores took 30 us).
+// Where heads and sequences do not fill the chip, workgroups of four waves leave no CU idle.
+template <int NK, int W>
+__global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep q) {
   typedef elem<B16>::T T;
-  constexpr int N = NK * 32, ROWS = 4 * NK, STAGE = (2 * ROWS + kScalarTotal) * 1024, PER = (kScalarTotal + 3) / 4;
+  constexpr int N = NK * 32, ROWS = 4 * NK, VF = 2 * W;   // fragments of 1 KiB: k, q; v
+  constexpr int AT_V = 2 * ROWS, AT = AT_V + VF, STAGE = (AT + kScalarTotal) * 1024, PER = (kScalarTotal + W - 1) / W;
   const MvDeltaArgs &p = q.a;
-  extern __shared__ __attribute__((aligned(16))) char smem[];   // 2 stages of k [4][NK] | q [4][NK] | T | B | factors, fragments of 1 KiB
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // 2 stages of k [4][NK] | q [4][NK] | v [64][W * 16] | T | B | factors
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  const int head = blockIdx.y, seq = blockIdx.z, tiles = p.p / 16, tile0 = blockIdx.x * 4 * CW, grp = head / (p.heads / p.groups);
+  // (workgroups are dealt to the 8 XCDs in turn: each gets a run of columns and heads, which share k and q)
+  const int wide = gridDim.x, all = wide * p.heads;
+  int at_head = blockIdx.y * wide + blockIdx.x;
+  if (!(all & 7)) at_head = (at_head & 7) * (all >> 3) + (at_head >> 3);
+  const int head = at_head / wide, seq = blockIdx.z, tiles = p.p / 16, tile0 = (at_head - head * wide) * W, grp = head / (p.heads / p.groups);
   const int q0 = p.cu_q[seq], len = p.cu_q[seq + 1] - q0;
   if (len <= 0) return;
   const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq];
@@ -156,231 +168,254 @@ __global__ void __launch_bounds__(256, 1) delta_scalar_walk_kernel(DeltaPrep q) 
   const char *ws = q.ws + ((int64_t)(q0 / L + seq) * p.heads + head) * kScalarTotal * 1024 + lane * 16;
   const T *x = (const T *)p.x + (int64_t)q0 * p.x_stride;
 
-  int col[CW];
-  bool live[CW];
-#pragma unroll
-  for (int w = 0; w < CW; ++w) {
-    const int t = tile0 + wave * CW + w;
-    live[w] = t < tiles, col[w] = min(t, tiles - 1) * 16 + r16;
-  }
-  auto state_at = [&](int half, int w, int i, int e) {
+  const bool live = tile0 + wave < tiles;
+  const int col = min(tile0 + wave, tiles - 1) * 16;
+  auto state_at = [&](int half, int i, int e) {
     const int n = (i >> 1) * 32 + g * 8 + (i & 1) * 4 + e;
-    return p.state + half * p.slots * size + (int64_t)(keep ? slot : 0) * size + ((int64_t)head * p.n + n) * p.p + col[w];
+    return p.state + half * p.slots * size + (int64_t)(keep ? slot : 0) * size + ((int64_t)head * p.n + n) * p.p + col + r16;
   };
-  f32x4 st[CW][2 * NK];
+  f32x4 st[2 * NK];
 #pragma unroll
-  for (int w = 0; w < CW; ++w)
+  for (int i = 0; i < 2 * NK; ++i)
 #pragma unroll
-    for (int i = 0; i < 2 * NK; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st[w][i][e] = keep && before > 0 ? *state_at(before & 1, w, i, e) : 0.f;
+    for (int e = 0; e < 4; ++e) st[i][e] = keep && before > 0 ? *state_at(before & 1, i, e) : 0.f;
 
   auto transfer = [&](const void *from, char *to) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from, (__attribute__((address_space(3))) void *)to, 16, 0, 0);
   };
-  // a wave brings the rows of one token tile and its share of the rest (rows behind the end: the last row again, with factors 0)
-  auto fetch = [&](int c) {
+  // Where this lane's pieces of 16 bytes come from: rows of k and q of one token tile (of half its channels, with eight waves), two runs of rows of v
+  // (whose pieces lie in an order that spreads eight rows over the banks), its share of the rest.  Rows behind the end: the last row again, with
+  // factors 0.
+  constexpr int VP = 2 * W, VR = 64 / VP;   // pieces of a row of v, rows of a fragment
+  auto v_swizzle = [](int row) { return (row << 1) & (VP - 1); };
+  constexpr int KQ = (NK + W / 4 - 1) / (W / 4) * 2, ALL = KQ + 2 + PER;   // transfers of a wave and chunk
+  auto fetch = [&](auto I, int c) __attribute__((always_inline)) {
+    constexpr int n = decltype(I)::value;
     char *to = smem + (c & 1) * STAGE;
-    const T *row = x + (int64_t)min(c * L + 16 * wave + (lane >> 2), len - 1) * p.x_stride + grp * N + row_chunk(lane) * 8;
-#pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      transfer(row + p.k_off + 32 * s, to + (wave * NK + s) * 1024);
-      transfer(row + p.q_off + 32 * s, to + (ROWS + wave * NK + s) * 1024);
-    }
-    const char *from = ws + c * stride;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int f = min(i * 4 + wave, kScalarTotal - 1);
-      transfer(from + f * 1024, to + (2 * ROWS + f) * 1024);
+    if constexpr (n < KQ) {
+      const int it = wave & 3, s = n / 2 * (W / 4) + (wave >> 2);
+      const T *row = x + (int64_t)min(c * L + 16 * it + (lane >> 2), len - 1) * p.x_stride + grp * N + row_chunk(lane) * 8;
+      if (NK % (W / 4) == 0 || s < NK) transfer(row + (n % 2 ? p.q_off : p.k_off) + 32 * s, to + (n % 2 * ROWS + it * NK + s) * 1024);
+    } else if constexpr (n < KQ + 2) {
+      const int f = 2 * wave + n - KQ, r = f * VR + lane / VP, piece = (lane % VP) ^ v_swizzle(r);
+      const T *from = x + (int64_t)min(c * L + r, len - 1) * p.x_stride + head * p.p + min(tile0 * 16 + piece * 8, p.p - 8);
+      transfer(from, to + (AT_V + f) * 1024);
+    } else {
+      const int f = min((n - KQ - 2) * W + wave, kScalarTotal - 1);
+      transfer(ws + c * stride + f * 1024, to + (AT + f) * 1024);
     }
   };
-  T v[CW][16];
-  auto fetch_v = [&](int c) {
+  // Results take the place of the wave's columns of v in LDS; at the next chunk a wave takes the rows from there that it brings v of, whole lines
+  // of them, and stores them.
+  u32x4 done[2];
+  const bool pieces = !(((uintptr_t)p.out & 15) | (p.out_stride & 7));   // (rows of the output may stand anywhere)
+  auto store = [&](int c, int i) __attribute__((always_inline)) {
+    const int r = (2 * wave + i) * VR + lane / VP, t = c * L + r, at = tile0 * 16 + ((lane % VP) ^ v_swizzle(r)) * 8;
+    if (t >= len || at >= p.p) return;
+    T *to = (T *)p.out + (int64_t)(q0 + t) * p.out_stride + head * p.p + at;
+    if (pieces) {
+      *(u32x4 *)to = done[i];
+    } else {
 #pragma unroll
-    for (int w = 0; w < CW; ++w)
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        v[w][i] = x[(int64_t)min(c * L + 16 * (i >> 2) + 4 * g + (i & 3), len - 1) * p.x_stride + head * p.p + col[w]];
+      for (int e = 0; e < 8; ++e) to[e] = (T)(done[i][e >> 1] >> (e & 1) * 16);
+    }
   };
-  f32x4 o[CW][4];
-  auto store = [&](int c) {
-#pragma unroll
-    for (int w = 0; w < CW; ++w)
-#pragma unroll
-      for (int it = 0; it < 4; ++it)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int t = c * L + 16 * it + 4 * g + e;
-          if (live[w] && t < len) ((T *)p.out)[(int64_t)(q0 + t) * p.out_stride + head * p.p + col[w]] = elem<B16>::st(o[w][it][e]);
-        }
+  // What a chunk's transfers and stores cost is their way through the memory pipeline, which a wave that asks for all of them at once waits out: they
+  // are asked for a few at a time, between its products.
+  constexpr int POINTS = NK + 1;
+  auto between = [&](auto I, int c, int chunks) __attribute__((always_inline)) {
+    constexpr int n = decltype(I)::value, lo = ALL * n / POINTS, hi = ALL * (n + 1) / POINTS;
+    if constexpr (n == 0) lds_wait<8>(done[0], done[1]);   // (read ahead of the rows; the transfers of v come behind)
+    if (c + 1 < chunks) static_for<hi - lo>([&](auto J) { fetch(std::integral_constant<int, lo + decltype(J)::value>{}, c + 1); });
+    if (n < 2 && c > 0) store(c - 1, n);
   };
   const uint32_t lds = lds_address(smem);
   const int chunks = (len + L - 1) / L;
-  fetch(0);
-  fetch_v(0);
+  static_for<ALL>([&](auto I) { fetch(I, 0); });
   for (int c = 0; c < chunks; ++c) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     lds_barrier();   // this chunk has landed; every wave is done with the one before
-    f32x4 rest[CW][4];   // v, then R
-#pragma unroll
-    for (int w = 0; w < CW; ++w)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) rest[w][i >> 2][i & 3] = elem<B16>::ld(v[w][i]);
-    if (c > 0) store(c - 1);
-    if (c + 1 < chunks) {
-      fetch(c + 1);
-      fetch_v(c + 1);
-    }
-    const uint32_t at = lds + (c & 1) * STAGE, rows = at + row_place(r16, g) * 16, rest_at = at + 2 * ROWS * 1024;
+    const uint32_t at = lds + (c & 1) * STAGE, rows = at + row_place(r16, g) * 16, rest_at = at + AT * 1024;
     const uint32_t fl = rest_at + lane * 16, ff = rest_at + kFactors * 1024 + g * 16;
     const uint32_t tr = at + row_place(4 * g + (r16 >> 2), r16 & 3) * 16;
-    // ---- k S and q S
-    f32x4 ksum[CW][4];
+    const int vrow = 4 * g + (r16 >> 2);   // (rows 16 apart have the same order)
+    const uint32_t vt = at + AT_V * 1024 + vrow * W * 32 + ((2 * wave + ((r16 & 3) >> 1)) ^ v_swizzle(vrow)) * 16 + (r16 & 1) * 8;
+    // ---- k S (tokens by columns) and q S (columns by tokens); what comes out of LDS is asked for one step ahead, here and below
+    f32x4 ksum[4], o[4];
 #pragma unroll
-    for (int w = 0; w < CW; ++w)
-#pragma unroll
-      for (int it = 0; it < 4; ++it) ksum[w][it] = o[w][it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int it = 0; it < 4; ++it) ksum[it] = o[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 fk[2][4], fq[2][4], raw[2][4];
+    u32x2 v[4];
+    float to_o[4], last;
+    auto read_rows = [&](auto S) __attribute__((always_inline)) {
+      constexpr int s = decltype(S)::value;
+      static_for<4>([&](auto I) {
+        constexpr int it = decltype(I)::value;
+        lds_read128<(it * NK + s) * 1024>(fk[s & 1][it], rows);
+        lds_read128<(ROWS + it * NK + s) * 1024>(fq[s & 1][it], rows);
+      });
+    };
+    const uint32_t results = lds + ((c + 1) & 1) * STAGE + (AT_V + 2 * wave) * 1024 + lane * 16;
+    lds_read128<0>(done[0], results);
+    lds_read128<1024>(done[1], results);
+    read_rows(std::integral_constant<int, 0>{});
     static_for<NK>([&](auto S) {
       constexpr int s = decltype(S)::value;
-      u32x4 fk[4], fq[4], sh[CW], sl[CW];
+      u32x4 sh, sl;
+      if constexpr (s + 1 < NK) {
+        read_rows(std::integral_constant<int, s + 1>{});
+      } else {
+        static_for<4>([&](auto I) {
+          constexpr int it = decltype(I)::value;
+          lds_read64_tr<it * 16 * W * 32>(v[it], vt);
+          lds_read128<it * 64>(raw[0][it], ff);
+        });
+      }
+      split44(st[2 * s], st[2 * s + 1], sh, sl);
       static_for<4>([&](auto I) {
         constexpr int it = decltype(I)::value;
-        lds_read128<(it * NK + s) * 1024>(fk[it], rows);
-        lds_read128<(ROWS + it * NK + s) * 1024>(fq[it], rows);
-      });
-#pragma unroll
-      for (int w = 0; w < CW; ++w) split44(st[w][2 * s], st[w][2 * s + 1], sh[w], sl[w]);
-      static_for<4>([&](auto I) {
-        constexpr int it = decltype(I)::value;
-        lds_wait<2 * (3 - it)>(fk[it], fq[it]);
+        lds_wait<8>(fk[s & 1][it], fq[s & 1][it]);
       });
 #pragma unroll
       for (int part = 0; part < 2; ++part)
 #pragma unroll
-        for (int it = 0; it < 4; ++it)
-#pragma unroll
-          for (int w = 0; w < CW; ++w) {
-            ksum[w][it] = mfma16x16x32<B16>(fk[it], part ? sl[w] : sh[w], ksum[w][it]);
-            o[w][it] = mfma16x16x32<B16>(fq[it], part ? sl[w] : sh[w], o[w][it]);
-          }
+        for (int it = 0; it < 4; ++it) {
+          ksum[it] = mfma16x16x32<B16>(fk[s & 1][it], part ? sl : sh, ksum[it]);
+          o[it] = mfma16x16x32<B16>(part ? sl : sh, fq[s & 1][it], o[it]);
+        }
+      between(S, c, chunks);
     });
     // ---- R, U = T R
-    u32x4 raw[3][4];
+    u32x4 ft[2][kTriangle][2];   // T, B
+    auto read_triangle = [&](auto B) __attribute__((always_inline)) {
+      constexpr int b = decltype(B)::value;
+      static_for<kTriangle>([&](auto M) {
+        constexpr int m = decltype(M)::value;
+        lds_read128<b * kB * 1024 + m * 2048>(ft[b][m][0], fl);
+        lds_read128<b * kB * 1024 + m * 2048 + 1024>(ft[b][m][1], fl);
+      });
+    };
+    read_triangle(std::integral_constant<int, 0>{});
     static_for<4>([&](auto I) {
       constexpr int it = decltype(I)::value;
-      lds_read128<it * 64>(raw[0][it], ff);
-      lds_read128<it * 64 + 256>(raw[1][it], ff);
-      lds_read128<it * 64 + 512>(raw[2][it], ff);
+      lds_wait<2 * kTriangle>(raw[0][it]);
+      lds_wait<2 * kTriangle>(v[it]);
     });
-    float last;
-    lds_read32<kFactors * 1024 + 768>(last, rest_at);
-    u32x4 ft[kTriangle][2];
-    static_for<kTriangle>([&](auto M) {
-      constexpr int m = decltype(M)::value;
-      lds_read128<m * 2048>(ft[m][0], fl);
-      lds_read128<m * 2048 + 1024>(ft[m][1], fl);
-    });
-    static_for<4>([&](auto I) {
-      constexpr int it = decltype(I)::value;
-      lds_wait<2 * kTriangle>(raw[0][it], raw[1][it]);
-      lds_wait<2 * kTriangle>(raw[2][it]);
-    });
-    lds_wait<2 * kTriangle>(last);
-    u32x4 uh[CW][2], ul[CW][2];
+    u32x4 uh[2], ul[2];
+    f32x4 rest[4];
 #pragma unroll
-    for (int w = 0; w < CW; ++w) {
+    for (int it = 0; it < 4; ++it) {
+      const f32x4 f = __builtin_bit_cast(f32x4, raw[0][it]) * ksum[it];
 #pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        rest[w][it] -= __builtin_bit_cast(f32x4, raw[0][it]) * ksum[w][it];
-        o[w][it] *= __builtin_bit_cast(f32x4, raw[1][it]);
+      for (int e = 0; e < 2; ++e) {
+        rest[it][2 * e] = u2f(v[it][e] << 16) - f[2 * e];
+        rest[it][2 * e + 1] = u2f(v[it][e] & 0xffff0000u) - f[2 * e + 1];
       }
-#pragma unroll
-      for (int s = 0; s < 2; ++s) split44(rest[w][2 * s], rest[w][2 * s + 1], uh[w][s], ul[w][s]);
     }
-    f32x4 u[CW][4];
 #pragma unroll
-    for (int w = 0; w < CW; ++w)
+    for (int s = 0; s < 2; ++s) split44(rest[2 * s], rest[2 * s + 1], uh[s], ul[s]);
+    f32x4 u[4];
 #pragma unroll
-      for (int it = 0; it < 4; ++it) u[w][it] = f32x4{0.f, 0.f, 0.f, 0.f};
-    static_for<kTriangle>([&](auto M) { lds_wait<0>(ft[decltype(M)::value][0], ft[decltype(M)::value][1]); });
+    for (int it = 0; it < 4; ++it) u[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    static_for<kTriangle>([&](auto M) { lds_wait<0>(ft[0][decltype(M)::value][0], ft[0][decltype(M)::value][1]); });
+    static_for<4>([&](auto I) {
+      constexpr int it = decltype(I)::value;
+      lds_read32<kFactors * 1024 + 256 + it * 64>(to_o[it], rest_at + r16 * 4);
+    });
+    read_triangle(std::integral_constant<int, 1>{});
 #pragma unroll
     for (int part = 0; part < 3; ++part)
       static_for<4>([&](auto I) {
         constexpr int it = decltype(I)::value;
         static_for<it / 2 + 1>([&](auto S) {
           constexpr int s = decltype(S)::value;
-#pragma unroll
-          for (int w = 0; w < CW; ++w) u[w][it] = mfma16x16x32<B16>(ft[triangle(it, s)][part == 2], part == 1 ? ul[w][s] : uh[w][s], u[w][it]);
+          u[it] = mfma16x16x32<B16>(ft[0][triangle(it, s)][part == 2], part == 1 ? ul[s] : uh[s], u[it]);
         });
       });
+    between(std::integral_constant<int, NK>{}, c, chunks);
     // ---- o += B U
-    static_for<kTriangle>([&](auto M) {
-      constexpr int m = decltype(M)::value;
-      lds_read128<kB * 1024 + m * 2048>(ft[m][0], fl);
-      lds_read128<kB * 1024 + m * 2048 + 1024>(ft[m][1], fl);
+    static_for<4>([&](auto I) {
+      constexpr int it = decltype(I)::value;
+      lds_wait<2 * kTriangle>(to_o[it]);
+      o[it] *= to_o[it];
     });
 #pragma unroll
-    for (int w = 0; w < CW; ++w)
-#pragma unroll
-      for (int s = 0; s < 2; ++s) split44(u[w][2 * s], u[w][2 * s + 1], uh[w][s], ul[w][s]);
-    static_for<kTriangle>([&](auto M) { lds_wait<0>(ft[decltype(M)::value][0], ft[decltype(M)::value][1]); });
-#pragma unroll
-    for (int part = 0; part < 3; ++part)
-      static_for<4>([&](auto I) {
-        constexpr int it = decltype(I)::value;
-        static_for<it / 2 + 1>([&](auto S) {
-          constexpr int s = decltype(S)::value;
-#pragma unroll
-          for (int w = 0; w < CW; ++w) o[w][it] = mfma16x16x32<B16>(ft[triangle(it, s)][part == 2], part == 1 ? ul[w][s] : uh[w][s], o[w][it]);
-        });
-      });
-    // ---- S <- decay S + k^T (e^{r_last - r} f u); k transposed: row r16 of a state tile, tokens 16 (e >> 2) + 4 g + (e & 3) of a step of 32
-#pragma unroll
-    for (int w = 0; w < CW; ++w) {
-#pragma unroll
-      for (int it = 0; it < 4; ++it) u[w][it] *= __builtin_bit_cast(f32x4, raw[2][it]);
-#pragma unroll
-      for (int s = 0; s < 2; ++s) split44(u[w][2 * s], u[w][2 * s + 1], uh[w][s], ul[w][s]);
-#pragma unroll
-      for (int i = 0; i < 2 * NK; ++i) st[w][i] *= last;
-    }
-    static_for<NK>([&](auto P) {
+    for (int s = 0; s < 2; ++s) split44(u[2 * s], u[2 * s + 1], uh[s], ul[s]);
+    static_for<kTriangle>([&](auto M) { lds_wait<0>(ft[1][decltype(M)::value][0], ft[1][decltype(M)::value][1]); });
+    // ---- k transposed: row r16 of a state tile, tokens 16 (e >> 2) + 4 g + (e & 3) of a step of 32
+    u32x2 kt[2][2][2][2];   // [which][state tile][step of 32 tokens][its half]
+    auto read_pair = [&](auto P) __attribute__((always_inline)) {
       constexpr int pair = decltype(P)::value;
-      u32x2 kt[2][2][2];   // [state tile][step of 32 tokens][its half]
       static_for<2>([&](auto D) {
         constexpr int d = decltype(D)::value;
         static_for<4>([&](auto I) {
           constexpr int it = decltype(I)::value;
-          lds_read64_tr<(it * NK + pair) * 1024 + d * 8>(kt[d][it >> 1][it & 1], tr);
+          lds_read64_tr<(it * NK + pair) * 1024 + d * 8>(kt[pair & 1][d][it >> 1][it & 1], tr);
         });
       });
+    };
+    static_for<4>([&](auto I) {
+      constexpr int it = decltype(I)::value;
+      lds_read128<it * 64 + 512>(raw[1][it], ff);
+    });
+    lds_read32<kFactors * 1024 + 768>(last, rest_at);
+    read_pair(std::integral_constant<int, 0>{});
+#pragma unroll
+    for (int part = 0; part < 3; ++part)
+      static_for<4>([&](auto I) {
+        constexpr int it = decltype(I)::value;
+        static_for<it / 2 + 1>([&](auto S) {
+          constexpr int s = decltype(S)::value;
+          o[it] = mfma16x16x32<B16>(part == 1 ? ul[s] : uh[s], ft[1][triangle(it, s)][part == 2], o[it]);
+        });
+      });
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const int row = 16 * it + r16;
+      *(u32x2 *)(smem + (c & 1) * STAGE + AT_V * 1024 + row * W * 32 + ((2 * wave + (g >> 1)) ^ v_swizzle(row)) * 16 + (g & 1) * 8) = pack_quad<B16>(o[it]);
+    }
+    // ---- S <- decay S + k^T (e^{r_last - r} f u)
+    static_for<4>([&](auto I) {
+      constexpr int it = decltype(I)::value;
+      lds_wait<8>(raw[1][it]);
+      u[it] *= __builtin_bit_cast(f32x4, raw[1][it]);
+    });
+    lds_wait<8>(last);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) split44(u[2 * s], u[2 * s + 1], uh[s], ul[s]);
+#pragma unroll
+    for (int i = 0; i < 2 * NK; ++i) st[i] *= last;
+    static_for<NK>([&](auto P) {
+      constexpr int pair = decltype(P)::value;
+      if constexpr (pair + 1 < NK) read_pair(std::integral_constant<int, pair + 1>{});
       static_for<2>([&](auto D) {
         constexpr int d = decltype(D)::value;
-        lds_wait<0>(kt[d][0][0], kt[d][0][1]);
-        lds_wait<0>(kt[d][1][0], kt[d][1][1]);
+        lds_wait<(pair + 1 < NK ? 8 : 0)>(kt[pair & 1][d][0][0], kt[pair & 1][d][0][1]);
+        lds_wait<(pair + 1 < NK ? 8 : 0)>(kt[pair & 1][d][1][0], kt[pair & 1][d][1][1]);
       });
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          const u32x4 k = {kt[d][s][0][0], kt[d][s][0][1], kt[d][s][1][0], kt[d][s][1][1]};
+        for (int part = 0; part < 2; ++part)
 #pragma unroll
-          for (int part = 0; part < 2; ++part)
-#pragma unroll
-            for (int w = 0; w < CW; ++w) st[w][2 * pair + d] = mfma16x16x32<B16>(k, part ? ul[w][s] : uh[w][s], st[w][2 * pair + d]);
-        }
+          for (int d = 0; d < 2; ++d) {
+            const u32x2 &lo = kt[pair & 1][d][s][0], &hi = kt[pair & 1][d][s][1];
+            st[2 * pair + d] = mfma16x16x32<B16>(u32x4{lo[0], lo[1], hi[0], hi[1]}, part ? ul[s] : uh[s], st[2 * pair + d]);
+          }
     });
   }
-  store(chunks - 1);
-  if (keep) {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  lds_barrier();
 #pragma unroll
-    for (int w = 0; w < CW; ++w)
-      if (live[w]) {
+  for (int i = 0; i < 2; ++i) {
+    done[i] = *(const u32x4 *)(smem + ((chunks - 1) & 1) * STAGE + (AT_V + 2 * wave + i) * 1024 + lane * 16);
+    store(chunks - 1, i);
+  }
+  if (keep && live) {
 #pragma unroll
-        for (int i = 0; i < 2 * NK; ++i)
+    for (int i = 0; i < 2 * NK; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) *state_at((before + len) & 1, w, i, e) = st[w][i][e];
-      }
+      for (int e = 0; e < 4; ++e) *state_at((before + len) & 1, i, e) = st[i][e];
   }
 }
 
@@ -389,14 +424,15 @@ int launch(const DeltaPrep &q, hipStream_t stream) {
   const MvDeltaArgs &a = q.a;
   hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK>), dim3((unsigned)chunk_slots(a.n_seqs, a.total_q), a.heads), dim3(256), 0, stream, q);
   MV_LAUNCH_CHECK();
-  // two column tiles a wave share every operand read, where that still leaves a workgroup per CU
-  const int tiles = a.p / 16, wide = (tiles + 7) / 8, lds = 2 * (8 * NK + kScalarTotal) * 1024;
-  if (tiles > 4 && (int64_t)wide * a.heads * a.n_seqs >= 256) {
-    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 2>>()) return rc;
-    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 2>), dim3(wide, a.heads, a.n_seqs), dim3(256), lds, stream, q);
+  // Eight waves where workgroups of four would be more than the CUs, of which each holds one
+  const int tiles = a.p / 16, wide = (tiles + 7) / 8, narrow = (tiles + 3) / 4;
+  const auto lds = [](int waves) { return 2 * (8 * NK + 2 * waves + kScalarTotal) * 1024; };
+  if (tiles > 4 && lds(8) <= 160 * 1024 && (int64_t)narrow * a.heads * a.n_seqs > 256) {
+    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 8>>()) return rc;
+    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 8>), dim3(wide, a.heads, a.n_seqs), dim3(512), lds(8), stream, q);
   } else {
-    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 1>>()) return rc;
-    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 1>), dim3((tiles + 3) / 4, a.heads, a.n_seqs), dim3(256), lds, stream, q);
+    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 4>>()) return rc;
+    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 4>), dim3(narrow, a.heads, a.n_seqs), dim3(256), lds(4), stream, q);
   }
   MV_LAUNCH_CHECK();
   return MV_OK;
