@@ -291,15 +291,27 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(De
 
 // Workgroup = 4 waves x CW tiles of 16 columns of one head of one sequence; a wave keeps S of its columns in accumulators.  The
 // accumulators are the next product's operands as they are: the rows of S are dealt so that tiles 2 s and 2 s + 1 together hold
-// n = 32 s + 8 g .. + 7 in lane group g.  LDS holds the operands of one phase while those of the other phase land.
+// n = 32 s + 8 g .. + 7 in lane group g.  O is computed transposed (columns by tokens), so that a lane stores four columns of a token.
+// Bound by the chain of a chunk and by the way of its 129 KB through the memory pipeline of a CU.  LDS holds one chunk, in groups in the order of their
+// use: as soon as all waves have used a group, its part of the next chunk is asked for, so that transfers run all the time and none is waited for
+// that was not asked for a chunk before (3 sequences of 4011 tokens and less, 8 heads of 128 x 128: 283 us with two phases, each fetched as a whole
+// while the other was used -> 247).
 template <typename Tag, int NK, int CW>
 __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
   typedef typename elem<Tag>::T T;
-  constexpr int F1 = 16 * NK + 16 * CW, F2 = 8 * NK + 17, N1 = F1 / 4, N2 = (F2 + 3) / 4;   // fragments of a phase; a wave's
+  constexpr int F1 = 16 * NK + 16 * CW, GROUPS = 2 * NK + 1;   // fragments of W, Q and U0; steps of W and Q (U0 in the first) | B | pairs of tiles of K
+  // transfers of a wave: for a group, for those behind it, for all
+  constexpr auto own = [](int n) { return n < NK ? (n ? 4 : 4 + 4 * CW) : n == NK ? 5 : 2; };
+  constexpr auto behind = [](int n) { return n < NK ? 4 * (NK - 1 - n) + 5 + 2 * NK : 2 * (GROUPS - 1 - n); };
+  constexpr int ALL = 4 * CW + 4 * NK + 5 + 2 * NK;
   const MvDeltaArgs &p = q.a;
   extern __shared__ __attribute__((aligned(16))) char smem[];   // [F1][1 KiB] | [F2][1 KiB]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  const int head = blockIdx.y, seq = blockIdx.z, tiles = p.p / 16, tile0 = blockIdx.x * 4 * CW;
+  // (workgroups are dealt to the 8 XCDs in turn: each gets a run of columns and heads, which share all but their part of U0)
+  const int wide = gridDim.x, all = wide * p.heads;
+  int at_head = blockIdx.y * wide + blockIdx.x;
+  if (!(all & 7)) at_head = (at_head & 7) * (all >> 3) + (at_head >> 3);
+  const int head = at_head / wide, seq = blockIdx.z, tiles = p.p / 16, tile0 = (at_head - head * wide) * 4 * CW;
   const int q0 = p.cu_q[seq], len = p.cu_q[seq + 1] - q0;
   if (len <= 0) return;
   const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq];
@@ -332,31 +344,53 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(from + (int64_t)frag * 1024),
                                      (__attribute__((address_space(3))) void *)to, 16, 0, 0);
   };
-  auto fetch1 = [&](const char *from) {
+  auto fetch_group = [&](auto G, int c) __attribute__((always_inline)) {
+    constexpr int n = decltype(G)::value;
+    const char *from = ws + c * stride;
+    if constexpr (n < NK) {
 #pragma unroll
-    for (int i = 0; i < N1; ++i) {
-      const int f = i * 4 + wave, u = f - 16 * NK;   // u: (column tile, token tile)
-      fetch(from, f < 16 * NK ? f : lay.u0 + min(tile0 + (u >> 2), tiles - 1) * 4 + (u & 3), smem + f * 1024);
-    }
-  };
-  auto fetch2 = [&](const char *from) {
+      for (int i = 0; i < 4; ++i) {
+        const int which = i * 4 + wave, f = (which >> 3) * 8 * NK + (((which >> 1) & 3) * NK + n) * 2 + (which & 1);
+        fetch(from, f, smem + f * 1024);
+      }
+      if constexpr (n == 0) {
 #pragma unroll
-    for (int i = 0; i < N2; ++i) {
-      const int f = min(i * 4 + wave, F2 - 1);
-      fetch(from, lay.k + f, smem + (F1 + f) * 1024);
+        for (int i = 0; i < 4 * CW; ++i) {
+          const int f = i * 4 + wave;   // (column tile, token tile)
+          fetch(from, lay.u0 + min(tile0 + (f >> 2), tiles - 1) * 4 + (f & 3), smem + (16 * NK + f) * 1024);
+        }
+      }
+    } else {
+      constexpr int first = n == NK ? 8 * NK : (n - NK - 1) * 8, last = n == NK ? 8 * NK + 16 : first + 7;
+#pragma unroll
+      for (int i = 0; i < own(n); ++i) {
+        const int f = min(first + i * 4 + wave, last);
+        fetch(from, lay.k + f, smem + (F1 + f) * 1024);
+      }
     }
   };
   const uint32_t base = lds_address(smem) + lane * 16;
   const uint32_t aw = base, aq = base + 8 * NK * 1024, au = base + (16 * NK + wave * CW * 4) * 1024;
   const uint32_t ak = base + F1 * 1024, ab = ak + 8 * NK * 1024, at = lds_address(smem) + (F1 + 8 * NK + 16) * 1024 + g * 32;
   const int chunks = (len + L - 1) / L;
-  fetch1(ws);
-  fetch2(ws);
+  const bool quads = !(((uintptr_t)p.out & 7) | (p.out_stride & 3));   // (rows of the output may stand anywhere)
+  static_for<GROUPS>([&](auto G) { fetch_group(G, 0); });
   for (int c = 0; c < chunks; ++c) {
     const bool more = c + 1 < chunks;
-    ws += stride;
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N2) : "memory");   // (the newest N2: the other phase's)
-    lds_barrier();
+    // Before a group is used: it has landed (the transfers of the others may be under way; stores only make the wait longer), and every wave is done
+    // with the group before, whose place the next chunk's takes.
+    auto begin = [&](auto G) __attribute__((always_inline)) {
+      constexpr int n = decltype(G)::value;
+      if (n == 0 || more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(ALL - own(n) - own((n + GROUPS - 1) % GROUPS)) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(behind(n)) : "memory");
+      lds_barrier();
+      if constexpr (n == 0) {
+        if (c > 0) fetch_group(std::integral_constant<int, GROUPS - 1>{}, c);
+      } else {
+        if (more) fetch_group(std::integral_constant<int, n - 1>{}, c + 1);
+      }
+    };
+    begin(std::integral_constant<int, 0>{});
     // ---- U = U0 - W S, O = Q S
     f32x4 u[CW][4], o[CW][4];
 #pragma unroll
@@ -375,6 +409,7 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
     static_for<NK>([&](auto S) {
       constexpr int s = decltype(S)::value;
       u32x4 fw[4][2], fo[4][2], sh[CW], sl[CW];
+      if constexpr (s > 0) begin(S);
       static_for<4>([&](auto I) {
         constexpr int it = decltype(I)::value;
         lds_read128<((it * NK + s) * 2) * 1024>(fw[it][0], aw);
@@ -396,17 +431,10 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
 #pragma unroll
           for (int w = 0; w < CW; ++w) {
             u[w][it] = mfma16x16x32<B16>(fw[it][part == 2], part == 1 ? sl[w] : sh[w], u[w][it]);
-            o[w][it] = mfma16x16x32<B16>(fo[it][part == 2], part == 1 ? sl[w] : sh[w], o[w][it]);
+            o[w][it] = mfma16x16x32<B16>(part == 1 ? sl[w] : sh[w], fo[it][part == 2], o[w][it]);
           }
     });
-    lds_barrier();   // every wave has read phase 1
-    if (more) {
-      fetch1(ws);
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N1) : "memory");
-    } else {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    lds_barrier();
+    begin(std::integral_constant<int, NK>{});
     // ---- O += B U, S = decay S + K U
     u32x4 uh[CW][2], ul[CW][2];
 #pragma unroll
@@ -427,15 +455,37 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
         static_for<it / 2 + 1>([&](auto S) {
           constexpr int s = decltype(S)::value;
 #pragma unroll
-          for (int w = 0; w < CW; ++w) o[w][it] = mfma16x16x32<B16>(fb[s][part == 2], part == 1 ? ul[w][s] : uh[w][s], o[w][it]);
+          for (int w = 0; w < CW; ++w) o[w][it] = mfma16x16x32<B16>(part == 1 ? ul[w][s] : uh[w][s], fb[s][part == 2], o[w][it]);
         });
+    });
+#pragma unroll
+    for (int w = 0; w < CW; ++w)
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int t = c * L + 16 * it + r16;
+        T *to = (T *)p.out + (int64_t)(q0 + t) * p.out_stride + head * p.p + col[w] - r16 + 4 * g;
+        if (!live[w] || t >= len) continue;
+        if (quads) {
+          *(u32x2 *)to = pack_quad<Tag>(o[w][it]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) to[e] = elem<Tag>::st(o[w][it][e]);
+        }
+      }
+    u32x4 tail[2 * NK];   // (comes with B)
+    static_for<2 * NK>([&](auto I) { lds_read128<(decltype(I)::value >> 1) * 128 + (decltype(I)::value & 1) * 16>(tail[decltype(I)::value], at); });
+    static_for<2 * NK>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      lds_wait<0>(tail[i]);
+#pragma unroll
+      for (int w = 0; w < CW; ++w) st[w][i] *= __builtin_bit_cast(f32x4, tail[i]);
     });
     static_for<NK>([&](auto P) {   // two state tiles at a time
       constexpr int i0 = 2 * decltype(P)::value;
-      u32x4 fk[2][2][2], tail[2];
+      u32x4 fk[2][2][2];
+      begin(std::integral_constant<int, NK + 1 + decltype(P)::value>{});
       static_for<2>([&](auto D) {
         constexpr int d = decltype(D)::value;
-        lds_read128<((i0 + d) >> 1) * 128 + ((i0 + d) & 1) * 16>(tail[d], at);
         static_for<2>([&](auto S) {
           constexpr int s = decltype(S)::value;
           lds_read128<(((i0 + d) * 2 + s) * 2) * 1024>(fk[d][s][0], ak);
@@ -444,11 +494,8 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
       });
       static_for<2>([&](auto D) {
         constexpr int d = decltype(D)::value;
-        lds_wait<0>(tail[d]);
         lds_wait<0>(fk[d][0][0], fk[d][0][1]);
         lds_wait<0>(fk[d][1][0], fk[d][1][1]);
-#pragma unroll
-        for (int w = 0; w < CW; ++w) st[w][i0 + d] *= __builtin_bit_cast(f32x4, tail[d]);
       });
 #pragma unroll
       for (int s = 0; s < 2; ++s)
@@ -460,17 +507,6 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
             for (int w = 0; w < CW; ++w)
               st[w][i0 + d] = mfma16x16x32<B16>(fk[d][s][part == 2], part == 1 ? ul[w][s] : uh[w][s], st[w][i0 + d]);
     });
-#pragma unroll
-    for (int w = 0; w < CW; ++w)
-#pragma unroll
-      for (int it = 0; it < 4; ++it)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int t = c * L + 16 * it + 4 * g + e;
-          if (live[w] && t < len) ((T *)p.out)[(int64_t)(q0 + t) * p.out_stride + head * p.p + col[w]] = elem<Tag>::st(o[w][it][e]);
-        }
-    lds_barrier();   // every wave has read phase 2
-    if (more) fetch2(ws);
   }
   if (keep) {
 #pragma unroll

@@ -58,3 +58,40 @@ def test_many_sequences_are_as_each_alone(H, heads, groups, p, n, skew):
     # token by token: the operands are the same 16-bit rows, the sums run in another order; outputs of size sqrt(n) at most, rounded to 8 bits
     scan, _ = run(0, len(spans), slice(0, total), flags=H.MV_DELTA_SCAN)
     assert (out.double() - scan.double()).abs().max() <= 2**-6 * max(1.0, scan.double().abs().max().item())
+
+
+# one decay per channel (csrc/delta_chunk.hip): two column tiles a wave for many heads and sequences, one for few; groups of operands refilled a chunk ahead
+@pytest.mark.parametrize("heads, p, n", [(8, 128, 128), (6, 208, 32), (12, 80, 64), (16, 144, 96), (9, 64, 128), (4, 256, 160), (5, 16, 32)])
+@pytest.mark.parametrize("dtype, skew", [(torch.bfloat16, 0), (torch.bfloat16, 1), (torch.float16, 0)])
+def test_many_sequences_with_channel_decay_are_as_each_alone(H, heads, p, n, dtype, skew):
+    g = torch.Generator(device=DEV).manual_seed(heads * p + n)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    spans = SPANS * (1 + 256 // (heads * len(SPANS) * -(-p // 128)))
+    total, slots = sum(t for t, _ in spans), len(spans) - 1
+    s = H.DeltaShape(heads, heads, p, n, heads * p, heads * (p + n), p, n ** -0.5, True)
+    x, beta, a = (rand(total, c).to(dtype) for c in (s.channels, heads + -heads % 8, heads * n))
+    beta, bias, a_log = beta[:, :heads], rand(heads * n).to(dtype), rand(heads).to(dtype)
+    state = rand(2, slots, heads, n, p) * 0.1
+
+    def run(first, last, rows, flags=0):
+        left, part = state.clone(), spans[first:last]
+        cu = lambda v: ints([0] + torch.tensor(v).cumsum(0).tolist())
+        out = torch.full((rows.stop - rows.start, heads * p + 8 + skew), 7.0, dtype=dtype, device=DEV)
+        at = [i if i < slots else -1 for i in range(first, last)]
+        H.delta_prefill(s, x[rows], beta[rows], a[rows], bias, a_log, left, ints(at), cu([t for t, _ in part]), cu([t + b for t, b in part]),
+                        max(t for t, _ in part), out=out[:, skew:skew + heads * p], flags=flags)
+        assert (out[:, skew + heads * p:] == 7).all() and (out[:, :skew] == 7).all()
+        return out[:, skew:skew + heads * p], left
+
+    out, left = run(0, len(spans), slice(0, total))
+    begin = 0
+    for i, (t, before) in enumerate(spans):
+        if i < len(SPANS) or i >= slots - 1:
+            alone, state_alone = run(i, i + 1, slice(begin, begin + t))
+            assert torch.equal(out[begin:begin + t], alone), f"sequence {i}: {t} tokens behind {before}"
+            if i < slots:
+                assert torch.equal(left[(before + t) & 1, i], state_alone[(before + t) & 1, i])
+        begin += t
+    scan, _ = run(0, len(spans), slice(0, total), flags=H.MV_DELTA_SCAN)   # (bounds as above)
+    assert (out.double() - scan.double()).abs().max() <= 2**-6 * max(1.0, scan.double().abs().max().item())
