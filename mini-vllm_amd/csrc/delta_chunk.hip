@@ -295,7 +295,11 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(De
 // Bound by the chain of a chunk and by the way of its 129 KB through the memory pipeline of a CU.  LDS holds one chunk, in groups in the order of their
 // use: as soon as all waves have used a group, its part of the next chunk is asked for, so that transfers run all the time and none is waited for
 // that was not asked for a chunk before (3 sequences of 4011 tokens and less, 8 heads of 128 x 128: 283 us with two phases, each fetched as a whole
-// while the other was used -> 247).
+// while the other was used, 247 with operands read as they were used -> 224).
+// (reads that a barrier has waited for: the registers count as written here)
+__device__ __forceinline__ void lds_landed(u32x4 &a) { asm volatile("" : "+v"(a)); }
+__device__ __forceinline__ void lds_landed(u32x4 &a, u32x4 &b) { asm volatile("" : "+v"(a), "+v"(b)); }
+
 template <typename Tag, int NK, int CW>
 __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
   typedef typename elem<Tag>::T T;
@@ -390,72 +394,97 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
         if (more) fetch_group(std::integral_constant<int, n - 1>{}, c + 1);
       }
     };
-    begin(std::integral_constant<int, 0>{});
-    // ---- U = U0 - W S, O = Q S
-    f32x4 u[CW][4], o[CW][4];
-#pragma unroll
-    for (int w = 0; w < CW; ++w)
-#pragma unroll
-      for (int it = 0; it < 4; ++it) o[w][it] = f32x4{0.f, 0.f, 0.f, 0.f};
-    static_for<CW>([&](auto W) {
-      constexpr int w = decltype(W)::value;
-      u32x4 raw[4];
-      static_for<4>([&](auto I) { lds_read128<(w * 4 + decltype(I)::value) * 1024>(raw[decltype(I)::value], au); });
-      static_for<4>([&](auto I) {
-        lds_wait<0>(raw[decltype(I)::value]);
-        u[w][decltype(I)::value] = __builtin_bit_cast(f32x4, raw[decltype(I)::value]);
-      });
-    });
-    static_for<NK>([&](auto S) {
+    // The operands of a group are read while the products of the one before run.
+    u32x4 fw[2][4][2], fo[2][4][2], u0[CW][4], fb[kTriangle][2], tail[2 * NK], fk[2][2][2][2];
+    auto read_step = [&](auto S) __attribute__((always_inline)) {
       constexpr int s = decltype(S)::value;
-      u32x4 fw[4][2], fo[4][2], sh[CW], sl[CW];
-      if constexpr (s > 0) begin(S);
       static_for<4>([&](auto I) {
         constexpr int it = decltype(I)::value;
-        lds_read128<((it * NK + s) * 2) * 1024>(fw[it][0], aw);
-        lds_read128<((it * NK + s) * 2 + 1) * 1024>(fw[it][1], aw);
-        lds_read128<((it * NK + s) * 2) * 1024>(fo[it][0], aq);
-        lds_read128<((it * NK + s) * 2 + 1) * 1024>(fo[it][1], aq);
+        static_for<2>([&](auto P) {
+          constexpr int h = decltype(P)::value;
+          lds_read128<((it * NK + s) * 2 + h) * 1024>(fw[s & 1][it][h], aw);
+          lds_read128<((it * NK + s) * 2 + h) * 1024>(fo[s & 1][it][h], aq);
+        });
       });
+    };
+    auto read_pair = [&](auto P) __attribute__((always_inline)) {
+      constexpr int pair = decltype(P)::value;
+      static_for<8>([&](auto I) {
+        constexpr int i = decltype(I)::value;
+        lds_read128<(pair * 8 + i) * 1024>(fk[pair & 1][i >> 2][(i >> 1) & 1][i & 1], ak);
+      });
+    };
+    auto begin_step = [&](auto N) __attribute__((always_inline)) {   // the group behind the one that is about to be multiplied
+      constexpr int n = decltype(N)::value;
+      begin(N);
+      if constexpr (n < NK) {
+        read_step(N);
+      } else if constexpr (n == NK) {
+        static_for<kTriangle>([&](auto M) {
+          constexpr int m = decltype(M)::value, it = m < 2 ? m : m / 2 + 1, s = m < 2 ? 0 : m % 2;
+          lds_read128<((it * 2 + s) * 2) * 1024>(fb[m][0], ab);
+          lds_read128<((it * 2 + s) * 2 + 1) * 1024>(fb[m][1], ab);
+        });
+        static_for<2 * NK>([&](auto I) { lds_read128<(decltype(I)::value >> 1) * 128 + (decltype(I)::value & 1) * 16>(tail[decltype(I)::value], at); });
+      } else {
+        read_pair(std::integral_constant<int, n - NK - 1>{});
+      }
+    };
+    begin(std::integral_constant<int, 0>{});
+    static_for<4 * CW>([&](auto I) { lds_read128<decltype(I)::value * 1024>(u0[decltype(I)::value / 4][decltype(I)::value % 4], au); });
+    read_step(std::integral_constant<int, 0>{});
+    // ---- U = U0 - W S, O = Q S
+    f32x4 u[CW][4], o[CW][4];
+    static_for<NK>([&](auto S) {
+      constexpr int s = decltype(S)::value;
+      u32x4 sh[CW], sl[CW];
 #pragma unroll
       for (int w = 0; w < CW; ++w) split44(st[w][2 * s], st[w][2 * s + 1], sh[w], sl[w]);
+      begin_step(std::integral_constant<int, s + 1>{});   // (its barrier comes behind all reads of this group)
       static_for<4>([&](auto I) {
-        constexpr int it = decltype(I)::value, left = 4 * (3 - it);
-        lds_wait<left>(fw[it][0], fw[it][1]);
-        lds_wait<left>(fo[it][0], fo[it][1]);
+        constexpr int it = decltype(I)::value;
+        lds_landed(fw[s & 1][it][0], fw[s & 1][it][1]);
+        lds_landed(fo[s & 1][it][0], fo[s & 1][it][1]);
       });
+      if constexpr (s == 0)
+        static_for<4 * CW>([&](auto I) {
+          constexpr int w = decltype(I)::value / 4, it = decltype(I)::value % 4;
+          lds_landed(u0[w][it]);
+          u[w][it] = __builtin_bit_cast(f32x4, u0[w][it]), o[w][it] = f32x4{0.f, 0.f, 0.f, 0.f};
+        });
 #pragma unroll
       for (int part = 0; part < 3; ++part)
 #pragma unroll
         for (int it = 0; it < 4; ++it)
 #pragma unroll
           for (int w = 0; w < CW; ++w) {
-            u[w][it] = mfma16x16x32<B16>(fw[it][part == 2], part == 1 ? sl[w] : sh[w], u[w][it]);
-            o[w][it] = mfma16x16x32<B16>(part == 1 ? sl[w] : sh[w], fo[it][part == 2], o[w][it]);
+            u[w][it] = mfma16x16x32<B16>(fw[s & 1][it][part == 2], part == 1 ? sl[w] : sh[w], u[w][it]);
+            o[w][it] = mfma16x16x32<B16>(part == 1 ? sl[w] : sh[w], fo[s & 1][it][part == 2], o[w][it]);
           }
     });
-    begin(std::integral_constant<int, NK>{});
     // ---- O += B U, S = decay S + K U
     u32x4 uh[CW][2], ul[CW][2];
 #pragma unroll
     for (int w = 0; w < CW; ++w)
 #pragma unroll
       for (int s = 0; s < 2; ++s) split44(u[w][2 * s], u[w][2 * s + 1], uh[w][s], ul[w][s]);
+    begin_step(std::integral_constant<int, NK + 1>{});
+    static_for<kTriangle>([&](auto M) { lds_landed(fb[decltype(M)::value][0], fb[decltype(M)::value][1]); });
+    static_for<2 * NK>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      lds_landed(tail[i]);
+#pragma unroll
+      for (int w = 0; w < CW; ++w) st[w][i] *= __builtin_bit_cast(f32x4, tail[i]);
+    });
     static_for<4>([&](auto I) {
       constexpr int it = decltype(I)::value;
-      u32x4 fb[2][2];
-      static_for<it / 2 + 1>([&](auto S) {
-        constexpr int s = decltype(S)::value;
-        lds_read128<((it * 2 + s) * 2) * 1024>(fb[s][0], ab);
-        lds_read128<((it * 2 + s) * 2 + 1) * 1024>(fb[s][1], ab);
-      });
-      static_for<it / 2 + 1>([&](auto S) { lds_wait<0>(fb[decltype(S)::value][0], fb[decltype(S)::value][1]); });
 #pragma unroll
       for (int part = 0; part < 3; ++part)
         static_for<it / 2 + 1>([&](auto S) {
           constexpr int s = decltype(S)::value;
 #pragma unroll
-          for (int w = 0; w < CW; ++w) o[w][it] = mfma16x16x32<B16>(part == 1 ? ul[w][s] : uh[w][s], fb[s][part == 2], o[w][it]);
+          for (int w = 0; w < CW; ++w)
+            o[w][it] = mfma16x16x32<B16>(part == 1 ? ul[w][s] : uh[w][s], fb[triangle(it, s)][part == 2], o[w][it]);
         });
     });
 #pragma unroll
@@ -472,30 +501,14 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
           for (int e = 0; e < 4; ++e) to[e] = elem<Tag>::st(o[w][it][e]);
         }
       }
-    u32x4 tail[2 * NK];   // (comes with B)
-    static_for<2 * NK>([&](auto I) { lds_read128<(decltype(I)::value >> 1) * 128 + (decltype(I)::value & 1) * 16>(tail[decltype(I)::value], at); });
-    static_for<2 * NK>([&](auto I) {
-      constexpr int i = decltype(I)::value;
-      lds_wait<0>(tail[i]);
-#pragma unroll
-      for (int w = 0; w < CW; ++w) st[w][i] *= __builtin_bit_cast(f32x4, tail[i]);
-    });
     static_for<NK>([&](auto P) {   // two state tiles at a time
-      constexpr int i0 = 2 * decltype(P)::value;
-      u32x4 fk[2][2][2];
-      begin(std::integral_constant<int, NK + 1 + decltype(P)::value>{});
+      constexpr int pair = decltype(P)::value, i0 = 2 * pair;
+      if constexpr (pair + 1 < NK) begin_step(std::integral_constant<int, NK + 2 + pair>{});
+      else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       static_for<2>([&](auto D) {
         constexpr int d = decltype(D)::value;
-        static_for<2>([&](auto S) {
-          constexpr int s = decltype(S)::value;
-          lds_read128<(((i0 + d) * 2 + s) * 2) * 1024>(fk[d][s][0], ak);
-          lds_read128<(((i0 + d) * 2 + s) * 2 + 1) * 1024>(fk[d][s][1], ak);
-        });
-      });
-      static_for<2>([&](auto D) {
-        constexpr int d = decltype(D)::value;
-        lds_wait<0>(fk[d][0][0], fk[d][0][1]);
-        lds_wait<0>(fk[d][1][0], fk[d][1][1]);
+        lds_landed(fk[pair & 1][d][0][0], fk[pair & 1][d][0][1]);
+        lds_landed(fk[pair & 1][d][1][0], fk[pair & 1][d][1][1]);
       });
 #pragma unroll
       for (int s = 0; s < 2; ++s)
@@ -505,7 +518,7 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
           for (int d = 0; d < 2; ++d)
 #pragma unroll
             for (int w = 0; w < CW; ++w)
-              st[w][i0 + d] = mfma16x16x32<B16>(fk[d][s][part == 2], part == 1 ? ul[w][s] : uh[w][s], st[w][i0 + d]);
+              st[w][i0 + d] = mfma16x16x32<B16>(fk[pair & 1][d][s][part == 2], part == 1 ? ul[w][s] : uh[w][s], st[w][i0 + d]);
     });
   }
   if (keep) {
