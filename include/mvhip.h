@@ -207,7 +207,7 @@ int mv_rope_paged_decode_ex(const void *q, int64_t q_stride_tok, const void *k, 
  *               sequence i are its first seqlen_k tokens in the cache)
  * Causal mask is bottom-right aligned: query j of sequence i (0-based in its
  * seqlen_q) attends keys 0 .. seqlen_k-seqlen_q+j (attention.py:584-588).
- * flags: MV_PREFILL_SIMPLE routes 16-bit tensors through the vector-ALU kernel (debug aid); 0 = default. */
+ * flags: MV_PREFILL_SIMPLE routes tensors of every dtype through the vector-ALU kernel (debug aid); 0 = default. */
 enum { MV_PREFILL_SIMPLE = 1 };
 int mv_prefill_varlen(const void *q, int64_t q_stride_tok, const void *k,
                       const void *v, int64_t k_stride_tok, int64_t v_stride_tok,

@@ -289,6 +289,10 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(De
   }
 }
 
+// (reads that a barrier has waited for: the registers count as written here)
+__device__ __forceinline__ void lds_landed(u32x4 &a) { asm volatile("" : "+v"(a)); }
+__device__ __forceinline__ void lds_landed(u32x4 &a, u32x4 &b) { asm volatile("" : "+v"(a), "+v"(b)); }
+
 // Workgroup = 4 waves x CW tiles of 16 columns of one head of one sequence; a wave keeps S of its columns in accumulators.  The
 // accumulators are the next product's operands as they are: the rows of S are dealt so that tiles 2 s and 2 s + 1 together hold
 // n = 32 s + 8 g .. + 7 in lane group g.  O is computed transposed (columns by tokens), so that a lane stores four columns of a token.
@@ -296,10 +300,6 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(De
 // use: as soon as all waves have used a group, its part of the next chunk is asked for, so that transfers run all the time and none is waited for
 // that was not asked for a chunk before (3 sequences of 4011 tokens and less, 8 heads of 128 x 128: 283 us with two phases, each fetched as a whole
 // while the other was used, 247 with operands read as they were used -> 224).
-// (reads that a barrier has waited for: the registers count as written here)
-__device__ __forceinline__ void lds_landed(u32x4 &a) { asm volatile("" : "+v"(a)); }
-__device__ __forceinline__ void lds_landed(u32x4 &a, u32x4 &b) { asm volatile("" : "+v"(a), "+v"(b)); }
-
 template <typename Tag, int NK, int CW>
 __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
   typedef typename elem<Tag>::T T;
