@@ -260,6 +260,12 @@ struct AttnMask {
   const void *gate = nullptr;       // a row of [heads * D] per query: the output is multiplied by its sigmoid
   int64_t gate_stride = 0;
 };
+// The sink as the start of a row's maximum (log2 units) and sum, the latter on the lane that counts it.  The maximum starts no lower than without a
+// sink: from -inf (no sink, or one so low that the product overflows) a step whose keys are all masked would take -inf from -inf.
+__device__ __forceinline__ void sink_start(float sink, bool counts, float &m, float &l) {
+  const float s = sink * 1.4426950408889634f;
+  m = fmaxf(s, -1e30f), l = counts ? __builtin_amdgcn_exp2f(s - m) : 0.f;
+}
 // what an output element is multiplied by
 template <typename Tag>
 __device__ __forceinline__ float attn_factor(const AttnMask &m, int64_t row, int col) {

@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
   const float cap = GENERAL ? p.mask.softcap : 0.f, to_cap = cap > 0.f ? p.scale / cap : 0.f, cap_log2 = cap * 1.4426950408889634f;
   float m = -1e30f, l = 0.f;
   int apart = 0;   // a tile with masked keys holds values of V that are not finite
-  if (p.mask.sink) m = ((const float *)p.mask.sink)[head] * 1.4426950408889634f, l = half == 0 && turn == 0 ? 1.f : 0.f;
+  if (p.mask.sink) sink_start(((const float *)p.mask.sink)[head], half == 0 && turn == 0, m, l);
   f32x16 o[DT];
 #pragma unroll
   for (int t = 0; t < DT; ++t)
