@@ -172,10 +172,7 @@ __global__ void __launch_bounds__(NW * 64, 2) prefill_mfma_kernel(PrefillParams 
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
   float m_run = -1e30f, l_run = 0.f;
-  if (WINDOW && p.mask.sink) {   // (a row's two half-waves: the sink counts once)
-    m_run = elem<Tag>::ld(((const T *)p.mask.sink)[head]) * 1.4426950408889634f;
-    l_run = h == 0 ? 1.f : 0.f;
-  }
+  if (WINDOW && p.mask.sink) sink_start(elem<Tag>::ld(((const T *)p.mask.sink)[head]), h == 0, m_run, l_run);   // (a row's two half-waves: it counts once)
   const bool capped = WINDOW && p.mask.softcap > 0.f;
   const float cap_log2 = p.mask.softcap * 1.4426950408889634f, to_cap = capped ? p.scale / p.mask.softcap : 0.f;
   const float scale_log2 = capped ? 1.f : p.scale * 1.4426950408889634f;

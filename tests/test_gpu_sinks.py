@@ -62,7 +62,7 @@ def _pages(ks, vs, block, lost=()):
     return kc.to(DEV), vc.to(DEV), table.to(DEV)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("spans", [[(150, 150), (65, 65)], [(70, 77), (33, 40)]], ids=["whole", "behind 7 keys"])
 @pytest.mark.parametrize("window, chunk", [(0, 0), (9, 0), (40, 0), (0, 32), (0, 50)])
