@@ -142,10 +142,8 @@ __device__ __forceinline__ void paged_decode_body(const DecodeParams &p, const i
   for (int g = 0; g < G; ++g) {
     m[g] = NEG_BIG;
     l[g] = 0.f;
-    if (p.mask.sink && split == 0 && wave == 0 && (WIDE || grp == 0) && ctx > 0) {
-      m[g] = elem<Tag>::ld(((const T *)p.mask.sink)[h0 + (g < g_live ? g : 0)]) * 1.4426950408889634f;
-      l[g] = 1.f;
-    }
+    if (p.mask.sink && split == 0 && wave == 0 && (WIDE || grp == 0) && ctx > 0)
+      sink_start(elem<Tag>::ld(((const T *)p.mask.sink)[h0 + (g < g_live ? g : 0)]), true, m[g], l[g]);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) acc[g][j] = 0.f;
   }

@@ -190,10 +190,8 @@ __global__ void __launch_bounds__(256, KLDS ? 2 : 4) paged_decode_mfma_kernel(De
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = -1e30f, l_run = 0.f;
-  if (p.mask.sink && split == 0 && wave == 0 && ctx > 0) {
-    m_run = elem<Tag>::ld(((const T *)p.mask.sink)[h0 + min(i16, g_live - 1)]) * 1.4426950408889634f;
-    l_run = quad == 0 ? 1.f : 0.f;
-  }
+  if (p.mask.sink && split == 0 && wave == 0 && ctx > 0)
+    sink_start(elem<Tag>::ld(((const T *)p.mask.sink)[h0 + min(i16, g_live - 1)]), quad == 0, m_run, l_run);
   const float softcap = p.mask.softcap, to_cap = softcap > 0.f ? p.scale_log2 * 0.6931471805599453f / softcap : 0.f;
 
   const int32_t *table = p.block_tables + (int64_t)b * p.table_stride;

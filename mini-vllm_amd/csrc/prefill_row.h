@@ -47,7 +47,7 @@ __device__ __forceinline__ void prefill_row(const PrefillParams &p, int seq, int
   const T *qp = (const T *)p.q + (int64_t)tok * p.q_stride + (int64_t)h * D + sub * VEC;
   const u32x4 qraw = *reinterpret_cast<const u32x4 *>(qp);
   float m = -1e30f, l = 0.f, acc[VEC];
-  if (p.mask.sink && grp == 0) m = elem<Tag>::ld(((const T *)p.mask.sink)[h]) * 1.4426950408889634f, l = 1.f;
+  if (p.mask.sink && grp == 0) sink_start(elem<Tag>::ld(((const T *)p.mask.sink)[h]), true, m, l);
 #pragma unroll
   for (int j = 0; j < VEC; ++j) acc[j] = 0.f;
   const float scale_log2 = p.scale * 1.4426950408889634f;

@@ -22,7 +22,7 @@ def _sink(dtype):
 
 def _attend(q, k, v, scale, seen, sink):
     """q [nq, H, D], k / v [nk, KV, D], seen [nq, nk] in fp64."""
-    k, v = (t.double().repeat_interleave(HEADS // KV, 1).transpose(0, 1).contiguous() for t in (k, v))
+    k, v = (t.double().repeat_interleave(q.shape[1] // k.shape[1], 1).transpose(0, 1).contiguous() for t in (k, v))
     s = (torch.matmul(q.double().transpose(0, 1), k.transpose(1, 2)) * scale).masked_fill(~seen, -float("inf"))
     s = torch.cat([s, sink.double()[:, None, None].expand(-1, s.shape[1], 1)], -1)
     return torch.matmul(s.softmax(-1).nan_to_num(0.0)[..., :-1], v).transpose(0, 1)
@@ -39,9 +39,9 @@ def _close(got, want, dtype):
     torch.testing.assert_close(got.double().cpu(), want, rtol=2 * EPS[dtype], atol=2 * EPS[dtype])
 
 
-def _inputs(spans, dtype, d):
+def _inputs(spans, dtype, d, kv=KV):
     g = torch.Generator().manual_seed(d)
-    return ([torch.randn(n[i], h, d, generator=g).to(dtype) for n in spans] for i, h in ((0, HEADS), (1, KV), (1, KV)))
+    return ([torch.randn(n[i], h, d, generator=g).to(dtype) for n in spans] for i, h in ((0, HEADS), (1, kv), (1, kv)))
 
 
 def _cu(ns):
@@ -76,3 +76,36 @@ def test_prompts(H, dtype, d, spans, window, chunk):
     _close(H.prefill_varlen(q, k, v, cq, ck, mq, mk, d ** -0.5, chunk=chunk, mask=mask), want, dtype)
     kc, vc, table = _pages(ks, vs, 64)
     _close(H.prefill_varlen(q, None, None, cq, ck, mq, mk, d ** -0.5, k_cache=kc, v_cache=vc, block_tables=table, chunk=chunk, mask=mask), want, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_the_vector_kernel_and_a_page_that_is_not_there(H, dtype, d):
+    spans, lost = [(150, 150), (33, 97)], 0
+    qs, ks, vs = _inputs(spans, dtype, d)
+    sink, there = _sink(dtype), torch.arange(150) >= 16
+    want = torch.cat([_attend(q, k, v, d ** -0.5, _seen(q.shape[0], k.shape[0], 0, 0) & there[:k.shape[0]], sink) for q, k, v in zip(qs, ks, vs)])
+    kc, vc, table = _pages(ks, vs, 16, [lost])
+    args = (torch.cat(qs).to(DEV), None, None, _cu([a for a, _ in spans]), _cu([b for _, b in spans]), 150, 150, d ** -0.5)
+    for flags in (0, H.MV_PREFILL_SIMPLE):
+        _close(H.prefill_varlen(*args, k_cache=kc, v_cache=vc, block_tables=table, flags=flags, mask=H.AttnMask(sink=sink.to(DEV))), want, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kv, d", [(1, 64), (2, 64), (4, 64), (1, 128), (2, 128), (4, 128), (2, 256)])
+@pytest.mark.parametrize("window, lost", [(0, ()), (5, ()), (90, ()), (0, (0,)), (200, (0, 2))])
+def test_decode(H, dtype, kv, d, window, lost):
+    lens = [1, 64, 65, 130, 200, 517, 1100]
+    if lost:
+        lens = lens[2:]
+    qs, ks, vs = _inputs([(1, n) for n in lens], dtype, d, kv)
+    sink, there = _sink(dtype), torch.ones(max(lens), dtype=torch.bool)
+    for i in lost:
+        there[i * 64:(i + 1) * 64] = False
+    want = torch.cat([_attend(q, k, v, d ** -0.5, _seen(1, k.shape[0], window, 0) & there[:k.shape[0]], sink) for q, k, v in zip(qs, ks, vs)])
+    kc, vc, table = _pages(ks, vs, 64, lost)
+    q, at, mask = torch.cat(qs).to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV), H.AttnMask(window=window, sink=sink.to(DEV))
+    for flags in [0] if dtype == torch.float32 else [0, H.MV_DECODE_VECTOR, H.MV_DECODE_MFMA, H.MV_DECODE_MFMA | H.MV_DECODE_KLDS_ON]:
+        _close(H.paged_decode(q, kc, vc, table, at, d ** -0.5, flags=flags, mask=mask), want, dtype)
+    for s in range(len(lens)):   # alone: the context in many parts
+        _close(H.paged_decode(q[s:s + 1], kc, vc, table[s:s + 1], at[s:s + 1], d ** -0.5, mask=mask), want[s:s + 1], dtype)
