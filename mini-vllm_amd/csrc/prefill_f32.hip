@@ -1,14 +1,21 @@
 // K2 (fp32) — packed varlen causal prefill attention on the fp32 matrix cores (v_mfma_f32_32x32x2_f32: exact products, fp32 sums).
 //
-// Bound by the matrix cores: a flash tile of 32 keys x 32 queries is 64 of these products at head dim 64 (4096 cycles) beside some 800 of
+// Bound by the matrix cores: a flash tile of 32 keys x 32 queries is 64 of these products at head dim 64 (4096 cycles) beside some 1400 of
 // vector arithmetic and 16 KiB of LDS reads.  One workgroup = 64 queries of one head, 32 to a wave, and two waves for the same queries that
 // take the tiles in turn and meet at the end: blocks of rows differ in length, and short chains of tiles even them out (128 queries a workgroup, four
-// waves, each over all tiles: 179 us where this takes 151).  S^T = K Q^T puts a query on a lane (and its partner 32 lanes on), so that the row maximum is one exchange and P, as it lies in the accumulators, is the
-// operand of O^T += V^T P^T: register r of lane half h holds key 8 (r / 4) + 4 h + r % 4, and V is read in that order.  Rows of O^T are
-// dealt so that D / 32 adjacent dims of a key are one read of V and one piece of an output row.
+// waves, each over all tiles: 179 us where two in turn took 151).  S^T = K Q^T puts a query on a lane (and its partner 32 lanes on), so that the row
+// maximum is one exchange and P, as it lies in the accumulators, is the operand of O^T += V^T P^T: register r of lane half h holds key
+// 8 (r / 4) + 4 h + r % 4, and V is read in that order.  Rows of O^T are dealt so that D / 32 adjacent dims of a key are one read of V and one piece of
+// an output row.  The rows of K come into LDS while the products of V run, those of V while the scores do: one set of registers holds them.
+//
+// Sums are short chains of products, added up like a tree, and a score is scaled where its exponent is formed: as far from 64 bits as the vector kernel
+// for rows of a few tokens, nearer for longer ones.  Relative error, this / the vector kernel, 1e-7 (unit normal inputs):
+//   head dim 64:  20 tokens 0.81 / 0.81, 50 0.95 / 0.97, 300 1.18 / 1.32, 1000 1.36 / 1.73     (chains of 16 products: 0.92, 1.10, 1.35, 1.50)
+//   head dim 128: 20 tokens 0.84 / 0.85, 50 0.99 / 1.05, 300 1.20 / 1.59, 1000 1.37 / 2.26     (chains of 32: 1.05, 1.28, 1.73, 2.25)
+// What the tree costs and gives, attention of a layer (us): 6131 tokens in 8 prompts, 12 heads of 64: vector kernel 801, chains of 16 products 137, this
+// 148 (62 TFLOP/s of visible pairs; 4 x 2048: 91); 16 x 1024, 16 heads of 128: 958 -> 771 (89), where the longer chains and rows of K and V
+// side by side left 69 registers in memory; now 4 (paged or masked: 12; head dim 64: 1, 6).
 // The vector kernel (prefill_simple.hip: a wave per query and head, every query reads its keys again) stays for head dim 256.
-// 6131 tokens in 8 prompts, 12 heads of 64: 801 -> 151 us (61 TFLOP/s of visible pairs; 4 x 2048: 89); 16 x 1024, 16 heads of 128: 75 TFLOP/s.
-// Relative error against 64 bits, this / the vector kernel: 50 tokens 1.1e-7 / 0.9e-7, 300 1.3e-7 / 1.3e-7, 1000 1.5e-7 / 1.7e-7, 3000 1.7e-7 / 2.4e-7.
 // Reference: minivllm/models/layers/attention.py:467-504,554-597.
 #include "prefill_row.h"
 
@@ -16,6 +23,7 @@ namespace {
 
 constexpr int BN = 32, WAVES = 4, GROUPS = 2, TURNS = WAVES / GROUPS, BM = GROUPS * 32;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 // first key of its own that a position sees (chunk or window)
 __device__ __forceinline__ int first_key_of(const PrefillParams &p, int pos) {
@@ -26,6 +34,8 @@ __device__ __forceinline__ int first_key_of(const PrefillParams &p, int pos) {
 template <int D, bool GENERAL>
 __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kernel(PrefillParams p) {
   constexpr int CPR = D / 4, PER = TURNS * BN * CPR / (WAVES * 64), DT = D / 32;   // 16-byte pieces of a row, of a thread; tiles of 32 dims
+  // head dim 64 has the registers to add a chain of products up while the next one runs, and to add two chains of keys to each other first
+  constexpr bool BEHIND = D == 64, PAIRS = D == 64;
   constexpr bool QL = D == 64;   // queries in LDS (at head dim 128 they would halve the workgroups of a CU)
   typedef __attribute__((ext_vector_type(DT))) float fdt;
   __shared__ __attribute__((aligned(16))) f32x4 tiles_lds[2][TURNS * BN * CPR];   // K | V
@@ -41,7 +51,7 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
   if (qb >= sq) return;
   const int keep = GENERAL ? p.mask.keep_first : 0;
   const bool paged = GENERAL && p.block_tables != nullptr;
-  auto first_key = [&](int at) { return GENERAL ? first_key_of(p, at) : 0; };
+  auto first_key = [&](int at) __attribute__((always_inline)) { return GENERAL ? first_key_of(p, at) : 0; };
   // positions of the workgroup's, the wave's and the lane's queries (queries behind the end repeat the last one)
   const int shift = sk - sq, last = min(qb + BM, sq) - 1;
   const int wq = min(qb + group * 32, sq - 1), qi = min(qb + group * 32 + col, sq - 1), pos = qi + shift;
@@ -51,7 +61,7 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
   const int end = min(sk, last + shift + 1), to = end > 0 ? (end + BN - 1) / BN : 0;
   const int from = min(first_key(qb + shift) / BN, to), heads = min((min(keep, sk) + BN - 1) / BN, from);
   const int tiles = heads + to - from;
-  auto tile_at = [&](int i) { return i < heads ? i : from + i - heads; };
+  auto tile_at = [&](int i) __attribute__((always_inline)) { return i < heads ? i : from + i - heads; };
 
   const float *qp = (const float *)p.q + (int64_t)(q0 + qi) * p.q_stride + (int64_t)head * D + half * (D / 2);
   f32x4 q[QL ? 1 : CPR / 2];   // dims half * D / 2 .. of the lane's query
@@ -63,57 +73,65 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
     else q[j] = w;
   }
 
-  f32x4 kr[PER], vr[PER];
-  int ok[PER];
-  // where piece n of this thread lies in K (V); false: no page
-  auto piece = [&](int i0, int n, const void *rows, const void *cache, int64_t stride, const float *&at) {
-    const int i = tid + n * WAVES * 64, row = i / CPR, c = i % CPR;
-    const int key = min(tile_at(min(i0 + row / BN, tiles - 1)) * BN + row % BN, sk - 1);   // (clamped rows are masked)
-    if (!paged) {
-      at = (const float *)rows + (int64_t)(k0 + key) * stride + (int64_t)hkv * D + 4 * c;
-      return true;
-    }
-    const int bi = key / p.block_size, blk = bi < p.table_width ? p.block_tables[(int64_t)seq * p.table_stride + bi] : -1;
-    const bool is = blk >= 0 && blk < p.num_blocks;
-    at = (const float *)cache + (((is ? (int64_t)blk * p.block_size : 0) + (key - bi * p.block_size)) * p.n_kv_heads + hkv) * D + 4 * c;
-    return is;
+  f32x4 raw[PER];   // rows on their way to LDS: K during the products of V, V during the scores
+  unsigned pages = 0;   // bit n: piece n has one
+  // (addresses are worked out at each tile: kept, they take the registers of a chain of products)
+  auto anew = [](unsigned x) __attribute__((always_inline)) {
+    asm volatile("" : "+v"(x));
+    return x;
   };
-  auto fetch_k = [&](int i0) {
+  constexpr int STEP = WAVES * 64 / CPR;   // rows from one piece of a thread to its next
+  auto fetch = [&](int i0, const void *rows, const void *cache, int64_t stride) __attribute__((always_inline)) {
+    const unsigned here = anew(tid);
+    const int row = here / CPR, c = here % CPR;
 #pragma unroll
     for (int n = 0; n < PER; ++n) {
-      const float *at;
-      ok[n] = piece(i0, n, p.k, p.k_cache, p.k_stride, at);
-      kr[n] = *(const f32x4 *)at;
-      if (paged && !ok[n]) kr[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int from = tile_at(min(i0 + n * STEP / BN, tiles - 1)) * BN;
+      const int in = min(row + n * STEP % BN, sk - 1 - from);   // (clamped rows are masked)
+      if (!paged) {
+        raw[n] = *(const f32x4 *)((const float *)rows + (int64_t)(k0 + from) * stride + (int64_t)hkv * D + (in * stride + 4 * c));
+      } else {
+        const int key = from + in, bi = key / p.block_size, blk = bi < p.table_width ? p.block_tables[(int64_t)seq * p.table_stride + bi] : -1;
+        const bool is = blk >= 0 && blk < p.num_blocks;
+        const int64_t at = (is ? (int64_t)blk * p.block_size : 0) + (key - bi * p.block_size);
+        pages = n == 0 ? is : pages | (unsigned)is << n;
+        raw[n] = *(const f32x4 *)((const float *)cache + (at * p.n_kv_heads + hkv) * D + 4 * c);
+      }
+    }
+    if (paged) {
+#pragma unroll
+      for (int n = 0; n < PER; ++n)
+        if (!(pages >> n & 1)) raw[n] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
   };
-  auto fetch_v = [&](int i0) {
+  auto fetch_k = [&](int i0) __attribute__((always_inline)) { fetch(i0, p.k, p.k_cache, p.k_stride); };
+  auto fetch_v = [&](int i0) __attribute__((always_inline)) { fetch(i0, p.v, p.v_cache, p.v_stride); };
+  auto put_k = [&]() __attribute__((always_inline)) {   // in an order that spreads the rows over the banks
+    const unsigned here = anew(tid);
+    const int row = here / CPR, c = here % CPR;
 #pragma unroll
     for (int n = 0; n < PER; ++n) {
-      const float *at;
-      const bool is = piece(i0, n, p.v, p.v_cache, p.v_stride, at);
-      vr[n] = *(const f32x4 *)at;
-      if (paged && !is) vr[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+      ks[(row + n * STEP) * CPR + (c ^ ((row + n * STEP) & 15))] = raw[n];
+      if (paged && c == 0) there[n * STEP / BN][row + n * STEP % BN] = pages >> n & 1;
     }
   };
-  auto put = [&]() {   // K's pieces in an order that spreads the rows over the banks
-#pragma unroll
-    for (int n = 0; n < PER; ++n) {
-      const int i = tid + n * WAVES * 64, row = i / CPR, c = i % CPR;
-      ks[row * CPR + (c ^ (row & 15))] = kr[n], vs[i] = vr[n];
-      if (paged && c == 0) there[row / BN][row % BN] = ok[n];
-    }
+  auto put_v = [&]() __attribute__((always_inline)) {
     float z = 0.f;
 #pragma unroll
-    for (int n = 0; n < PER; ++n)
+    for (int n = 0; n < PER; ++n) {
+      vs[tid + n * WAVES * 64] = raw[n];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) z = fmaf(vr[n][e], 0.f, z);
+      for (int e = 0; e < 4; ++e) z = fmaf(raw[n][e], 0.f, z);
+    }
     const int any = __any(z != 0.f) ? 1 : 0;   // (NaN)
     if (lane == 0) wild[wave] = any;
   };
 
   const float scale_log2 = p.scale * 1.4426950408889634f;
   const float cap = GENERAL ? p.mask.softcap : 0.f, to_cap = cap > 0.f ? p.scale / cap : 0.f, cap_log2 = cap * 1.4426950408889634f;
+  // scores are multiplied by `mul` where their exponent is formed, without a rounding between
+  const bool late = !(cap > 0.f) && scale_log2 > 0.f;
+  const float mul = late ? scale_log2 : 1.f;
   float m = -1e30f, l = 0.f;
   int apart = 0;   // a tile with masked keys holds values of V that are not finite
   if (p.mask.sink) sink_start(((const float *)p.mask.sink)[head], half == 0 && turn == 0, m, l);
@@ -125,57 +143,80 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
 
   if (tiles > 0) {
     fetch_k(0);
+    put_k();
     fetch_v(0);
   }
   for (int i0 = 0; i0 < tiles; i0 += TURNS) {
-    __syncthreads();   // every wave is done with the tiles before
-    put();
-    __syncthreads();
-    if (i0 + TURNS < tiles) fetch_k(i0 + TURNS);
+    __syncthreads();   // K is there; every wave is done with V of the tiles before
+    put_v();
+    const bool more = i0 + TURNS < tiles;
+    if (more) fetch_k(i0 + TURNS);
     const int tile = tile_at(min(i0 + turn, tiles - 1)), key0 = tile * BN;
     const f32x4 *kt = ks + turn * BN * CPR, *vt = vs + turn * BN * CPR;
     // of the wave's queries sees a key of it
     const bool some = i0 + turn < tiles && key0 <= wave_hi && (key0 + BN > first_key(wave_lo) || key0 < keep);
+    bool masked = false;
     f32x16 s;
     if (some) {
-      // a score's D products in four chains: one alone has twice the rounding error of the vector kernel's, whose lanes meet in a tree
+      // A score's D products in chains of eight, four chains to a group, (0 + 1) + (2 + 3)
+      const int swizzle = anew(col & 15);
+      f32x16 group, pair, before;
+      auto join = [&](int c, const f32x16 &x) __attribute__((always_inline)) {
+        if (c % 4 == 0) group = x;
+        else if (c % 4 == 1) group += x;
+        else if (c % 4 == 2) pair = x;
+        else group += pair + x;
+        if (c % 4 == 3) s = c == 3 ? group : s + group;
+        // (here, not where the sum is used: a chain's registers are free)
+        if (c % 4 == 2) asm volatile("" : "+v"(pair));
+        else asm volatile("" : "+v"(group));
+        if (c % 4 == 3) asm volatile("" : "+v"(s));
+      };
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (int c = 0; c < CPR / 2; ++c) {
+        const int at = (half * (CPR / 2) + c) ^ swizzle;
+        const f32x4 k = kt[col * CPR + at], w = QL ? qt[at] : q[QL ? 0 : c];
         f32x16 chain = {};
 #pragma unroll
-        for (int j = c * CPR / 8; j < (c + 1) * CPR / 8; ++j) {
-          const int at = (half * (CPR / 2) + j) ^ (col & 15);
-          const f32x4 k = kt[col * CPR + at], w = QL ? qt[at] : q[QL ? 0 : j];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) chain = __builtin_amdgcn_mfma_f32_32x32x2f32(k[e], w[e], chain, 0, 0, 0);
-        }
-        if (c == 0) s = chain;
-        else s += chain;
-        __builtin_amdgcn_sched_barrier(0);   // (one chain's registers at a time)
+        for (int e = 0; e < 4; ++e) chain = __builtin_amdgcn_mfma_f32_32x32x2f32(k[e], w[e], chain, 0, 0, 0);
+        if (!BEHIND) join(c, chain);
+        else if (c > 0) join(c - 1, before);
+        before = chain;
       }
-    }
-    if (i0 + TURNS < tiles) fetch_v(i0 + TURNS);   // (not before: the registers of a chain are free now)
-    if (some) {
+      if (BEHIND) join(CPR / 2 - 1, before);
       if (cap > 0.f) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] = capped_log2<f32_tag>(s[r], to_cap, cap_log2);
-      } else {
+      } else if (!late) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] *= scale_log2;
       }
-      if (paged || key0 + BN - 1 > wave_lo || key0 + BN > sk || key0 < first_key(wave_hi)) {
+      masked = paged || key0 + BN - 1 > wave_lo || key0 + BN > sk || key0 < first_key(wave_hi);
+      if (masked) {   // register r of lane half h holds key 8 (r / 4) + 4 h + r % 4 of the tile
+        const int upto = min(pos, sk - 1) - key0 - 4 * half, since = first - key0 - 4 * half, kept = keep - key0 - 4 * half;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int j = 8 * (r >> 2) + 4 * half + (r & 3), key = key0 + j;
-          const bool seen = key <= pos && key < sk && (!GENERAL || key >= first || key < keep) && (!paged || there[turn][j]);
-          s[r] = seen ? s[r] : -INFINITY;
+        for (int c = 0; c < 4; ++c) {
+          i32x4 is = {1, 1, 1, 1};
+          if (paged) is = *(const i32x4 *)&there[turn][8 * c + 4 * half];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = 8 * c + e;
+            s[4 * c + e] = j <= upto && (!GENERAL || j >= since || j < kept) && is[e] ? s[4 * c + e] : -INFINITY;
+          }
         }
-        apart |= wild[0] | wild[1] | wild[2] | wild[3];
       }
+    }
+    __syncthreads();   // V is there; every wave is done with K
+    if (more) {
+      put_k();
+      fetch_v(i0 + TURNS);
+    }
+    if (some) {
+      if (masked) apart |= wild[0] | wild[1] | wild[2] | wild[3];
       float mx = s[0];
 #pragma unroll
       for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
-      mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)));
+      mx = fmaxf(m, fmaxf(mx, __shfl_xor(mx, 32, 64)) * mul);
       if (__any(mx > m)) {
         const float alpha = __builtin_amdgcn_exp2f(m - mx);
         l *= alpha;
@@ -186,25 +227,40 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
         m = mx;
       }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(s[r] - m);
+      for (int r = 0; r < 16; ++r) s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], mul, -m));
       l += (((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))) + (((s[8] + s[9]) + (s[10] + s[11])) + ((s[12] + s[13]) + (s[14] + s[15])));
-      // Head dim 64: a tile's 32 keys in two chains, apart from the sums so far: fewer roundings on a path, as with the scores.  (At 128 the
-      // registers are not there; its rows have fewer roundings behind the scores than ahead of them.)
+      // the keys apart from the sums so far, in chains of eight; of four where rows may have few
+      auto values = [&](auto N) __attribute__((always_inline)) {
+        constexpr int M = decltype(N)::value;
+        f32x16 before, part[DT];
+        auto join = [&](int i, const f32x16 &x) __attribute__((always_inline)) {
+          const int c = i / DT, t = i % DT;
+          if (PAIRS && M == 2 && c % 2 == 0) {
+            part[t] = x;
+            return;
+          }
+          o[t] += PAIRS && M == 2 ? part[t] + x : x;
+          asm volatile("" : "+v"(o[t]));
+        };
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        f32x16 sums[DT];
+        for (int c = 0; c < 16 / M; ++c) {
+          fdt v[M];
 #pragma unroll
-        for (int t = 0; t < DT; ++t) sums[t] = D == 64 ? f32x16{} : o[t];
+          for (int r = 0; r < M; ++r) v[r] = ((const fdt *)vt)[(8 * ((c * M + r) >> 2) + 4 * half + ((c * M + r) & 3)) * 32 + col];
 #pragma unroll
-        for (int r = 8 * c; r < 8 * c + 8; ++r) {
-          const fdt v = ((const fdt *)vt)[(8 * (r >> 2) + 4 * half + (r & 3)) * 32 + col];
+          for (int t = 0; t < DT; ++t) {
+            f32x16 sums = {};
 #pragma unroll
-          for (int t = 0; t < DT; ++t) sums[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[t], s[r], sums[t], 0, 0, 0);
+            for (int r = 0; r < M; ++r) sums = __builtin_amdgcn_mfma_f32_32x32x2f32(v[r][t], s[M * c + r], sums, 0, 0, 0);
+            if (!BEHIND) join(c * DT + t, sums);
+            else if (c + t > 0) join(c * DT + t - 1, before);
+            before = sums;
+          }
         }
-#pragma unroll
-        for (int t = 0; t < DT; ++t) o[t] = D == 64 ? o[t] + sums[t] : sums[t];
-        if constexpr (D == 64) __builtin_amdgcn_sched_barrier(0);
-      }
+        if (BEHIND) join(16 / M * DT - 1, before);
+      };
+      if (masked) values(std::integral_constant<int, 2>{});
+      else values(std::integral_constant<int, 4>{});
     }
   }
   // the second wave of each query group hands its part over
