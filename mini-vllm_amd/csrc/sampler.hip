@@ -335,12 +335,46 @@ struct RowOnChip {
   static __device__ __forceinline__ short least_of_key(uint32_t key) { return key >= 0x8000u ? (short)(key - 0x8000u) : kAll; }
 };
 
+// Largest element of a thread's vectors (those of RowOnChip) and the first index that has it; -inf and no index if none is larger.  One comparison
+// a vector; four vectors in flight (7, 10 or 19: as fast or slower).
+template <typename Tag>
+__device__ __forceinline__ int greedy_pass(const uint16_t *row, int nvec, float &best) {
+  constexpr int U = 4;
+  u32x4 top = {0u, 0u, 0u, 0u};
+  int at = -1;
+  for (int c0 = 0; c0 < nvec; c0 += kThreads * U) {
+    u32x4 raw[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) raw[u] = *reinterpret_cast<const u32x4 *>(row + (int64_t)min(c0 + u * kThreads + (int)threadIdx.x, nvec - 1) * 8);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (c0 + u * kThreads >= nvec) break;
+      float f[8];
+      unpack8<Tag>(raw[u], f);
+      float m = f[0];
+#pragma unroll
+      for (int j = 1; j < 8; ++j) m = fmaxf(m, f[j]);
+      const int c = c0 + u * kThreads + (int)threadIdx.x;
+      if (c < nvec && m > best) best = m, at = c, top = raw[u];
+    }
+  }
+  if (at < 0) return 0x7fffffff;
+  float f[8];
+  unpack8<Tag>(top, f);
+  int first = 0;
+#pragma unroll
+  for (int j = 7; j >= 0; --j) first = f[j] == best ? j : first;
+  return at * 8 + first;
+}
+
 // NR >= 0: the row stays on the CU (16-bit logits in whole, aligned vectors, no mask asked for; RowOnChip); -1: every pass reads memory.
 // A row is one pass for the maximum, one for the histogram of a filter, one for ties, one for the masses; 256 rows of 151 936 logits are one
 // workgroup a CU, 304 KB each: more than the LDS and, beside what the passes need, more than the registers, but not more than half in each.  Kept
 // there, the passes behind the first read no memory, and those behind a filter skip what cannot be kept.
-// 256 rows of 151 936 bf16 logits, us: greedy 19 -> 21, plain 59 -> 33, top-k 40 91 -> 41, top-p 0.9 83 -> 59, min-p 56 -> 30; one row 16 -> 12, 52 -> 22,
-// 81 -> 30, 73 -> 47, 49 -> 20.  What is left is vector arithmetic: an exponential and four instructions an element where every weight counts.
+// A greedy row is one pass and stays nowhere (greedy_pass).
+// 151 936 bf16 logits, us, memory in every pass -> now; 256 rows: greedy 18.9 -> 13.9, plain 58 -> 30, top-k 40 89 -> 37, top-p 0.9 81 -> 55, min-p
+// 55 -> 27; one row: 15.5 -> 6.3, 51 -> 20, 81 -> 28, 73 -> 45, 49 -> 18 (a greedy row brought to its CU like the others: 18.4, 9.8).  What is left is
+// vector arithmetic: an exponential and four instructions an element where every weight counts.
 template <typename Tag, int NR>
 __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   typedef typename elem<Tag>::T T;
@@ -365,8 +399,12 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   int best_i = 0x7fffffff;
   Row chip;
   if constexpr (CHIP) {
-    chip.load(row, V / 8, row_lds);
-    best = chip.largest();
+    if (temp == 0.0f) {   // one pass is all of it: nothing is kept but the vector that has the thread's maximum
+      best_i = greedy_pass<Tag>(row, V / 8, best);
+    } else {
+      chip.load(row, V / 8, row_lds);
+      best = chip.largest();
+    }
   } else {
     row_foreach<Tag, U>(row, V, vec_ok, [&](int i, T raw, bool ok) {
       const float x = elem<Tag>::ld(raw);
@@ -376,10 +414,9 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   const float xmax = block_max(best, sh);
   if (temp == 0.0f) {  // greedy (argmax, not multinomial over softmax(l/1e-8))
     if constexpr (CHIP) {
-      const short least = xmax > 0.f ? Row::least_of_key(make_key<Tag>(elem<Tag>::st(xmax))) : Row::kAll;
-      if (best == xmax)
-        chip.foreach_from(least, [&](int i, T raw) {
-          if (elem<Tag>::ld(raw) == xmax) best_i = min(best_i, i);
+      if (xmax == -INFINITY)   // (no element is above it: the first that is not NaN)
+        row_foreach<Tag, 1>(row, V, vec_ok, [&](int i, T raw, bool ok) {
+          if (ok && elem<Tag>::ld(raw) == xmax) best_i = min(best_i, i);
         });
     }
     int cand = (best == xmax) ? best_i : 0x7fffffff;

@@ -63,3 +63,24 @@ def test_rows_with_nan_end_and_name_a_word(H):
     logits[:, 123] = -float("nan")
     _both(H, logits.bfloat16())
     _both(H, torch.full_like(logits, float("nan")).bfloat16())
+
+
+@pytest.mark.parametrize("vocab", [8, 4096, 32_000, 50_272, 19 * 8192, 19 * 8192 + 8, 4099])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_greedy_rows_name_the_first_of_the_largest(H, vocab, dtype):
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    x = torch.empty(40, vocab, device=DEV).normal_(0, 3, generator=g).round()            # many ties
+    x[1], x[2, vocab // 2:] = -float("inf"), -float("inf")
+    x[3], x[3, -1], x[4] = float("nan"), -float("inf"), float("nan")
+    x[5, ::3], x[6, 1::2], x[7] = float("nan"), float("inf"), -x[7].abs() * 1e-30 + 0.0  # (the last: zeros of both signs, tiny values)
+    x[8, :7], x[9] = -float("inf"), -x[9].abs() - 1
+    x = x.to(dtype)
+    t = torch.zeros(40, device=DEV)
+    t[30:] = 0.7                                                                         # beside sampled rows
+    got, stats = H.sample(x, t, None, None, None, return_stats=True)
+    top = x.double().nan_to_num(-float("inf"), float("inf"), -float("inf")).amax(1, keepdim=True)
+    is_top = x.double() == top
+    want = torch.where(is_top.any(1), is_top.double().argmax(1), 0)
+    assert torch.equal(got[:30], want[:30])
+    assert torch.equal(stats[:30, 0].double(), top[:30, 0]) and (stats[:30, 1] == 1).all()
+    assert torch.equal(got, H.sample(x, t, None, None, None, return_mask=True)[0])
