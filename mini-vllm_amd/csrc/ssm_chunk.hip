@@ -331,6 +331,7 @@ inline int column_tiles(int p) {
 inline int pick_segment(int n_seqs, int total_q, int max_q, int heads, int p) {
   const int64_t per_chunk = (int64_t)heads * (p / 16 / column_tiles(p)), longest = (max_q + L - 1) / L;
   if (per_chunk * n_seqs >= 512) return 0;
+  if (total_q < max_q) return 0;   // (no bound of the rows, from which the segments are counted)
   const int64_t chunks = (total_q + L - 1) / L, seg = std::max<int64_t>({4, (longest + 7) / 8, (chunks * per_chunk + 1023) / 1024});
   return longest * 3 > seg * 4 ? (int)seg : 0;
 }

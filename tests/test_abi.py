@@ -39,6 +39,18 @@ def test_workspace_size_queries_are_host_only():
     assert hip_ops.paged_decode_workspace_bytes(1, 16, 8, 96, 64, 64) == 256         # unsupported D: nothing
 
 
+def test_when_state_space_prompts_are_cut():
+    """Scratch memory is asked for where sequences are cut into segments: six chunks of 64 tokens and more, fewer than 512 workgroups."""
+    from minivllm_amd import hip_ops
+
+    need = lambda seqs, rows, longest, heads=4, dtype=hip_ops.MV_BF16: hip_ops.lib().mv_ssm_prefill_workspace_bytes(seqs, rows, longest, heads, 64, 128, dtype)
+    assert need(1, 320, 320) == 0 < need(1, 321, 321)
+    assert need(7, 7000, 1000, heads=64) > 0 == need(8, 8000, 1000, heads=64)
+    assert need(1, 4000, 4000, dtype=hip_ops.MV_F32) == 0
+    for rows in (0, -1, 999):          # fewer rows than the longest sequence: no bound that segments could be counted from
+        assert need(1, rows, 1000) == 0
+
+
 def test_struct_layouts_of_the_binding_match_the_library():
     """mv_decode_layers_persistent takes two structs by pointer: the ctypes declarations must have the library's layout."""
     from minivllm_amd import hip_ops
