@@ -542,16 +542,19 @@ int launch(const DeltaPrep &q, hipStream_t stream) {
   hipLaunchKernelGGL((delta_prepare_kernel<Tag, NK>), dim3((unsigned)chunk_slots(a.n_seqs, a.total_q), a.heads),
                      dim3(kPrepareWaves * 64), L * RS * 4 + L * KS * 2 + QB + (3 + kPrepareWaves) * L * 4, stream, q);
   MV_LAUNCH_CHECK();
-  // two column tiles a wave share every operand read, where that still leaves a workgroup per CU
+  // two column tiles a wave share every operand read, where that still leaves a workgroup per CU and LDS holds their chunk (up to 128 channels)
   const int tiles = a.p / 16, wide = (tiles + 7) / 8;
-  if (tiles > 4 && (int64_t)wide * a.heads * a.n_seqs >= 256 && 24 * NK + 32 + 17 <= 160) {
-    if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 2>>()) return rc;
-    hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 2>), dim3(wide, a.heads, a.n_seqs), dim3(256), (24 * NK + 32 + 17) * 1024, stream, q);
-  } else {
-    if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 1>>()) return rc;
-    hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 1>), dim3((tiles + 3) / 4, a.heads, a.n_seqs), dim3(256), (24 * NK + 16 + 17) * 1024,
-                       stream, q);
+  constexpr auto lds = [](int columns) { return (24 * NK + 16 * columns + 17) * 1024; };
+  if constexpr (lds(2) <= 160 * 1024) {
+    if (tiles > 4 && (int64_t)wide * a.heads * a.n_seqs >= 256) {
+      if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 2>>()) return rc;
+      hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 2>), dim3(wide, a.heads, a.n_seqs), dim3(256), lds(2), stream, q);
+      MV_LAUNCH_CHECK();
+      return MV_OK;
+    }
   }
+  if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 1>>()) return rc;
+  hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 1>), dim3((tiles + 3) / 4, a.heads, a.n_seqs), dim3(256), lds(1), stream, q);
   MV_LAUNCH_CHECK();
   return MV_OK;
 }

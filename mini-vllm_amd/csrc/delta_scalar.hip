@@ -424,16 +424,20 @@ int launch(const DeltaPrep &q, hipStream_t stream) {
   const MvDeltaArgs &a = q.a;
   hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK>), dim3((unsigned)chunk_slots(a.n_seqs, a.total_q), a.heads), dim3(256), 0, stream, q);
   MV_LAUNCH_CHECK();
-  // Eight waves where workgroups of four would be more than the CUs, of which each holds one
+  // Eight waves where workgroups of four would be more than the CUs, of which each holds one, and LDS holds their chunk (up to 128 channels: at
+  // 160 four waves of one tile it is, 16 heads and 16 sequences of 1000 tokens 201 us, where four waves of two tiles took 211)
   const int tiles = a.p / 16, wide = (tiles + 7) / 8, narrow = (tiles + 3) / 4;
-  const auto lds = [](int waves) { return 2 * (8 * NK + 2 * waves + kScalarTotal) * 1024; };
-  if (tiles > 4 && lds(8) <= 160 * 1024 && (int64_t)narrow * a.heads * a.n_seqs > 256) {
-    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 8>>()) return rc;
-    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 8>), dim3(wide, a.heads, a.n_seqs), dim3(512), lds(8), stream, q);
-  } else {
-    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 4>>()) return rc;
-    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 4>), dim3(narrow, a.heads, a.n_seqs), dim3(256), lds(4), stream, q);
+  constexpr auto lds = [](int waves) { return 2 * (8 * NK + 2 * waves + kScalarTotal) * 1024; };
+  if constexpr (lds(8) <= 160 * 1024) {
+    if (tiles > 4 && (int64_t)narrow * a.heads * a.n_seqs > 256) {
+      if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 8>>()) return rc;
+      hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 8>), dim3(wide, a.heads, a.n_seqs), dim3(512), lds(8), stream, q);
+      MV_LAUNCH_CHECK();
+      return MV_OK;
+    }
   }
+  if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 4>>()) return rc;
+  hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 4>), dim3(narrow, a.heads, a.n_seqs), dim3(256), lds(4), stream, q);
   MV_LAUNCH_CHECK();
   return MV_OK;
 }
