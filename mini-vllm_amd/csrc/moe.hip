@@ -128,15 +128,16 @@ __device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c,
 }
 
 // A workgroup: TT tiles of 16 tokens.  Latencies: the inputs are split over the waves, every operand of U steps is asked for before the first is
-// used (16 waves: all of 2048 inputs at once), and a token's choice stays in one wave's registers.  Few tokens: 16 waves share a tile, so that a wave
-// chooses for one token; many: 8 waves and two tiles, which read the weights once.  34 outputs of 2048 inputs: 24 tokens 18.8 -> 11.0 us, 9001
-// 37 -> 31 us.
+// used (16 waves: all of 2048 inputs at once), and the choice of a token with up to 64 outputs stays in one wave's registers.  Few tokens: 16 waves
+// share a tile, so that a wave chooses for one token; many: eight waves (mv_moe_route).  34 outputs of 2048 inputs, alone: 24 tokens 18.8 -> 11.0 us; one
+// launch behind the other, eight waves with a step's loads at a time -> now: 24 tokens 14.7 -> 9.7, 9001 24 -> 16; 128 outputs of 512 inputs: one token
+// 12.7 -> 12.8, 24 20.5 -> 15.4, 20000 53 -> 51; fp32, 34 outputs of 2048 inputs, 4400 tokens: 392 -> 131.
 template <typename Tag, int WAVES, int TT>
 __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
   typedef typename elem<Tag>::T T;
-  constexpr int TOKENS = 16 * TT, U = TT == 1 ? 4 : 2;
+  constexpr int TOKENS = 16 * TT, U = WAVES == 16 ? 4 : 2;
   extern __shared__ float lds[];   // logits [TOKENS][outputs] | scratch [TOKENS][outputs] | (16-bit) partial tiles
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m0 = blockIdx.x * TOKENS, R = p.outputs;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m0 = blockIdx.x * TOKENS, R = p.outputs;
   float *sc = lds, *ch = sc + TOKENS * R;
   const T *x = (const T *)p.x, *w = (const T *)p.w;
   const float correction = p.correction ? elem<Tag>::ld(((const T *)p.correction)[min(lane, R - 1)]) : 0.f;   // (asked for ahead of the products)
@@ -146,7 +147,15 @@ __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
       const int t = i / R, r = i - t * R;
       const T *xr = x + (int64_t)min(m0 + t, p.rows - 1) * p.x_stride, *wr = w + (int64_t)r * p.k;
       float z = 0.f;
-      for (int k = l; k < p.k; k += 16) z = fmaf(xr[k], wr[k], z);
+      int k = l;
+      for (; k < p.k - 112; k += 128) {   // (eight steps' loads in flight, one sum)
+        float a[8], b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a[u] = xr[k + 16 * u], b[u] = wr[k + 16 * u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) z = fmaf(a[u], b[u], z);
+      }
+      for (; k < p.k; k += 16) z = fmaf(xr[k], wr[k], z);
       z = row16_sum(z);
       if (l == 0) sc[i] = z;
     }
@@ -168,13 +177,14 @@ __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
         for (int s = steps * wave / WAVES; s < hi; s += U) {
           u32x4 a[U][NT], b[U][TT];
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int at = min(s + u, hi - 1) * 32;
+          for (int u = 0; u < U; ++u)
+            if (s + u < hi) {   // (of the wave: few inputs are not asked for several times)
+              const int at = (s + u) * 32;
 #pragma unroll
-            for (int t = 0; t < TT; ++t) b[u][t] = *(const u32x4 *)(xr[t] + at);
+              for (int t = 0; t < TT; ++t) b[u][t] = *(const u32x4 *)(xr[t] + at);
 #pragma unroll
-            for (int j = 0; j < NT; ++j) a[u][j] = *(const u32x4 *)(wr[j] + at);
-          }
+              for (int j = 0; j < NT; ++j) a[u][j] = *(const u32x4 *)(wr[j] + at);
+            }
 #pragma unroll
           for (int u = 0; u < U; ++u)
             if (s + u < hi) {
@@ -668,10 +678,19 @@ extern "C" int mv_moe_route(const void *x, int64_t x_stride, const void *w, cons
     return MV_E_SHAPE;
   if (!mv_aligned16(x) || !mv_aligned16(w) || x_stride % (dtype == MV_F32 ? 4 : 8)) return MV_E_ALIGN;
   const RouteParams p{x, w, correction, ids, weights, x_stride, rows, k, outputs, top, groups, keep, flags, scale};
-  // A tile of 16 tokens to a workgroup while that fills no more than the chip; and more than 256 outputs,
-  // of which the LDS does not hold the scores of two tiles
+  // A tile of 16 tokens over 16 waves while that fills no more than the chip, and for more than 256 outputs, whose scores leave room for one
+  // workgroup a CU.  More tokens: eight waves, so that the workgroups of a CU choose beside each other (20000 tokens of 512 inputs, 128 outputs: 51 us,
+  // 16 waves 74, eight waves of two tiles 105).  Two tiles, which read the weights once, where those are long: 34 outputs of 4096 inputs, 4400 tokens
+  // 23 us, one tile 28.  More than 64 outputs leave two tiles one workgroup a CU, so its rounds over the chip have to be full: 128 outputs of 4096
+  // inputs, 4400 tokens 73 us, 12000 145; one tile 87 and 122.
   MV_DISPATCH_DTYPE(dtype, {
-    if (int rc = rows <= 16 * 256 || outputs > 256 ? launch_route<Tag, 16, 1>(p, (hipStream_t)stream) : launch_route<Tag, 8, 2>(p, (hipStream_t)stream)) return rc;
+    const hipStream_t st = (hipStream_t)stream;
+    const bool full = k > 2048 && (rows <= 8192 || (k >= 4096 && (rows - 1) % 8192 >= 4096));
+    int rc;
+    if (rows <= 16 * 256 || outputs > 256) rc = launch_route<Tag, 16, 1>(p, st);
+    else if (dtype != MV_F32 && (outputs <= 64 ? k >= 2048 : full)) rc = launch_route<Tag, 8, 2>(p, st);
+    else rc = launch_route<Tag, 8, 1>(p, st);
+    if (rc) return rc;
   });
   MV_LAUNCH_CHECK();
   return MV_OK;

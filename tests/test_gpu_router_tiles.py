@@ -1,4 +1,5 @@
-"""The router's workgroups (csrc/moe.hip): one tile of 16 tokens or two, choices out of registers (up to 64 outputs in up to 8 groups) or LDS."""
+"""The router's workgroups (csrc/moe.hip): one tile of 16 tokens over 16 or eight waves, or two tiles (long rows of inputs); choices out of registers
+(up to 64 outputs in up to 8 groups) or LDS."""
 import pytest
 import torch
 
@@ -26,7 +27,7 @@ def _choose(scores, corr, top, groups, keep):
 # rows around a tile, two tiles and the line between the two workgroups; steps of K that the waves share unevenly; outputs around 64, groups around 8
 @pytest.mark.parametrize("rows", [1, 15, 17, 33, 4096, 4097])
 @pytest.mark.parametrize("k, outputs, top, groups, keep", [(32, 1, 1, 1, 1), (544, 17, 17, 1, 1), (96, 63, 5, 3, 2), (2048, 64, 64, 8, 8), (160, 64, 3, 16, 5),
-                                                           (1056, 72, 9, 8, 3), (64, 512, 6, 1, 1)])
+                                                           (1056, 72, 9, 8, 3), (64, 512, 6, 1, 1), (2080, 96, 8, 4, 2)])
 @pytest.mark.parametrize("dtype, sigmoid", [(torch.bfloat16, True), (torch.float16, False), (torch.float32, True)])
 def test_choices_at_the_edges_of_the_tiles(H, rows, k, outputs, top, groups, keep, dtype, sigmoid):
     """Logits are multiples of 1/8 below 16 in size, exact in any order; corrections of r/16 (8 bits hold them) order what would tie."""
