@@ -325,14 +325,23 @@ inline int column_tiles(int p) {
   const int tiles = p / 16;
   return tiles % 4 == 0 ? 4 : tiles % 3 == 0 ? 3 : tiles % 2 == 0 ? 2 : 1;
 }
-// chunks of a segment; 0: whole sequences.  Two workgroups fit a CU, so sequences that make 512 are left whole (8 x 1900 tokens, 64 heads: 262 us, in
-// segments 332); about four a CU even out; a segment is at least four chunks (its start is a load of the states before it) and a sequence at
-// most eight segments.
-inline int pick_segment(int n_seqs, int total_q, int max_q, int heads, int p) {
-  const int64_t per_chunk = (int64_t)heads * (p / 16 / column_tiles(p)), longest = (max_q + L - 1) / L;
-  if (per_chunk * n_seqs >= 512) return 0;
+// Chunks of a segment; 0: whole sequences.  Cut, all chunks run once more for their states, so that it pays where whole sequences leave the chip idle:
+// `busy`, the part of the CUs that have work while the longest sequence runs, each workgroup counted by what it takes of a CU, has to be below a line that rises
+// with the length, over which the start of a segment and the second launch are spread.  us, whole and cut; column tiles x state rows:
+//   4 x 128: 8 chunks busy 0.25 33 and 31, 0.38 34 and 39; 16: 0.50 60 and 48, 0.88 62 and 73; 32: 0.50 110 and 88, 0.75 109 and 111; 63: 0.50 209 and 133,
+//   0.75 209 and 184, 1.5 291 and 353; 7 chunks lose at any (28 and 30).   4 x 256: 16: 0.31 95 and 87, 0.62 95 and 124; 63: 0.62 353 and 365.
+//   4 x 64: 16: 0.88 55 and 54; 32: 0.75 96 and 88.   3 x 128: 16: 0.50 77 and 73; 61: 0.75 275 and 339.   2 x 128: 6: 0.12 35 and 37, 7: 42 and 37; 16: 0.88 87 and 80; 8: 1.5 49 and 67.
+//   1 x 96: 6: 0.23 62 and 56; 16: 0.94 143 and 97, 1.9 147 and 171; 61: 1.4 531 and 426.
+// About four workgroups a CU even out; a segment is at least four chunks (its start is a load of the states before it) and a sequence at most eight segments.
+inline int pick_segment(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
+  const int tiles = column_tiles(p);
+  const int64_t per_chunk = (int64_t)heads * (p / 16 / tiles), longest = (max_q + L - 1) / L, chunks = (total_q + L - 1) / L;
+  if (per_chunk * n_seqs >= 512 || longest < (tiles == 1 ? 6 : tiles < 4 ? 7 : 8)) return 0;
   if (total_q < max_q) return 0;   // (no bound of the rows, from which the segments are counted)
-  const int64_t chunks = (total_q + L - 1) / L, seg = std::max<int64_t>({4, (longest + 7) / 8, (chunks * per_chunk + 1023) / 1024});
+  const double takes = (tiles == 1 ? 0.5 : tiles == 2 ? 0.65 : tiles == 3 && n > 64 ? 1.2 : 1.0) * (n > 192 ? 1.4 : n > 64 ? 1.0 : 0.75);
+  const double busy = (double)(chunks * per_chunk) / (256.0 * longest) * takes;
+  if (busy > 0.92 - 4.5 / (double)longest) return 0;
+  const int64_t seg = std::max<int64_t>({4, (longest + 7) / 8, (chunks * per_chunk + 1023) / 1024});
   return longest * 3 > seg * 4 ? (int)seg : 0;
 }
 
@@ -370,7 +379,7 @@ int launch(const MvSsmArgs &a, int seg, void *workspace, int total_q, hipStream_
 
 // states and decays of the segments, and the states that sequences come with
 size_t mv_ssm_chunk_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
-  const int seg = pick_segment(n_seqs, total_q, max_q, heads, p);
+  const int seg = pick_segment(n_seqs, total_q, max_q, heads, p, n);
   if (!seg) return 0;
   const int64_t slots = total_q / (seg * L) + n_seqs;
   if (slots > 65535) return 0;
@@ -379,7 +388,7 @@ size_t mv_ssm_chunk_workspace(int n_seqs, int total_q, int max_q, int heads, int
 
 int mv_ssm_chunk_launch(const MvSsmArgs &a, void *workspace, size_t ws_bytes, int total_q, int dtype, hipStream_t stream) {
   const size_t need = workspace ? mv_ssm_chunk_workspace(a.n_seqs, total_q, a.max_q, a.heads, a.p, a.n) : 0;
-  const int seg = need && ws_bytes >= need ? pick_segment(a.n_seqs, total_q, a.max_q, a.heads, a.p) : 0;
+  const int seg = need && ws_bytes >= need ? pick_segment(a.n_seqs, total_q, a.max_q, a.heads, a.p, a.n) : 0;
 #define MV_SN(N_) \
   if (a.n == N_) return dtype == MV_BF16 ? launch<bf16_tag, N_ / 32>(a, seg, workspace, total_q, stream) \
                                          : launch<f16_tag, N_ / 32>(a, seg, workspace, total_q, stream)

@@ -1423,7 +1423,8 @@ def ssm_prefill(x, dt, dt_bias, a_log, d, shape, ssm_state, state_slots, cu_q, c
     a = _ssm_args(shape, x, state_slots, out, ssm_state=ssm_state, dt=dt, dt_bias=dt_bias, a_log=a_log, d=d)
     a.cu_q, a.cu_k, a.max_q = cu_q.data_ptr(), cu_k.data_ptr(), int(max_q)
     rows = x.shape[0]
-    n = 0 if flags & MV_SSM_SCAN else int(_lib.mv_ssm_prefill_workspace_bytes(a.n_seqs, rows, a.max_q, a.heads, a.p, a.n, _dt(x)))
+    # (five chunks of 64 tokens and fewer are never cut)
+    n = 0 if flags & MV_SSM_SCAN or a.max_q <= 320 else int(_lib.mv_ssm_prefill_workspace_bytes(a.n_seqs, rows, a.max_q, a.heads, a.p, a.n, _dt(x)))
     ws = torch.empty((n,), dtype=torch.uint8, device=x.device) if n else None
     _check(_lib.mv_ssm_prefill_ws(ctypes.byref(a), _ptr(ws), n, rows, _dt(x), int(flags), _stream()), "mv_ssm_prefill")
     return out

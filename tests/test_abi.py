@@ -40,12 +40,18 @@ def test_workspace_size_queries_are_host_only():
 
 
 def test_when_state_space_prompts_are_cut():
-    """Scratch memory is asked for where sequences are cut into segments: six chunks of 64 tokens and more, fewer than 512 workgroups."""
+    """Scratch memory is asked for where sequences are cut into segments: eight chunks of 64 tokens and more (six where a workgroup has one column tile), and
+    few enough workgroups."""
     from minivllm_amd import hip_ops
 
-    need = lambda seqs, rows, longest, heads=4, dtype=hip_ops.MV_BF16: hip_ops.lib().mv_ssm_prefill_workspace_bytes(seqs, rows, longest, heads, 64, 128, dtype)
-    assert need(1, 320, 320) == 0 < need(1, 321, 321)
-    assert need(7, 7000, 1000, heads=64) > 0 == need(8, 8000, 1000, heads=64)
+    need = lambda seqs, rows, longest, heads=4, p=64, n=128, dtype=hip_ops.MV_BF16: hip_ops.lib().mv_ssm_prefill_workspace_bytes(
+        seqs, rows, longest, heads, p, n, dtype)
+    assert need(1, 448, 448) == 0 < need(1, 449, 449)
+    assert need(1, 320, 320, p=80) == 0 < need(1, 321, 321, p=80)
+    assert need(2, 2000, 1000, heads=64) > 0 == need(4, 4000, 1000, heads=64)            # half of the CUs have work, or all
+    assert need(4, 5000, 4000, heads=64) > 0 == need(4, 16000, 4000, heads=64)           # one long sequence, or four
+    assert need(2, 8000, 4000, heads=80) > 0 == need(2, 8000, 4000, heads=80, n=256)     # two workgroups to a CU, or one
+    assert need(8, 8000, 8000, heads=64) == 0                                            # 512 workgroups
     assert need(1, 4000, 4000, dtype=hip_ops.MV_F32) == 0
     for rows in (0, -1, 999):          # fewer rows than the longest sequence: no bound that segments could be counted from
         assert need(1, rows, 1000) == 0

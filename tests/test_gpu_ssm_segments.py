@@ -48,8 +48,8 @@ def _both(H, monkeypatch, case, dtype):
     assert torch.isfinite(got).all()
 
 
-# around the lengths at which a sequence gets one more segment (four chunks of 64 tokens and up; from 321 tokens on), beside short ones and empty slots
-@pytest.mark.parametrize("spans", [[(321, 7)], [(384, 0), (1, 0)], [(385, 3), (64, 0)], [(513, 7), (70, 0), (512, 3)], [(2500, 0), (33, 5)],
+# around the lengths at which a sequence gets one more segment (four chunks of 64 tokens and up; from 449 tokens on), beside short ones and empty slots
+@pytest.mark.parametrize("spans", [[(449, 7)], [(512, 0), (1, 0)], [(576, 3), (64, 0)], [(513, 7), (70, 0), (512, 3)], [(2500, 0), (33, 5)],
                                    [(1000, 2), (999, 1), (40, 0)]], ids=str)
 @pytest.mark.parametrize("heads, groups, p, n", [(4, 2, 64, 128), (3, 1, 48, 32), (2, 1, 80, 160), (6, 1, 32, 64)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -57,9 +57,9 @@ def test_segments_are_whole_sequences(H, monkeypatch, spans, heads, groups, p, n
     _both(H, monkeypatch, _case(spans, heads, groups, p, n, dtype, H), dtype)
 
 
-@pytest.mark.parametrize("spans", [[(2100, 5), (1999, 0), (1500, 64), (2047, 1)], [(2500, 0), (129, 3), (64, 0)]], ids=str)
+@pytest.mark.parametrize("spans", [[(4000, 5), (3500, 0), (2000, 64)], [(2500, 0), (2400, 3), (900, 1)]], ids=str)
 def test_segments_sized_by_the_work_of_many_heads(H, monkeypatch, spans):
-    """Eight and three chunks where the longest sequence alone would take five: the workgroups of all heads even out at about four a CU."""
+    """Ten and six chunks where the longest sequence alone would take eight and five: the workgroups of all heads even out at about four a CU."""
     _both(H, monkeypatch, _case(spans, 64, 8, 64, 128, torch.bfloat16, H), torch.bfloat16)
 
 
@@ -72,7 +72,7 @@ def _call(H, entry, case, *rest):
     return out, state
 
 
-@pytest.mark.parametrize("spans", [[(900, 0), (400, 3)], [(321, 1)]], ids=str)
+@pytest.mark.parametrize("spans", [[(900, 0), (400, 3)], [(470, 1)]], ids=str)
 def test_calls_that_cannot_be_cut_are_whole_sequences(H, spans):
     """The entry point without scratch memory, too little of it, and a number of rows that no bound can be."""
     case = _case(spans, 4, 2, 64, 128, torch.bfloat16, H)
