@@ -335,8 +335,8 @@ struct RowOnChip {
   static __device__ __forceinline__ short least_of_key(uint32_t key) { return key >= 0x8000u ? (short)(key - 0x8000u) : kAll; }
 };
 
-// Largest element of a thread's vectors (those of RowOnChip) and the first index that has it; -inf and no index if none is larger.  One comparison
-// a vector; four vectors in flight (7, 10 or 19: as fast or slower).
+// Greedy rows that LDS does not hold: largest element of a thread's vectors (those of RowOnChip) and the first index that has it; -inf and no index if none
+// is larger.  One comparison a vector; four vectors in flight (7, 10 or 19: as fast or slower).
 template <typename Tag>
 __device__ __forceinline__ int greedy_pass(const uint16_t *row, int nvec, float &best) {
   constexpr int U = 4;
@@ -371,20 +371,25 @@ __device__ __forceinline__ int greedy_pass(const uint16_t *row, int nvec, float 
 // A row is one pass for the maximum, one for the histogram of a filter, one for ties, one for the masses; 256 rows of 151 936 logits are one
 // workgroup a CU, 304 KB each: more than the LDS and, beside what the passes need, more than the registers, but not more than half in each.  Kept
 // there, the passes behind the first read no memory, and those behind a filter skip what cannot be kept.
-// A greedy row is one pass and stays nowhere (greedy_pass).
+// A long greedy row is one pass and stays nowhere (greedy_pass).
 // 151 936 bf16 logits, us, memory in every pass -> now; 256 rows: greedy 18.9 -> 13.9, plain 58 -> 30, top-k 40 89 -> 37, top-p 0.9 81 -> 55, min-p
-// 55 -> 27; one row: 15.5 -> 6.3, 51 -> 20, 81 -> 28, 73 -> 45, 49 -> 18 (a greedy row brought to its CU like the others: 18.4, 9.8).  What is left is
+// 55 -> 27; one row: 15.5 -> 6.3, 51 -> 20, 81 -> 28, 73 -> 45, 49 -> 18 (brought to its CU like the others: 18.4, 9.8).  What is left is
 // vector arithmetic: an exponential and four instructions an element where every weight counts.
 template <typename Tag, int NR>
 __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   typedef typename elem<Tag>::T T;
   constexpr int KBITS = keyinfo<Tag>::BITS;
   constexpr int LEVELS = KBITS / 8;
-  constexpr bool CHIP = NR >= 0;
+  constexpr bool CHIP = NR >= 0, STREAM = NR > 0;
   typedef RowOnChip<Tag, CHIP ? NR : 0> Row;
   constexpr int U = CHIP ? 1 : 4;   // (beside a row in registers only rare passes read memory: little of it in flight)
   extern __shared__ __attribute__((aligned(16))) char smem[];   // Shared | the row's first vectors
-  Shared &sh = *(Shared *)smem;
+  Shared *shared = (Shared *)smem;
+  if constexpr (!CHIP) {   // (at a constant address: the radix select of fp32 rows takes 2 to 3 % longer behind the other)
+    __shared__ Shared own;
+    shared = &own;
+  }
+  Shared &sh = *shared;
   char *row_lds = smem + sizeof(Shared);
 
   const int rowi = blockIdx.x;
@@ -399,7 +404,7 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   int best_i = 0x7fffffff;
   Row chip;
   if constexpr (CHIP) {
-    if (temp == 0.0f) {   // one pass is all of it: nothing is kept but the vector that has the thread's maximum
+    if (STREAM && temp == 0.0f) {   // one pass is all of it: nothing is kept but the vector that has the thread's maximum
       best_i = greedy_pass<Tag>(row, V / 8, best);
     } else {
       chip.load(row, V / 8, row_lds);
@@ -413,10 +418,16 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
   }
   const float xmax = block_max(best, sh);
   if (temp == 0.0f) {  // greedy (argmax, not multinomial over softmax(l/1e-8))
-    if constexpr (CHIP) {
+    if constexpr (STREAM) {
       if (xmax == -INFINITY)   // (no element is above it: the first that is not NaN)
         row_foreach<Tag, 1>(row, V, vec_ok, [&](int i, T raw, bool ok) {
           if (ok && elem<Tag>::ld(raw) == xmax) best_i = min(best_i, i);
+        });
+    } else if constexpr (CHIP) {
+      const short least = xmax > 0.f ? Row::least_of_key(make_key<Tag>(elem<Tag>::st(xmax))) : Row::kAll;
+      if (best == xmax)
+        chip.foreach_from(least, [&](int i, T raw) {
+          if (elem<Tag>::ld(raw) == xmax) best_i = min(best_i, i);
         });
     }
     int cand = (best == xmax) ? best_i : 0x7fffffff;
@@ -497,15 +508,15 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
       if constexpr (CHIP) {
         // What is asked of the whole row besides (top-p: its mass) is a pass without branches.  With top-k, at least k elements reach the k-th
         // largest of the threads' maxima, so few elements are left to count; a bound that is no use (fewer maxima than k) is the whole window.
-        if (topk_on) {
+        if (topk_on && k_raw <= kThreads) {
           clear();
           if (best > -INFINITY) count(elem<Tag>::st(best), kWin);
           scan();
-          const unsigned least_c = (unsigned)min(k_raw, (int64_t)kThreads + 1);
+          const unsigned least_c = (unsigned)k_raw;
           if (pc < least_c && least_c <= pc + c0 + c1) sh.bcast_u[0] = 2 * threadIdx.x + (pc + c0 < least_c ? 1 : 0);
           __syncthreads();
           win = sh.bcast_u[0] + 1u;
-        } else {
+        } else if (!topk_on) {
           float z = 0.f;
           chip.foreach([&](T raw) { z += weight(elem<Tag>::ld(raw)); });
           all_m = block_sum_f(z, sh);
@@ -1360,7 +1371,7 @@ int launch_sample(const SampleParams &p, int batch, hipStream_t st) {
       }
     }
   }
-  hipLaunchKernelGGL((sample_kernel<Tag, -1>), grid, block, sizeof(Shared), st, p);
+  hipLaunchKernelGGL((sample_kernel<Tag, -1>), grid, block, 0, st, p);
   return MV_OK;
 }
 }  // namespace
