@@ -207,8 +207,9 @@ int mv_rope_paged_decode_ex(const void *q, int64_t q_stride_tok, const void *k, 
  *               sequence i are its first seqlen_k tokens in the cache)
  * Causal mask is bottom-right aligned: query j of sequence i (0-based in its
  * seqlen_q) attends keys 0 .. seqlen_k-seqlen_q+j (attention.py:584-588).
- * flags: MV_PREFILL_SIMPLE routes tensors of every dtype through the vector-ALU kernel (debug aid); 0 = default. */
-enum { MV_PREFILL_SIMPLE = 1 };
+ * flags (debug aids; 0 = default): MV_PREFILL_SIMPLE routes tensors of every dtype through the vector-ALU kernel, MV_PREFILL_TILES fp32 tensors of
+ * head dims 64 and 128 through the matrix cores whatever their sizes (by default: where that is the quicker). */
+enum { MV_PREFILL_SIMPLE = 1, MV_PREFILL_TILES = 2 };
 int mv_prefill_varlen(const void *q, int64_t q_stride_tok, const void *k,
                       const void *v, int64_t k_stride_tok, int64_t v_stride_tok,
                       const void *k_cache, const void *v_cache,

@@ -16,8 +16,8 @@ struct PrefillParams {
   int64_t out_stride;   // elements between token rows of out
 };
 
-// fp32 flash path on the matrix cores (D in {64,128}); returns MV_E_SHAPE when it does not apply
-int mv_prefill_f32_launch(const PrefillParams &p, hipStream_t stream);
+// fp32 flash path on the matrix cores (D in {64,128}); returns MV_E_SHAPE when it does not apply, or (unless `always`) the vector kernel is the quicker
+int mv_prefill_f32_launch(const PrefillParams &p, bool always, hipStream_t stream);
 // generic vector-ALU path (every dtype, D in {64,128,256})
 int mv_prefill_simple_launch(const PrefillParams &p, int64_t max_total_q, int dtype, hipStream_t stream);
 // MFMA flash path (bf16/f16, D in {64,128}); returns MV_E_SHAPE when it does not apply

@@ -45,9 +45,9 @@ extern "C" int mv_prefill_varlen_ex(const void *q, int64_t q_stride_tok, const v
   p.mask = mv_attn_mask(opts);
   p.out_stride = out_stride;
   hipStream_t st = (hipStream_t)stream;
-  // MV_PREFILL_SIMPLE routes every dtype through the vector-ALU kernel (debug aid)
+  // debug aids: MV_PREFILL_SIMPLE routes every dtype through the vector-ALU kernel, MV_PREFILL_TILES every fp32 call that has one through the other
   if (!(flags & MV_PREFILL_SIMPLE)) {
-    const int rc = dtype == MV_F32 ? mv_prefill_f32_launch(p, st) : mv_prefill_mfma_launch(p, dtype, flags >> 4, st);
+    const int rc = dtype == MV_F32 ? mv_prefill_f32_launch(p, flags & MV_PREFILL_TILES, st) : mv_prefill_mfma_launch(p, dtype, flags >> 4, st);
     if (rc != MV_E_SHAPE) return rc;
   }
   return mv_prefill_simple_launch(p, (int64_t)n_seqs * max_seqlen_q, dtype, st);

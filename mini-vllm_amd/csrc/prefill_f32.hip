@@ -15,7 +15,8 @@
 // What the tree costs and gives, attention of a layer (us): 6131 tokens in 8 prompts, 12 heads of 64: vector kernel 801, chains of 16 products 137, this
 // 148 (62 TFLOP/s of visible pairs; 4 x 2048: 91); 16 x 1024, 16 heads of 128: 958 -> 771 (89), where the longer chains and rows of K and V
 // side by side left 69 registers in memory; now 4 (paged or masked: 12; head dim 64: 1, 6).
-// The vector kernel (prefill_simple.hip: a wave per query and head, every query reads its keys again) stays for head dim 256.
+// The vector kernel (prefill_simple.hip: a wave per query and head, every query reads its keys again) stays for head dim 256, and where queries see few
+// keys or are few themselves: vector_is_quicker below.
 // Reference: minivllm/models/layers/attention.py:467-504,554-597.
 #include "prefill_row.h"
 
@@ -310,9 +311,28 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
   }
 }
 
+// Both kernels' times in ns, as they grew over 1700 shapes (1 .. 400 queries of 1 .. 2000 keys, 4 .. 32 heads, 1 .. 256 sequences): the vector kernel takes
+// 3 us, the walk to the sequence, and 0.11 us a key (twice that at head dim 128) or its reads of K and V, whichever is more; a tile of 64 queries 9 us for
+// the first 64 keys and 4 for each further 64, or what its turns on the chip take.  The other kernel is quicker by more than 5 % in 5 % of them, by 45 % at most.
+// Vector kernel / this, us: one prompt of 8 tokens, 12 heads of 64 (128) 4 / 9 (4 / 15); 64 of 8 tokens 14 / 14 (16 / 31), of 16 24 / 14 (28 / 32);
+// one of 64 tokens 10 / 9 (17 / 15); 256 single queries of 400 paged keys, 32 heads of 64 (128) 193 / 953 (349 / 2270).
+// From 320 keys on, where the vector kernel is further from 64 bits, it has to take half as long or less.
+bool vector_is_quicker(const PrefillParams &p) {
+  const int64_t seen = p.max_seqlen_k, wide = p.head_dim / 64, beside = min(p.max_seqlen_q, BM) + BN - 2;   // keys that only other queries of a tile see
+  const int64_t limit = p.chunk > 0 ? p.chunk : p.mask.window > 0 ? (int64_t)p.mask.window + p.mask.keep_first : seen;
+  const int64_t keys = min(seen, limit), pieces = (min(seen, limit < seen ? limit + beside : seen) + 63) / 64;
+  const int64_t rows = (int64_t)p.n_heads * p.n_seqs * p.max_seqlen_q, groups = (int64_t)p.n_heads * p.n_seqs * ((p.max_seqlen_q + BM - 1) / BM);
+  const int64_t read = rows * keys * wide / 25 / (p.n_heads >= 4 * p.n_kv_heads ? 2 : 1);
+  const int64_t vector = 3000 + 70 * p.n_seqs + max(22 * wide * keys * (p.block_tables ? 6 : 5), read) + rows * p.n_seqs * 14 / 1000;
+  const int64_t tiles = max(4700 + 4000 * pieces, groups * (7 + 12 * pieces)) * (wide > 1 ? 7 : 4) / 4 *
+                        (p.block_tables ? 14 : limit < seen || p.mask.softcap > 0.f ? 12 : 10) / 10;
+  return vector * (keys > 320 ? 2 : 1) <= tiles;
+}
+
 }  // namespace
 
-int mv_prefill_f32_launch(const PrefillParams &p, hipStream_t stream) {
+int mv_prefill_f32_launch(const PrefillParams &p, bool always, hipStream_t stream) {
+  if (p.head_dim > 128 || (!always && vector_is_quicker(p))) return MV_E_SHAPE;
   const dim3 grid(p.n_heads, p.n_seqs, (p.max_seqlen_q + BM - 1) / BM);
   if (grid.y > 65535 || grid.z > 65535) return MV_E_SHAPE;
   const bool general = p.block_tables || p.chunk > 0 || p.mask.window > 0 || p.mask.softcap > 0.f;

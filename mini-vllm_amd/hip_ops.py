@@ -287,6 +287,7 @@ def _out_rows(out, rows: int, h: int, d: int):
 # The C-ABI reads no environment: the overrides below are read HERE, once, and passed as explicit arguments.
 MV_DECODE_VECTOR, MV_DECODE_MFMA, MV_DECODE_KLDS_OFF, MV_DECODE_KLDS_ON, MV_DECODE_PER_HEAD = 1, 2, 4, 8, 16
 MV_PREFILL_SIMPLE = 1
+MV_PREFILL_TILES = 2
 MV_E_SHAPE = -2   # include/mvhip.h
 
 

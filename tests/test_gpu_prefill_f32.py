@@ -14,6 +14,11 @@ def H():
     return hip_ops
 
 
+@pytest.fixture(autouse=True)
+def tiles(H, monkeypatch):
+    monkeypatch.setattr(H, "PREFILL_FLAGS", H.MV_PREFILL_TILES)      # (also where the vector kernel is the quicker)
+
+
 def _attend(q, k, v, scale, seen, cap=0.0, sink=None):
     """q [nq, H, D], k / v [nk, Hkv, D], seen [nq, nk] in fp64."""
     g = q.shape[1] // k.shape[1]
@@ -132,5 +137,25 @@ def test_no_further_from_64_bits_than_the_vector_kernel(H, n, seqs, d):
     s = torch.matmul(lanes(q), lanes(k).transpose(1, 2).contiguous()) * d ** -0.5
     s.masked_fill_(torch.ones(n, n, dtype=torch.bool, device=DEV).triu(1), -float("inf"))
     want = torch.matmul(s.softmax(-1), lanes(v))
-    error = [(lanes(H.prefill_varlen(q, k, v, cu, cu, n, n, d ** -0.5, flags=f)) - want).norm() / want.norm() for f in (0, H.MV_PREFILL_SIMPLE)]
+    error = [(lanes(H.prefill_varlen(q, k, v, cu, cu, n, n, d ** -0.5, flags=f)) - want).norm() / want.norm() for f in (H.MV_PREFILL_TILES, H.MV_PREFILL_SIMPLE)]
     assert error[0] <= 1.01 * error[1], (error[0].item(), error[1].item())
+
+
+# by what the vector kernel and the tiles take: few keys, single queries of paged keys; long prompts, many of a few tokens; a window, a chunk
+@pytest.mark.parametrize("seqs, nq, nk, kw, vector", [(1, 8, 8, {}, True), (1, 40, 40, {}, True), (256, 1, 200, dict(paged=True), True), (1, 8, 400, dict(window=32), True),
+                                                      (1, 300, 300, dict(chunk=16), True), (1, 100, 100, {}, False), (256, 16, 16, {}, False), (2, 500, 500, {}, False),
+                                                      (1, 8, 400, dict(window=300), False)], ids=str)
+@pytest.mark.parametrize("d", [64, 128])
+def test_kernel_by_size(H, d, seqs, nq, nk, kw, vector):
+    g = torch.Generator(device=DEV).manual_seed(nk)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    cu = lambda n: torch.arange(0, seqs * n + 1, n, dtype=torch.int32, device=DEV)
+    q, k, v, cache = rand(seqs * nq, 8, d), rand(seqs * nk, 2, d), rand(seqs * nk, 2, d), {}
+    if kw.get("paged"):
+        kc, vc = (t.view(-1, 40, 2, d) for t in (k, v))
+        k, v, cache = None, None, dict(k_cache=kc, v_cache=vc, block_tables=torch.arange(seqs * nk // 40, dtype=torch.int32, device=DEV).view(seqs, -1))
+    call = lambda flags: H.prefill_varlen(q, k, v, cu(nq), cu(nk), nq, nk, d ** -0.5, flags=flags, chunk=kw.get("chunk", 0), mask=H.AttnMask(kw.get("window", 0)), **cache)
+    by_size, one, other = call(0), call(H.MV_PREFILL_SIMPLE), call(H.MV_PREFILL_TILES)
+    assert not torch.equal(one, other)
+    assert torch.equal(by_size, one if vector else other)
+    torch.testing.assert_close(one, other, rtol=1e-5, atol=1e-5)      # (as above)

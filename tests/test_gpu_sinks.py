@@ -73,9 +73,10 @@ def test_prompts(H, dtype, d, spans, window, chunk):
     q, k, v = (torch.cat(t).to(DEV) for t in (qs, ks, vs))
     cq, ck, mq, mk = _cu([a for a, _ in spans]), _cu([b for _, b in spans]), max(a for a, _ in spans), max(b for _, b in spans)
     mask = H.AttnMask(window=window, sink=sink.to(DEV))
-    _close(H.prefill_varlen(q, k, v, cq, ck, mq, mk, d ** -0.5, chunk=chunk, mask=mask), want, dtype)
     kc, vc, table = _pages(ks, vs, 64)
-    _close(H.prefill_varlen(q, None, None, cq, ck, mq, mk, d ** -0.5, k_cache=kc, v_cache=vc, block_tables=table, chunk=chunk, mask=mask), want, dtype)
+    for flags in (0, H.MV_PREFILL_TILES):
+        _close(H.prefill_varlen(q, k, v, cq, ck, mq, mk, d ** -0.5, flags=flags, chunk=chunk, mask=mask), want, dtype)
+        _close(H.prefill_varlen(q, None, None, cq, ck, mq, mk, d ** -0.5, k_cache=kc, v_cache=vc, block_tables=table, flags=flags, chunk=chunk, mask=mask), want, dtype)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
@@ -87,7 +88,7 @@ def test_the_vector_kernel_and_a_page_that_is_not_there(H, dtype, d):
     want = torch.cat([_attend(q, k, v, d ** -0.5, _seen(q.shape[0], k.shape[0], 0, 0) & there[:k.shape[0]], sink) for q, k, v in zip(qs, ks, vs)])
     kc, vc, table = _pages(ks, vs, 16, [lost])
     args = (torch.cat(qs).to(DEV), None, None, _cu([a for a, _ in spans]), _cu([b for _, b in spans]), 150, 150, d ** -0.5)
-    for flags in (0, H.MV_PREFILL_SIMPLE):
+    for flags in (0, H.MV_PREFILL_TILES, H.MV_PREFILL_SIMPLE):
         _close(H.prefill_varlen(*args, k_cache=kc, v_cache=vc, block_tables=table, flags=flags, mask=H.AttnMask(sink=sink.to(DEV))), want, dtype)
 
 
