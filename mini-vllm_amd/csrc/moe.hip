@@ -678,17 +678,17 @@ extern "C" int mv_moe_route(const void *x, int64_t x_stride, const void *w, cons
     return MV_E_SHAPE;
   if (!mv_aligned16(x) || !mv_aligned16(w) || x_stride % (dtype == MV_F32 ? 4 : 8)) return MV_E_ALIGN;
   const RouteParams p{x, w, correction, ids, weights, x_stride, rows, k, outputs, top, groups, keep, flags, scale};
-  // A tile of 16 tokens over 16 waves while that fills no more than the chip, and for more than 256 outputs, whose scores leave room for one
-  // workgroup a CU.  More tokens: eight waves, so that the workgroups of a CU choose beside each other (20000 tokens of 512 inputs, 128 outputs: 51 us,
-  // 16 waves 74, eight waves of two tiles 105).  Two tiles, which read the weights once, where those are long: 34 outputs of 4096 inputs, 4400 tokens
+  // A tile of 16 tokens over 16 waves while that fills no more than the chip.  More tokens: eight waves, so that the workgroups of a CU choose beside
+  // each other (20000 tokens of 512 inputs, 128 outputs: 51 us, 16 waves 74, eight waves of two tiles 105; 384 outputs, whose scores leave room for one
+  // workgroup a CU, 16 waves 123, eight 91).  Two tiles, which read the weights once, where those are long: 34 outputs of 4096 inputs, 4400 tokens
   // 23 us, one tile 28.  More than 64 outputs leave two tiles one workgroup a CU, so its rounds over the chip have to be full: 128 outputs of 4096
-  // inputs, 4400 tokens 73 us, 12000 145; one tile 87 and 122.
+  // inputs, 4400 tokens 73 us, 12000 145; one tile 87 and 122.  LDS has the scores of two tiles up to 256 outputs.
   MV_DISPATCH_DTYPE(dtype, {
     const hipStream_t st = (hipStream_t)stream;
     const bool full = k > 2048 && (rows <= 8192 || (k >= 4096 && (rows - 1) % 8192 >= 4096));
     int rc;
-    if (rows <= 16 * 256 || outputs > 256) rc = launch_route<Tag, 16, 1>(p, st);
-    else if (dtype != MV_F32 && (outputs <= 64 ? k >= 2048 : full)) rc = launch_route<Tag, 8, 2>(p, st);
+    if (rows <= 16 * 256) rc = launch_route<Tag, 16, 1>(p, st);
+    else if (dtype != MV_F32 && (outputs <= 64 ? k >= 2048 : outputs <= 256 && full)) rc = launch_route<Tag, 8, 2>(p, st);
     else rc = launch_route<Tag, 8, 1>(p, st);
     if (rc) return rc;
   });
