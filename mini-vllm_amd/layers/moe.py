@@ -18,7 +18,9 @@ from .linear import Segment, SegmentedLinear, gated_linear, pad_to
 
 __all__ = ["ExpertMLP"]
 
-# pairs per expert up to which a launch works on tiles of that many rows
+# Pairs per expert up to which a launch works on tiles of that many rows.  The last line was drawn for workgroups of 256 x 256 rows and outputs; their successors,
+# two of 128 x 256 to a CU, are ahead from fewer pairs on.  Both products, tiles of 64 / 128 / 256 rows, us: 32 experts of 2048 -> 768, 64 pairs each 101 / 76 / 68,
+# 256 188 / 194 / 131, 768 400 / 392 / 294; of 1024 -> 384 31 / 36 / 32, 75 / 78 / 42, 134 / 143 / 88; 8 experts of 2048 -> 768 39 / 49 / 49, 49 / 58 / 51, 104 / 110 / 82.
 TILES = ((8, 16), (40, 32), (96, 64), (768, 128))
 
 
