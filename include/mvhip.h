@@ -731,6 +731,8 @@ typedef struct MvDeltaArgs {
 /* out[t] = o, [T][heads * p], from convolved channels; writes state.  flags: MV_DELTA_SCAN = token by token */
 enum { MV_DELTA_SCAN = 1 };
 size_t mv_delta_prefill_workspace_bytes(int n_seqs, int total_q, int heads, int p, int n, int dtype);
+/* scratch beyond that with which few long sequences are worked on in several places at once (0: none is of use) */
+size_t mv_delta_prefill_segments_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int channel_decay, int dtype);
 int mv_delta_prefill(const MvDeltaArgs *args, int dtype, int flags, void *stream);
 /* one token per sequence, from projected channels: convolution, recurrence and mv_head_norm_gate in one launch; writes both states */
 int mv_delta_step(const MvDeltaArgs *args, int dtype, void *stream);

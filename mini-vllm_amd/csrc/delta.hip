@@ -292,6 +292,11 @@ extern "C" size_t mv_delta_prefill_workspace_bytes(int n_seqs, int total_q, int 
   return dtype == MV_F32 ? 0 : mv_delta_chunk_workspace(n_seqs, total_q, heads, p, n);
 }
 
+extern "C" size_t mv_delta_prefill_segments_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int channel_decay, int dtype) {
+  // (bf16 with one decay per head: delta_scalar.hip, whole sequences)
+  return dtype == MV_F32 || (dtype == MV_BF16 && !channel_decay) ? 0 : mv_delta_segments_workspace(n_seqs, total_q, max_q, heads, p, n);
+}
+
 extern "C" int mv_delta_prefill(const MvDeltaArgs *a, int dtype, int flags, void *stream) {
   if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
   if (int e = check_delta(a, dtype)) return e;

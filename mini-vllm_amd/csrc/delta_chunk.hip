@@ -17,6 +17,9 @@
 // Exponentials never overflow: A and B are computed by blocks of 16 x 16 tokens with the sums taken relative to r at the end of the
 // block in front of the rows' (both factors at most 1), or in the middle of a diagonal block; where a block decays by more than
 // 2^kRange a diagonal block is summed pair by pair instead.
+#include <algorithm>
+#include <cmath>
+
 #include "delta_chunk.h"
 
 namespace {
@@ -293,6 +296,15 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(De
 __device__ __forceinline__ void lds_landed(u32x4 &a) { asm volatile("" : "+v"(a)); }
 __device__ __forceinline__ void lds_landed(u32x4 &a, u32x4 &b) { asm volatile("" : "+v"(a), "+v"(b)); }
 
+// segments of `len` tokens: what they add to the state ahead of them [slot][heads][n * p], what becomes of that state [slot][heads] (n x n as
+// operands), the states that sequences of several segments come with [sequence][heads][n * p]; a sequence's slots start at cu_q / len + its number
+struct Segments {
+  float *added, *first;
+  char *carry;
+  int len;
+};
+enum { WHOLE, SEGMENTS, ADDED, CARRY };   // workgroups are sequences, or segments; ADDED, CARRY: only what a segment does to the state
+
 // Workgroup = 4 waves x CW tiles of 16 columns of one head of one sequence; a wave keeps S of its columns in accumulators.  The
 // accumulators are the next product's operands as they are: the rows of S are dealt so that tiles 2 s and 2 s + 1 together hold
 // n = 32 s + 8 g .. + 7 in lane group g.  O is computed transposed (columns by tokens), so that a lane stores four columns of a token.
@@ -300,30 +312,49 @@ __device__ __forceinline__ void lds_landed(u32x4 &a, u32x4 &b) { asm volatile(""
 // use: as soon as all waves have used a group, its part of the next chunk is asked for, so that transfers run all the time and none is waited for
 // that was not asked for a chunk before (3 sequences of 4011 tokens and less, 8 heads of 128 x 128: 283 us with two phases, each fetched as a whole
 // while the other was used, 247 with operands read as they were used -> 224).
-template <typename Tag, int NK, int CW>
-__global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
+// Few long sequences leave most CUs idle in it, and are cut into segments of whole chunks (pick_segment).  What a segment does to the state ahead
+// of it is linear, S <- M S + C: a first launch walks the segments for C (from zeros, or what the sequence comes with) and M (from the identity, without
+// values), with neither q nor B; the second starts a segment from the state that the C and M of those before it give, and is otherwise the walk.  Of the
+// sequences above: 224 -> 53 + 58 us (11 chunks a segment; 5 - 8 times as many workgroups as sequences, heads and halves of them).
+template <typename Tag, int NK, int CW, int MODE>
+__device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int wide, int at_head) {
   typedef typename elem<Tag>::T T;
-  constexpr int F1 = 16 * NK + 16 * CW, GROUPS = 2 * NK + 1;   // fragments of W, Q and U0; steps of W and Q (U0 in the first) | B | pairs of tiles of K
+  constexpr bool OUT = MODE == WHOLE || MODE == SEGMENTS, VALUES = MODE != CARRY;
+  // fragments of W, Q and U0; steps of W and Q (U0 in the first) | B, decay | pairs of tiles of K
+  constexpr int QF = OUT ? 8 * NK : 0, BF = OUT ? 16 : 0, F1 = 8 * NK + QF + (VALUES ? 16 * CW : 0), GROUPS = 2 * NK + 1;
   // transfers of a wave: for a group, for those behind it, for all
-  constexpr auto own = [](int n) { return n < NK ? (n ? 4 : 4 + 4 * CW) : n == NK ? 5 : 2; };
-  constexpr auto behind = [](int n) { return n < NK ? 4 * (NK - 1 - n) + 5 + 2 * NK : 2 * (GROUPS - 1 - n); };
-  constexpr int ALL = 4 * CW + 4 * NK + 5 + 2 * NK;
+  constexpr int STEP = OUT ? 4 : 2, MIDDLE = OUT ? 5 : 1;
+  constexpr auto own = [](int n) { return n < NK ? (n || !VALUES ? STEP : STEP + 4 * CW) : n == NK ? MIDDLE : 2; };
+  constexpr auto behind = [](int n) { return n < NK ? STEP * (NK - 1 - n) + MIDDLE + 2 * NK : 2 * (GROUPS - 1 - n); };
+  constexpr int ALL = own(0) + behind(0);
   const MvDeltaArgs &p = q.a;
-  extern __shared__ __attribute__((aligned(16))) char smem[];   // [F1][1 KiB] | [F2][1 KiB]
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // [F1][1 KiB] | K | B | decay
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  // (workgroups are dealt to the 8 XCDs in turn: each gets a run of columns and heads, which share all but their part of U0)
-  const int wide = gridDim.x, all = wide * p.heads;
-  int at_head = blockIdx.y * wide + blockIdx.x;
-  if (!(all & 7)) at_head = (at_head & 7) * (all >> 3) + (at_head >> 3);
-  const int head = at_head / wide, seq = blockIdx.z, tiles = p.p / 16, tile0 = (at_head - head * wide) * 4 * CW;
-  const int q0 = p.cu_q[seq], len = p.cu_q[seq + 1] - q0;
+  const int head = at_head / wide, tiles = MODE == CARRY ? 2 * NK : p.p / 16, tile0 = (at_head - head * wide) * 4 * CW;
+  int seq = blockIdx.z, from = 0, q0 = 0, len = 0, all = 0;
+  if constexpr (MODE == WHOLE) {
+    q0 = p.cu_q[seq], all = len = p.cu_q[seq + 1] - q0;
+  } else {
+    seq = 0;
+    for (int hi = p.n_seqs; hi - seq > 1;) {   // the sequence that the slot belongs to
+      const int mid = (seq + hi) >> 1;
+      if (p.cu_q[mid] / sg.len + mid <= (int)blockIdx.z) seq = mid;
+      else hi = mid;
+    }
+    q0 = p.cu_q[seq], all = p.cu_q[seq + 1] - q0;
+    from = ((int)blockIdx.z - q0 / sg.len - seq) * sg.len;
+    len = min(sg.len, all - from);
+    // (nobody asks for what the last one adds, nor for what becomes of the state ahead of the first)
+    if (from < 0 || (!OUT && from + sg.len >= all) || (MODE == CARRY && from == 0)) return;
+  }
   if (len <= 0) return;
-  const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq];
+  const int before = p.cu_k[seq + 1] - p.cu_k[seq] - all, slot = p.state_slots[seq];
   const bool keep = slot >= 0 && slot < p.slots;
   const int64_t size = (int64_t)p.heads * p.n * p.p;
   const Layout lay(NK, p.p);
   const int64_t stride = (int64_t)p.heads * lay.total * 1024;
-  const char *ws = q.ws + ((int64_t)(q0 / L + seq) * p.heads + head) * lay.total * 1024 + lane * 16;
+  const char *ws = q.ws + ((int64_t)(q0 / L + seq + from / L) * p.heads + head) * lay.total * 1024 + lane * 16;
+  q0 += from;
 
   int col[CW];
   bool live[CW];
@@ -332,17 +363,10 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
     const int t = tile0 + wave * CW + w;
     live[w] = t < tiles, col[w] = min(t, tiles - 1) * 16 + r16;
   }
-  auto state_at = [&](int half, int w, int i, int e) {
-    const int n = (i >> 1) * 32 + g * 8 + (i & 1) * 4 + e;
-    return p.state + half * p.slots * size + (int64_t)(keep ? slot : 0) * size + ((int64_t)head * p.n + n) * p.p + col[w];
-  };
+  auto state_row = [&](int i, int e) { return (i >> 1) * 32 + g * 8 + (i & 1) * 4 + e; };
+  auto in_head = [&](int w, int i, int e) { return ((int64_t)head * p.n + state_row(i, e)) * p.p + col[w]; };
+  auto state_at = [&](int half, int w, int i, int e) { return p.state + half * p.slots * size + (int64_t)(keep ? slot : 0) * size + in_head(w, i, e); };
   f32x4 st[CW][2 * NK];
-#pragma unroll
-  for (int w = 0; w < CW; ++w)
-#pragma unroll
-    for (int i = 0; i < 2 * NK; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) st[w][i][e] = keep && before > 0 ? *state_at(before & 1, w, i, e) : 0.f;
 
   auto fetch = [&](const char *from, int frag, char *to) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(from + (int64_t)frag * 1024),
@@ -353,17 +377,19 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
     const char *from = ws + c * stride;
     if constexpr (n < NK) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < STEP; ++i) {   // (W's eight, then Q's)
         const int which = i * 4 + wave, f = (which >> 3) * 8 * NK + (((which >> 1) & 3) * NK + n) * 2 + (which & 1);
         fetch(from, f, smem + f * 1024);
       }
-      if constexpr (n == 0) {
+      if constexpr (n == 0 && VALUES) {
 #pragma unroll
         for (int i = 0; i < 4 * CW; ++i) {
           const int f = i * 4 + wave;   // (column tile, token tile)
-          fetch(from, lay.u0 + min(tile0 + (f >> 2), tiles - 1) * 4 + (f & 3), smem + (16 * NK + f) * 1024);
+          fetch(from, lay.u0 + min(tile0 + (f >> 2), tiles - 1) * 4 + (f & 3), smem + (8 * NK + QF + f) * 1024);
         }
       }
+    } else if constexpr (n == NK && !OUT) {
+      fetch(from, lay.tail, smem + (F1 + 8 * NK) * 1024);   // (every wave: the same bytes)
     } else {
       constexpr int first = n == NK ? 8 * NK : (n - NK - 1) * 8, last = n == NK ? 8 * NK + 16 : first + 7;
 #pragma unroll
@@ -373,12 +399,111 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
       }
     }
   };
-  const uint32_t base = lds_address(smem) + lane * 16;
-  const uint32_t aw = base, aq = base + 8 * NK * 1024, au = base + (16 * NK + wave * CW * 4) * 1024;
-  const uint32_t ak = base + F1 * 1024, ab = ak + 8 * NK * 1024, at = lds_address(smem) + (F1 + 8 * NK + 16) * 1024 + g * 32;
+  const uint32_t base = lds_address(smem) + lane * 16;   // (fragments)
+  const uint32_t aw = base, aq = base + 8 * NK * 1024, au = base + (8 * NK + QF + wave * CW * 4) * 1024;
+  const uint32_t ak = base + F1 * 1024, ab = ak + 8 * NK * 1024, at = lds_address(smem) + (F1 + 8 * NK + BF) * 1024 + g * 32;
   const int chunks = (len + L - 1) / L;
   const bool quads = !(((uintptr_t)p.out & 7) | (p.out_stride & 3));   // (rows of the output may stand anywhere)
-  static_for<GROUPS>([&](auto G) { fetch_group(G, 0); });
+  if constexpr (MODE != SEGMENTS) static_for<GROUPS>([&](auto G) { fetch_group(G, 0); });
+
+  // ---- the state ahead
+  const int64_t first_at = (int64_t)seq * size;
+#pragma unroll
+  for (int w = 0; w < CW; ++w)
+#pragma unroll
+    for (int i = 0; i < 2 * NK; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = 0.f;
+        if constexpr (MODE == CARRY) {
+          v = state_row(i, e) == col[w] ? 1.f : 0.f;
+        } else if (from == 0 && keep && before > 0) {
+          // (the pool's state of a cut sequence is read by the first launch alone: the second may write it)
+          v = MODE == SEGMENTS && all > len ? sg.first[first_at + in_head(w, i, e)] : *state_at(before & 1, w, i, e);
+        }
+        if (MODE == ADDED && from == 0 && before > 0 && live[w]) sg.first[first_at + in_head(w, i, e)] = v;
+        st[w][i][e] = v;
+      }
+  if constexpr (MODE == SEGMENTS) {
+    // .. of a later segment: that at the end of the first, and from segment to segment one product, whose left operand lands in LDS while
+    // the one before is multiplied (where LDS holds two: up to 128 channels).  Read by each wave as it was used, a segment took 4.5 us.
+    constexpr int CF = 4 * NK * NK, BUFFERS = 2 * CF <= F1 + 8 * NK + BF + 1 ? 2 : 1;   // fragments
+    const int ahead = from / sg.len, first = (int)blockIdx.z - ahead;
+    auto fetch_carry = [&](int j) __attribute__((always_inline)) {
+      const char *of = sg.carry + ((int64_t)(first + j) * p.heads + head) * (CF * 1024) + lane * 16;
+#pragma unroll
+      for (int i = 0; i < NK * NK; ++i) fetch(of, i * 4 + wave, smem + ((j % BUFFERS) * CF + i * 4 + wave) * 1024);
+    };
+    f32x4 next[CW][2 * NK];
+    auto load_added = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int w = 0; w < CW; ++w)
+#pragma unroll
+        for (int i = 0; i < 2 * NK; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) next[w][i][e] = sg.added[(first + j) * size + in_head(w, i, e)];
+    };
+    if (ahead > 0) {
+      if (ahead > 1) fetch_carry(1);
+      load_added(0);
+#pragma unroll
+      for (int w = 0; w < CW; ++w)
+#pragma unroll
+        for (int i = 0; i < 2 * NK; ++i) st[w][i] = next[w][i];
+      if (ahead > 1) load_added(1);
+      for (int j = 1; j < ahead; ++j) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        lds_barrier();
+        u32x4 sh[CW][NK], sl[CW][NK], f[2][NK][2];
+#pragma unroll
+        for (int w = 0; w < CW; ++w) {
+#pragma unroll
+          for (int s = 0; s < NK; ++s) split44(st[w][2 * s], st[w][2 * s + 1], sh[w][s], sl[w][s]);
+#pragma unroll
+          for (int i = 0; i < 2 * NK; ++i) st[w][i] = next[w][i];
+        }
+        if (j + 1 < ahead) {
+          if constexpr (BUFFERS == 2) fetch_carry(j + 1);
+          load_added(j + 1);
+        }
+        const uint32_t left = base + (j % BUFFERS) * CF * 1024;
+        auto read_tile = [&](auto I) __attribute__((always_inline)) {
+          constexpr int i = decltype(I)::value;
+          static_for<2 * NK>([&](auto M) {
+            constexpr int m = decltype(M)::value;
+            lds_read128<m * 1024>(f[i & 1][m >> 1][m & 1], left + i * NK * 2048);
+          });
+        };
+        read_tile(std::integral_constant<int, 0>{});
+        static_for<2 * NK>([&](auto I) {
+          constexpr int i = decltype(I)::value;
+          static_for<NK>([&](auto S) { lds_wait<0>(f[i & 1][decltype(S)::value][0], f[i & 1][decltype(S)::value][1]); });
+          if constexpr (i + 1 < 2 * NK) read_tile(std::integral_constant<int, i + 1>{});
+          f32x4 half[CW];   // (two sums: a product waits for the one before it)
+#pragma unroll
+          for (int w = 0; w < CW; ++w) half[w] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int part = 0; part < 3; ++part)
+#pragma unroll
+            for (int s = 0; s < NK; ++s)
+#pragma unroll
+              for (int w = 0; w < CW; ++w) {
+                f32x4 &to = (part * NK + s) & 1 ? half[w] : st[w][i];
+                to = mfma16x16x32<B16>(f[i & 1][s][part == 2], part == 1 ? sl[w][s] : sh[w][s], to);
+              }
+#pragma unroll
+          for (int w = 0; w < CW; ++w) st[w][i] += half[w];
+        });
+        if (BUFFERS == 1 && j + 1 < ahead) {
+          lds_barrier();
+          fetch_carry(j + 1);
+        }
+      }
+      lds_barrier();
+    }
+    static_for<GROUPS>([&](auto G) { fetch_group(G, 0); });
+  }
+
   for (int c = 0; c < chunks; ++c) {
     const bool more = c + 1 < chunks;
     // Before a group is used: it has landed (the transfers of the others may be under way; stores only make the wait longer), and every wave is done
@@ -403,7 +528,7 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
         static_for<2>([&](auto P) {
           constexpr int h = decltype(P)::value;
           lds_read128<((it * NK + s) * 2 + h) * 1024>(fw[s & 1][it][h], aw);
-          lds_read128<((it * NK + s) * 2 + h) * 1024>(fo[s & 1][it][h], aq);
+          if constexpr (OUT) lds_read128<((it * NK + s) * 2 + h) * 1024>(fo[s & 1][it][h], aq);
         });
       });
     };
@@ -420,7 +545,7 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
       if constexpr (n < NK) {
         read_step(N);
       } else if constexpr (n == NK) {
-        static_for<kTriangle>([&](auto M) {
+        static_for<(OUT ? kTriangle : 0)>([&](auto M) {
           constexpr int m = decltype(M)::value, it = m < 2 ? m : m / 2 + 1, s = m < 2 ? 0 : m % 2;
           lds_read128<((it * 2 + s) * 2) * 1024>(fb[m][0], ab);
           lds_read128<((it * 2 + s) * 2 + 1) * 1024>(fb[m][1], ab);
@@ -431,7 +556,7 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
       }
     };
     begin(std::integral_constant<int, 0>{});
-    static_for<4 * CW>([&](auto I) { lds_read128<decltype(I)::value * 1024>(u0[decltype(I)::value / 4][decltype(I)::value % 4], au); });
+    static_for<(VALUES ? 4 * CW : 0)>([&](auto I) { lds_read128<decltype(I)::value * 1024>(u0[decltype(I)::value / 4][decltype(I)::value % 4], au); });
     read_step(std::integral_constant<int, 0>{});
     // ---- U = U0 - W S, O = Q S
     f32x4 u[CW][4], o[CW][4];
@@ -444,13 +569,16 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
       static_for<4>([&](auto I) {
         constexpr int it = decltype(I)::value;
         lds_landed(fw[s & 1][it][0], fw[s & 1][it][1]);
-        lds_landed(fo[s & 1][it][0], fo[s & 1][it][1]);
+        if constexpr (OUT) lds_landed(fo[s & 1][it][0], fo[s & 1][it][1]);
       });
       if constexpr (s == 0)
         static_for<4 * CW>([&](auto I) {
           constexpr int w = decltype(I)::value / 4, it = decltype(I)::value % 4;
-          lds_landed(u0[w][it]);
-          u[w][it] = __builtin_bit_cast(f32x4, u0[w][it]), o[w][it] = f32x4{0.f, 0.f, 0.f, 0.f};
+          o[w][it] = u[w][it] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if constexpr (VALUES) {
+            lds_landed(u0[w][it]);
+            u[w][it] = __builtin_bit_cast(f32x4, u0[w][it]);
+          }
         });
 #pragma unroll
       for (int part = 0; part < 3; ++part)
@@ -459,7 +587,7 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
 #pragma unroll
           for (int w = 0; w < CW; ++w) {
             u[w][it] = mfma16x16x32<B16>(fw[s & 1][it][part == 2], part == 1 ? sl[w] : sh[w], u[w][it]);
-            o[w][it] = mfma16x16x32<B16>(part == 1 ? sl[w] : sh[w], fo[s & 1][it][part == 2], o[w][it]);
+            if constexpr (OUT) o[w][it] = mfma16x16x32<B16>(part == 1 ? sl[w] : sh[w], fo[s & 1][it][part == 2], o[w][it]);
           }
     });
     // ---- O += B U, S = decay S + K U
@@ -469,38 +597,40 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
 #pragma unroll
       for (int s = 0; s < 2; ++s) split44(u[w][2 * s], u[w][2 * s + 1], uh[w][s], ul[w][s]);
     begin_step(std::integral_constant<int, NK + 1>{});
-    static_for<kTriangle>([&](auto M) { lds_landed(fb[decltype(M)::value][0], fb[decltype(M)::value][1]); });
+    static_for<(OUT ? kTriangle : 0)>([&](auto M) { lds_landed(fb[decltype(M)::value][0], fb[decltype(M)::value][1]); });
     static_for<2 * NK>([&](auto I) {
       constexpr int i = decltype(I)::value;
       lds_landed(tail[i]);
 #pragma unroll
       for (int w = 0; w < CW; ++w) st[w][i] *= __builtin_bit_cast(f32x4, tail[i]);
     });
-    static_for<4>([&](auto I) {
-      constexpr int it = decltype(I)::value;
+    if constexpr (OUT) {
+      static_for<4>([&](auto I) {
+        constexpr int it = decltype(I)::value;
 #pragma unroll
-      for (int part = 0; part < 3; ++part)
-        static_for<it / 2 + 1>([&](auto S) {
-          constexpr int s = decltype(S)::value;
+        for (int part = 0; part < 3; ++part)
+          static_for<it / 2 + 1>([&](auto S) {
+            constexpr int s = decltype(S)::value;
 #pragma unroll
-          for (int w = 0; w < CW; ++w)
-            o[w][it] = mfma16x16x32<B16>(part == 1 ? ul[w][s] : uh[w][s], fb[triangle(it, s)][part == 2], o[w][it]);
-        });
-    });
+            for (int w = 0; w < CW; ++w)
+              o[w][it] = mfma16x16x32<B16>(part == 1 ? ul[w][s] : uh[w][s], fb[triangle(it, s)][part == 2], o[w][it]);
+          });
+      });
 #pragma unroll
-    for (int w = 0; w < CW; ++w)
+      for (int w = 0; w < CW; ++w)
 #pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        const int t = c * L + 16 * it + r16;
-        T *to = (T *)p.out + (int64_t)(q0 + t) * p.out_stride + head * p.p + col[w] - r16 + 4 * g;
-        if (!live[w] || t >= len) continue;
-        if (quads) {
-          *(u32x2 *)to = pack_quad<Tag>(o[w][it]);
-        } else {
+        for (int it = 0; it < 4; ++it) {
+          const int t = c * L + 16 * it + r16;
+          T *to = (T *)p.out + (int64_t)(q0 + t) * p.out_stride + head * p.p + col[w] - r16 + 4 * g;
+          if (!live[w] || t >= len) continue;
+          if (quads) {
+            *(u32x2 *)to = pack_quad<Tag>(o[w][it]);
+          } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) to[e] = elem<Tag>::st(o[w][it][e]);
+            for (int e = 0; e < 4; ++e) to[e] = elem<Tag>::st(o[w][it][e]);
+          }
         }
-      }
+    }
     static_for<NK>([&](auto P) {   // two state tiles at a time
       constexpr int pair = decltype(P)::value, i0 = 2 * pair;
       if constexpr (pair + 1 < NK) begin_step(std::integral_constant<int, NK + 2 + pair>{});
@@ -521,20 +651,84 @@ __global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q) {
               st[w][i0 + d] = mfma16x16x32<B16>(fk[pair & 1][d][s][part == 2], part == 1 ? ul[w][s] : uh[w][s], st[w][i0 + d]);
     });
   }
-  if (keep) {
+  if constexpr (MODE == ADDED) {
 #pragma unroll
     for (int w = 0; w < CW; ++w)
       if (live[w]) {
 #pragma unroll
         for (int i = 0; i < 2 * NK; ++i)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) *state_at((before + len) & 1, w, i, e) = st[w][i][e];
+          for (int e = 0; e < 4; ++e) sg.added[(int64_t)blockIdx.z * size + in_head(w, i, e)] = st[w][i][e];
+      }
+  } else if constexpr (MODE == CARRY) {
+    // by rows through LDS: the left operand of the product with the state ahead, in the order of its accumulators
+    constexpr int CS = 64 * CW + 4;   // row stride
+    float *cs = (float *)smem;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < CW; ++w)
+#pragma unroll
+      for (int i = 0; i < 2 * NK; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cs[state_row(i, e) * CS + (wave * CW + w) * 16 + r16] = st[w][i][e];
+    __syncthreads();
+    char *carry = sg.carry + ((int64_t)blockIdx.z * p.heads + head) * (4 * NK * NK * 1024) + lane * 16;
+    for (int f = wave; f < 2 * NK * 2 * CW; f += 4) {
+      const int i = f / (2 * CW), s = f - i * (2 * CW), to = tile0 / 2 + s;
+      if (to >= NK) continue;
+      const float *row = cs + ((i >> 1) * 32 + (r16 >> 2) * 8 + (i & 1) * 4 + (r16 & 3)) * CS + 32 * s + 8 * g;
+      u32x4 hi, lo;
+      split44(*(const f32x4 *)row, *(const f32x4 *)(row + 4), hi, lo);
+      *(u32x4 *)(carry + ((i * NK + to) * 2) * 1024) = hi;
+      *(u32x4 *)(carry + ((i * NK + to) * 2 + 1) * 1024) = lo;
+    }
+  } else if (keep && from + len >= all) {
+#pragma unroll
+    for (int w = 0; w < CW; ++w)
+      if (live[w]) {
+#pragma unroll
+        for (int i = 0; i < 2 * NK; ++i)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) *state_at((before + all) & 1, w, i, e) = st[w][i][e];
       }
   }
 }
 
+// (workgroups are dealt to the 8 XCDs in turn: each gets a run of columns and heads, which share all but their part of U0)
+__device__ __forceinline__ int by_xcd(int wide, int heads) {
+  const int all = wide * heads, at = blockIdx.y * wide + blockIdx.x;
+  return all & 7 ? at : (at & 7) * (all >> 3) + (at >> 3);
+}
+template <typename Tag, int NK, int CW, int MODE>
+__global__ void __launch_bounds__(256, 1) delta_walk_kernel(DeltaPrep q, Segments sg) {
+  walk<Tag, NK, CW, MODE>(q, sg, gridDim.x, by_xcd(gridDim.x, q.a.heads));
+}
+// what the segments add, and what becomes of the state ahead of them: workgroups of either beside each other
+template <typename Tag, int NK, int CW>
+__global__ void __launch_bounds__(256, 1) delta_segments_kernel(DeltaPrep q, Segments sg, int added) {
+  const int wide = gridDim.x, at = by_xcd(wide, q.a.heads), head = at / wide, x = at - head * wide;
+  if (x < added) walk<Tag, NK, CW, ADDED>(q, sg, added, head * added + x);
+  else walk<Tag, NK, CW, CARRY>(q, sg, wide - added, head * (wide - added) + x - added);
+}
+
+inline int64_t segment_slots(int n_seqs, int total_q, int seg) { return (int64_t)total_q / (seg * L) + n_seqs; }
+// Chunks of a segment; 0: whole sequences.  A chunk of a whole sequence being 1, one of both launches is 2.1 (3 of 32 key channels), a product with the state ahead 0.6 and
+// the second launch 2.5; a segment of the square root of a third of the longest is the shortest way through both, and there are to be no more
+// workgroups than CUs (each holds one: rounds behind the first cost what they save).  us of the whole call, whole and cut; n x p, heads x sequences:
+//   128 x 128: 4 x 1, 8 chunks 54 and 53, 12: 68 and 58, 24: 115 and 76, 63: 249 and 97; 8 x 3 (the later ones shorter), 24: 122 and 90, 63: 317 and 199;
+//   16 x 3, 12: 82 and 85, 24: 155 and 153, 63: 411 and 382.    64 x 64: 16 x 1, 12: 50 and 42, 63: 177 and 84; 16 x 3, 24: 95 and 77.
+//   32 x 128: 4 x 10 of 2148 tokens at most 106 and 112.   160 x 128: 8 x 1, 24: 136 and 93; 16 x 3, 24: 219 and 219.   128 x 256: 16 x 1, 24: 123 and 103; 16 x 3, 63: 433 and 524.
+inline int pick_segment(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
+  const int tiles = p / 16, workgroups = std::max((tiles + 3) / 4, (tiles + 7) / 8 + (n / 16 + 7) / 8) * heads;   // (of either launch)
+  const int64_t longest = ((int64_t)max_q + L - 1) / L, chunks = ((int64_t)total_q + L - 1) / L;
+  const int64_t room = 256 - (int64_t)n_seqs * workgroups / 2;   // (a sequence's last segment is half a segment)
+  if (room <= 0) return 0;
+  const int64_t seg = std::max<int64_t>({2, (int64_t)std::ceil(std::sqrt(longest / 3.0)), (chunks * workgroups + room - 1) / room});
+  return (n > 32 ? 2.1 : 3.0) * seg + 0.6 * longest / seg + 2.5 < longest ? (int)seg : 0;
+}
+
 template <typename Tag, int NK>
-int launch(const DeltaPrep &q, hipStream_t stream) {
+int launch(const DeltaPrep &q, int seg, hipStream_t stream) {
   const MvDeltaArgs &a = q.a;
   constexpr int RS = NK * 32 + 4, KS = NK * 32 + 8;
   constexpr int QB = L * KS * 2 > L * (L + 4) * 4 ? L * KS * 2 : L * (L + 4) * 4;
@@ -542,19 +736,35 @@ int launch(const DeltaPrep &q, hipStream_t stream) {
   hipLaunchKernelGGL((delta_prepare_kernel<Tag, NK>), dim3((unsigned)chunk_slots(a.n_seqs, a.total_q), a.heads),
                      dim3(kPrepareWaves * 64), L * RS * 4 + L * KS * 2 + QB + (3 + kPrepareWaves) * L * 4, stream, q);
   MV_LAUNCH_CHECK();
-  // two column tiles a wave share every operand read, where that still leaves a workgroup per CU and LDS holds their chunk (up to 128 channels)
-  const int tiles = a.p / 16, wide = (tiles + 7) / 8;
+  const int tiles = a.p / 16, wide = (tiles + 7) / 8, narrow = (tiles + 3) / 4;
   constexpr auto lds = [](int columns) { return (24 * NK + 16 * columns + 17) * 1024; };
+  if (seg) {
+    Segments sg;
+    sg.len = seg * L;
+    const int64_t slots = segment_slots(a.n_seqs, a.total_q, seg), state = (int64_t)a.heads * a.n * a.p;
+    sg.added = (float *)(q.ws + mv_delta_chunk_workspace(a.n_seqs, a.total_q, a.heads, a.p, a.n));
+    sg.first = sg.added + slots * state, sg.carry = (char *)(sg.first + a.n_seqs * state);
+    const int carried = (2 * NK + 7) / 8, by_rows = 32 * NK * (64 * 2 + 4) * 4;
+    const int need = std::max((16 * NK + 32 + 1) * 1024, by_rows);
+    if (int rc = mv_allow_lds<delta_segments_kernel<Tag, NK, 2>>()) return rc;
+    hipLaunchKernelGGL((delta_segments_kernel<Tag, NK, 2>), dim3(wide + carried, a.heads, (unsigned)slots), dim3(256), need, stream, q, sg, wide);
+    MV_LAUNCH_CHECK();
+    if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 1, SEGMENTS>>()) return rc;
+    hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 1, SEGMENTS>), dim3(narrow, a.heads, (unsigned)slots), dim3(256), lds(1), stream, q, sg);
+    MV_LAUNCH_CHECK();
+    return MV_OK;
+  }
+  // two column tiles a wave share every operand read, where that still leaves a workgroup per CU and LDS holds their chunk (up to 128 channels)
   if constexpr (lds(2) <= 160 * 1024) {
     if (tiles > 4 && (int64_t)wide * a.heads * a.n_seqs >= 256) {
-      if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 2>>()) return rc;
-      hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 2>), dim3(wide, a.heads, a.n_seqs), dim3(256), lds(2), stream, q);
+      if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 2, WHOLE>>()) return rc;
+      hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 2, WHOLE>), dim3(wide, a.heads, a.n_seqs), dim3(256), lds(2), stream, q, Segments{});
       MV_LAUNCH_CHECK();
       return MV_OK;
     }
   }
-  if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 1>>()) return rc;
-  hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 1>), dim3((tiles + 3) / 4, a.heads, a.n_seqs), dim3(256), lds(1), stream, q);
+  if (int rc = mv_allow_lds<delta_walk_kernel<Tag, NK, 1, WHOLE>>()) return rc;
+  hipLaunchKernelGGL((delta_walk_kernel<Tag, NK, 1, WHOLE>), dim3(narrow, a.heads, a.n_seqs), dim3(256), lds(1), stream, q, Segments{});
   MV_LAUNCH_CHECK();
   return MV_OK;
 }
@@ -566,6 +776,16 @@ size_t mv_delta_chunk_workspace(int n_seqs, int total_q, int heads, int p, int n
   return (size_t)chunk_slots(n_seqs, total_q) * heads * Layout(n / 32, p).total * 1024;
 }
 
+// (behind the above)
+size_t mv_delta_segments_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
+  if (!mv_delta_chunk_workspace(n_seqs, total_q, heads, p, n)) return 0;
+  const int seg = pick_segment(n_seqs, total_q, max_q, heads, p, n);
+  if (!seg) return 0;
+  const int64_t slots = segment_slots(n_seqs, total_q, seg);
+  if (slots > 65535) return 0;
+  return ((slots + n_seqs) * p + slots * n) * (size_t)heads * n * 4;
+}
+
 int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, hipStream_t stream) {
   const size_t need = mv_delta_chunk_workspace(a.n_seqs, a.total_q, a.heads, a.p, a.n);
   if (!need || !a.workspace) return MV_E_SHAPE;   // larger states: token by token
@@ -574,8 +794,10 @@ int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, hipStream_t stream) {
   if (a.channel_decay && (!mv_aligned16(a.a) || (a.a_stride & 7) || !mv_aligned16(a.dt_bias))) return MV_E_ALIGN;
   const DeltaPrep q{a, (char *)a.workspace};
   if (!a.channel_decay && dtype == MV_BF16) return mv_delta_scalar_launch(a, stream);
+  const size_t more = mv_delta_segments_workspace(a.n_seqs, a.total_q, a.max_q, a.heads, a.p, a.n);
+  const int seg = more && (size_t)a.ws_bytes >= need + more ? pick_segment(a.n_seqs, a.total_q, a.max_q, a.heads, a.p, a.n) : 0;
 #define MV_DN(NK_) \
-  if (a.n == 32 * NK_) return dtype == MV_BF16 ? launch<bf16_tag, NK_>(q, stream) : launch<f16_tag, NK_>(q, stream)
+  if (a.n == 32 * NK_) return dtype == MV_BF16 ? launch<bf16_tag, NK_>(q, seg, stream) : launch<f16_tag, NK_>(q, seg, stream)
   MV_DN(1);
   MV_DN(2);
   MV_DN(3);
