@@ -6,7 +6,7 @@
 //     B_ij = g_i f_j e^{r_i - r_j} (q_i k_j)             o_i = e^{r_i} g_i (q_i S) + sum_{j <= i} B_ij u_j
 //     S <- e^{r_last} S + sum_j k_j (e^{r_last - r_j} f_j u_j)^T
 // so k and q enter every product as they are in memory (exact in bf16) and only T, B, S and U are sums of two bf16 numbers.  Two launches:
-//   prepare: T, B and three factors per token, one workgroup per (chunk, head), 25 KiB of workspace;
+//   prepare: T, B and three factors per token, one workgroup per (chunk, pair of heads with the same k and q), 25 KiB of workspace a head;
 //   walk:    chunks one behind the other, one workgroup per (sequence, head, columns); rows of k, q and v come from the inputs, transposed out of
 //            LDS where the state takes them in; the next chunk lands while this one is multiplied.
 #include "delta_chunk.h"
@@ -21,115 +21,137 @@ constexpr int kB = 2 * kTriangle, kFactors = 4 * kTriangle, kScalarTotal = kFact
 __device__ __forceinline__ int row_chunk(int lane) { return (lane & 3) ^ ((lane >> 4) & 3); }
 __device__ __forceinline__ int row_place(int row, int chunk) { return row * 4 + (chunk ^ ((row >> 2) & 3)); }
 
-template <int NK>
-__global__ void __launch_bounds__(256, NK < 5 ? 4 : 3) delta_scalar_prepare_kernel(DeltaPrep q) {
+// Workgroup = HEADS heads of four waves each that share k and q of a chunk: the products k k^T and q k^T are theirs in common, decays, solution and results
+// their own.  Bound by the latency of its phases, which 16 to 20 waves a CU cover in part: everything is asked for from memory at the start.
+template <int NK, int HEADS>
+__global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(DeltaPrep q) {
   typedef uint16_t T;
-  constexpr int N = NK * 32, KS = N + 8;   // LDS row stride
+  typedef elem<B16>::T E;
+  constexpr int N = NK * 32, KS = N + 8, W = 4 * HEADS, PARTS = W;   // LDS row stride; threads a token
   const MvDeltaArgs &p = q.a;
-  constexpr int QB = L * KS * 2 > L * TS * 4 ? L * KS * 2 : L * TS * 4;
-  __shared__ __attribute__((aligned(16))) char smem[L * KS * 2 + QB + 4 * L * 4];
-  T *ks = (T *)smem, *qs = ks + L * KS;   // [L][KS]; later (from qs on) -A, then T
-  float *ts = (float *)qs, *fk = (float *)(smem + L * KS * 2 + QB), *fq = fk + L, *bt = fq + L, *rs = bt + L;
+  constexpr int QB = L * KS * 2 > L * TS * 4 ? L * KS * 2 : L * TS * 4, KB = HEADS > 1 ? QB : L * KS * 2;
+  __shared__ __attribute__((aligned(16))) char smem[KB + QB + (2 + 2 * HEADS) * L * 4];
+  T *ks = (T *)smem, *qs = (T *)(smem + KB);   // [L][KS]; later -A, then T, of the first head from qs on, of the second from ks on
+  float *fk = (float *)(smem + KB + QB), *fq = fk + L, *bts = fq + L, *rss = bts + HEADS * L;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
-  const int head = blockIdx.y, seq = chunk_sequence(p, blockIdx.x);
+  const int of = HEADS > 1 ? wave >> 2 : 0, head = blockIdx.y * HEADS + of;   // (of this wave)
+  const int seq = chunk_sequence(p, blockIdx.x);
   const int q0 = p.cu_q[seq], len = p.cu_q[seq + 1] - q0, t0 = ((int)blockIdx.x - q0 / L - seq) * L;
   if (t0 >= len) return;
   const int nt = min(L, len - t0), grp = head / (p.heads / p.groups);
   char *ws = q.ws + ((int64_t)blockIdx.x * p.heads + head) * kScalarTotal * 1024;
   const T *x = (const T *)p.x + (int64_t)(q0 + t0) * p.x_stride;
+  float *ts = (float *)(of ? (char *)ks : (char *)qs), *bt = bts + of * L, *rs = rss + of * L;
 
-  // ---- k, q (tokens behind the end: zeros) and their lengths: four threads a token
+  // ---- k, q (tokens behind the end: zeros) and their lengths: PARTS threads a token; a head's first wave its betas and log2 decays, a lane a token
   {
-    const int t = tid >> 2, part = tid & 3;
+    const int t = tid / PARTS, part = tid % PARTS;
     const T *row = x + (int64_t)min(t, nt - 1) * p.x_stride + grp * N;
+    constexpr int PIECES = N / 8, PER = (PIECES + PARTS - 1) / PARTS;
+    u32x4 a[PER], b[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = min(part + PARTS * i, PIECES - 1) * 8;
+      a[i] = *(const u32x4 *)(row + p.k_off + c), b[i] = *(const u32x4 *)(row + p.q_off + c);
+    }
+    const bool leads = (wave & 3) == 0;
+    float beta = 0.f, decay = 0.f, bias = 0.f, rate = 0.f;
+    if (leads) {
+      const int64_t at = q0 + t0 + min(lane, nt - 1);
+      beta = elem<B16>::ld(((const E *)p.beta)[at * p.beta_stride + head]), decay = elem<B16>::ld(((const E *)p.a)[at * p.a_stride + head]);
+      rate = elem<B16>::ld(((const E *)p.a_log)[head]), bias = elem<B16>::ld(((const E *)p.dt_bias)[head]);
+    }
     float sk = 0.f, sq = 0.f;
 #pragma unroll
-    for (int s = 0; s < NK; ++s) {
-      const int c = part * 8 + 32 * s;
-      u32x4 a = *(const u32x4 *)(row + p.k_off + c), b = *(const u32x4 *)(row + p.q_off + c);
-      if (t >= nt) a = b = u32x4{0u, 0u, 0u, 0u};
+    for (int i = 0; i < PER; ++i) {
+      const int c = (part + PARTS * i) * 8;
+      if (PIECES % PARTS && c >= N) continue;
+      if (t >= nt) a[i] = b[i] = u32x4{0u, 0u, 0u, 0u};
       float fa[8], fb[8];
-      unpack8<B16>(a, fa);
-      unpack8<B16>(b, fb);
+      unpack8<B16>(a[i], fa);
+      unpack8<B16>(b[i], fb);
 #pragma unroll
       for (int j = 0; j < 8; ++j) sk = fmaf(fa[j], fa[j], sk), sq = fmaf(fb[j], fb[j], sq);
-      *(u32x4 *)(ks + t * KS + c) = a;
-      *(u32x4 *)(qs + t * KS + c) = b;
+      *(u32x4 *)(ks + t * KS + c) = a[i];
+      *(u32x4 *)(qs + t * KS + c) = b[i];
     }
-    sk += __shfl_xor(sk, 1, 64), sq += __shfl_xor(sq, 1, 64);
-    sk += __shfl_xor(sk, 2, 64), sq += __shfl_xor(sq, 2, 64);
-    if (part == 0) {
-      fk[t] = 1.f / sqrtf(sk + p.unit_eps), fq[t] = p.q_scale / sqrtf(sq + p.unit_eps);
-      bt[t] = t < nt ? sigmoid_f32(elem<B16>::ld(((const elem<B16>::T *)p.beta)[(int64_t)(q0 + t0 + t) * p.beta_stride + head])) : 0.f;
-    }
-  }
-  if (wave == 0) {   // log2 decays, summed over the tokens
-    typedef elem<B16>::T E;
-    const float rate = -expf(elem<B16>::ld(((const E *)p.a_log)[head])) * 1.4426950408889634f;
-    const float z = elem<B16>::ld(((const E *)p.a)[(int64_t)(q0 + t0 + min(lane, nt - 1)) * p.a_stride + head]) + elem<B16>::ld(((const E *)p.dt_bias)[head]);
-    float sum = lane < nt ? rate * softplus_fast(z) : 0.f;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const float left = __shfl_up(sum, o, 64);
-      if (lane >= o) sum += left;
+    for (int o = 1; o < PARTS; o <<= 1) sk += __shfl_xor(sk, o, 64), sq += __shfl_xor(sq, o, 64);
+    if (part == 0) fk[t] = 1.f / sqrtf(sk + p.unit_eps), fq[t] = p.q_scale / sqrtf(sq + p.unit_eps);
+    if (leads) {
+      rate = -expf(rate) * 1.4426950408889634f;
+      float sum = lane < nt ? rate * softplus_fast(decay + bias) : 0.f;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const float left = __shfl_up(sum, o, 64);
+        if (lane >= o) sum += left;
+      }
+      rs[lane] = sum, bt[lane] = lane < nt ? sigmoid_f32(beta) : 0.f;
     }
-    rs[lane] = sum;
   }
   __syncthreads();
-  if (tid < L) {
+  if ((wave & 3) == 0) {
     float *f = (float *)(ws + kFactors * 1024);
     const float last = rs[L - 1];
-    const bool is = tid < nt;
-    f[tid] = is ? fk[tid] * __builtin_amdgcn_exp2f(rs[tid]) : 0.f;
-    f[L + tid] = is ? fq[tid] * __builtin_amdgcn_exp2f(rs[tid]) : 0.f;
-    f[2 * L + tid] = is ? fk[tid] * __builtin_amdgcn_exp2f(last - rs[tid]) : 0.f;
-    f[3 * L + tid] = __builtin_amdgcn_exp2f(last);
+    const bool is = lane < nt;
+    f[lane] = is ? fk[lane] * __builtin_amdgcn_exp2f(rs[lane]) : 0.f;
+    f[L + lane] = is ? fq[lane] * __builtin_amdgcn_exp2f(rs[lane]) : 0.f;
+    f[2 * L + lane] = is ? fk[lane] * __builtin_amdgcn_exp2f(last - rs[lane]) : 0.f;
+    f[3 * L + lane] = __builtin_amdgcn_exp2f(last);
   }
 
   // ---- A and B by blocks of 16 x 16 tokens; a lane gets row r16, columns 4 g ..
-  f32x4 blk[3];
+  constexpr int BW = (10 + W - 1) / W;
+  f32x4 blk[BW][HEADS];
 #pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    const int idx = wave + 4 * m;
+  for (int m = 0; m < BW; ++m) {
+    const int idx = wave + W * m;
     if (idx >= 10) continue;
     int I, J;
     block_place(idx, I, J);
     const T *ki = ks + (16 * I + r16) * KS + 8 * g, *kj = ks + (16 * J + r16) * KS + 8 * g, *qi = qs + (16 * I + r16) * KS + 8 * g;
-    f32x4 A = {0.f, 0.f, 0.f, 0.f}, B = A;
+    f32x4 kk = {0.f, 0.f, 0.f, 0.f}, qk = kk;
 #pragma unroll
     for (int s = 0; s < NK; ++s) {
       const u32x4 right = *(const u32x4 *)(kj + 32 * s);
-      A = mfma16x16x32<B16>(right, *(const u32x4 *)(ki + 32 * s), A);
-      B = mfma16x16x32<B16>(right, *(const u32x4 *)(qi + 32 * s), B);
+      kk = mfma16x16x32<B16>(right, *(const u32x4 *)(ki + 32 * s), kk);
+      qk = mfma16x16x32<B16>(right, *(const u32x4 *)(qi + 32 * s), qk);
     }
     const int i = 16 * I + r16, j0 = 16 * J + 4 * g;
-    const float ri = rs[i], fi = -bt[i] * fk[i], gi = fq[i];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float f = fk[j0 + e] * __builtin_amdgcn_exp2f(j0 + e <= i ? ri - rs[j0 + e] : 0.f);
-      A[e] = j0 + e < i ? A[e] * (fi * f) : 0.f;
-      B[e] = j0 + e <= i ? B[e] * (gi * f) : 0.f;
+    for (int h = 0; h < HEADS; ++h) {
+      const float *r = rss + h * L;
+      const float ri = r[i], fi = -bts[h * L + i] * fk[i], gi = fq[i];
+      f32x4 A, B;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float f = fk[j0 + e] * __builtin_amdgcn_exp2f(j0 + e <= i ? ri - r[j0 + e] : 0.f);
+        A[e] = j0 + e < i ? kk[e] * (fi * f) : 0.f;
+        B[e] = j0 + e <= i ? qk[e] * (gi * f) : 0.f;
+      }
+      blk[m][h] = A;   // (the negative)
+      u32x2 hi, lo;
+      split4(B, hi, lo);
+      u32x2 *dst = (u32x2 *)(ws + (h - of) * kScalarTotal * 1024 + (kB + triangle(I, J >> 1) * 2) * 1024 + lane * 16) + (J & 1);
+      dst[0] = hi;
+      dst[128] = lo;
+      if (I == J && (I & 1) == 0) dst[1] = dst[129] = u32x2{0u, 0u};   // the columns behind, in the same step of 32
     }
-    blk[m] = A;   // (the negative)
-    u32x2 hi, lo;
-    split4(B, hi, lo);
-    u32x2 *dst = (u32x2 *)(ws + (kB + triangle(I, J >> 1) * 2) * 1024 + lane * 16) + (J & 1);
-    dst[0] = hi;
-    dst[128] = lo;
-    if (I == J && (I & 1) == 0) dst[1] = dst[129] = u32x2{0u, 0u};   // the columns behind, in the same step of 32
   }
-  __syncthreads();   // q is done with
+  __syncthreads();   // k and q are done with
 #pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    const int idx = wave + 4 * m;
+  for (int m = 0; m < BW; ++m) {
+    const int idx = wave + W * m;
     if (idx >= 10) continue;
     int I, J;
     block_place(idx, I, J);
-    *(f32x4 *)(ts + (16 * I + r16) * TS + 16 * J + 4 * g) = blk[m];
+#pragma unroll
+    for (int h = 0; h < HEADS; ++h)
+      *(f32x4 *)((float *)(h ? (char *)ks : (char *)qs) + (16 * I + r16) * TS + 16 * J + 4 * g) = blk[m][h];
   }
   __syncthreads();
-  solve_chunk(ts, bt, wave, lane);
-  for (int m = wave; m < kTriangle; m += 4) {
+  solve_chunk(ts, bt, wave & 3, lane);
+  for (int m = wave & 3; m < kTriangle; m += 4) {
     u32x4 hi, lo;
     solution_operand(ts, m, lane, hi, lo);
     u32x4 *dst = (u32x4 *)(ws + m * 2 * 1024) + lane;
@@ -422,7 +444,9 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
 template <int NK>
 int launch(const DeltaPrep &q, hipStream_t stream) {
   const MvDeltaArgs &a = q.a;
-  hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK>), dim3((unsigned)chunk_slots(a.n_seqs, a.total_q), a.heads), dim3(256), 0, stream, q);
+  const unsigned slots = (unsigned)chunk_slots(a.n_seqs, a.total_q);
+  if (a.heads / a.groups % 2 == 0) hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 2>), dim3(slots, a.heads / 2), dim3(512), 0, stream, q);
+  else hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 1>), dim3(slots, a.heads), dim3(256), 0, stream, q);
   MV_LAUNCH_CHECK();
   // Eight waves where workgroups of four would be more than the CUs, of which each holds one, and LDS holds their chunk (up to 128 channels: at
   // 160 four waves of one tile it is, 16 heads and 16 sequences of 1000 tokens 201 us, where four waves of two tiles took 211)
