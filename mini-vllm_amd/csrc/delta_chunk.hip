@@ -24,6 +24,9 @@
 
 namespace {
 
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
 constexpr float kRange = 60.f;     // log2
 constexpr int kPrepareWaves = 8;
 
@@ -34,14 +37,19 @@ struct Layout {
   __host__ __device__ constexpr Layout(int nk, int p) : u0(16 * nk), k(16 * nk + p / 4), b(24 * nk + p / 4), tail(24 * nk + p / 4 + 16), total(24 * nk + p / 4 + 17) {}
 };
 
+// Workgroup = 8 waves of a (chunk, head).  Bound by its vector arithmetic (some 15 000 instructions of a wave, a tenth of them exponentials) and by the latency
+// of its phases: everything is asked for from memory at the start, blocks of one row of A and B share that row's factors, K is made beside the
+// solution, and the solution is split into operands once.  3 sequences of 4011 tokens and less, 8 heads of 128 x 128 (1256 workgroups, two a CU):
+// 107 us with every block's factors, all of K and W by four waves, and operands of T by each item -> 84.
 template <typename Tag, int NK>
-__global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(DeltaPrep q) {
+__global__ void __launch_bounds__(kPrepareWaves * 64, NK < 5 ? 4 : 2) delta_prepare_kernel(DeltaPrep q) {
   typedef typename elem<Tag>::T T;
   constexpr int N = NK * 32, W = kPrepareWaves, RS = N + 4, KS = N + 8;   // LDS row strides: fp32, 16-bit
+  static_assert(W == 8, "the blocks are dealt to eight waves");
   const MvDeltaArgs &p = q.a;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   float *rs = (float *)smem;                              // [L][RS] running log2 decays
-  T *ks = (T *)(smem + L * RS * 4), *qs = ks + L * KS;    // [L][KS]; later (from qs on) -A, then T
+  T *ks = (T *)(smem + L * RS * 4), *qs = ks + L * KS;    // [L][KS]; later (from qs on) -A, then T, then its operands
   float *ts = (float *)qs;                                // [L][TS]
   constexpr int QB = L * KS * 2 > L * TS * 4 ? L * KS * 2 : L * TS * 4;
   float *fk = (float *)((char *)qs + QB), *fq = fk + L, *bt = fq + L, *part_sums = bt + L;   // [W][64]
@@ -55,49 +63,82 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(De
   char *ws = q.ws + ((int64_t)blockIdx.x * p.heads + head) * lay.total * 1024;
   const T *x = (const T *)p.x + (int64_t)(q0 + t0) * p.x_stride;
 
-  // ---- k, q (tokens behind the end: zeros) and their lengths: eight threads a token
+  // ---- everything that comes from memory: k and q, eight threads a token; the decays; v of this wave's (first) 16 columns
+  constexpr int KQ = (N + 63) / 64, AP = (L * N / 8 + W * 64 - 1) / (W * 64);   // pieces of 8 channels a thread
+  const int tt = tid >> 3, part = tid & 7, columns = p.p / 16;
+  u32x4 kraw[KQ], qraw[KQ], araw[AP], braw[AP];
   {
-    const int t = tid >> 3, part = tid & 7;
-    const T *row = x + (int64_t)min(t, nt - 1) * p.x_stride;
+    const T *row = x + (int64_t)min(tt, nt - 1) * p.x_stride + grp * N;
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) {
+      const int c = min(part * 8 + 64 * i, N - 8);
+      kraw[i] = *(const u32x4 *)(row + p.k_off + c), qraw[i] = *(const u32x4 *)(row + p.q_off + c);
+    }
+  }
+  const T *a = (const T *)p.a + (int64_t)(q0 + t0) * p.a_stride, *bias = (const T *)p.dt_bias;
+  const T *of_beta = (const T *)p.beta + (int64_t)(q0 + t0 + min(tt, nt - 1)) * p.beta_stride + head;
+  const float beta = elem<Tag>::ld(*of_beta), log_rate = elem<Tag>::ld(((const T *)p.a_log)[head]);
+  float a_head = 0.f, b_head = 0.f;
+  if (p.channel_decay) {
+#pragma unroll
+    for (int i = 0; i < AP; ++i) {
+      const int at = min(tid + i * W * 64, L * N / 8 - 1), t = at / (N / 8), c = (at - t * (N / 8)) * 8;
+      araw[i] = *(const u32x4 *)(a + (int64_t)min(t, nt - 1) * p.a_stride + head * N + c);
+      braw[i] = *(const u32x4 *)(bias + head * N + c);
+    }
+  } else {
+    a_head = elem<Tag>::ld(a[(int64_t)min(tt, nt - 1) * p.a_stride + head]), b_head = elem<Tag>::ld(bias[head]);
+  }
+  T vraw[16];
+  auto load_values = [&](int ct) __attribute__((always_inline)) {
+    const T *v = x + head * p.p + ct * 16 + r16;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) vraw[e] = v[(int64_t)min(16 * (e >> 2) + 4 * g + (e & 3), nt - 1) * p.x_stride];
+  };
+  load_values(min(wave, columns - 1));
+
+  // ---- k, q (tokens behind the end: zeros) and their lengths
+  {
     float sk = 0.f, sq = 0.f;
-    for (int c = part * 8; c < N; c += 64) {
-      u32x4 a = *(const u32x4 *)(row + p.k_off + grp * N + c), b = *(const u32x4 *)(row + p.q_off + grp * N + c);
-      if (t >= nt) a = b = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) {
+      const int c = part * 8 + 64 * i;
+      if (N % 64 && c >= N) continue;
+      if (tt >= nt) kraw[i] = qraw[i] = u32x4{0u, 0u, 0u, 0u};
       float fa[8], fb[8];
-      unpack8<Tag>(a, fa);
-      unpack8<Tag>(b, fb);
+      unpack8<Tag>(kraw[i], fa);
+      unpack8<Tag>(qraw[i], fb);
 #pragma unroll
       for (int j = 0; j < 8; ++j) sk = fmaf(fa[j], fa[j], sk), sq = fmaf(fb[j], fb[j], sq);
-      *(u32x4 *)(ks + t * KS + c) = a;
-      *(u32x4 *)(qs + t * KS + c) = b;
+      *(u32x4 *)(ks + tt * KS + c) = kraw[i];
+      *(u32x4 *)(qs + tt * KS + c) = qraw[i];
     }
 #pragma unroll
     for (int o = 1; o <= 4; o <<= 1) sk += __shfl_xor(sk, o, 64), sq += __shfl_xor(sq, o, 64);
     if (part == 0) {
-      fk[t] = 1.f / sqrtf(sk + p.unit_eps), fq[t] = p.q_scale / sqrtf(sq + p.unit_eps);
-      bt[t] = t < nt ? sigmoid_f32(elem<Tag>::ld(((const T *)p.beta)[(int64_t)(q0 + t0 + t) * p.beta_stride + head])) : 0.f;
+      fk[tt] = 1.f / sqrtf(sk + p.unit_eps), fq[tt] = p.q_scale / sqrtf(sq + p.unit_eps);
+      bt[tt] = tt < nt ? sigmoid_f32(beta) : 0.f;
     }
   }
   // ---- log2 decays, summed over the tokens
   {
-    const float rate = -expf(elem<Tag>::ld(((const T *)p.a_log)[head])) * 1.4426950408889634f;
-    const T *a = (const T *)p.a + (int64_t)(q0 + t0) * p.a_stride, *bias = (const T *)p.dt_bias;
+    const float rate = -expf(log_rate) * 1.4426950408889634f;
     if (p.channel_decay) {
-      for (int i = tid; i < L * N / 8; i += W * 64) {
-        const int t = i / (N / 8), c = (i - t * (N / 8)) * 8;
+#pragma unroll
+      for (int i = 0; i < AP; ++i) {
+        const int at = tid + i * W * 64, t = at / (N / 8), c = (at - t * (N / 8)) * 8;
+        if (L * N / 8 % (W * 64) && at >= L * N / 8) continue;
         float f[8], b[8];
-        unpack8<Tag>(*(const u32x4 *)(a + (int64_t)min(t, nt - 1) * p.a_stride + head * N + c), f);
-        unpack8<Tag>(*(const u32x4 *)(bias + head * N + c), b);
+        unpack8<Tag>(araw[i], f);
+        unpack8<Tag>(braw[i], b);
 #pragma unroll
         for (int j = 0; j < 8; ++j) f[j] = t < nt ? rate * softplus_fast(f[j] + b[j]) : 0.f;
         f32x4 *dst = (f32x4 *)(rs + t * RS + c);
         dst[0] = f32x4{f[0], f[1], f[2], f[3]}, dst[1] = f32x4{f[4], f[5], f[6], f[7]};
       }
     } else {
-      const float b = elem<Tag>::ld(bias[head]);
-      const int t = tid >> 3;
-      const float v = t < nt ? rate * softplus_fast(elem<Tag>::ld(a[(int64_t)t * p.a_stride + head]) + b) : 0.f;
-      for (int c = tid & 7; c < N; c += 8) rs[t * RS + c] = v;
+      const float v = tt < nt ? rate * softplus_fast(a_head + b_head) : 0.f;
+      for (int c = part; c < N; c += 8) rs[tt * RS + c] = v;
     }
     __syncthreads();
     // a thread TW of a channel's tokens (the threads of a wave: adjacent channels); then the sums ahead are added
@@ -125,170 +166,206 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, 4) delta_prepare_kernel(De
   }
   __syncthreads();
 
-  // ---- A and B by blocks of 16 x 16 tokens (rows I, columns J <= I), ten of them over the waves; a lane gets row r16, columns 4 g ..
-  constexpr int BW = (10 + W - 1) / W;
-  f32x4 blk[BW];
+  // ---- A and B by blocks of 16 x 16 tokens (rows I, columns J <= I); a lane gets row r16, columns 4 g ..  A wave has one diagonal block or one or two
+  // others of a row, which share the row's factors: 3: 0 1 | 2: 0 1 | 3: 2 | 1: 0 | the diagonal
+  const int I = wave >= 4 ? 7 - wave : wave == 3 ? 1 : wave == 1 ? 2 : 3, J0 = wave >= 4 ? I : wave == 2 ? 2 : 0, blocks = wave < 2 ? 2 : 1;
+  f32x4 blkA[2], blkB[2];
+  {
+    const bool diagonal = wave >= 4;
+    const int ref = diagonal ? 16 * I + 7 : 16 * I - 1;
+    const float *ri = rs + (16 * I + r16) * RS + 8 * g, *rr = rs + ref * RS + 8 * g;
+    const T *ki = ks + (16 * I + r16) * KS + 8 * g, *qi = qs + (16 * I + r16) * KS + 8 * g;
 #pragma unroll
-  for (int m = 0; m < BW; ++m) {
-    const int idx = wave + W * m;
-    if (idx >= 10) continue;
-    int I, J;
-    block_place(idx, I, J);
-    const int ref = I == J ? 16 * I + 7 : 16 * I - 1;
-    const float *ri = rs + (16 * I + r16) * RS + 8 * g, *rj = rs + (16 * J + r16) * RS + 8 * g, *rr = rs + ref * RS + 8 * g;
-    const T *ki = ks + (16 * I + r16) * KS + 8 * g, *kj = ks + (16 * J + r16) * KS + 8 * g, *qi = qs + (16 * I + r16) * KS + 8 * g;
-    f32x4 A = {0.f, 0.f, 0.f, 0.f}, B = A;
+    for (int m = 0; m < 2; ++m) blkA[m] = blkB[m] = f32x4{0.f, 0.f, 0.f, 0.f};
     bool fits = true;   // (the sums fall, so the ends of a diagonal block decide)
-    if (I == J)
+    if (diagonal)
       for (int c = lane; c < N; c += 64)
         fits = fits && rs[16 * I * RS + c] - rs[ref * RS + c] <= kRange && rs[ref * RS + c] - rs[(16 * I + 15) * RS + c] <= kRange;
 #pragma unroll
     for (int s = 0; s < NK; ++s) {
-      float fi[8], fj[8], fp[8];
+      float fi[8], fp[8], rc[8];
       unpack8<Tag>(*(const u32x4 *)(ki + 32 * s), fi);
-      unpack8<Tag>(*(const u32x4 *)(kj + 32 * s), fj);
       unpack8<Tag>(*(const u32x4 *)(qi + 32 * s), fp);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const f32x4 a = *(const f32x4 *)(ri + 32 * s + 4 * h), b = *(const f32x4 *)(rj + 32 * s + 4 * h), c = *(const f32x4 *)(rr + 32 * s + 4 * h);
+        const f32x4 ra = *(const f32x4 *)(ri + 32 * s + 4 * h), c = *(const f32x4 *)(rr + 32 * s + 4 * h);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float el = __builtin_amdgcn_exp2f(a[e] - c[e]);
-          fi[4 * h + e] *= el, fp[4 * h + e] *= el;
-          fj[4 * h + e] *= __builtin_amdgcn_exp2f(c[e] - b[e]);
+          const float el = __builtin_amdgcn_exp2f(ra[e] - c[e]);
+          fi[4 * h + e] *= el, fp[4 * h + e] *= el, rc[4 * h + e] = c[e];
         }
       }
-      u32x4 ih, il, jh, jl, ph, pl;
+      u32x4 ih, il, ph, pl;
       split8(fi, ih, il);
-      split8(fj, jh, jl);
       split8(fp, ph, pl);
-      A = mfma3(jh, jl, ih, il, A);
-      B = mfma3(jh, jl, ph, pl, B);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        if (m >= blocks) continue;
+        const int j = 16 * (J0 + m) + r16;
+        const float *rj = rs + j * RS + 8 * g + 32 * s;
+        float fj[8];
+        unpack8<Tag>(*(const u32x4 *)(ks + j * KS + 8 * g + 32 * s), fj);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 rb = *(const f32x4 *)(rj + 4 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) fj[4 * h + e] *= __builtin_amdgcn_exp2f(rc[4 * h + e] - rb[e]);
+        }
+        u32x4 jh, jl;
+        split8(fj, jh, jl);
+        blkA[m] = mfma3(jh, jl, ih, il, blkA[m]);
+        blkB[m] = mfma3(jh, jl, ph, pl, blkB[m]);
+      }
     }
-    const int i = 16 * I + r16, j0 = 16 * J + 4 * g;
-    if (I == J && !__all(fits)) {
+    const int i = 16 * I + r16;
+    if (diagonal && !__all(fits)) {
+      const int j0 = 16 * I + 4 * g;
       for (int e = 0; e < 4; ++e) {
-        float a = 0.f, b = 0.f;
+        float sa = 0.f, sb = 0.f;
         if (j0 + e <= i)
           for (int c = 0; c < N; ++c) {
             const float k = elem<Tag>::ld(ks[(j0 + e) * KS + c]) * __builtin_amdgcn_exp2f(rs[i * RS + c] - rs[(j0 + e) * RS + c]);
-            a = fmaf(elem<Tag>::ld(ks[i * KS + c]), k, a);
-            b = fmaf(elem<Tag>::ld(qs[i * KS + c]), k, b);
+            sa = fmaf(elem<Tag>::ld(ks[i * KS + c]), k, sa);
+            sb = fmaf(elem<Tag>::ld(qs[i * KS + c]), k, sb);
           }
-        A[e] = a, B[e] = b;
+        blkA[0][e] = sa, blkB[0][e] = sb;
       }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      A[e] = j0 + e < i ? -A[e] * (bt[i] * fk[i] * fk[j0 + e]) : 0.f;
-      B[e] = j0 + e <= i ? B[e] * (fq[i] * fk[j0 + e]) : 0.f;
+    for (int m = 0; m < 2; ++m) {
+      if (m >= blocks) continue;
+      const int J = J0 + m, j0 = 16 * J + 4 * g;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        blkA[m][e] = j0 + e < i ? -blkA[m][e] * (bt[i] * fk[i] * fk[j0 + e]) : 0.f;   // (the negative)
+        blkB[m][e] = j0 + e <= i ? blkB[m][e] * (fq[i] * fk[j0 + e]) : 0.f;
+      }
+      // B as an operand whose k order is that of an accumulator pair: key 16 (e >> 2) + 4 g + (e & 3) of a step of 32
+      u32x2 hi, lo;
+      split4(blkB[m], hi, lo);
+      u32x2 *dst = (u32x2 *)(ws + (lay.b + (I * 2 + (J >> 1)) * 2) * 1024 + lane * 16) + (J & 1);
+      dst[0] = hi;
+      dst[128] = lo;
+      if (I == J && (I & 1) == 0) dst[1] = dst[129] = u32x2{0u, 0u};   // the columns behind, in the same step of 32
     }
-    blk[m] = A;   // (the negative)
-    // B as an operand whose k order is that of an accumulator pair: key 16 (e >> 2) + 4 g + (e & 3) of a step of 32
-    u32x2 hi, lo;
-    split4(B, hi, lo);
-    u32x2 *dst = (u32x2 *)(ws + (lay.b + (I * 2 + (J >> 1)) * 2) * 1024 + lane * 16) + (J & 1);
-    dst[0] = hi;
-    dst[128] = lo;
-    if (I == J && (I & 1) == 0) dst[1] = dst[129] = u32x2{0u, 0u};   // the columns behind, in the same step of 32
   }
 
-  // ---- the operands that meet S and U: e^r q by rows; e^(r_last - r) k by state rows, in the order of the walk's accumulators
-  for (int f = wave; f < 4 * NK; f += W) {
-    const int it = f / NK, s = f - it * NK, t = 16 * it + r16, c = 32 * s + 8 * g;
-    float v[8];
-    u32x4 hi, lo;
-    unpack8<Tag>(*(const u32x4 *)(qs + t * KS + c), v);
-    const float w = fq[t];
+  // ---- e^r q by rows (the waves with one block)
+  if (wave >= 2) {
+    for (int f = wave - 2; f < 4 * NK; f += W - 2) {
+      const int it = f / NK, s = f - it * NK, t = 16 * it + r16, c = 32 * s + 8 * g;
+      float v[8];
+      u32x4 hi, lo;
+      unpack8<Tag>(*(const u32x4 *)(qs + t * KS + c), v);
+      const float w = fq[t];
+      const f32x4 r0 = *(const f32x4 *)(rs + t * RS + c), r1 = *(const f32x4 *)(rs + t * RS + c + 4);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] *= w * __builtin_amdgcn_exp2f(rs[t * RS + c + e]);
-    split8(v, hi, lo);
-    u32x4 *dst = (u32x4 *)(ws + (8 * NK + f * 2) * 1024) + lane;
-    dst[0] = hi, dst[64] = lo;
+      for (int e = 0; e < 8; ++e) v[e] *= w * __builtin_amdgcn_exp2f(e < 4 ? r0[e & 3] : r1[e & 3]);
+      split8(v, hi, lo);
+      u32x4 *dst = (u32x4 *)(ws + (8 * NK + f * 2) * 1024) + lane;
+      dst[0] = hi, dst[64] = lo;
+    }
   }
   for (int c = tid; c < N; c += W * 64) ((float *)(ws + lay.tail * 1024))[c] = __builtin_amdgcn_exp2f(rs[(L - 1) * RS + c]);
   __syncthreads();   // q is done with
 #pragma unroll
-  for (int m = 0; m < BW; ++m) {
-    const int idx = wave + W * m;
-    if (idx >= 10) continue;
-    int I, J;
-    block_place(idx, I, J);
-    *(f32x4 *)(ts + (16 * I + r16) * TS + 16 * J + 4 * g) = blk[m];
-  }
+  for (int m = 0; m < 2; ++m)
+    if (m < blocks) *(f32x4 *)(ts + (16 * I + r16) * TS + 16 * (J0 + m) + 4 * g) = blkA[m];
   __syncthreads();
 
-  solve_chunk(ts, bt, wave, lane);
-
-  // ---- by 32 channels: K = e^(r_last - r) k by state rows, in the order of the walk's accumulators, and -W = -T e^r k by tokens;
-  // by 16 columns of v: U0 = T v
-  for (int item = wave; item < NK + p.p / 16; item += W) {
-    if (item < NK) {
-      f32x4 acc[2][4];
+  // k of a state tile (in the order of the walk's accumulators), scaled: tokens 32 s + 16 (e >> 2) + 4 g + (e & 3) of channel c; and its sums of decays
+  auto columns_of = [&](int i, int s, int &c, float (&k)[8], float (&r)[8]) __attribute__((always_inline)) {
+    c = (i >> 1) * 32 + (r16 >> 2) * 8 + (i & 1) * 4 + (r16 & 3);
+    const T *from = ks + (32 * s + 4 * g + (r16 >> 2)) * KS + (i >> 1) * 32 + (r16 & 3) * 8 + (i & 1) * 4;
+    u32x2 h[2];
 #pragma unroll
-      for (int it = 0; it < 4; ++it) acc[0][it] = acc[1][it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 2; ++e)
+      h[e] = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(from + 16 * e * KS)));
+    unpack8<Tag>(u32x4{h[0][0], h[0][1], h[1][0], h[1][1]}, k);
+    const f32x4 f0 = *(const f32x4 *)(fk + 32 * s + 4 * g), f1 = *(const f32x4 *)(fk + 32 * s + 16 + 4 * g);
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        u32x4 th[4], tl[4];
-#pragma unroll
-        for (int it = 2 * s; it < 4; ++it) solution_operand(ts, triangle(it, s), lane, th[it], tl[it]);
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          const int i = 2 * item + d, c = item * 32 + (r16 >> 2) * 8 + d * 4 + (r16 & 3);
-          const float last = rs[(L - 1) * RS + c];
-          float v[8], w[8];
-          u32x4 hi, lo;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int t = 32 * s + 16 * (e >> 2) + 4 * g + (e & 3);
-            const float k = elem<Tag>::ld(ks[t * KS + c]) * fk[t], r = rs[t * RS + c];
-            v[e] = k * __builtin_amdgcn_exp2f(last - r);
-            w[e] = k * __builtin_amdgcn_exp2f(r);
-          }
-          split8(v, hi, lo);
-          u32x4 *dst = (u32x4 *)(ws + (lay.k + (i * 2 + s) * 2) * 1024) + lane;
-          dst[0] = hi, dst[64] = lo;
-          split8(w, hi, lo);
-#pragma unroll
-          for (int it = 2 * s; it < 4; ++it) acc[d][it] = mfma3(hi, lo, th[it], tl[it], acc[d][it]);
-        }
-      }
-#pragma unroll
-      for (int it = 0; it < 4; ++it) {
-        u32x4 hi, lo;
-        split44(-acc[0][it], -acc[1][it], hi, lo);
-        u32x4 *dst = (u32x4 *)(ws + (it * NK + item) * 2 * 1024) + lane;
-        dst[0] = hi, dst[64] = lo;
-      }
-    } else {
-      const int ct = item - NK;
-      const T *v = x + head * p.p + ct * 16 + r16;
-      T raw[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) raw[e] = v[(int64_t)min(16 * (e >> 2) + 4 * g + (e & 3), nt - 1) * p.x_stride];
-      f32x4 acc[4];
-#pragma unroll
-      for (int it = 0; it < 4; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        float f[8];
-        u32x4 hi, lo;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = elem<Tag>::ld(raw[8 * s + e]);
-        split8(f, hi, lo);
-#pragma unroll
-        for (int it = 2 * s; it < 4; ++it) {
-          u32x4 th, tl;
-          solution_operand(ts, triangle(it, s), lane, th, tl);
-          acc[it] = mfma16x16x32<B16>(th, hi, acc[it]);
-          acc[it] = mfma16x16x32<B16>(tl, hi, acc[it]);
-          if constexpr (!__is_same(Tag, B16)) acc[it] = mfma16x16x32<B16>(th, lo, acc[it]);
-        }
-      }
-      // in the layout of an accumulator: column lane & 15, tokens 4 (lane >> 4) ..
-#pragma unroll
-      for (int it = 0; it < 4; ++it) *((f32x4 *)(ws + (lay.u0 + ct * 4 + it) * 1024) + lane) = acc[it];
+    for (int e = 0; e < 8; ++e) {
+      k[e] *= e < 4 ? f0[e & 3] : f1[e & 3];
+      r[e] = rs[(32 * s + 16 * (e >> 2) + 4 * g + (e & 3)) * RS + c];
     }
+  };
+  // ---- K = e^(r_last - r) k by state rows, by the waves that have no part in the solution
+  if (wave >= 4) {
+    for (int f = wave - 4; f < 4 * NK; f += 4) {
+      const int i = f >> 1, s = f & 1;
+      int c;
+      float k[8], r[8];
+      columns_of(i, s, c, k, r);
+      const float last = rs[(L - 1) * RS + c];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) k[e] *= __builtin_amdgcn_exp2f(last - r[e]);
+      u32x4 hi, lo;
+      split8(k, hi, lo);
+      u32x4 *dst = (u32x4 *)(ws + (lay.k + f * 2) * 1024) + lane;
+      dst[0] = hi, dst[64] = lo;
+    }
+  }
+  solve_chunk(ts, bt, wave, lane);
+  {
+    u32x4 hi, lo;
+    if (wave < kTriangle) solution_operand(ts, wave, lane, hi, lo);
+    __syncthreads();
+    if (wave < kTriangle) {
+      u32x4 *dst = (u32x4 *)qs + wave * 128 + lane;
+      dst[0] = hi, dst[64] = lo;
+    }
+    __syncthreads();
+  }
+  const u32x4 *solution = (const u32x4 *)qs + lane;   // [kTriangle][high, rest][64]
+
+  // ---- by 16 channels: -W = -T e^r k by tokens; by 16 columns of v: U0 = T v
+  for (int i = wave; i < 2 * NK; i += W) {
+    f32x4 acc[4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      int c;
+      float k[8], r[8];
+      columns_of(i, s, c, k, r);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) k[e] *= __builtin_amdgcn_exp2f(r[e]);
+      u32x4 hi, lo;
+      split8(k, hi, lo);
+#pragma unroll
+      for (int it = 2 * s; it < 4; ++it) acc[it] = mfma3(hi, lo, solution[triangle(it, s) * 128], solution[triangle(it, s) * 128 + 64], acc[it]);
+    }
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      u32x2 hi, lo;
+      split4(-acc[it], hi, lo);
+      u32x2 *dst = (u32x2 *)(ws + (it * NK + (i >> 1)) * 2 * 1024 + lane * 16) + (i & 1);
+      dst[0] = hi, dst[128] = lo;
+    }
+  }
+  for (int ct = wave; ct < columns; ct += W) {
+    if (ct != wave) load_values(ct);
+    f32x4 acc[4];
+#pragma unroll
+    for (int it = 0; it < 4; ++it) acc[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      float f[8];
+      u32x4 hi, lo;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = elem<Tag>::ld(vraw[8 * s + e]);
+      split8(f, hi, lo);
+#pragma unroll
+      for (int it = 2 * s; it < 4; ++it) {
+        const u32x4 th = solution[triangle(it, s) * 128], tl = solution[triangle(it, s) * 128 + 64];
+        acc[it] = mfma16x16x32<B16>(th, hi, acc[it]);
+        acc[it] = mfma16x16x32<B16>(tl, hi, acc[it]);
+        if constexpr (!__is_same(Tag, B16)) acc[it] = mfma16x16x32<B16>(th, lo, acc[it]);
+      }
+    }
+    // in the layout of an accumulator: column lane & 15, tokens 4 (lane >> 4) ..
+#pragma unroll
+    for (int it = 0; it < 4; ++it) *((f32x4 *)(ws + (lay.u0 + ct * 4 + it) * 1024) + lane) = acc[it];
   }
 }
 
