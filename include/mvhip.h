@@ -816,6 +816,19 @@ size_t mv_gru_prefill_workspace_bytes(int n_seqs, int total_q, int max_q, int n)
 int mv_gru_prefill(const MvGruArgs *args, int dtype, void *stream);
 int mv_gru_step(const MvGruArgs *args, int dtype, void *stream);
 
+/* ---- K20 — projections with inputs and outputs of their own over the same rows (16-bit): out[:, first_output + i] = x[:, first_input ..] W[first_output + i,
+ * first_input ..]^T, i < outputs.  W [outputs of all][k] dense (what lies beside the blocks is not read); inputs 64 or 128; first_*, outputs and strides
+ * multiples of 8, pointers of 16 bytes. */
+enum { MV_BLOCK_LINEAR_MAX = 4 };
+typedef struct MvBlockLinearArgs {
+  const void *x, *w;
+  void *out;
+  int64_t x_stride, out_stride;
+  int rows, k, inputs, blocks;
+  int first_input[MV_BLOCK_LINEAR_MAX], first_output[MV_BLOCK_LINEAR_MAX], outputs[MV_BLOCK_LINEAR_MAX];
+} MvBlockLinearArgs;
+int mv_block_linear(const MvBlockLinearArgs *args, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -126,6 +126,7 @@ _SIGNATURES = {
                                                     c_void_p, c_float, c_void_p, c_void_p, c_int64, c_int, c_int,
                                                     c_int, c_int, c_int, c_void_p]),
     "mv_packed_weight_elems": (c_size_t, [c_int, c_int]),
+    "mv_block_linear": (c_int, [c_void_p, c_int, c_void_p]),
     "mv_pack_weight": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "mv_linear_mid_m": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                 c_int, c_int, c_int, c_void_p]),
@@ -975,6 +976,37 @@ def norm_linear_small_m(x, residual, norm_weight, eps: float, weight_packed, n: 
         return None
     _check(rc, "mv_norm_linear_small_m_packed")
     return out, res_out
+
+
+# ---------------------------------------------------------------- K20
+MV_BLOCK_LINEAR_MAX = 4
+
+
+class MvBlockLinearArgs(ctypes.Structure):
+    """include/mvhip.h: MvBlockLinearArgs."""
+    _fields_ = [("x", c_void_p), ("w", c_void_p), ("out", c_void_p), ("x_stride", c_int64), ("out_stride", c_int64), ("rows", c_int), ("k", c_int),
+                ("inputs", c_int), ("blocks", c_int), ("first_input", c_int * MV_BLOCK_LINEAR_MAX), ("first_output", c_int * MV_BLOCK_LINEAR_MAX),
+                ("outputs", c_int * MV_BLOCK_LINEAR_MAX)]
+
+
+def block_linear(x, weight, blocks):
+    """x [T, K], weight [N, K], blocks of (first input, inputs, first output, outputs), all outputs together -> [T, N]; None: shapes that the kernel
+    does not take (the caller uses the whole weight)."""
+    n, k = weight.shape
+    if not (x.is_cuda and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float16) and weight.dtype == x.dtype and weight.is_contiguous()
+            and x.shape[1] == k and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= k and n % 8 == 0 and 0 < len(blocks) <= MV_BLOCK_LINEAR_MAX
+            and blocks[0][1] in (64, 128) and all(b[1] == blocks[0][1] and not any(v % 8 for v in b) for b in blocks)
+            and sum(b[3] for b in blocks) == n and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
+        return None
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+        return None
+    out = torch.empty((x.shape[0], n), dtype=x.dtype, device=x.device)
+    a = MvBlockLinearArgs(x=x.data_ptr(), w=weight.data_ptr(), out=out.data_ptr(), x_stride=x.stride(0), out_stride=n, rows=x.shape[0], k=k,
+                          inputs=blocks[0][1], blocks=len(blocks))
+    for i, (at, _, to, outputs) in enumerate(blocks):
+        a.first_input[i], a.first_output[i], a.outputs[i] = at, to, outputs
+    _check(_lib.mv_block_linear(ctypes.byref(a), _dt(x), _stream()), "mv_block_linear")
+    return out
 
 
 # ---------------------------------------------------------------- K11

@@ -418,6 +418,7 @@ class BlockLinear(LinearBase):
             n, k = n + g.local(1), k + pad_to(inputs)
         super().__init__(k, n)
         self.weight.data.zero_()
+        self._places = [(k, pad_to(inputs), self.offsets[name], g.local(1)) for name, (inputs, k, g) in self.blocks.items()]
 
     def weight_loader(self, param, loaded_weight, loaded_shard_id: str | None = None, *args, **kwargs):
         inputs, k, g = self.blocks[loaded_shard_id]
@@ -428,4 +429,8 @@ class BlockLinear(LinearBase):
         dst[:, :g.unit].copy_(materialize(loaded_weight).unflatten(0, (g.units, g.unit)))
 
     def forward(self, x):
+        if x.shape[0] > max(MID_M_MAX, SMALL_M_MAX):    # (a decode step's kernels read the whole weight)
+            out = hip_ops.block_linear(x, self.weight, self._places)
+            if out is not None:
+                return out
         return linear(x, self.weight, None, self.weight_packed)
