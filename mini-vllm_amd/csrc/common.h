@@ -84,15 +84,16 @@ __device__ __forceinline__ void unpack8(const u32x4 &v, float (&f)[8]) {
   }
 }
 template <typename Tag>
+__device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
+  if constexpr (__is_same(Tag, bf16_tag))
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2_t));
+  else
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, f16x2_t));
+}
+// (pairs: a conversion for both, where two single ones and their union are three instructions)
+template <typename Tag>
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
-  u32x4 v;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t lo = elem<Tag>::st(f[2 * i]);
-    uint32_t hi = elem<Tag>::st(f[2 * i + 1]);
-    v[i] = lo | (hi << 16);
-  }
-  return v;
+  return u32x4{pack_pair<Tag>(f[0], f[1]), pack_pair<Tag>(f[2], f[3]), pack_pair<Tag>(f[4], f[5]), pack_pair<Tag>(f[6], f[7])};
 }
 
 // ---- cross-lane ----------------------------------------------------------
