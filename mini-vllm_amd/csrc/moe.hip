@@ -3,6 +3,9 @@
 //   mv_moe_group:  pairs sorted by expert, and the tiles of at most tile_m rows of one expert each;
 //   mv_moe_linear: out[place] = W[expert of the place] x[token of the place], with the gate's activation if asked for.
 // The weighted sum over a token's choices rides in mv_residual_update.
+#include <algorithm>
+#include <type_traits>
+
 #include "latent.h"
 
 namespace {
@@ -222,46 +225,56 @@ __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
   for (int t = wave; t < TOKENS && m0 + t < p.rows; t += WAVES) choose<Tag>(p, sc + t * R, ch + t * R, m0 + t, correction);   // (no barrier in it)
 }
 
-// ---- grouping.  Workgroup e = expert e: its pairs start behind those of the experts before it.  Each wave walks a part of the
-// pairs, in order, so places are the same in every run.
+// ---- grouping.  Workgroup (e, part): the pairs of expert e, which start behind those of the experts before it.  Each wave walks a run of all
+// pairs, in order, so places are the same in every run: all of its run to count, then the part of it whose pairs it places.  Latencies and the stores
+// to scattered places bound it, and instructions that are fetched for the first time: all of a run's choices at once, kept in registers for the second
+// walk, made a program that took longer to arrive than the second reading (36004 pairs, eight parts 25.6 us).  36004 pairs of 32 experts: one part
+// 17.4 us, eight 10.1; 160000 pairs 61.6 and 27.8; 4000 pairs 5.9 and 5.9.
 constexpr int kGroupThreads = 1024, kGroupWaves = kGroupThreads / 64, kGroupAhead = 8;   // kGroupAhead: choices of a lane requested at a time
+constexpr int kGroupParts = 8;
 
 __global__ void __launch_bounds__(kGroupThreads) moe_group_kernel(const int32_t *ids, int pairs, int top, int experts, int tile_m,
                                                                   int max_tiles, int32_t *rows, int32_t *tokens, int32_t *tiles,
                                                                   const float *weights, float *weights_out) {
   __shared__ int less[kGroupWaves], equal[kGroupWaves];
-  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int per = (pairs + kGroupWaves * 64 - 1) / (kGroupWaves * 64) * 64, lo = wave * per, hi = min(pairs, lo + per);
-  int nl = 0, ne = 0;
-  // the choices i0 + 64 u + lane of this wave's part (-1 behind its end)
-  auto choices = [&](int i0, int (&v)[kGroupAhead]) {
+  const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int runs = (pairs + kGroupWaves * 64 - 1) / (kGroupWaves * 64), lo = wave * runs * 64, hi = min(pairs, lo + runs * 64);
+  // the pairs of its run that the wave places: from `from` on, ahead of `to`
+  const int parts = gridDim.y, part = blockIdx.y;
+  const int from = lo + runs * part / parts * 64, to = min(hi, lo + runs * (part + 1) / parts * 64);
+  int nl = 0, ne = 0, nb = 0;   // choices of lower experts, of this one, of this one ahead of `from`
+  // the choices i0 + 64 u + lane, ahead of `end` (-1 behind it)
+  auto choices = [&](int i0, int end, int (&v)[kGroupAhead]) {
 #pragma unroll
     for (int u = 0; u < kGroupAhead; ++u) {
       const int i = i0 + 64 * u + lane;
       v[u] = ids[min(i, pairs - 1)];
-      if (i >= hi) v[u] = -1;
+      if (i >= end) v[u] = -1;
     }
   };
   for (int i0 = lo; i0 < hi; i0 += 64 * kGroupAhead) {
     int v[kGroupAhead];
-    choices(i0, v);
+    choices(i0, hi, v);
 #pragma unroll
-    for (int u = 0; u < kGroupAhead; ++u) nl += v[u] >= 0 && v[u] < e, ne += v[u] == e;
+    for (int u = 0; u < kGroupAhead; ++u) {
+      const int is = v[u] == e;
+      nl += v[u] >= 0 && v[u] < e, ne += is, nb += i0 + 64 * u < from ? is : 0;
+    }
   }
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) nl += __shfl_xor(nl, o, 64), ne += __shfl_xor(ne, o, 64);
+  for (int o = 32; o >= 1; o >>= 1) nl += __shfl_xor(nl, o, 64), ne += __shfl_xor(ne, o, 64), nb += __shfl_xor(nb, o, 64);
   if (lane == 0) less[wave] = nl, equal[wave] = ne;
   __syncthreads();
-  int start = 0, count = 0, ahead = 0;
+  int start = 0, count = 0, ahead = nb;
   for (int w = 0; w < kGroupWaves; ++w) {
     start += less[w], count += equal[w];
     if (w < wave) ahead += equal[w];
   }
   int at = start + ahead;
-  for (int i0 = lo; i0 < hi; i0 += 64 * kGroupAhead) {
+  for (int i0 = from; i0 < to; i0 += 64 * kGroupAhead) {
     int v[kGroupAhead];
     float w[kGroupAhead];
-    choices(i0, v);
+    choices(i0, to, v);
 #pragma unroll
     for (int u = 0; u < kGroupAhead; ++u)
       if (weights && v[u] == e) w[u] = weights[i0 + 64 * u + lane];
@@ -278,6 +291,7 @@ __global__ void __launch_bounds__(kGroupThreads) moe_group_kernel(const int32_t 
       at += __popcll(mask);
     }
   }
+  if (part) return;
   // tiles of this expert: entries start / tile_m + e on, up to the next expert's; the last expert also clears what is left
   const int t0 = start / tile_m + e, t1 = e + 1 < experts ? (start + count) / tile_m + e + 1 : max_tiles;
   for (int t = t0 + tid; t < t1; t += kGroupThreads) {
@@ -701,7 +715,9 @@ extern "C" int mv_moe_group(const int32_t *ids, int pairs, int top, int experts,
   if (pairs == 0) return MV_OK;
   if (!ids || !rows || !tokens || !tiles || (weights && !weights_out)) return MV_E_NULLPTR;
   if (pairs < 0 || top <= 0 || experts <= 0 || experts > 65535 || tile_m <= 0 || max_tiles < pairs / tile_m + experts) return MV_E_SHAPE;
-  hipLaunchKernelGGL(moe_group_kernel, dim3(experts), dim3(kGroupThreads), 0, (hipStream_t)stream, ids, pairs, top, experts, tile_m,
+  // (every part counts all pairs; a part is worth having for some 1024 of them to place)
+  const int parts = std::max(1, std::min({kGroupParts, 256 / experts, pairs / 1024}));
+  hipLaunchKernelGGL(moe_group_kernel, dim3(experts, parts), dim3(kGroupThreads), 0, (hipStream_t)stream, ids, pairs, top, experts, tile_m,
                      max_tiles, rows, tokens, tiles, weights, weights_out);
   MV_LAUNCH_CHECK();
   return MV_OK;
