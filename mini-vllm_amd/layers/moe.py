@@ -8,6 +8,8 @@ where the weight multiplies the expert's input instead, it multiplies the sums o
 Expert weights are kept in ONE form: as the checkpoint has them in fp32, fragment-ordered in 16 bits (``finish_weights``)."""
 from __future__ import annotations
 
+import math
+
 import torch
 from torch import nn
 
@@ -18,10 +20,14 @@ from .linear import Segment, SegmentedLinear, gated_linear, pad_to
 
 __all__ = ["ExpertMLP"]
 
-# Pairs per expert up to which a launch works on tiles of that many rows.  The last line was drawn for workgroups of 256 x 256 rows and outputs; their successors,
-# two of 128 x 256 to a CU, are ahead from fewer pairs on.  Both products, tiles of 64 / 128 / 256 rows, us: 32 experts of 2048 -> 768, 64 pairs each 101 / 76 / 68,
-# 256 188 / 194 / 131, 768 400 / 392 / 294; of 1024 -> 384 31 / 36 / 32, 75 / 78 / 42, 134 / 143 / 88; 8 experts of 2048 -> 768 39 / 49 / 49, 49 / 58 / 51, 104 / 110 / 82.
-TILES = ((8, 16), (40, 32), (96, 64), (768, 128))
+# Rows of the tiles that a launch works on, by the pairs per expert.  Both products, us, tiles of 16 / 32 / 64 / 256 rows:
+#   few pairs: the next tile is ahead from 10 (32 experts of 2048 -> 768: 8 62 / 58, 12 67 / 62; 8 experts 24 / 22, 26 / 24) and, for the 64 rows' longer runs
+#   of a weight, from 16 where experts are many (32: 16 67 / 62, 24 82 / 65; 128: 245 / 236, 297 / 241), from 28 else (8: 16 26 / 37, 28 38 / 37).
+#   256 rows (two workgroups of 128 x 256 to a CU) against 64: ahead as soon as their workgroups fill five eighths of the chip: 32 of 2048 -> 768 (192 workgroups)
+#   24 pairs 65 / 64, 64 84 / 68, 256 176 / 128; of 1024 -> 384 64 pairs (96) 30 / 33, 160 (192) 51 / 37; 8 of 2048 -> 768 256 (96) 46 / 52, 384 (144) 59 / 55, 800
+#   103 / 83; 2 of 2048 -> 768 1100 (108) 46 / 56, 2500 (240) 88 / 70; the worst found: 2 of 4096 -> 1024, 1500 pairs (192) 102 / 111.
+#   128 rows (tiles of the 64's kind) are nowhere ahead of both.
+FEW, MANY_EXPERTS, WIDE_GROUPS = 8, 32, 160
 
 
 class ExpertMLP(nn.Module):
@@ -72,7 +78,10 @@ class ExpertMLP(nn.Module):
         if self.router.dtype == torch.float32:
             return 16
         per = tokens * self.top / self.experts
-        return next((rows for most, rows in TILES if per <= most), 256)
+        if per <= (16 if self.experts >= MANY_EXPERTS else 28):
+            return 16 if per <= FEW else 32
+        wide = self.experts * math.ceil(per / 128) * math.ceil(2 * self.f / 256)      # workgroups of the gated product
+        return 256 if wide >= WIDE_GROUPS else 64
 
     def route(self, h):
         """-> (weights [T, top], the pairs sorted by expert)."""
