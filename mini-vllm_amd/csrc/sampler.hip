@@ -314,7 +314,7 @@ struct RowOnChip {
       }
     });
   }
-  // f(top - bits) of every element, `top` the bits of a positive value: up to `top` the places of the values from `top` down to zero, more for
+  // f(raw, top - bits) of every element, `top` the bits of a positive value: up to `top` the places of the values from `top` down to zero, more for
   // negative values, larger ones and NaN
   template <typename F>
   __device__ __forceinline__ void foreach_place(uint32_t top, F &&f) const {
@@ -325,7 +325,7 @@ struct RowOnChip {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t d = __builtin_bit_cast(uint32_t, t - __builtin_bit_cast(u16x2, (uint32_t)v[j]));
-          f(d & 0xffffu), f(d >> 16);
+          f((uint16_t)(v[j] & 0xffffu), d & 0xffffu), f((uint16_t)(v[j] >> 16), d >> 16);
         }
       }
     });
@@ -372,8 +372,8 @@ __device__ __forceinline__ int greedy_pass(const uint16_t *row, int nvec, float 
 // workgroup a CU, 304 KB each: more than the LDS and, beside what the passes need, more than the registers, but not more than half in each.  Kept
 // there, the passes behind the first read no memory, and those behind a filter skip what cannot be kept.
 // A long greedy row is one pass and stays nowhere (greedy_pass).
-// 151 936 bf16 logits, us, memory in every pass -> now; 256 rows: greedy 18.9 -> 13.9, plain 58 -> 30, top-k 40 89 -> 37, top-p 0.9 81 -> 55, min-p
-// 55 -> 27; one row: 15.5 -> 6.3, 51 -> 20, 81 -> 28, 73 -> 45, 49 -> 18 (brought to its CU like the others: 18.4, 9.8).  What is left is
+// 151 936 bf16 logits, us, memory in every pass -> now; 256 rows: greedy 18.9 -> 13.9, plain 58 -> 30, top-k 40 89 -> 37, top-p 0.9 81 -> 50 (58 with mass and
+// counts in a pass each and keys made for the last), min-p 55 -> 27; one row: 15.5 -> 6.3, 51 -> 20, 81 -> 28, 73 -> 38, 49 -> 18 (brought to its CU like the others: 18.4, 9.8).  What is left is
 // vector arithmetic: an exponential and four instructions an element where every weight counts.
 template <typename Tag, int NR>
 __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
@@ -505,6 +505,7 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
       };
       uint32_t win = kWin;    // bins counted
       float all_m = 0.f;      // the row's mass (asked for when top-k is off)
+      bool counted = false;
       if constexpr (CHIP) {
         // What is asked of the whole row besides (top-p: its mass) is a pass without branches.  With top-k, at least k elements reach the k-th
         // largest of the threads' maxima, so few elements are left to count; a bound that is no use (fewer maxima than k) is the whole window.
@@ -517,8 +518,18 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
           __syncthreads();
           win = sh.bcast_u[0] + 1u;
         } else if (!topk_on) {
+          // (the window ends above zero: one pass for mass and counts, whose additions in LDS run beside the exponentials)
           float z = 0.f;
-          chip.foreach([&](T raw) { z += weight(elem<Tag>::ld(raw)); });
+          counted = kmax >= 0x8000u + kWin - 1u;
+          if (counted) {
+            clear();
+            chip.foreach_place(kmax - 0x8000u, [&](T raw, uint32_t bin) {
+              z += weight(elem<Tag>::ld(raw));
+              if (bin < (uint32_t)kWin) atomicAdd(&sh.wcnt[bin], 1u);
+            });
+          } else {
+            chip.foreach([&](T raw) { z += weight(elem<Tag>::ld(raw)); });
+          }
           all_m = block_sum_f(z, sh);
         }
       }
@@ -527,11 +538,14 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
         unsigned under_cnt = 0;
         float z1;
         ok_fast = true;
-        __syncthreads();
-        clear();
+        if (!counted) {
+          __syncthreads();
+          clear();
+        }
         if constexpr (CHIP) {
-          if (win < (uint32_t)kWin) chip.foreach_from(kmax >= win ? Row::least_of_key(kmax - win + 1) : Row::kAll, [&](int i, T raw) { count(raw, win); });
-          else if (kmax >= 0x8000u + kWin - 1u) chip.foreach_place(kmax - 0x8000u, [&](uint32_t bin) {   // (the window ends above zero)
+          if (counted) {
+          } else if (win < (uint32_t)kWin) chip.foreach_from(kmax >= win ? Row::least_of_key(kmax - win + 1) : Row::kAll, [&](int i, T raw) { count(raw, win); });
+          else if (kmax >= 0x8000u + kWin - 1u) chip.foreach_place(kmax - 0x8000u, [&](T raw, uint32_t bin) {
             if (bin < (uint32_t)kWin) atomicAdd(&sh.wcnt[bin], 1u);
           });
           else chip.foreach([&](T raw) { count(raw, kWin); });
@@ -733,7 +747,13 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(SampleParams p) {
           const float w = weight(elem<Tag>::ld(raw));
           if (kept(make_key<Tag>(raw), w)) mine += w;
         });
-      else   // (many are kept: turns over a vector cost more than all of its elements)
+      else if (key_p > 0x8000u && !minp_on) {   // many are kept: turns over a vector cost more than all of its elements
+        const short least = Row::least_of_key(key_p);   // (a positive value: bits as signed numbers are in the keys' order)
+        chip.foreach([&](T raw) {
+          const float w = weight(elem<Tag>::ld(raw));
+          mine += (short)raw < least ? 0.f : w;
+        });
+      } else
         chip.foreach([&](T raw) {
           const float w = weight(elem<Tag>::ld(raw));
           const bool out = make_key<Tag>(raw) < key_p || (minp_on && w < min_p);
