@@ -241,7 +241,8 @@ __global__ void __launch_bounds__(kGroupThreads) moe_group_kernel(const int32_t 
   const int runs = (pairs + kGroupWaves * 64 - 1) / (kGroupWaves * 64), lo = wave * runs * 64, hi = min(pairs, lo + runs * 64);
   // the pairs of its run that the wave places: from `from` on, ahead of `to`
   const int parts = gridDim.y, part = blockIdx.y;
-  const int from = lo + runs * part / parts * 64, to = min(hi, lo + runs * (part + 1) / parts * 64);
+  int from = lo, to = hi;
+  if (parts > 1) from = lo + runs * part / parts * 64, to = min(hi, lo + runs * (part + 1) / parts * 64);
   int nl = 0, ne = 0, nb = 0;   // choices of lower experts, of this one, of this one ahead of `from`
   // the choices i0 + 64 u + lane, ahead of `end` (-1 behind it)
   auto choices = [&](int i0, int end, int (&v)[kGroupAhead]) {
@@ -262,7 +263,11 @@ __global__ void __launch_bounds__(kGroupThreads) moe_group_kernel(const int32_t 
     }
   }
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) nl += __shfl_xor(nl, o, 64), ne += __shfl_xor(ne, o, 64), nb += __shfl_xor(nb, o, 64);
+  for (int o = 32; o >= 1; o >>= 1) nl += __shfl_xor(nl, o, 64), ne += __shfl_xor(ne, o, 64);
+  if (part) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) nb += __shfl_xor(nb, o, 64);
+  }
   if (lane == 0) less[wave] = nl, equal[wave] = ne;
   __syncthreads();
   int start = 0, count = 0, ahead = nb;
