@@ -714,10 +714,10 @@ enum { MV_GATE_SILU = 0, MV_GATE_SIGMOID = 1 };
 typedef struct MvDeltaArgs {
   const void *x;                    /* [T] rows of channels at x_stride: projected (step) or convolved (prefill) */
   const void *beta, *a;             /* raw: [T] rows of heads; of heads, or (channel_decay) heads * n */
-  const void *gate;                 /* step: raw, [T] rows of heads * p */
+  const void *gate;                 /* step, MV_DELTA_NORM: raw, [T] rows of heads * p */
   const void *conv_w;               /* step: [taps][channels], no bias */
   const void *dt_bias, *a_log;      /* [heads] or [heads * n]; [heads] */
-  const void *norm_w;               /* step: [p] */
+  const void *norm_w;               /* step, MV_DELTA_NORM: [p] */
   void *conv_state;
   float *state;
   const int32_t *state_slots;       /* [n_seqs] */
@@ -728,8 +728,10 @@ typedef struct MvDeltaArgs {
   int n_seqs, max_q, total_q, channels, taps, heads, groups, p, p_true, n, k_off, q_off, channel_decay, gate_kind;
   float eps, unit_eps, q_scale, out_scale;
 } MvDeltaArgs;
-/* out[t] = o, [T][heads * p], from convolved channels; writes state.  flags: MV_DELTA_SCAN = token by token */
-enum { MV_DELTA_SCAN = 1 };
+/* out[t] = o, [T][heads * p], from convolved channels; writes state.  flags: MV_DELTA_SCAN = token by token; MV_DELTA_NORM = behind it mv_head_norm_gate with
+ * the arguments' gate, norm_w, p_true, eps, gate_kind and out_scale, where rows of `out` are whole, aligned vectors of 16 bytes, in the same launches
+ * where a workgroup has a head's columns */
+enum { MV_DELTA_SCAN = 1, MV_DELTA_NORM = 2 };
 size_t mv_delta_prefill_workspace_bytes(int n_seqs, int total_q, int heads, int p, int n, int dtype);
 /* scratch beyond that with which few long sequences are worked on in several places at once (0: none is of use) */
 size_t mv_delta_prefill_segments_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int channel_decay, int dtype);

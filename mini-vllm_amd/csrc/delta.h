@@ -3,11 +3,19 @@
 #include "ssm.h"
 
 __device__ __forceinline__ float sigmoid_f32(float z) { return 1.0f / (1.0f + expf(-z)); }
+// what norm and gate of a head's outputs make of one of them, in 16 bits: hardware root, exponential and reciprocal (1 ulp of fp32 each)
+__device__ __forceinline__ float head_rms_16(float squares, float share, float eps, float out_scale) {
+  return out_scale * __builtin_amdgcn_rsqf(fmaf(squares, share, eps));
+}
+__device__ __forceinline__ float gate_16(float z, int kind) {
+  return (kind == MV_GATE_SIGMOID ? 1.f : z) * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
+}
 // log of the decay factor: -exp(a_log) * softplus(a + bias)
 __device__ __forceinline__ float decay_log(float rate, float a, float bias) { return -rate * softplus_f32(a + bias); }
 
 // chunked form (16-bit); MV_E_SHAPE when it does not apply
 size_t mv_delta_chunk_workspace(int n_seqs, int total_q, int heads, int p, int n);
 size_t mv_delta_segments_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n);   // beside it, where sequences are cut
-int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, hipStream_t stream);
-int mv_delta_scalar_launch(const MvDeltaArgs &a, hipStream_t stream);   // (from the above: bf16, one decay per head)
+// `normed` (NULL: not asked for): set where norm and gate are already in the output
+int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, bool *normed, hipStream_t stream);
+int mv_delta_scalar_launch(const MvDeltaArgs &a, bool *normed, hipStream_t stream);   // (from the above: bf16, one decay per head)

@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(256) head_norm_gate_kernel(const typename elem
     }
     float rs;
     if constexpr (__is_same(Tag, f32_tag)) rs = out_scale / sqrtf(ss / (float)p_true + eps);
-    else rs = out_scale * __builtin_amdgcn_rsqf(fmaf(ss, share, eps));
+    else rs = head_rms_16(ss, share, eps, out_scale);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int c = (sub + i * LPT) * VEC;
@@ -315,7 +315,7 @@ __global__ void __launch_bounds__(256) head_norm_gate_kernel(const typename elem
         for (int j = 0; j < VEC; ++j) {
           float act;
           if constexpr (__is_same(Tag, f32_tag)) act = gate_kind == MV_GATE_SIGMOID ? sigmoid_f32(g[j]) : silu_f32(g[j]);
-          else act = (gate_kind == MV_GATE_SIGMOID ? 1.f : g[j]) * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g[j]));
+          else act = gate_16(g[j], gate_kind);
           o[j] = f[i][j] * rs * wv[j] * act;
         }
         store_vec_row<Tag>(out + rows[k] * out_stride + cols[k] + c, o);
@@ -337,6 +337,18 @@ int check_delta(const MvDeltaArgs *a, int dtype) {
   return (a->state && !mv_aligned16(a->state)) ? MV_E_ALIGN : MV_OK;
 }
 
+int check_norm(const void *y, int64_t y_stride, const void *gate, int64_t gate_stride, const void *w, const void *out, int64_t out_stride, int rows,
+               int heads, int p, int p_true, int gate_kind, int dtype) {
+  if (!y || !gate || !w || !out) return MV_E_NULLPTR;
+  if (rows < 0 || heads <= 0 || p_true <= 0 || p < p_true || (p & 7) || p > 1024 || y_stride < (int64_t)heads * p ||
+      gate_stride < (int64_t)heads * p || out_stride < (int64_t)heads * p)
+    return MV_E_SHAPE;
+  if (gate_kind != MV_GATE_SILU && gate_kind != MV_GATE_SIGMOID) return MV_E_RANGE;
+  const int vec = dtype == MV_F32 ? 4 : 8;
+  return !mv_aligned16(y) || !mv_aligned16(gate) || !mv_aligned16(w) || !mv_aligned16(out) || y_stride % vec || gate_stride % vec || out_stride % vec
+             ? MV_E_ALIGN : MV_OK;
+}
+
 }  // namespace
 
 extern "C" size_t mv_delta_prefill_workspace_bytes(int n_seqs, int total_q, int heads, int p, int n, int dtype) {
@@ -353,15 +365,26 @@ extern "C" int mv_delta_prefill(const MvDeltaArgs *a, int dtype, int flags, void
   if (int e = check_delta(a, dtype)) return e;
   if (!a->cu_q || !a->cu_k) return MV_E_NULLPTR;
   if (a->max_q < 0) return MV_E_SHAPE;
+  const bool norm = flags & MV_DELTA_NORM;
+  if (norm)
+    if (int e = check_norm(a->out, a->out_stride, a->gate, a->gate_stride, a->norm_w, a->out, a->out_stride, a->total_q, a->heads, a->p, a->p_true,
+                           a->gate_kind, dtype))
+      return e;
+  const auto behind = [&](int rc, bool normed) {
+    return rc != MV_OK || !norm || normed ? rc
+                                          : mv_head_norm_gate(a->out, a->out_stride, a->gate, a->gate_stride, a->norm_w, a->out, a->out_stride, a->total_q,
+                                                              a->heads, a->p, a->p_true, a->eps, a->gate_kind, a->out_scale, dtype, stream);
+  };
   if (dtype != MV_F32 && !(flags & MV_DELTA_SCAN)) {
-    const int rc = mv_delta_chunk_launch(*a, dtype, (hipStream_t)stream);
-    if (rc != MV_E_SHAPE) return rc;
+    bool normed = false;
+    const int rc = mv_delta_chunk_launch(*a, dtype, norm ? &normed : nullptr, (hipStream_t)stream);
+    if (rc != MV_E_SHAPE) return behind(rc, normed);
   }
   const size_t lds = (size_t)(3 * kScanRows * a->n + kScanRows * 17) * 4;
   const dim3 grid(a->p / 16, a->heads, a->n_seqs);
   MV_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((delta_scan_kernel<Tag>), grid, dim3(256), lds, (hipStream_t)stream, *a));
   MV_LAUNCH_CHECK();
-  return MV_OK;
+  return behind(MV_OK, false);
 }
 
 extern "C" int mv_delta_step(const MvDeltaArgs *a, int dtype, void *stream) {
@@ -388,15 +411,8 @@ extern "C" int mv_head_norm_gate(const void *y, int64_t y_stride, const void *ga
                                  int64_t out_stride, int rows, int heads, int p, int p_true, float eps, int gate_kind, float out_scale,
                                  int dtype, void *stream) {
   if (rows == 0) return MV_OK;
-  if (!y || !gate || !w || !out) return MV_E_NULLPTR;
-  if (rows < 0 || heads <= 0 || p_true <= 0 || p < p_true || (p & 7) || p > 1024 || y_stride < (int64_t)heads * p ||
-      gate_stride < (int64_t)heads * p || out_stride < (int64_t)heads * p)
-    return MV_E_SHAPE;
-  if (gate_kind != MV_GATE_SILU && gate_kind != MV_GATE_SIGMOID) return MV_E_RANGE;
+  if (int e = check_norm(y, y_stride, gate, gate_stride, w, out, out_stride, rows, heads, p, p_true, gate_kind, dtype)) return e;
   const int vec = dtype == MV_F32 ? 4 : 8;
-  if (!mv_aligned16(y) || !mv_aligned16(gate) || !mv_aligned16(w) || !mv_aligned16(out) || y_stride % vec || gate_stride % vec ||
-      out_stride % vec)
-    return MV_E_ALIGN;
   const int64_t items = (int64_t)rows * heads;
   const int vecs = p / vec;
   // four items a thread where that leaves four workgroups a CU (19 000 x 16 heads of 128: one item 44.6 us, four 39.2)

@@ -159,6 +159,11 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
   }
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_to(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+
 // Workgroup = W waves = W tiles of 16 columns of one head of one sequence; a wave keeps S of its columns in accumulators, whose rows are
 // dealt so that tiles 2 s and 2 s + 1 together hold n = 32 s + 8 g .. + 7 in lane group g: operands of the next product as they are.  o is
 // computed transposed (columns by tokens), so that a lane holds four columns of a token; the rows of v land in LDS like those of k and q and are
@@ -168,7 +173,11 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
 // elements; 158 with eight waves of one tile, two on a SIMD, that fill each other's gaps, and v by LDS; 144 with transfers asked for between the
 // products (all at once they held a wave up for 3000 of 12000 cycles) and k, q on one XCD; 135 with o by lines (by 32 bytes its stores took 30 us).
 // Where heads and sequences do not fill the chip, workgroups of four waves leave no CU idle.
-template <int NK, int W>
+// NORM (the workgroup has all of a head's columns): the rows leave normed and gated.  A row of the head lies on 2 W adjacent lanes when it is stored, as in
+// head_norm_gate_kernel, whose rounding points and order of the sum these are; the gate's pieces come with the chunk.  Bound by the same
+// chain, of which this is vector arithmetic: the walk above 122 -> 148 us, where a launch behind it took 43 and a pass over o; the layer 271 -> 242.  Half of
+// the waves later than the others, so that one of two on a SIMD multiplies meanwhile: 267.
+template <int NK, int W, bool NORM>
 __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep q) {
   typedef elem<B16>::T T;
   constexpr int N = NK * 32, ROWS = 4 * NK, VF = 2 * W;   // fragments of 1 KiB: k, q; v
@@ -229,7 +238,39 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
   };
   // Results take the place of the wave's columns of v in LDS; at the next chunk a wave takes the rows from there that it brings v of, whole lines
   // of them, and stores them.
-  u32x4 done[2];
+  u32x4 done[2], gate[2] = {}, norm_w[2];   // (gate: of the chunk's rows, on their way with it)
+  const bool padded = p.p_true < W * 16;
+  const float share = NORM ? 1.0f / (float)p.p_true : 0.f;
+  auto col_of = [&](int i) { return ((lane % VP) ^ v_swizzle((2 * wave + i) * VR + lane / VP)) * 8; };   // (the head's first column is the workgroup's)
+  if constexpr (NORM) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) norm_w[i] = *(const u32x4 *)((const T *)p.norm_w + min(col_of(i), p.p - 8));
+  }
+  auto ask_gate = [&](int c, int i) __attribute__((always_inline)) {
+    const int t = min(c * L + (2 * wave + i) * VR + lane / VP, len - 1);
+    gate[i] = *(const u32x4 *)((const T *)p.gate + (int64_t)(q0 + t) * p.gate_stride + head * p.p + min(col_of(i), p.p - 8));
+  };
+  auto norm_gate = [&](int i) __attribute__((always_inline)) {   // done[i] becomes what norm and gate make of it
+    float f[8], z[8], w[8], ss = 0.f;
+    unpack8<B16>(done[i], f);
+    unpack8<B16>(gate[i], z);
+    unpack8<B16>(norm_w[i], w);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (padded && col_of(i) + j >= p.p_true) f[j] = 0.f;
+      ss = fmaf(f[j], f[j], ss);
+    }
+    if constexpr (VP == 16) {
+      ss = row16_sum(ss);
+    } else {
+      static_assert(VP == 16 || VP == 8, "lanes of a row");
+      ss += dpp_to<0xB1>(ss), ss += dpp_to<0x4E>(ss), ss += dpp_to<0x141>(ss);   // lanes ^ 1, ^ 2, the other four of eight
+    }
+    const float rs = head_rms_16(ss, share, p.eps, p.out_scale);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) f[j] = f[j] * rs * w[j] * gate_16(z[j], p.gate_kind);
+    done[i] = pack8<B16>(f);
+  };
   const bool pieces = !(((uintptr_t)p.out & 15) | (p.out_stride & 7));   // (rows of the output may stand anywhere)
   auto store = [&](int c, int i) __attribute__((always_inline)) {
     const int r = (2 * wave + i) * VR + lane / VP, t = c * L + r, at = tile0 * 16 + ((lane % VP) ^ v_swizzle(r)) * 8;
@@ -249,7 +290,13 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
     constexpr int n = decltype(I)::value, lo = ALL * n / POINTS, hi = ALL * (n + 1) / POINTS;
     if constexpr (n == 0) lds_wait<8>(done[0], done[1]);   // (read ahead of the rows; the transfers of v come behind)
     if (c + 1 < chunks) static_for<hi - lo>([&](auto J) { fetch(std::integral_constant<int, lo + decltype(J)::value>{}, c + 1); });
-    if (n < 2 && c > 0) store(c - 1, n);
+    if constexpr (n < 2) {
+      if (c > 0) {
+        if constexpr (NORM) norm_gate(n);
+        store(c - 1, n);
+      }
+      if constexpr (NORM) ask_gate(c, n);
+    }
   };
   const uint32_t lds = lds_address(smem);
   const int chunks = (len + L - 1) / L;
@@ -257,6 +304,8 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
   for (int c = 0; c < chunks; ++c) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     lds_barrier();   // this chunk has landed; every wave is done with the one before
+    // (the compiler's own wait for the gate belongs here, where nothing is under way: behind, it would take in the next chunk's transfers)
+    if constexpr (NORM) asm volatile("" : "+v"(gate[0]), "+v"(gate[1]));
     const uint32_t at = lds + (c & 1) * STAGE, rows = at + row_place(r16, g) * 16, rest_at = at + AT * 1024;
     const uint32_t fl = rest_at + lane * 16, ff = rest_at + kFactors * 1024 + g * 16;
     const uint32_t tr = at + row_place(4 * g + (r16 >> 2), r16 & 3) * 16;
@@ -431,6 +480,7 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     done[i] = *(const u32x4 *)(smem + ((chunks - 1) & 1) * STAGE + (AT_V + 2 * wave + i) * 1024 + lane * 16);
+    if constexpr (NORM) norm_gate(i);
     store(chunks - 1, i);
   }
   if (keep && live) {
@@ -441,8 +491,26 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
   }
 }
 
+template <int NK, int W>
+int launch_walk(const DeltaPrep &q, int slices, int lds, bool *normed, hipStream_t stream) {
+  const dim3 grid(slices, q.a.heads, q.a.n_seqs), block(W * 64);
+  // Norm and gate in the walk lengthen the chain of the longest sequence, by 1.1 us a chunk with eight waves (16 sequences of up to 1490 tokens, 16 heads of 128:
+  // 26 us) and 0.47 with four (3 of up to 1490, 16 heads of 64: 11); a launch behind it takes some 3.5 us and the time of its rows (43 and 7).
+  const double chunks = (q.a.max_q + L - 1) / L, in_chain = chunks * (W == 8 ? 1.1 : 0.47), behind = 3.5 + (double)q.a.total_q * q.a.heads * q.a.p * 6 / 5.7e6;
+  if (normed && slices == 1 && in_chain <= behind) {
+    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, W, true>>()) return rc;
+    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, W, true>), grid, block, lds, stream, q);
+    *normed = true;
+  } else {
+    if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, W, false>>()) return rc;
+    hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, W, false>), grid, block, lds, stream, q);
+  }
+  MV_LAUNCH_CHECK();
+  return MV_OK;
+}
+
 template <int NK>
-int launch(const DeltaPrep &q, hipStream_t stream) {
+int launch(const DeltaPrep &q, bool *normed, hipStream_t stream) {
   const MvDeltaArgs &a = q.a;
   const unsigned slots = (unsigned)chunk_slots(a.n_seqs, a.total_q);
   if (a.heads / a.groups % 2 == 0) hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 2>), dim3(slots, a.heads / 2), dim3(512), 0, stream, q);
@@ -453,30 +521,22 @@ int launch(const DeltaPrep &q, hipStream_t stream) {
   const int tiles = a.p / 16, wide = (tiles + 7) / 8, narrow = (tiles + 3) / 4;
   constexpr auto lds = [](int waves) { return 2 * (8 * NK + 2 * waves + kScalarTotal) * 1024; };
   if constexpr (lds(8) <= 160 * 1024) {
-    if (tiles > 4 && (int64_t)narrow * a.heads * a.n_seqs > 256) {
-      if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 8>>()) return rc;
-      hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 8>), dim3(wide, a.heads, a.n_seqs), dim3(512), lds(8), stream, q);
-      MV_LAUNCH_CHECK();
-      return MV_OK;
-    }
+    if (tiles > 4 && (int64_t)narrow * a.heads * a.n_seqs > 256) return launch_walk<NK, 8>(q, wide, lds(8), normed, stream);
   }
-  if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, 4>>()) return rc;
-  hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, 4>), dim3(narrow, a.heads, a.n_seqs), dim3(256), lds(4), stream, q);
-  MV_LAUNCH_CHECK();
-  return MV_OK;
+  return launch_walk<NK, 4>(q, narrow, lds(4), normed, stream);
 }
 
 }  // namespace
 
 // (arguments checked by mv_delta_chunk_launch, whose workspace is larger)
-int mv_delta_scalar_launch(const MvDeltaArgs &a, hipStream_t stream) {
+int mv_delta_scalar_launch(const MvDeltaArgs &a, bool *normed, hipStream_t stream) {
   const DeltaPrep q{a, (char *)a.workspace};
   switch (a.n / 32) {
-    case 1: return launch<1>(q, stream);
-    case 2: return launch<2>(q, stream);
-    case 3: return launch<3>(q, stream);
-    case 4: return launch<4>(q, stream);
-    case 5: return launch<5>(q, stream);
+    case 1: return launch<1>(q, normed, stream);
+    case 2: return launch<2>(q, normed, stream);
+    case 3: return launch<3>(q, normed, stream);
+    case 4: return launch<4>(q, normed, stream);
+    case 5: return launch<5>(q, normed, stream);
   }
   return MV_E_SHAPE;
 }

@@ -1495,7 +1495,7 @@ def gated_group_norm(y, z, w, heads: int, p: int, p_true: int, groups: int, eps:
 
 
 # ---------------------------------------------------------------- K16
-MV_DELTA_SCAN = 1
+MV_DELTA_SCAN, MV_DELTA_NORM = 1, 2
 GATES = {"silu": 0, "sigmoid": 1}
 
 
@@ -1547,8 +1547,10 @@ def _delta_args(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots, o
     return g
 
 
-def delta_prefill(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots, cu_q, cu_k, max_q: int, out=None, flags: int = 0):
-    """The gated delta rule over convolved channels [T, channels], raw beta [T, heads] and raw decays -> o [T, heads * p]."""
+def delta_prefill(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots, cu_q, cu_k, max_q: int, out=None, flags: int = 0,
+                  gate=None, norm_w=None, gate_kind: str = "silu", out_scale: float = 1.0):
+    """The gated delta rule over convolved channels [T, channels], raw beta [T, heads] and raw decays -> o [T, heads * p]; with ``gate``
+    [T, heads * p] and ``norm_w``: ``head_norm_gate`` of it."""
     if out is None:
         out = torch.empty((x.shape[0], s.heads * s.p), dtype=x.dtype, device=x.device)
     g = _delta_args(s, x, beta, a, dt_bias, a_log, state, state_slots, out)
@@ -1558,6 +1560,13 @@ def delta_prefill(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots,
         n += int(_lib.mv_delta_prefill_segments_bytes(g.n_seqs, g.total_q, g.max_q, s.heads, s.p, s.n, g.channel_decay, _dt(x)))
     ws = torch.empty((n,), dtype=torch.uint8, device=x.device) if n else None
     g.workspace, g.ws_bytes = _ptr(ws), n
+    if gate is not None:
+        _need_cuda(gate, norm_w)
+        _rows_ok("gate", gate, s.heads * s.p, x.dtype)
+        if norm_w.dtype != x.dtype or norm_w.numel() < s.p or gate.shape[0] != x.shape[0] or out.shape[0] != x.shape[0]:
+            raise MvHipError(f"norm weight of {s.p} {x.dtype} and as many rows of the gate and the output required")
+        g.gate, g.gate_stride, g.norm_w, g.gate_kind, g.out_scale = gate.data_ptr(), gate.stride(0), norm_w.data_ptr(), GATES[gate_kind], float(out_scale)
+        flags |= MV_DELTA_NORM
     _check(_lib.mv_delta_prefill(ctypes.byref(g), _dt(x), int(flags), _stream()), "mv_delta_prefill")
     return out
 

@@ -96,5 +96,5 @@ class GatedDeltaRule(nn.Module):
             cu_q, cu_k, max_q = ((ctx.rest_cum_seqlens_q, ctx.rest_cum_seqlens_k, ctx.rest_max_seqlen_q) if nd else
                                  (ctx.cum_seqlens_q, ctx.cum_seqlens_k, ctx.max_seqlen_q))
             xc = hip_ops.causal_conv(x[nd:], self.conv, None, s.conv, self.conv_state, slots[nd:], cu_q, cu_k, max_q)
-            y = hip_ops.delta_prefill(s, xc, beta[nd:], a[nd:], self.dt_bias, self.A_log, self.state, slots[nd:], cu_q, cu_k, max_q)
-            hip_ops.head_norm_gate(y, gate[nd:], self.norm, s.heads, s.p, s.p_true, s.eps, self.gate, self.out_scale, out=out[nd:])
+            hip_ops.delta_prefill(s, xc, beta[nd:], a[nd:], self.dt_bias, self.A_log, self.state, slots[nd:], cu_q, cu_k, max_q, out=out[nd:],
+                                  gate=gate[nd:], norm_w=self.norm, gate_kind=self.gate, out_scale=self.out_scale)
