@@ -19,7 +19,8 @@
 // to itself, half of it in throughput.  Few long sequences are therefore cut into segments of whole chunks (pick_segment): a first launch
 // carries the state through every segment but the last from zeros (the recurrence is linear: b, x and step sizes only), the second starts a
 // segment from S = the sum of those before it, each decayed by the segments between.  64 heads of 64 x 128 with the convolution and the
-// norm: 4 sequences of up to 3900 tokens 315 -> 271 us (the recurrence 232 -> 139 + 69 under the profiler), 1 x 1900 127 -> 71; 32 heads, 1 x 3900 229 -> 83.
+// norm: 4 sequences of up to 3900 tokens 315 -> 271 us (the recurrence 232 -> 139 + 69 under the profiler), 1 x 1900 127 -> 71; 32 heads, 1 x 3900 229 -> 83.  Step
+// sizes and decays of a batch of chunks by all waves instead of the next chunk's by one: 271 -> 257 (the states 71 -> 56).
 #include <algorithm>
 
 #include "ssm.h"
@@ -74,7 +75,8 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
   constexpr int PER = (PIECES + THREADS - 1) / THREADS, AHEAD = PER <= 20 ? PER : 20;
   __shared__ __attribute__((aligned(16))) char bs[L * RB], cs[OUT ? L * RB : 16], xs[L * RX];
   __shared__ u32x4 wf[2][OUT ? 4 : 1][2][64];  // weighted scores, high / remainder: [token tile][32 keys][lane]
-  __shared__ float steps[2][3][L];             // of this and the next chunk: r_i (log2), dt_i, exp(r_last - r_i) dt_i
+  constexpr int BATCH = 2 * PT;
+  __shared__ float steps[BATCH][3][L];         // of BATCH chunks: r_i (log2), dt_i, exp(r_last - r_i) dt_i
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
   const int slice = blockIdx.x, head = blockIdx.y;
   int seq = blockIdx.z, from = 0, q0 = p.cu_q[MODE == WHOLE ? seq : 0], len = 0, all = 0;
@@ -149,9 +151,7 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
     src[k] = x + (int64_t)rows[k] * p.x_stride + col;
   }
   u32x4 ahead[AHEAD];
-  float dt_ahead = 0.f;
   auto request = [&](int t0) {
-    if (wave == 0) dt_ahead = elem<Tag>::ld(dt[(int64_t)min(t0 + lane, len - 1) * p.dt_stride]);
     if (t0 + L <= len) {
       const int64_t off = (int64_t)t0 * p.x_stride;
 #pragma unroll
@@ -162,24 +162,44 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
         ahead[k] = *(const u32x4 *)(src[k] + (int64_t)(min(t0 + rows[k], len - 1) - rows[k]) * p.x_stride);
     }
   };
-  // step sizes and decays of the requested chunk (wave 0); tokens behind the end: dt = 0, no decay
-  auto scan = [&](int nt, float (*to)[L]) {
-    const float step = lane < nt ? softplus_f32(dt_ahead + bias) : 0.f;
-    float r = na2 * step;
+  // Step sizes and decays of BATCH chunks from c0 on, two a wave (tokens behind the end: dt = 0, no decay).  By one wave for the next chunk, they were what
+  // the others waited for at its barrier: 0.5 us a chunk.
+  float raw[2];
+  auto ask_steps = [&](int c0) {
 #pragma unroll
-    for (int o = 1; o < 64; o *= 2) {
-      const float v = __shfl_up(r, o, 64);
-      if (lane >= o) r += v;
-    }
-    to[0][lane] = r, to[1][lane] = step;
-    to[2][lane] = __builtin_amdgcn_exp2f(__shfl(r, 63, 64) - r) * step;
+    for (int j = 0; j < 2; ++j) raw[j] = elem<Tag>::ld(dt[(int64_t)min((c0 + wave + PT * j) * L + lane, len - 1) * p.dt_stride]);
   };
+  auto scan = [&](int c0) {
+    float step[2], r[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      step[j] = (c0 + wave + PT * j) * L + lane < len ? softplus_f32(raw[j] + bias) : 0.f;
+      r[j] = na2 * step[j];
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o *= 2)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float v = __shfl_up(r[j], o, 64);
+        if (lane >= o) r[j] += v;
+      }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float (*to)[L] = steps[wave + PT * j];
+      to[0][lane] = r[j], to[1][lane] = step[j];
+      to[2][lane] = __builtin_amdgcn_exp2f(__shfl(r[j], 63, 64) - r[j]) * step[j];
+    }
+  };
+  ask_steps(0);
   request(0);
-  if (wave == 0) scan(min(L, len), steps[0]);
 
   for (int t0 = 0; t0 < len; t0 += L) {
-    const int nt = min(L, len - t0), cur = (t0 / L) & 1;
+    const int nt = min(L, len - t0), chunk = t0 / L, cur = chunk % BATCH;
     const float *rs = steps[cur][0], *dts = steps[cur][1], *ws = steps[cur][2];
+    if (cur == 0) {   // (nobody needs the batch before: a barrier ended its last chunk)
+      scan(chunk);
+      if (t0 + BATCH * L < len) ask_steps(chunk + BATCH);
+    }
 #pragma unroll
     for (int k = 0; k < AHEAD; ++k) *(u32x4 *)dst[k] = ahead[k];   // (threads without a piece repeat the last one)
     if constexpr (PER > AHEAD) {
@@ -246,7 +266,6 @@ __global__ void __launch_bounds__(PT * 64, PT == 4 ? 2 : 1) ssm_chunk_kernel(MvS
         }
       }
     }
-    if (wave == 0 && t0 + L < len) scan(min(L, len - t0 - L), steps[cur ^ 1]);   // (wave 0 scored the fewest keys)
     if constexpr (OUT) __syncthreads();
     else decayed += rs[L - 1];
     // ---- sum over the chunk's keys; then the state moves on
