@@ -2,6 +2,8 @@
 // launch each) and decode_persistent.hip (phases of the persistent small-batch decode kernel, over virtual workgroups):
 // ONE statement of the arithmetic, so the two paths are bit-identical by construction.
 #pragma once
+#include <type_traits>
+
 #include "paged_decode.h"
 
 template <typename Tag>
@@ -344,40 +346,45 @@ __device__ __forceinline__ void paged_decode_reduce_body(const float *ws_acc, co
   lds_f *sf = (lds_f *)lds + 128 * 4;
   lds_f &s_l = ((lds_f *)lds)[128 * 4 + 64];
   const int q = tid / D4, c = tid - q * D4;
-  // rows first (they do not depend on the factors), then the pairs: one round trip covers both
-  f32x4 a[PER];
-  const f32x4 *row = reinterpret_cast<const f32x4 *>(ws_acc + bh * nsplit * D) + c;
-#pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int sp = q + u * NQ;
-    a[u] = ldf4<COH>(reinterpret_cast<const float *>(row + (int64_t)(sp < nsplit ? sp : 0) * D4));
-  }
-  float m = -1e30f, l = 0.f;
-  if (tid < nsplit) {
-    m = ldf<COH>(ws_ml + (bh * nsplit + tid) * 2);
-    l = ldf<COH>(ws_ml + (bh * nsplit + tid) * 2 + 1);
-  }
-  // maximum over the splits (<= 64: the first wave holds them all), factors, the sum of l * f
-  if (tid < 64) {
-    float M = m;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-    const float f = tid < nsplit ? __builtin_amdgcn_exp2f(m - M) : 0.f;
-    sf[tid] = f;
-    float L = l * f;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) L += __shfl_xor(L, off, 64);
-    if (tid == 0) s_l = L;
-  }
-  __syncthreads();
   f32x4 A = {0.f, 0.f, 0.f, 0.f};
+  // As many rows a thread as the splits need: rows asked for and added beside those, and sums over a wave through the LDS pipe, are time of the launch.
+  // A step of 28 layers with one launch each: one sequence of 100 tokens 1083 -> 1059 us, of 777 1097 -> 1082, eight of up to 500 1258 -> 1244.
+  auto combine = [&](auto ROWS) __attribute__((always_inline)) {
+    constexpr int rows = decltype(ROWS)::value;
+    // rows first (they do not depend on the factors), then the pairs: one round trip covers both
+    f32x4 a[rows];
+    const f32x4 *row = reinterpret_cast<const f32x4 *>(ws_acc + bh * nsplit * D) + c;
 #pragma unroll
-  for (int u = 0; u < PER; ++u) {
-    const int sp = q + u * NQ;
-    const float f = sp < nsplit ? sf[sp] : 0.f;
+    for (int u = 0; u < rows; ++u) {
+      const int sp = q + u * NQ;
+      a[u] = ldf4<COH>(reinterpret_cast<const float *>(row + (int64_t)(sp < nsplit ? sp : 0) * D4));
+    }
+    float m = -1e30f, l = 0.f;
+    if (tid < nsplit) {
+      m = ldf<COH>(ws_ml + (bh * nsplit + tid) * 2);
+      l = ldf<COH>(ws_ml + (bh * nsplit + tid) * 2 + 1);
+    }
+    // maximum over the splits (<= 64: the first wave holds them all), factors, the sum of l * f
+    if (tid < 64) {
+      const float M = wave_max(m);
+      const float f = tid < nsplit ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+      sf[tid] = f;
+      const float L = wave_sum(l * f);
+      if (tid == 0) s_l = L;
+    }
+    __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 4; ++e) A[e] += a[u][e] * f;
-  }
+    for (int u = 0; u < rows; ++u) {
+      const int sp = q + u * NQ;
+      const float f = sp < nsplit ? sf[sp] : 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) A[e] += a[u][e] * f;
+    }
+  };
+  if (nsplit <= 2 * NQ) combine(std::integral_constant<int, 2>{});
+  else if (nsplit <= PER / 4 * NQ) combine(std::integral_constant<int, PER / 4>{});
+  else if (nsplit <= PER / 2 * NQ) combine(std::integral_constant<int, PER / 2>{});
+  else combine(std::integral_constant<int, PER>{});
   part[q][c] = A;
   __syncthreads();
   if (q == 0 && write) {
