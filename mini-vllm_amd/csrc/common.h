@@ -137,6 +137,14 @@ __device__ __forceinline__ float wave_sum(float x) {
   swap32(a + b, a, b);
   return a + b;
 }
+// The sum in the order of a butterfly of 32, 16, 8, 4, 2, 1 lanes (behind an exchange the values repeat with its distance, so that a rotation by half
+// of that is an exchange): its bits, without the LDS pipe.
+__device__ __forceinline__ float wave_sum_halves(float x) {
+  float a, b;
+  swap32(x, a, b);
+  swap16(a + b, a, b);
+  return row16_sum(a + b);
+}
 __device__ __forceinline__ float wave_max(float x) {
   float a, b;
   swap16(row16_max(x), a, b);

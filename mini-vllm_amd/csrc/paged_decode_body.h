@@ -321,9 +321,8 @@ __global__ void __launch_bounds__(256) paged_decode_kernel(DecodeParams p) {
 
 // Split-KV combine: one workgroup (128 threads) per (sequence, head).  The partial rows were written by workgroups on other
 // XCDs, so every load is a ~2 us round trip and what counts is how many of them are DEPENDENT: the (m, l) pairs go
-// through LDS once; then thread (q, c) — q = threadIdx / (D/4) picks every QUARTER-th split, c the 16-byte column piece —
-// keeps all its rows (up to 16) in flight at once, and the four partial sums meet in LDS.  (Round 2: one thread per
-// output dim, eight 4-byte loads in flight, four rounds at 32 splits: 6.8 us per launch, 14 % of the B = 1 step.)
+// go to the first wave's lanes once; thread (q, c) — q = threadIdx / (D/4) picks every NQ-th split, c the 16-byte column piece —
+// keeps all its rows (as many as the splits need, up to 64 / NQ) in flight at once, and the NQ partial sums meet in LDS.
 // LDS of one (virtual) workgroup of paged_decode_reduce_body, in floats: part [NQ][D4] f32x4, then sf [64], then s_l
 template <int D>
 struct ReduceLds {
@@ -347,8 +346,9 @@ __device__ __forceinline__ void paged_decode_reduce_body(const float *ws_acc, co
   lds_f &s_l = ((lds_f *)lds)[128 * 4 + 64];
   const int q = tid / D4, c = tid - q * D4;
   f32x4 A = {0.f, 0.f, 0.f, 0.f};
-  // As many rows a thread as the splits need: rows asked for and added beside those, and sums over a wave through the LDS pipe, are time of the launch.
-  // A step of 28 layers with one launch each: one sequence of 100 tokens 1083 -> 1059 us, of 777 1097 -> 1082, eight of up to 500 1258 -> 1244.
+  // As many rows a thread as the splits need: rows asked for and added beside those are time of the launch.  A step of 28 layers with one launch each,
+  // one sequence of 777 tokens: 1099 -> 1085 us (those left out had a factor of 0: the same bits); another 5 (two runs differ by 4) by sums over
+  // a wave that do not go through the LDS pipe.
   auto combine = [&](auto ROWS) __attribute__((always_inline)) {
     constexpr int rows = decltype(ROWS)::value;
     // rows first (they do not depend on the factors), then the pairs: one round trip covers both
@@ -369,7 +369,7 @@ __device__ __forceinline__ void paged_decode_reduce_body(const float *ws_acc, co
       const float M = wave_max(m);
       const float f = tid < nsplit ? __builtin_amdgcn_exp2f(m - M) : 0.f;
       sf[tid] = f;
-      const float L = wave_sum(l * f);
+      const float L = wave_sum_halves(l * f);   // (in this order: sums of other shapes differ in the last bit, and a step's tokens with it)
       if (tid == 0) s_l = L;
     }
     __syncthreads();
