@@ -758,7 +758,10 @@ int mv_moe_group(const int32_t *ids, int pairs, int top, int experts, int tile_m
                  int32_t *tiles, const float *weights, float *weights_out, void *stream);
 /* out[place] = W[expert] x[tokens[place]] (tokens NULL: x[place]), W [experts][n][k]; act: W [experts][2][n][k], out = act(gate, up).
  * 16-bit: W packed per expert (mv_pack_weight of all rows), tile_m 16, 32, 64, 128 or 256; fp32: W as it is, tile_m 16.  n % 16 == 0,
- * k % 64 == 0.  in_scale [places] (may be NULL): the input x is multiplied by it (the sums are, in fp32, ahead of the activation). */
+ * k % 64 == 0.  in_scale [places] (may be NULL): the input x is multiplied by it (the sums are, in fp32, ahead of the activation).
+ * Sums: one behind the other for tile_m from 64 on; below that, and for tile_m 64 | MV_MOE_QUARTERS, of four quarters of the inputs: the same bits for any
+ * tile_m of either kind. */
+enum { MV_MOE_QUARTERS = 1 << 16 };
 typedef struct MvMoeLinearArgs {
   const void *x, *w;
   void *out;

@@ -391,7 +391,8 @@ __device__ __forceinline__ int row_place(int row, int chunk) { return row * 4 + 
 
 // many rows: BM x BN per workgroup of 2 x 2 waves, 64 inputs at a time.  Rows and weights reach LDS by DMA as fragments (16 rows x
 // 32 inputs, 1 KiB; weights in the order of the lanes); the next 64 inputs land while these are multiplied.
-template <typename Tag, int BM, int BN, bool GATED>
+// QUARTERS: sums as moe_small_kernel makes them, of four quarters of the inputs, so that an expert of some 30 rows gives the same bits from either.
+template <typename Tag, int BM, int BN, bool GATED, bool QUARTERS>
 __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
   typedef typename elem<Tag>::T T;
   constexpr int MT = BM / 16, NT = BN / 16, WM = MT / 2, WN = NT / 2, PIECES = 2 * (MT + NT), PER = PIECES / 4;
@@ -429,6 +430,23 @@ __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
   f32x4 acc[WN][WM] = {};
   const uint32_t base = lds_address(smem) + lane * 16, rows = lds_address(smem) + row_place(r16, g) * 16;
   const int trips = p.k / 64;
+  f32x4 half[QUARTERS ? 2 : 1][WN][WM] = {};
+  int quarter = 0;
+  auto settle = [&](int done) {   // the quarters that end behind `done` steps of 32 inputs
+    while (quarter < 3 && steps * (quarter + 1) / 4 == done) {
+#pragma unroll
+      for (int j = 0; j < WN; ++j)
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+          if (quarter == 2) half[1][j][i] = acc[j][i];
+          else if (quarter == 1) half[0][j][i] += acc[j][i];
+          else half[0][j][i] = acc[j][i];
+          acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      ++quarter;
+    }
+  };
+  if constexpr (QUARTERS) settle(0);
   fetch(0);
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   lds_barrier();
@@ -449,9 +467,16 @@ __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
       for (int j = 0; j < WN; ++j)
 #pragma unroll
         for (int i = 0; i < WM; ++i) acc[j][i] = mfma16x16x32<Tag>(a[h][j], b[h][i], acc[j][i]);
+      if constexpr (QUARTERS) settle(2 * t + h + 1);
     });
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
+  }
+  if constexpr (QUARTERS) {
+#pragma unroll
+    for (int j = 0; j < WN; ++j)
+#pragma unroll
+      for (int i = 0; i < WM; ++i) acc[j][i] = half[0][j][i] + (half[1][j][i] + acc[j][i]);
   }
 #pragma unroll
   for (int i = 0; i < WM; ++i) {
@@ -658,14 +683,17 @@ int launch_linear(const MoeLinear &p, int tile_m, int max_tiles, hipStream_t st)
   const int nt = p.n / 16;
   constexpr int TN = GATED ? 1 : 2;
   const dim3 small((nt + TN - 1) / TN, max_tiles);
+  const bool quarters = tile_m & MV_MOE_QUARTERS;
+  tile_m &= ~MV_MOE_QUARTERS;
   if (tile_m == 16) hipLaunchKernelGGL((moe_small_kernel<Tag, 1, TN, GATED>), small, dim3(256), 0, st, p);
   else if (tile_m == 32) hipLaunchKernelGGL((moe_small_kernel<Tag, 2, TN, GATED>), small, dim3(256), 0, st, p);
-  else if (tile_m == 64 || tile_m == 128) {
+  else if (tile_m == 64 || (tile_m == 128 && !quarters)) {
     constexpr int BN = 128;
     const dim3 grid((nt * 16 * (GATED ? 2 : 1) + BN - 1) / BN, max_tiles);
-    if (tile_m == 64) hipLaunchKernelGGL((moe_tile_kernel<Tag, 64, BN, GATED>), grid, dim3(256), (64 + BN) * 256, st, p);
-    else hipLaunchKernelGGL((moe_tile_kernel<Tag, 128, BN, GATED>), grid, dim3(256), (128 + BN) * 256, st, p);
-  } else if (tile_m == 256) {
+    if (tile_m == 128) hipLaunchKernelGGL((moe_tile_kernel<Tag, 128, BN, GATED, false>), grid, dim3(256), (128 + BN) * 256, st, p);
+    else if (quarters) hipLaunchKernelGGL((moe_tile_kernel<Tag, 64, BN, GATED, true>), grid, dim3(256), (64 + BN) * 256, st, p);
+    else hipLaunchKernelGGL((moe_tile_kernel<Tag, 64, BN, GATED, false>), grid, dim3(256), (64 + BN) * 256, st, p);
+  } else if (tile_m == 256 && !quarters) {
     const int nx = (nt * (GATED ? 2 : 1) + 15) / 16;
     if (int rc = mv_allow_lds<moe_wide_kernel<Tag, GATED>>()) return rc;
     hipLaunchKernelGGL((moe_wide_kernel<Tag, GATED>), dim3((unsigned)(((int64_t)max_tiles * 2 * nx + 7) / 8 * 8)), dim3(256),

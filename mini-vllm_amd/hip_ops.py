@@ -1631,6 +1631,9 @@ def moe_route(x, w, correction, top: int, groups: int = 1, keep: int = 1, scale:
     return ids, weights
 
 
+MV_MOE_QUARTERS = 1 << 16
+
+
 class ExpertGroups(NamedTuple):
     place: torch.Tensor      # int32 [pairs]; -1: no product
     tokens: torch.Tensor     # int32 [pairs], by place
@@ -1657,10 +1660,10 @@ def moe_group(ids, experts: int, tile_m: int, weights=None) -> ExpertGroups:
 
 
 def moe_linear(x, w, n: int, groups: ExpertGroups, act: GateAct | None = None, gather: bool = False, experts: int = 0,
-               in_scale=None):
+               in_scale=None, quarters: bool = False):
     """Rows by place: out[i] = W[expert of i] x[i] (``gather``: x[token of i]), W the experts' weights [experts, n, K] -- fp32: as
     they are, 16-bit: packed per expert; ``act``: [experts, 2, n, K], out = act(gate, up).  ``in_scale`` (fp32 by
-    place): the inputs are multiplied by it."""
+    place): the inputs are multiplied by it.  ``quarters`` (tiles of 64 rows): sums as from smaller tiles, the same bits."""
     _need_cuda(x, w, in_scale)
     pairs, k = groups.tokens.numel(), x.shape[1]
     _rows_ok("x", x, 1, w.dtype)
@@ -1671,7 +1674,8 @@ def moe_linear(x, w, n: int, groups: ExpertGroups, act: GateAct | None = None, g
         raise MvHipError("a dense fp32 factor per place required")
     a = MvMoeLinearArgs(x=x.data_ptr(), w=w.data_ptr(), out=out.data_ptr(), in_scale=_ptr(in_scale), tokens=groups.tokens.data_ptr() if gather else None,
                         tiles=groups.tiles.data_ptr(), act=ctypes.addressof(act) if act is not None else None, x_stride=x.stride(0),
-                        out_stride=out.stride(0), max_tiles=groups.tiles.shape[0], tile_m=groups.tile_m, n=n, k=k)
+                        out_stride=out.stride(0), max_tiles=groups.tiles.shape[0],
+                        tile_m=groups.tile_m | (MV_MOE_QUARTERS if quarters else 0), n=n, k=k)
     _check(_lib.mv_moe_linear(ctypes.byref(a), _dt(x), _stream()), "mv_moe_linear")
     return out
 

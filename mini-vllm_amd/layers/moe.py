@@ -27,7 +27,9 @@ __all__ = ["ExpertMLP"]
 #   24 pairs 65 / 64, 64 84 / 68, 256 176 / 128; of 1024 -> 384 64 pairs (96) 30 / 33, 160 (192) 51 / 37; 8 of 2048 -> 768 256 (96) 46 / 52, 384 (144) 59 / 55, 800
 #   103 / 83; 2 of 2048 -> 768 1100 (108) 46 / 56, 2500 (240) 88 / 70; the worst found: 2 of 4096 -> 1024, 1500 pairs (192) 102 / 111.
 #   128 rows (tiles of the 64's kind) are nowhere ahead of both.
-FEW, MANY_EXPERTS, WIDE_GROUPS = 8, 32, 160
+# Up to QUARTERS pairs per expert, tiles of 64 rows sum as those of 16 and 32 do: a call's bits are those of tiles of 32 rows, which it once had.
+# That costs nothing in them, but 256 rows, which have no such sums, would be ahead in the end: 32 experts of 2048 -> 768, 24 pairs 68 / 65, 40 74 / 66 (32 rows 78, 130).
+FEW, MANY_EXPERTS, WIDE_GROUPS, QUARTERS = 8, 32, 160, 40
 
 
 class ExpertMLP(nn.Module):
@@ -80,6 +82,8 @@ class ExpertMLP(nn.Module):
         per = tokens * self.top / self.experts
         if per <= (16 if self.experts >= MANY_EXPERTS else 28):
             return 16 if per <= FEW else 32
+        if per <= QUARTERS:
+            return 64
         wide = self.experts * math.ceil(per / 128) * math.ceil(2 * self.f / 256)      # workgroups of the gated product
         return 256 if wide >= WIDE_GROUPS else 64
 
@@ -92,8 +96,9 @@ class ExpertMLP(nn.Module):
     def forward(self, h):
         """-> (shared expert's output or None, the routed experts' part for ``hip_ops.residual_update``)."""
         weights, g = self.route(h)
-        z = hip_ops.moe_linear(h, self.gate_up, self.f, g, self.act, gather=True, experts=self.experts, in_scale=g.weights)
-        y = hip_ops.moe_linear(z, self.down, self.w, g, experts=self.experts)
+        quarters = g.tile_m == 64 and h.shape[0] * self.top <= QUARTERS * self.experts
+        z = hip_ops.moe_linear(h, self.gate_up, self.f, g, self.act, gather=True, experts=self.experts, in_scale=g.weights, quarters=quarters)
+        y = hip_ops.moe_linear(z, self.down, self.w, g, experts=self.experts, quarters=quarters)
         shared = None
         if self.shared_gate_up is not None:
             shared = self.shared_down(gated_linear(h, self.shared_gate_up, "silu"), partial_ok=True)

@@ -32,3 +32,48 @@ def test_groups_in_parts(pairs, top, experts, outputs, tile_m, weighed):
             assert 0 < n <= tile_m and bool((flat[order[first:first + n]] == e).all())
             seen[first:first + n] += 1
     assert bool((seen == 1).all())
+
+
+# inputs: quarters that are empty, that end within a trip of 64 inputs, whole ones
+@pytest.mark.parametrize("k", [64, 128, 192, 320, 768, 2048])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("gated, weighed", [(True, False), (False, False), (True, True)])
+def test_sums_by_quarters_are_those_of_small_tiles(k, dtype, gated, weighed):
+    from minivllm_amd import hip_ops as H
+
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=DEV)
+    experts, tokens, top, n = 5, 97, 2, 144
+    ids = torch.randint(0, experts + 1, (tokens, top), generator=gen, device=DEV, dtype=torch.int32)
+    scale = torch.rand(ids.shape, generator=gen, device=DEV) if weighed else None
+    x = rand(tokens, k).to(dtype)
+    w = H.pack_weight((rand(experts * n * (2 if gated else 1), k) * k ** -0.5).to(dtype))
+    outs = []
+    for tile, quarters in ((16, False), (32, False), (64, True)):
+        g = H.moe_group(ids, experts, tile, scale)
+        y = H.moe_linear(x, w, n, g, H.GateAct(0, 0.0, 0.0) if gated else None, gather=True, experts=experts, in_scale=g.weights, quarters=quarters)
+        outs.append(y[g.place[g.place >= 0].long()])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    with pytest.raises(H.MvHipError):
+        H.moe_linear(x, w, n, H.moe_group(ids, experts, 256), H.GateAct(0, 0.0, 0.0) if gated else None, gather=True, experts=experts, quarters=True)
+
+
+@pytest.mark.parametrize("tokens, top", [(129, 4), (160, 8), (231, 4), (320, 4)])
+@pytest.mark.parametrize("experts", [8, 32])
+def test_a_few_dozen_pairs_an_expert_sum_as_tiles_of_32(monkeypatch, tokens, top, experts):
+    """Up to 40 pairs an expert, whatever the tiles that they are worked on in."""
+    from minivllm_amd.layers import ExpertMLP
+
+    tokens = tokens * experts // 32
+    gen = torch.Generator(device=DEV).manual_seed(tokens)
+    with torch.device(DEV):
+        layer = ExpertMLP(512, experts, 0, top, 1, 1, 1.0, 384).to(torch.bfloat16)
+    for p in layer.parameters():
+        p.requires_grad_(False).copy_(torch.randn(p.shape, generator=gen, device=DEV) * 0.05)
+    layer.finish_weights()
+    h = torch.randn(tokens, 512, generator=gen, device=DEV).bfloat16()
+    assert tokens * top <= 40 * experts
+    out = lambda: (lambda y, place: y[place.long()])(*layer(h)[1][:2])
+    got = out()
+    monkeypatch.setattr(ExpertMLP, "tile_rows", lambda self, tokens: 32)
+    assert torch.equal(got, out())
