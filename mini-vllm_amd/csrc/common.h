@@ -90,9 +90,19 @@ __device__ __forceinline__ uint32_t pack_pair(float lo, float hi) {
   else
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, f16x2_t));
 }
-// (pairs: a conversion for both, where two single ones and their union are three instructions)
+// bf16 in pairs: a conversion for both, where two single ones and their union are three instructions.  f16 one by one: there the conversion joins the
+// product in front of it (v_fma_mixlo_f16), which is then rounded once instead of twice.
 template <typename Tag>
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
+  if constexpr (__is_same(Tag, f16_tag)) {
+    u32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t lo = elem<Tag>::st(f[2 * i]), hi = elem<Tag>::st(f[2 * i + 1]);
+      v[i] = lo | (hi << 16);
+    }
+    return v;
+  }
   return u32x4{pack_pair<Tag>(f[0], f[1]), pack_pair<Tag>(f[2], f[3]), pack_pair<Tag>(f[4], f[5]), pack_pair<Tag>(f[6], f[7])};
 }
 
