@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/mvhip.h"
 
 #define MV_WAVE 64
@@ -139,6 +141,29 @@ __device__ __forceinline__ void swap16(float x, float &a, float &b) {
 __device__ __forceinline__ void swap32(float x, float &a, float &b) {
   a = x, b = x;
   asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+// Sum over groups of LANES adjacent lanes in the order of a butterfly of 1, 2, 4 .. lanes, without the LDS pipe (behind an exchange of 2 lanes four adjacent
+// ones are alike, so that the mirror of eight is an exchange of 4; likewise 8); every lane gets its group's.
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float x) {
+  auto other = [](float v, auto CTRL) {
+    return u2f((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f2u(v), decltype(CTRL)::value, 0xf, 0xf, false));
+  };
+  if constexpr (LANES >= 2) x += other(x, std::integral_constant<int, 0xB1>{});    // quad_perm 1 0 3 2
+  if constexpr (LANES >= 4) x += other(x, std::integral_constant<int, 0x4E>{});    // quad_perm 2 3 0 1
+  if constexpr (LANES >= 8) x += other(x, std::integral_constant<int, 0x141>{});   // row_half_mirror
+  if constexpr (LANES >= 16) x += other(x, std::integral_constant<int, 0x140>{});  // row_mirror
+  if constexpr (LANES >= 32) {
+    float a, b;
+    swap16(x, a, b);
+    x = a + b;
+  }
+  if constexpr (LANES >= 64) {
+    float a, b;
+    swap32(x, a, b);
+    x = a + b;
+  }
+  return x;
 }
 // Full 64-lane reductions (every lane gets the result).
 __device__ __forceinline__ float wave_sum(float x) {

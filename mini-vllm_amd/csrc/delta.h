@@ -3,10 +3,9 @@
 #include "ssm.h"
 
 __device__ __forceinline__ float sigmoid_f32(float z) { return 1.0f / (1.0f + expf(-z)); }
-// what norm and gate of a head's outputs make of one of them, in 16 bits: hardware root, exponential and reciprocal (1 ulp of fp32 each)
-__device__ __forceinline__ float head_rms_16(float squares, float share, float eps, float out_scale) {
-  return out_scale * __builtin_amdgcn_rsqf(fmaf(squares, share, eps));
-}
+// what norm and gate of a head's outputs make of one of them: its root and division as in mv_delta_step; in 16 bits the gate by hardware exponential and
+// reciprocal (1 ulp of fp32 each)
+__device__ __forceinline__ float head_rms(float squares, int channels, float eps, float out_scale) { return out_scale / sqrtf(squares / (float)channels + eps); }
 __device__ __forceinline__ float gate_16(float z, int kind) {
   return (kind == MV_GATE_SIGMOID ? 1.f : z) * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
 }

@@ -225,8 +225,8 @@ __global__ void __launch_bounds__(THREADS) delta_step_kernel(MvDeltaArgs p) {
 
 // ---- rms over each head of y, a weight shared by the heads, act(gate): LPT lanes per (token, head), PER vectors per lane, ITEMS of them
 // one behind the other.  Bound by vector arithmetic beside memory: a workgroup's inputs are asked for at once, only its first item's row comes from a
-// division, sums stay out of the LDS pipe, and 16-bit rows take the hardware's reciprocal root (1 ulp).  18 250 tokens, 16 heads of 128: 45.5 us
-// (4.9 TB/s) -> 39.2 (5.7; an addition of the same rows 38.3).
+// division, and sums stay out of the LDS pipe.  18 250 tokens, 16 heads of 128: 45.5 us (4.9 TB/s) -> 41.0 (5.5; an addition of the same rows 38.2; with
+// the hardware's reciprocal root, 1 ulp, in place of root and division 39.2).
 template <typename Tag, int LPT, int PER, int ITEMS>
 __global__ void __launch_bounds__(256) head_norm_gate_kernel(const typename elem<Tag>::T *y, int64_t y_stride,
                                                              const typename elem<Tag>::T *z, int64_t z_stride,
@@ -270,7 +270,6 @@ __global__ void __launch_bounds__(256) head_norm_gate_kernel(const typename elem
     ws[i] = u32x4{0u, 0u, 0u, 0u};
     if (c < p) ws[i] = *(const u32x4 *)(w + c);
   }
-  const float share = 1.0f / (float)p_true;
   auto values = [](const u32x4 &raw, float (&f)[VEC]) {
     if constexpr (VEC == 8) {
       unpack8<Tag>(raw, f);
@@ -293,17 +292,7 @@ __global__ void __launch_bounds__(256) head_norm_gate_kernel(const typename elem
         ss = fmaf(f[i][j], f[i][j], ss);
       }
     }
-    if constexpr (LPT >= 16) {   // (within a row of 16 lanes on the vector unit)
-      ss = row16_sum(ss);
-#pragma unroll
-      for (int off = 16; off < LPT; off <<= 1) ss += __shfl_xor(ss, off, 64);
-    } else {
-#pragma unroll
-      for (int off = 1; off < LPT; off <<= 1) ss += __shfl_xor(ss, off, 64);
-    }
-    float rs;
-    if constexpr (__is_same(Tag, f32_tag)) rs = out_scale / sqrtf(ss / (float)p_true + eps);
-    else rs = head_rms_16(ss, share, eps, out_scale);
+    const float rs = head_rms(lanes_sum<LPT>(ss), p_true, eps, out_scale);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int c = (sub + i * LPT) * VEC;
@@ -415,7 +404,7 @@ extern "C" int mv_head_norm_gate(const void *y, int64_t y_stride, const void *ga
   const int vec = dtype == MV_F32 ? 4 : 8;
   const int64_t items = (int64_t)rows * heads;
   const int vecs = p / vec;
-  // four items a thread where that leaves four workgroups a CU (19 000 x 16 heads of 128: one item 44.6 us, four 39.2)
+  // four items a thread where that leaves four workgroups a CU (19 000 x 16 heads of 128, with the hardware's reciprocal root: one item 44.6 us, four 39.2)
   const int lpt = vecs <= 4 ? 4 : vecs <= 8 ? 8 : vecs <= 16 ? 16 : vecs <= 32 ? 32 : 64;
   const bool many = vecs <= 64 && items * lpt / 256 >= 4096;
 #define MV_HNI(LPT, PER, ITEMS)                                                                                                   \

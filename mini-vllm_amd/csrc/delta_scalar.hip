@@ -159,11 +159,6 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
   }
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_to(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
-}
-
 // Workgroup = W waves = W tiles of 16 columns of one head of one sequence; a wave keeps S of its columns in accumulators, whose rows are
 // dealt so that tiles 2 s and 2 s + 1 together hold n = 32 s + 8 g .. + 7 in lane group g: operands of the next product as they are.  o is
 // computed transposed (columns by tokens), so that a lane holds four columns of a token; the rows of v land in LDS like those of k and q and are
@@ -240,7 +235,6 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
   // of them, and stores them.
   u32x4 done[2], gate[2] = {}, norm_w[2];   // (gate: of the chunk's rows, on their way with it)
   const bool padded = p.p_true < W * 16;
-  const float share = NORM ? 1.0f / (float)p.p_true : 0.f;
   auto col_of = [&](int i) { return ((lane % VP) ^ v_swizzle((2 * wave + i) * VR + lane / VP)) * 8; };   // (the head's first column is the workgroup's)
   if constexpr (NORM) {
 #pragma unroll
@@ -260,13 +254,7 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
       if (padded && col_of(i) + j >= p.p_true) f[j] = 0.f;
       ss = fmaf(f[j], f[j], ss);
     }
-    if constexpr (VP == 16) {
-      ss = row16_sum(ss);
-    } else {
-      static_assert(VP == 16 || VP == 8, "lanes of a row");
-      ss += dpp_to<0xB1>(ss), ss += dpp_to<0x4E>(ss), ss += dpp_to<0x141>(ss);   // lanes ^ 1, ^ 2, the other four of eight
-    }
-    const float rs = head_rms_16(ss, share, p.eps, p.out_scale);
+    const float rs = head_rms(lanes_sum<VP>(ss), p.p_true, p.eps, p.out_scale);
 #pragma unroll
     for (int j = 0; j < 8; ++j) f[j] = f[j] * rs * w[j] * gate_16(z[j], p.gate_kind);
     done[i] = pack8<B16>(f);
