@@ -373,10 +373,11 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, NK < 5 ? 4 : 2) delta_prep
 __device__ __forceinline__ void lds_landed(u32x4 &a) { asm volatile("" : "+v"(a)); }
 __device__ __forceinline__ void lds_landed(u32x4 &a, u32x4 &b) { asm volatile("" : "+v"(a), "+v"(b)); }
 
-// segments of `len` tokens: what they add to the state ahead of them [slot][heads][n * p], what becomes of that state [slot][heads] (n x n as
-// operands), the states that sequences of several segments come with [sequence][heads][n * p]; a sequence's slots start at cu_q / len + its number
+// segments of `len` tokens: what they add to the state ahead of them [slot][heads][n * p], what becomes of that state: a product whose diagonal
+// stays fp32 [slot][heads][n], the rest [slot][heads] (n x n as operands); the states that sequences of several segments come with [sequence][heads][n * p]; a sequence's slots
+// start at cu_q / len + its number
 struct Segments {
-  float *added, *first;
+  float *added, *first, *diagonal;
   char *carry;
   int len;
 };
@@ -504,6 +505,9 @@ __device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int
   if constexpr (MODE == SEGMENTS) {
     // .. of a later segment: that at the end of the first, and from segment to segment one product, whose left operand lands in LDS while
     // the one before is multiplied (where LDS holds two: up to 128 channels).  Read by each wave as it was used, a segment took 4.5 us.
+    // Within a segment the state crosses chunks in fp32 (S *= decay), and so that no more is lost from segment to segment, M's diagonal stays in fp32 and
+    // the product of the rests is not left out: the kept states are as far from 64 bits as those of whole sequences (0.999 of it over 60 shapes, lengths
+    // and decays; with all of M in two bf16 numbers and three products up to 1.10, where nothing decays).  That costs 1.5 of 248 us.
     constexpr int CF = 4 * NK * NK, BUFFERS = 2 * CF <= F1 + 8 * NK + BF + 1 ? 2 : 1;   // fragments
     const int ahead = from / sg.len, first = (int)blockIdx.z - ahead;
     auto fetch_carry = [&](int j) __attribute__((always_inline)) {
@@ -511,7 +515,7 @@ __device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int
 #pragma unroll
       for (int i = 0; i < NK * NK; ++i) fetch(of, i * 4 + wave, smem + ((j % BUFFERS) * CF + i * 4 + wave) * 1024);
     };
-    f32x4 next[CW][2 * NK];
+    f32x4 next[CW][2 * NK], diagonal[2 * NK];
     auto load_added = [&](int j) __attribute__((always_inline)) {
 #pragma unroll
       for (int w = 0; w < CW; ++w)
@@ -519,6 +523,9 @@ __device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int
         for (int i = 0; i < 2 * NK; ++i)
 #pragma unroll
           for (int e = 0; e < 4; ++e) next[w][i][e] = sg.added[(first + j) * size + in_head(w, i, e)];
+#pragma unroll
+      for (int i = 0; i < 2 * NK; ++i)
+        if (j > 0) diagonal[i] = *(const f32x4 *)(sg.diagonal + ((int64_t)(first + j) * p.heads + head) * p.n + state_row(i, 0));
     };
     if (ahead > 0) {
       if (ahead > 1) fetch_carry(1);
@@ -537,7 +544,9 @@ __device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int
 #pragma unroll
           for (int s = 0; s < NK; ++s) split44(st[w][2 * s], st[w][2 * s + 1], sh[w][s], sl[w][s]);
 #pragma unroll
-          for (int i = 0; i < 2 * NK; ++i) st[w][i] = next[w][i];
+          for (int i = 0; i < 2 * NK; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st[w][i][e] = fmaf(diagonal[i][e], st[w][i][e], next[w][i][e]);
         }
         if (j + 1 < ahead) {
           if constexpr (BUFFERS == 2) fetch_carry(j + 1);
@@ -560,13 +569,13 @@ __device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int
 #pragma unroll
           for (int w = 0; w < CW; ++w) half[w] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int part = 0; part < 3; ++part)
+          for (int part = 0; part < 4; ++part)
 #pragma unroll
             for (int s = 0; s < NK; ++s)
 #pragma unroll
               for (int w = 0; w < CW; ++w) {
                 f32x4 &to = (part * NK + s) & 1 ? half[w] : st[w][i];
-                to = mfma16x16x32<B16>(f[i & 1][s][part == 2], part == 1 ? sl[w][s] : sh[w][s], to);
+                to = mfma16x16x32<B16>(f[i & 1][s][part >= 2], part & 1 ? sl[w][s] : sh[w][s], to);
               }
 #pragma unroll
           for (int w = 0; w < CW; ++w) st[w][i] += half[w];
@@ -747,7 +756,11 @@ __device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int
 #pragma unroll
       for (int i = 0; i < 2 * NK; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) cs[state_row(i, e) * CS + (wave * CW + w) * 16 + r16] = st[w][i][e];
+        for (int e = 0; e < 4; ++e) {
+          const bool diagonal = live[w] && state_row(i, e) == col[w];
+          if (diagonal) sg.diagonal[((int64_t)blockIdx.z * p.heads + head) * p.n + col[w]] = st[w][i][e];
+          cs[state_row(i, e) * CS + (wave * CW + w) * 16 + r16] = diagonal ? 0.f : st[w][i][e];
+        }
     __syncthreads();
     char *carry = sg.carry + ((int64_t)blockIdx.z * p.heads + head) * (4 * NK * NK * 1024) + lane * 16;
     for (int f = wave; f < 2 * NK * 2 * CW; f += 4) {
@@ -795,6 +808,7 @@ inline int64_t segment_slots(int n_seqs, int total_q, int seg) { return (int64_t
 //   128 x 128: 4 x 1, 8 chunks 54 and 53, 12: 68 and 58, 24: 115 and 76, 63: 249 and 97; 8 x 3 (the later ones shorter), 24: 122 and 90, 63: 317 and 199;
 //   16 x 3, 12: 82 and 85, 24: 155 and 153, 63: 411 and 382.    64 x 64: 16 x 1, 12: 50 and 42, 63: 177 and 84; 16 x 3, 24: 95 and 77.
 //   32 x 128: 4 x 10 of 2148 tokens at most 106 and 112.   160 x 128: 8 x 1, 24: 136 and 93; 16 x 3, 24: 219 and 219.   128 x 256: 16 x 1, 24: 123 and 103; 16 x 3, 63: 433 and 524.
+// A sequence's segments, and so the last bits of its results, depend on the call's other sequences; a whole sequence has the same bits in any call.
 inline int pick_segment(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
   const int tiles = p / 16, workgroups = std::max((tiles + 3) / 4, (tiles + 7) / 8 + (n / 16 + 7) / 8) * heads;   // (of either launch)
   const int64_t longest = ((int64_t)max_q + L - 1) / L, chunks = ((int64_t)total_q + L - 1) / L;
@@ -820,7 +834,7 @@ int launch(const DeltaPrep &q, int seg, hipStream_t stream) {
     sg.len = seg * L;
     const int64_t slots = segment_slots(a.n_seqs, a.total_q, seg), state = (int64_t)a.heads * a.n * a.p;
     sg.added = (float *)(q.ws + mv_delta_chunk_workspace(a.n_seqs, a.total_q, a.heads, a.p, a.n));
-    sg.first = sg.added + slots * state, sg.carry = (char *)(sg.first + a.n_seqs * state);
+    sg.first = sg.added + slots * state, sg.diagonal = sg.first + a.n_seqs * state, sg.carry = (char *)(sg.diagonal + slots * a.heads * a.n);
     const int carried = (2 * NK + 7) / 8, by_rows = 32 * NK * (64 * 2 + 4) * 4;
     const int need = std::max((16 * NK + 32 + 1) * 1024, by_rows);
     if (int rc = mv_allow_lds<delta_segments_kernel<Tag, NK, 2>>()) return rc;
@@ -860,7 +874,7 @@ size_t mv_delta_segments_workspace(int n_seqs, int total_q, int max_q, int heads
   if (!seg) return 0;
   const int64_t slots = segment_slots(n_seqs, total_q, seg);
   if (slots > 65535) return 0;
-  return ((slots + n_seqs) * p + slots * n) * (size_t)heads * n * 4;
+  return ((slots + n_seqs) * p + slots + slots * n) * (size_t)heads * n * 4;
 }
 
 int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, bool *normed, hipStream_t stream) {

@@ -95,3 +95,70 @@ def test_less_scratch_is_whole_sequences(H, monkeypatch):
             m.setattr(H._lib, "mv_delta_prefill_segments_bytes", lambda *a: need - 1 if less else 0)
             outs.append(H.delta_prefill(*args, torch.zeros(2, 1, 2, 64, 64, device=DEV), cu[:1], cu, cu, t))
     assert torch.equal(*outs)
+
+
+def _call(H, s, ins, spans, state):
+    """ins: the rows of all sequences -> their outputs and the states left (sequence i at slot i)."""
+    cu = lambda v: torch.tensor([0, *torch.tensor(v).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    x, beta, a, bias, a_log = ins
+    left, slots = state.clone(), torch.arange(len(spans), dtype=torch.int32, device=DEV)
+    out = H.delta_prefill(s, x, beta, a, bias, a_log, left, slots, cu([t for t, _ in spans]), cu([t + b for t, b in spans]), max(t for t, _ in spans))
+    return out.double(), [left[(t + b) & 1, i].double() for i, (t, b) in enumerate(spans)]
+
+
+def _inputs(H, seed, tokens, heads, p, n, speed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    s = H.DeltaShape(heads, heads, p, n, heads * p, heads * (p + n), p, n ** -0.5, True)
+    bias = torch.full((heads * n,), speed, device=DEV).bfloat16() if speed is not None else rand(heads * n) - 4
+    return s, (rand(tokens, s.channels), rand(tokens, heads + 8)[:, :heads], rand(tokens, heads * n), bias, rand(heads)), rand
+
+
+# nothing decays: what a segment makes of the state ahead of it is then all but the state itself; segments of two chunks and more
+@pytest.mark.parametrize("tokens", [700, 1500])
+@pytest.mark.parametrize("heads, p, n", [(4, 128, 128), (2, 144, 160), (3, 48, 96)])
+@pytest.mark.parametrize("speed", [-20.0, None])
+def test_segments_keep_the_state_as_exactly_as_whole_sequences(H, monkeypatch, tokens, heads, p, n, speed):
+    """The kept state against the recurrence in 64 bits."""
+    ratios = []
+    for seed in range(4):
+        s, ins, rand = _inputs(H, seed, tokens, heads, p, n, speed)
+        x, beta, a, bias, a_log = (t.double() for t in ins)
+        state = rand(2, 1, heads, n, p).float() * 0.3
+        v, k, q = (t.unflatten(1, (heads, -1)) for t in x.split([heads * p, heads * n, heads * n], 1))
+        k = k / (k.square().sum(-1, keepdim=True) + 1e-6).sqrt()
+        decay = (-a_log.exp()[:, None] * torch.nn.functional.softplus((a + bias).unflatten(1, (heads, n)), threshold=60.0)).exp()
+        want = state[1, 0].double()
+        for t in range(tokens):
+            want = want * decay[t][:, :, None]
+            u = beta[t].sigmoid()[:, None] * (v[t] - (k[t][:, None] @ want)[:, 0])
+            want = want + k[t][:, :, None] * u[:, None]
+        got = _call(H, s, ins, [(tokens, 1)], state)[1][0]
+        with monkeypatch.context() as m:
+            m.setattr(H._lib, "mv_delta_prefill_segments_bytes", lambda *a: 0)
+            whole = _call(H, s, ins, [(tokens, 1)], state)[1][0]
+        assert not torch.equal(got, whole)
+        error, other = ((t - want).norm() / want.norm() for t in (got, whole))
+        # operands are sums of two bf16 numbers, 2^-17 of them off at most; a few such roundings of a state live at a time
+        assert error <= 2 ** -16
+        ratios.append(float(error / other))
+    # four draws scatter by 1 % around 1; with the diagonal in two bf16 numbers and the product of the rests left out 1.05 to 1.09 (700 tokens that do not decay)
+    assert sum(ratios) / len(ratios) <= 1.02, ratios
+
+
+def test_a_sequence_alone_and_among_others(H):
+    """Its segments depend on the others: the last bits may, the rest does not."""
+    lens, heads, p, n = [2500, 700, 1900, 130], 4, 128, 128
+    s, ins, rand = _inputs(H, 0, sum(lens), heads, p, n, None)
+    state = rand(2, len(lens), heads, n, p).float() * 0.3
+    out, states = _call(H, s, ins, [(t, 3) for t in lens], state)
+    at = 0
+    for i, t in enumerate(lens):
+        rows = [r[at:at + t] for r in ins[:3]] + list(ins[3:])
+        alone, kept = _call(H, s, rows, [(t, 3)], state[:, i:i + 1].contiguous())
+        got = out[at:at + t]
+        # (each 2^-17 of its operands off; results rounded once to 8 bits, which may fall either way)
+        assert (got - alone).norm() <= 2 ** -10 * alone.norm()
+        assert ((got - alone).abs() <= 2 ** -7 * alone.abs() + 2 ** -14 * alone.abs().max()).all()
+        assert (states[i] - kept[0]).norm() <= 2 ** -15 * kept[0].norm()
+        at += t
