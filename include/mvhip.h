@@ -733,7 +733,9 @@ typedef struct MvDeltaArgs {
  * where a workgroup has a head's columns */
 enum { MV_DELTA_SCAN = 1, MV_DELTA_NORM = 2 };
 size_t mv_delta_prefill_workspace_bytes(int n_seqs, int total_q, int heads, int p, int n, int dtype);
-/* scratch beyond that with which few long sequences are worked on in several places at once (0: none is of use) */
+/* scratch beyond that with which few long sequences are worked on in several places at once (0: none is of use, so always where the longest has
+ * at most MV_DELTA_WHOLE tokens) */
+enum { MV_DELTA_WHOLE = 512 };
 size_t mv_delta_prefill_segments_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int channel_decay, int dtype);
 int mv_delta_prefill(const MvDeltaArgs *args, int dtype, int flags, void *stream);
 /* one token per sequence, from projected channels: convolution, recurrence and mv_head_norm_gate in one launch; writes both states */

@@ -869,7 +869,7 @@ size_t mv_delta_chunk_workspace(int n_seqs, int total_q, int heads, int p, int n
 
 // (behind the above)
 size_t mv_delta_segments_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
-  if (!mv_delta_chunk_workspace(n_seqs, total_q, heads, p, n)) return 0;
+  if (max_q <= MV_DELTA_WHOLE || !mv_delta_chunk_workspace(n_seqs, total_q, heads, p, n)) return 0;
   const int seg = pick_segment(n_seqs, total_q, max_q, heads, p, n);
   if (!seg) return 0;
   const int64_t slots = segment_slots(n_seqs, total_q, seg);

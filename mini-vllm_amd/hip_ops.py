@@ -1495,7 +1495,7 @@ def gated_group_norm(y, z, w, heads: int, p: int, p_true: int, groups: int, eps:
 
 
 # ---------------------------------------------------------------- K16
-MV_DELTA_SCAN, MV_DELTA_NORM = 1, 2
+MV_DELTA_SCAN, MV_DELTA_NORM, MV_DELTA_WHOLE = 1, 2, 512
 GATES = {"silu": 0, "sigmoid": 1}
 
 
@@ -1556,7 +1556,7 @@ def delta_prefill(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots,
     g = _delta_args(s, x, beta, a, dt_bias, a_log, state, state_slots, out)
     g.cu_q, g.cu_k, g.max_q = cu_q.data_ptr(), cu_k.data_ptr(), int(max_q)
     n = 0 if flags & MV_DELTA_SCAN else int(_lib.mv_delta_prefill_workspace_bytes(g.n_seqs, g.total_q, s.heads, s.p, s.n, _dt(x)))
-    if n:
+    if n and g.max_q > MV_DELTA_WHOLE:      # (0 otherwise: a call less)
         n += int(_lib.mv_delta_prefill_segments_bytes(g.n_seqs, g.total_q, g.max_q, s.heads, s.p, s.n, g.channel_decay, _dt(x)))
     ws = torch.empty((n,), dtype=torch.uint8, device=x.device) if n else None
     g.workspace, g.ws_bytes = _ptr(ws), n
