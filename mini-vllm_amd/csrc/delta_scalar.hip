@@ -27,7 +27,7 @@ template <int NK, int HEADS>
 __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(DeltaPrep q) {
   typedef uint16_t T;
   typedef elem<B16>::T E;
-  constexpr int N = NK * 32, KS = N + 8, W = 4 * HEADS, PARTS = W;   // LDS row stride; threads a token
+  constexpr int N = NK * 32, KS = N + 8, W = 4 * HEADS;   // LDS row stride
   const MvDeltaArgs &p = q.a;
   constexpr int QB = L * KS * 2 > L * TS * 4 ? L * KS * 2 : L * TS * 4, KB = HEADS > 1 ? QB : L * KS * 2;
   __shared__ __attribute__((aligned(16))) char smem[KB + QB + (2 + 2 * HEADS) * L * 4];
@@ -43,16 +43,16 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
   const T *x = (const T *)p.x + (int64_t)(q0 + t0) * p.x_stride;
   float *ts = (float *)(of ? (char *)ks : (char *)qs), *bt = bts + of * L, *rs = rss + of * L;
 
-  // ---- k, q (tokens behind the end: zeros) and their lengths: PARTS threads a token; a head's first wave its betas and log2 decays, a lane a token
+  // ---- k, q (tokens behind the end: zeros) and their lengths, four threads a token: both, or with two heads k by one half, q by the other (a length is
+  // the same sum in either form); a head's first wave its betas and log2 decays, a lane a token
   {
-    const int t = tid / PARTS, part = tid % PARTS;
-    const T *row = x + (int64_t)min(t, nt - 1) * p.x_stride + grp * N;
-    constexpr int PIECES = N / 8, PER = (PIECES + PARTS - 1) / PARTS;
-    u32x4 a[PER], b[PER];
+    const int t = (tid & 255) >> 2, part = tid & 3;
+    const T *row = x + (int64_t)min(t, nt - 1) * p.x_stride + grp * N + part * 8;
+    u32x4 a[NK], b[HEADS > 1 ? 1 : NK];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c = min(part + PARTS * i, PIECES - 1) * 8;
-      a[i] = *(const u32x4 *)(row + p.k_off + c), b[i] = *(const u32x4 *)(row + p.q_off + c);
+    for (int i = 0; i < NK; ++i) {
+      a[i] = *(const u32x4 *)(row + (of ? p.q_off : p.k_off) + 32 * i);
+      if constexpr (HEADS == 1) b[i] = *(const u32x4 *)(row + p.q_off + 32 * i);
     }
     const bool leads = (wave & 3) == 0;
     float beta = 0.f, decay = 0.f, bias = 0.f, rate = 0.f;
@@ -61,23 +61,25 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
       beta = elem<B16>::ld(((const E *)p.beta)[at * p.beta_stride + head]), decay = elem<B16>::ld(((const E *)p.a)[at * p.a_stride + head]);
       rate = elem<B16>::ld(((const E *)p.a_log)[head]), bias = elem<B16>::ld(((const E *)p.dt_bias)[head]);
     }
-    float sk = 0.f, sq = 0.f;
+    auto length = [&](u32x4 *raw, T *to, float scale) {
+      float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c = (part + PARTS * i) * 8;
-      if (PIECES % PARTS && c >= N) continue;
-      if (t >= nt) a[i] = b[i] = u32x4{0u, 0u, 0u, 0u};
-      float fa[8], fb[8];
-      unpack8<B16>(a[i], fa);
-      unpack8<B16>(b[i], fb);
+      for (int i = 0; i < NK; ++i) {
+        if (t >= nt) raw[i] = u32x4{0u, 0u, 0u, 0u};
+        float f[8];
+        unpack8<B16>(raw[i], f);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sk = fmaf(fa[j], fa[j], sk), sq = fmaf(fb[j], fb[j], sq);
-      *(u32x4 *)(ks + t * KS + c) = a[i];
-      *(u32x4 *)(qs + t * KS + c) = b[i];
+        for (int j = 0; j < 8; ++j) sum = fmaf(f[j], f[j], sum);
+        *(u32x4 *)(to + t * KS + part * 8 + 32 * i) = raw[i];
+      }
+      return scale / sqrtf(lanes_sum<4>(sum) + p.unit_eps);
+    };
+    const float first = length(a, of ? qs : ks, of ? p.q_scale : 1.f);
+    if (part == 0) (of ? fq : fk)[t] = first;
+    if constexpr (HEADS == 1) {
+      const float second = length(b, qs, p.q_scale);
+      if (part == 0) fq[t] = second;
     }
-#pragma unroll
-    for (int o = 1; o < PARTS; o <<= 1) sk += __shfl_xor(sk, o, 64), sq += __shfl_xor(sq, o, 64);
-    if (part == 0) fk[t] = 1.f / sqrtf(sk + p.unit_eps), fq[t] = p.q_scale / sqrtf(sq + p.unit_eps);
     if (leads) {
       rate = -expf(rate) * 1.4426950408889634f;
       float sum = lane < nt ? rate * softplus_fast(decay + bias) : 0.f;
