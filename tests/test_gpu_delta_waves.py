@@ -95,3 +95,23 @@ def test_many_sequences_with_channel_decay_are_as_each_alone(H, heads, p, n, dty
         begin += t
     scan, _ = run(0, len(spans), slice(0, total), flags=H.MV_DELTA_SCAN)   # (bounds as above)
     assert (out.double() - scan.double()).abs().max() <= 2**-6 * max(1.0, scan.double().abs().max().item())
+
+
+@pytest.mark.parametrize("n", [32, 64, 96, 128, 160])
+def test_heads_that_share_keys_are_as_those_with_their_own(H, n):
+    """Prepared two at a time, or one: the same bits."""
+    g = torch.Generator(device=DEV).manual_seed(n)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    heads, groups, p, lens = 8, 2, 48, [130, 64, 1, 63]
+    total, cu = sum(lens), torch.tensor([0, *torch.tensor(lens).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+    v, k, q = rand(total, heads * p), rand(total, groups, n), rand(total, groups, n)
+    beta, a, bias, a_log = rand(total, heads), rand(total, heads), rand(heads), rand(heads)
+    state = torch.randn(2, len(lens), heads, n, p, generator=g, device=DEV)
+    results = []
+    for times in (1, heads // groups):
+        many = groups * times
+        s = H.DeltaShape(heads, many, p, n, heads * p, heads * p + many * n, p, n ** -0.5, False)
+        x = torch.cat([v, *(t.repeat_interleave(times, 1).flatten(1) for t in (k, q))], 1)
+        left = state.clone()
+        results.append((H.delta_prefill(s, x, beta, a, bias, a_log, left, torch.arange(len(lens), dtype=torch.int32, device=DEV), cu, cu, max(lens)), left))
+    assert all(torch.equal(*pair) for pair in zip(*results))
