@@ -730,8 +730,8 @@ typedef struct MvDeltaArgs {
 } MvDeltaArgs;
 /* out[t] = o, [T][heads * p], from convolved channels; writes state.  flags: MV_DELTA_SCAN = token by token; MV_DELTA_NORM = behind it mv_head_norm_gate with
  * the arguments' gate, norm_w, p_true, eps, gate_kind and out_scale, where rows of `out` are whole, aligned vectors of 16 bytes, in the same launches
- * where a workgroup has a head's columns */
-enum { MV_DELTA_SCAN = 1, MV_DELTA_NORM = 2 };
+ * where a workgroup has a head's columns and a rule on sizes says that this is the shorter way (MV_DELTA_NORM_WALK: whatever it says) */
+enum { MV_DELTA_SCAN = 1, MV_DELTA_NORM = 2, MV_DELTA_NORM_WALK = 4 };
 size_t mv_delta_prefill_workspace_bytes(int n_seqs, int total_q, int heads, int p, int n, int dtype);
 /* scratch beyond that with which few long sequences are worked on in several places at once (0: none is of use, so always where the longest has
  * at most MV_DELTA_WHOLE tokens) */

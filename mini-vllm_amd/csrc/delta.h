@@ -15,6 +15,6 @@ __device__ __forceinline__ float decay_log(float rate, float a, float bias) { re
 // chunked form (16-bit); MV_E_SHAPE when it does not apply
 size_t mv_delta_chunk_workspace(int n_seqs, int total_q, int heads, int p, int n);
 size_t mv_delta_segments_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n);   // beside it, where sequences are cut
-// `normed` (NULL: not asked for): set where norm and gate are already in the output
+// `normed` (NULL: not asked for): in: norm and gate in the walk whatever the rule on sizes says; out: they are already in the output
 int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, bool *normed, hipStream_t stream);
 int mv_delta_scalar_launch(const MvDeltaArgs &a, bool *normed, hipStream_t stream);   // (from the above: bf16, one decay per head)

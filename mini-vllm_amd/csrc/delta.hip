@@ -365,7 +365,7 @@ extern "C" int mv_delta_prefill(const MvDeltaArgs *a, int dtype, int flags, void
                                                               a->heads, a->p, a->p_true, a->eps, a->gate_kind, a->out_scale, dtype, stream);
   };
   if (dtype != MV_F32 && !(flags & MV_DELTA_SCAN)) {
-    bool normed = false;
+    bool normed = flags & MV_DELTA_NORM_WALK;
     const int rc = mv_delta_chunk_launch(*a, dtype, norm ? &normed : nullptr, (hipStream_t)stream);
     if (rc != MV_E_SHAPE) return behind(rc, normed);
   }

@@ -885,6 +885,7 @@ int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, bool *normed, hipStre
   if (a.channel_decay && (!mv_aligned16(a.a) || (a.a_stride & 7) || !mv_aligned16(a.dt_bias))) return MV_E_ALIGN;
   const DeltaPrep q{a, (char *)a.workspace};
   if (!a.channel_decay && dtype == MV_BF16) return mv_delta_scalar_launch(a, normed, stream);
+  if (normed) *normed = false;
   const size_t more = mv_delta_segments_workspace(a.n_seqs, a.total_q, a.max_q, a.heads, a.p, a.n);
   const int seg = more && (size_t)a.ws_bytes >= need + more ? pick_segment(a.n_seqs, a.total_q, a.max_q, a.heads, a.p, a.n) : 0;
 #define MV_DN(NK_) \

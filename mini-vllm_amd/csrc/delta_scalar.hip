@@ -487,10 +487,11 @@ int launch_walk(const DeltaPrep &q, int slices, int lds, bool *normed, hipStream
   // Norm and gate in the walk lengthen the chain of the longest sequence, by 1.1 us a chunk with eight waves (16 sequences of up to 1490 tokens, 16 heads of 128:
   // 26 us) and 0.47 with four (3 of up to 1490, 16 heads of 64: 11); a launch behind it takes some 3.5 us and the time of its rows (43 and 7).
   const double chunks = (q.a.max_q + L - 1) / L, in_chain = chunks * (W == 8 ? 1.1 : 0.47), behind = 3.5 + (double)q.a.total_q * q.a.heads * q.a.p * 6 / 5.7e6;
-  if (normed && slices == 1 && in_chain <= behind) {
+  const bool in_walk = normed && slices == 1 && (*normed || in_chain <= behind);
+  if (normed) *normed = in_walk;
+  if (in_walk) {
     if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, W, true>>()) return rc;
     hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, W, true>), grid, block, lds, stream, q);
-    *normed = true;
   } else {
     if (int rc = mv_allow_lds<delta_scalar_walk_kernel<NK, W, false>>()) return rc;
     hipLaunchKernelGGL((delta_scalar_walk_kernel<NK, W, false>), grid, block, lds, stream, q);

@@ -1495,7 +1495,7 @@ def gated_group_norm(y, z, w, heads: int, p: int, p_true: int, groups: int, eps:
 
 
 # ---------------------------------------------------------------- K16
-MV_DELTA_SCAN, MV_DELTA_NORM, MV_DELTA_WHOLE = 1, 2, 512
+MV_DELTA_SCAN, MV_DELTA_NORM, MV_DELTA_NORM_WALK, MV_DELTA_WHOLE = 1, 2, 4, 512
 GATES = {"silu": 0, "sigmoid": 1}
 
 
