@@ -687,13 +687,12 @@ int launch_linear(const MoeLinear &p, int tile_m, int max_tiles, hipStream_t st)
   tile_m &= ~MV_MOE_QUARTERS;
   if (tile_m == 16) hipLaunchKernelGGL((moe_small_kernel<Tag, 1, TN, GATED>), small, dim3(256), 0, st, p);
   else if (tile_m == 32) hipLaunchKernelGGL((moe_small_kernel<Tag, 2, TN, GATED>), small, dim3(256), 0, st, p);
-  else if (tile_m == 64 || (tile_m == 128 && !quarters)) {
+  else if (tile_m == 64) {
     constexpr int BN = 128;
     const dim3 grid((nt * 16 * (GATED ? 2 : 1) + BN - 1) / BN, max_tiles);
-    if (tile_m == 128) hipLaunchKernelGGL((moe_tile_kernel<Tag, 128, BN, GATED, false>), grid, dim3(256), (128 + BN) * 256, st, p);
-    else if (quarters) hipLaunchKernelGGL((moe_tile_kernel<Tag, 64, BN, GATED, true>), grid, dim3(256), (64 + BN) * 256, st, p);
+    if (quarters) hipLaunchKernelGGL((moe_tile_kernel<Tag, 64, BN, GATED, true>), grid, dim3(256), (64 + BN) * 256, st, p);
     else hipLaunchKernelGGL((moe_tile_kernel<Tag, 64, BN, GATED, false>), grid, dim3(256), (64 + BN) * 256, st, p);
-  } else if (tile_m == 256 && !quarters) {
+  } else if ((tile_m == 128 || tile_m == 256) && !quarters) {   // (tiles of 128 rows have one half)
     const int nx = (nt * (GATED ? 2 : 1) + 15) / 16;
     if (int rc = mv_allow_lds<moe_wide_kernel<Tag, GATED>>()) return rc;
     hipLaunchKernelGGL((moe_wide_kernel<Tag, GATED>), dim3((unsigned)(((int64_t)max_tiles * 2 * nx + 7) / 8 * 8)), dim3(256),

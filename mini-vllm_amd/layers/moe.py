@@ -26,7 +26,7 @@ __all__ = ["ExpertMLP"]
 #   256 rows (two workgroups of 128 x 256 to a CU) against 64: ahead as soon as their workgroups fill five eighths of the chip: 32 of 2048 -> 768 (192 workgroups)
 #   24 pairs 65 / 64, 64 84 / 68, 256 176 / 128; of 1024 -> 384 64 pairs (96) 30 / 33, 160 (192) 51 / 37; 8 of 2048 -> 768 256 (96) 46 / 52, 384 (144) 59 / 55, 800
 #   103 / 83; 2 of 2048 -> 768 1100 (108) 46 / 56, 2500 (240) 88 / 70; the worst found: 2 of 4096 -> 1024, 1500 pairs (192) 102 / 111.
-#   128 rows (tiles of the 64's kind) are nowhere ahead of both.
+#   128 rows: the 256's kernel, a tile a workgroup (tiles of the 64's kind, which they were, are nowhere ahead of both).
 # Up to QUARTERS pairs per expert, tiles of 64 rows sum as those of 16 and 32 do: a call's bits are those of tiles of 32 rows, which it once had.
 # That costs nothing in them, but 256 rows, which have no such sums, would be ahead in the end: 32 experts of 2048 -> 768, 24 pairs 68 / 65, 40 74 / 66 (32 rows 78, 130).
 FEW, MANY_EXPERTS, WIDE_GROUPS, QUARTERS = 8, 32, 160, 40
