@@ -23,13 +23,15 @@ __all__ = ["ExpertMLP"]
 # Rows of the tiles that a launch works on, by the pairs per expert.  Both products, us, tiles of 16 / 32 / 64 / 256 rows:
 #   few pairs: the next tile is ahead from 10 (32 experts of 2048 -> 768: 8 62 / 58, 12 67 / 62; 8 experts 24 / 22, 26 / 24) and, for the 64 rows' longer runs
 #   of a weight, from 16 where experts are many (32: 16 67 / 62, 24 82 / 65; 128: 245 / 236, 297 / 241), from 28 else (8: 16 26 / 37, 28 38 / 37).
-#   256 rows (two workgroups of 128 x 256 to a CU) against 64: ahead as soon as their workgroups fill five eighths of the chip: 32 of 2048 -> 768 (192 workgroups)
-#   24 pairs 65 / 64, 64 84 / 68, 256 176 / 128; of 1024 -> 384 64 pairs (96) 30 / 33, 160 (192) 51 / 37; 8 of 2048 -> 768 256 (96) 46 / 52, 384 (144) 59 / 55, 800
-#   103 / 83; 2 of 2048 -> 768 1100 (108) 46 / 56, 2500 (240) 88 / 70; the worst found: 2 of 4096 -> 1024, 1500 pairs (192) 102 / 111.
+#   256 rows (two workgroups of 128 x 256 to a CU) against 64: ahead where the workgroups of both products fill the chip in part, half of it the gated one's, 80 CUs the
+#   other's, which is the longer one where the experts are wide.  Workgroups of the two, pairs: 32 of 2048 -> 768 (192, 256) 64 pairs 100 / 66, 32 of 1024 -> 384 (96, 128)
+#   64 30 / 33, (192, 256) 160 51 / 37; 4 of 2048 -> 768 (144, 192) 768 61 / 53; 8 of 768 -> 3072 (192, 24) 64 51 / 62, (768, 96) 500 110 / 98; 16 of 1024 -> 2816 (352, 64) 44
+#   77 / 83; 2 of 4096 -> 1024 (192, 384) 1500 102 / 94; 1 of 1024 -> 2816 (440, 80) 2500 82 / 76.  Over 500 shapes (1 .. 128 experts, 44 .. 2500 pairs) 0.3 % behind the better
+#   of the two in the mean, 17 % at worst; without the second line eleven took up to 1.2 times as long as by the 64 or 128 rows that they once had.
 #   128 rows: the 256's kernel, a tile a workgroup (tiles of the 64's kind, which they were, are nowhere ahead of both).
 # Up to QUARTERS pairs per expert, tiles of 64 rows sum as those of 16 and 32 do: a call's bits are those of tiles of 32 rows, which it once had.
 # That costs nothing in them, but 256 rows, which have no such sums, would be ahead in the end: 32 experts of 2048 -> 768, 24 pairs 68 / 65, 40 74 / 66 (32 rows 78, 130).
-FEW, MANY_EXPERTS, WIDE_GROUPS, QUARTERS = 8, 32, 160, 40
+FEW, MANY_EXPERTS, WIDE_GROUPS, QUARTERS = 8, 32, (128, 80), 40
 
 
 class ExpertMLP(nn.Module):
@@ -84,8 +86,9 @@ class ExpertMLP(nn.Module):
             return 16 if per <= FEW else 32
         if per <= QUARTERS:
             return 64
-        wide = self.experts * math.ceil(per / 128) * math.ceil(2 * self.f / 256)      # workgroups of the gated product
-        return 256 if wide >= WIDE_GROUPS else 64
+        rows = self.experts * math.ceil(per / 128)        # workgroups of the two products
+        wide = rows * math.ceil(2 * self.f / 256) >= WIDE_GROUPS[0] and rows * math.ceil(self.w / 256) >= WIDE_GROUPS[1]
+        return 256 if wide else 64
 
     def route(self, h):
         """-> (weights [T, top], the pairs sorted by expert)."""
