@@ -21,8 +21,10 @@ from .linear import Segment, SegmentedLinear, gated_linear, pad_to
 __all__ = ["ExpertMLP"]
 
 # Rows of the tiles that a launch works on, by the pairs per expert.  Both products, us, tiles of 16 / 32 / 64 / 256 rows:
-#   few pairs: the next tile is ahead from 10 (32 experts of 2048 -> 768: 8 62 / 58, 12 67 / 62; 8 experts 24 / 22, 26 / 24) and, for the 64 rows' longer runs
-#   of a weight, from 16 where experts are many (32: 16 67 / 62, 24 82 / 65; 128: 245 / 236, 297 / 241), from 28 else (8: 16 26 / 37, 28 38 / 37).
+#   few pairs: 32 rows are ahead of 16 from 10 (32 experts of 2048 -> 768: 8 62 / 58, 12 67 / 62; 8 experts 24 / 22, 26 / 24).  64 rows against 32, for their longer
+#   runs of a weight: of 8 experts from 28 (2048 -> 768: 24 32 / 34, 29 37 / 34; 4096 -> 1536 24 78 / 85, 29 98 / 86), of fewer not up to 40 (2 of 4096 -> 1024, 34 pairs
+#   29 / 51), of 32 and more from 24 (4096 -> 1536: 17 226 / 263, 24 261 / 264, 28 314 / 269), but from 16 where their workgroups are no more than two a CU (32 of 2048 ->
+#   768: 17 70 / 62, 24 80 / 63; 64 of 1024 -> 384 17 39 / 34) or the second product is the long one (32 of 768 -> 3072: 17 116 / 110; 128 408 / 363).
 #   256 rows (two workgroups of 128 x 256 to a CU) against 64: ahead where the workgroups of both products fill the chip in part, half of it the gated one's, 80 CUs the
 #   other's, which is the longer one where the experts are wide.  Workgroups of the two, pairs: 32 of 2048 -> 768 (192, 256) 64 pairs 100 / 66, 32 of 1024 -> 384 (96, 128)
 #   64 30 / 33, (192, 256) 160 51 / 37; 4 of 2048 -> 768 (144, 192) 768 61 / 53; 8 of 768 -> 3072 (192, 24) 64 51 / 62, (768, 96) 500 110 / 98; 16 of 1024 -> 2816 (352, 64) 44
@@ -31,7 +33,7 @@ __all__ = ["ExpertMLP"]
 #   128 rows: the 256's kernel, a tile a workgroup (tiles of the 64's kind, which they were, are nowhere ahead of both).
 # Up to QUARTERS pairs per expert, tiles of 64 rows sum as those of 16 and 32 do: a call's bits are those of tiles of 32 rows, which it once had.
 # That costs nothing in them, but 256 rows, which have no such sums, would be ahead in the end: 32 experts of 2048 -> 768, 24 pairs 68 / 65, 40 74 / 66 (32 rows 78, 130).
-FEW, MANY_EXPERTS, WIDE_GROUPS, QUARTERS = 8, 32, (128, 80), 40
+FEW, WIDE_GROUPS, QUARTERS = 8, (128, 80), 40
 
 
 class ExpertMLP(nn.Module):
@@ -78,11 +80,18 @@ class ExpertMLP(nn.Module):
                 p.data = hip_ops.pack_weight(p.data.view(-1, p.shape[-1]))
             self.packed = True
 
+    def _rows32(self) -> int:
+        """Pairs per expert up to which tiles of 32 rows are ahead of 64."""
+        if self.experts < 32:
+            return 28 if self.experts >= 8 else 40
+        groups = self.experts * math.ceil(max(2 * self.f, self.w) / 128)      # workgroups of the 64's larger product
+        return 16 if groups <= 512 or self.f > self.w else 24
+
     def tile_rows(self, tokens: int) -> int:
         if self.router.dtype == torch.float32:
             return 16
         per = tokens * self.top / self.experts
-        if per <= (16 if self.experts >= MANY_EXPERTS else 28):
+        if per <= self._rows32():
             return 16 if per <= FEW else 32
         if per <= QUARTERS:
             return 64
