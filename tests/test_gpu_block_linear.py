@@ -45,8 +45,10 @@ def test_the_layer_takes_either_path():
         lin.requires_grad_(False)
         for name, (inputs, _, s) in lin.blocks.items():
             lin.weight_loader(lin.weight, torch.randn(s.units * s.unit, inputs, generator=g, device=DEV).bfloat16() * 0.1, name)
-        x = torch.randn(MID_M_MAX + 40, lin.input_size, generator=g, device=DEV).bfloat16()
+        many = 2 ** 20 // lin.weight.shape[0] + 1       # (two blocks of 128 inputs go by blocks from so many rows on)
+        x = torch.randn(many, lin.input_size, generator=g, device=DEV).bfloat16()
         want = x.float() @ lin.weight.float().T
-        for rows in (MID_M_MAX, MID_M_MAX + 1, MID_M_MAX + 40):
+        assert lin._by_blocks(many)
+        for rows in (MID_M_MAX, MID_M_MAX + 1, MID_M_MAX + 40, many):
             torch.testing.assert_close(lin(x[:rows]).float(), want[:rows], rtol=2 ** -8, atol=1e-5)
         assert (H.block_linear(x, lin.weight, lin._places) is None) == (lin.input_size == 192)
