@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
 // Where heads and sequences do not fill the chip, workgroups of four waves leave no CU idle.
 // NORM (the workgroup has all of a head's columns): the rows leave normed and gated.  A row of the head lies on 2 W adjacent lanes when it is stored, as in
 // head_norm_gate_kernel, whose rounding points and order of the sum these are; the gate's pieces come with the chunk.  Bound by the same
-// chain, of which this is vector arithmetic: the walk above 122 -> 148 us, where a launch behind it took 43 and a pass over o; the layer 271 -> 242.  Half of
+// chain, of which this is vector arithmetic: the walk above 140 -> 174 us under the profiler, where a launch behind it took 53 and a pass over o; the layer 271 -> 245.  Half of
 // the waves later than the others, so that one of two on a SIMD multiplies meanwhile: 267.
 template <int NK, int W, bool NORM>
 __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep q) {
@@ -484,9 +484,10 @@ __global__ void __launch_bounds__(W * 64, 1) delta_scalar_walk_kernel(DeltaPrep 
 template <int NK, int W>
 int launch_walk(const DeltaPrep &q, int slices, int lds, bool *normed, hipStream_t stream) {
   const dim3 grid(slices, q.a.heads, q.a.n_seqs), block(W * 64);
-  // Norm and gate in the walk lengthen the chain of the longest sequence, by 1.1 us a chunk with eight waves (16 sequences of up to 1490 tokens, 16 heads of 128:
-  // 26 us) and 0.47 with four (3 of up to 1490, 16 heads of 64: 11); a launch behind it takes some 3.5 us and the time of its rows (43 and 7).
-  const double chunks = (q.a.max_q + L - 1) / L, in_chain = chunks * (W == 8 ? 1.1 : 0.47), behind = 3.5 + (double)q.a.total_q * q.a.heads * q.a.p * 6 / 5.7e6;
+  // Norm and gate in the walk lengthen the chain of the longest sequence, by some 1.2 us a chunk with eight waves and 0.5 (64 key channels) to 0.7 with four; a launch
+  // behind it takes 2.5 us and the time of its rows, 4.6 TB/s.  us, in the walk and behind: 16 heads over 8 of 128 x 128, 40 sequences of up to 600 tokens 192 and 215; of 64 x 64,
+  // 16 of up to 1490 116 and 124, 3 of up to 600 44 and 41, 8 of up to 3000 168 and 162, over 16 191 and 206; 3 heads of 32 x 32, 40 of up to 600 45 and 42.
+  const double chunks = (q.a.max_q + L - 1) / L, in_chain = chunks * (W == 8 ? 1.2 : 0.65), behind = 2.5 + (double)q.a.total_q * q.a.heads * q.a.p * 6 / 4.6e6;
   const bool in_walk = normed && slices == 1 && (*normed || in_chain <= behind);
   if (normed) *normed = in_walk;
   if (in_walk) {
