@@ -40,7 +40,7 @@ struct Layout {
 // Workgroup = 8 waves of a (chunk, head).  Bound by its vector arithmetic (some 15 000 instructions of a wave, a tenth of them exponentials) and by the latency
 // of its phases: everything is asked for from memory at the start, blocks of one row of A and B share that row's factors, K is made beside the
 // solution, and the solution is split into operands once.  3 sequences of 4011 tokens and less, 8 heads of 128 x 128 (1256 workgroups, two a CU):
-// 107 us with every block's factors, all of K and W by four waves, and operands of T by each item -> 84.
+// 105 us with every block's factors, all of K and W by four waves, and operands of T by each item -> 83.
 template <typename Tag, int NK>
 __global__ void __launch_bounds__(kPrepareWaves * 64, NK < 5 ? 4 : 2) delta_prepare_kernel(DeltaPrep q) {
   typedef typename elem<Tag>::T T;
@@ -393,7 +393,7 @@ enum { WHOLE, SEGMENTS, ADDED, CARRY };   // workgroups are sequences, or segmen
 // Few long sequences leave most CUs idle in it, and are cut into segments of whole chunks (pick_segment).  What a segment does to the state ahead
 // of it is linear, S <- M S + C: a first launch walks the segments for C (from zeros, or what the sequence comes with) and M (from the identity, without
 // values), with neither q nor B; the second starts a segment from the state that the C and M of those before it give, and is otherwise the walk.  Of the
-// sequences above: 224 -> 53 + 58 us (11 chunks a segment; 5 - 8 times as many workgroups as sequences, heads and halves of them).
+// sequences above: 223 -> 54 + 63 us (11 chunks a segment; 5 - 8 times as many workgroups as sequences, heads and halves of them).
 template <typename Tag, int NK, int CW, int MODE>
 __device__ __forceinline__ void walk(const DeltaPrep &q, const Segments &sg, int wide, int at_head) {
   typedef typename elem<Tag>::T T;

@@ -20,7 +20,7 @@
 // carries the state through every segment but the last from zeros (the recurrence is linear: b, x and step sizes only), the second starts a
 // segment from S = the sum of those before it, each decayed by the segments between.  64 heads of 64 x 128 with the convolution and the
 // norm: 4 sequences of up to 3900 tokens 315 -> 271 us (the recurrence 232 -> 139 + 69 under the profiler), 1 x 1900 127 -> 71; 32 heads, 1 x 3900 229 -> 83.  Step
-// sizes and decays of a batch of chunks by all waves instead of the next chunk's by one: 271 -> 257 (the states 71 -> 56).
+// sizes and decays of a batch of chunks by all waves instead of the next chunk's by one: 272 -> 259 (under the profiler states 74 -> 59, segments 149 and 152).
 #include <algorithm>
 
 #include "ssm.h"
