@@ -91,8 +91,10 @@ class ExpertMLP(nn.Module):
         if self.router.dtype == torch.float32:
             return 16
         per = tokens * self.top / self.experts
+        if per <= FEW:
+            return 16
         if per <= self._rows32():
-            return 16 if per <= FEW else 32
+            return 32
         if per <= QUARTERS:
             return 64
         rows = self.experts * math.ceil(per / 128)        # workgroups of the two products
