@@ -430,7 +430,7 @@ __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
   f32x4 acc[WN][WM] = {};
   const uint32_t base = lds_address(smem) + lane * 16, rows = lds_address(smem) + row_place(r16, g) * 16;
   const int trips = p.k / 64;
-  f32x4 half[QUARTERS ? 2 : 1][WN][WM] = {};
+  f32x4 half[2][WN][WM] = {};   // (of the first two quarters, of the third)
   int quarter = 0;
   auto settle = [&](int done) {   // the quarters that end behind `done` steps of 32 inputs
     while (quarter < 3 && steps * (quarter + 1) / 4 == done) {
