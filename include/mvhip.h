@@ -836,6 +836,32 @@ typedef struct MvBlockLinearArgs {
 } MvBlockLinearArgs;
 int mv_block_linear(const MvBlockLinearArgs *args, int dtype, void *stream);
 
+/* ---- K21 — fp32 projections from operands in parts: each number as three of bf16 that add up to it, [16 rows][32 columns][part][8 columns of 4][row][8].
+ * mv_split_f32: up to MV_SPLIT_F32_MAX matrices [rows][k] of fp32, k a multiple of 32, rows `stride` apart (a multiple of 4); dst of
+ * mv_split_f32_bytes(rows, k) bytes; norm_w (NULL: none), norm_b (may be NULL): a LayerNorm over the k columns of the first matrix, in front.
+ * mv_linear_f32: out[rows][n] = x[rows][k] w[n][k]^T + bias[n] (may be NULL), no less than 0 if `relu`, + residual[rows][n] (may be NULL); fp32, or with
+ * `parts_out` in parts (n a multiple of 32, no residual).  n and strides multiples of 4, pointers of 16 bytes.  tile: 0 by the sizes, 1: 128 x 128 outputs a
+ * workgroup, 2: 64 x 64. */
+enum { MV_SPLIT_F32_MAX = 4 };
+typedef struct MvSplitF32Args {
+  const void *src[MV_SPLIT_F32_MAX];
+  void *dst[MV_SPLIT_F32_MAX];
+  int64_t stride[MV_SPLIT_F32_MAX];
+  int rows[MV_SPLIT_F32_MAX], k[MV_SPLIT_F32_MAX];
+  const void *norm_w, *norm_b;
+  float eps;
+  int count;
+} MvSplitF32Args;
+size_t mv_split_f32_bytes(int rows, int k);
+int mv_split_f32(const MvSplitF32Args *args, void *stream);
+typedef struct MvLinearF32Args {
+  const void *x, *w, *bias, *residual;
+  void *out;
+  int64_t residual_stride, out_stride;
+  int rows, n, k, relu, parts_out, tile;
+} MvLinearF32Args;
+int mv_linear_f32(const MvLinearF32Args *args, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,19 +1,26 @@
 """OPT decoder glue (mirror of minivllm/models/opt.py): learned positions (offset 2), MHA,
 LayerNorm, ReLU MLP, pre- or post-LN.  Attention runs on the same HIP kernels (D = 64 for
 OPT-125M); LayerNorm/ReLU/bias adds stay torch ops — OPT is the reference's CPU plumbing
-config, not a throughput target."""
+config, not a throughput target — but in fp32 prompts, where they ride in the projections (csrc/linear_f32.hip)."""
 from __future__ import annotations
 
 from typing import Any
 
+import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .. import hip_ops
 from ..layers import (Attention, ColumnParallelLinear, ParallelLMHead, QKVParallelLinear, RowParallelLinear,
                       VocabParallelEmbedding)
+from ..layers.linear import f32_tiles
 from ..parallel_state import get_tensor_parallel_world_size
 
 __all__ = ["OPTForCausalLM"]
+
+# fp32 layers go by parts of bf16 as a whole (norms, ReLU and residual sums within the projections' launches) from so many tiles of 64 x 64 hidden features
+# on.  us, 768 features, projections and what is between them, as modules / as a whole: 1000 rows (192 tiles) 154 / 170, 1300 (252) 188 / 183, 1600 (300) 230 / 215
+F32_LAYER_TILES_MIN = 264
 
 
 class OPTLearnedPositionalEmbedding(nn.Embedding):
@@ -41,12 +48,14 @@ class OPTAttention(nn.Module):
         self.attn = Attention(self.num_heads, self.head_dim, self.scaling, self.num_heads)
 
     def forward(self, positions, hidden_states):
-        t = hidden_states.shape[0]
-        qkv = self.qkv_proj(hidden_states)
+        return self.out_proj(self.attend(self.qkv_proj(hidden_states)))
+
+    def attend(self, qkv):
+        t = qkv.shape[0]
         width = self.num_heads * self.head_dim
         q, k, v = (qkv[:, i * width:(i + 1) * width].view(t, self.num_heads, self.head_dim) for i in range(3))
         o = self.attn(q, k, v)  # stores K/V, then prefill / paged decode
-        return self.out_proj(o.reshape(t, width))
+        return o.reshape(t, width)
 
 
 class OPTDecoderLayer(nn.Module):
@@ -60,7 +69,24 @@ class OPTDecoderLayer(nn.Module):
         self.fc2 = RowParallelLinear(config.ffn_dim, d, bias=config.enable_bias)
         self.final_layer_norm = nn.LayerNorm(d)
 
+    def _by_parts(self, x) -> bool:
+        att = self.self_attn
+        linears, norms = (att.qkv_proj, att.out_proj, self.fc1, self.fc2), (self.self_attn_layer_norm, self.final_layer_norm)
+        return (x.dtype == torch.float32 and self.do_layer_norm_before and f32_tiles(x.shape[0], x.shape[1]) >= F32_LAYER_TILES_MIN
+                and all(lin.tp_size == 1 for lin in linears) and not any(m._forward_hooks or m._forward_pre_hooks for m in (*linears, *norms, att))
+                and hip_ops.linear_f32_ok(x, *(t for m in (*linears, *norms) for t in (m.weight, m.bias))))
+
+    def _forward_parts(self, x):
+        att, fc1, fc2 = self.self_attn, self.fc1, self.fc2
+        rows, w_qkv, w_out = hip_ops.split_f32(x, att.qkv_proj.weight, att.out_proj.weight, norm=self.self_attn_layer_norm)
+        rows, = hip_ops.split_f32(att.attend(hip_ops.linear_f32(rows, w_qkv, att.qkv_proj.bias)))
+        x = hip_ops.linear_f32(rows, w_out, att.out_proj.bias, residual=x)
+        rows, w1, w2 = hip_ops.split_f32(x, fc1.weight, fc2.weight, norm=self.final_layer_norm)
+        return hip_ops.linear_f32(hip_ops.linear_f32(rows, w1, fc1.bias, relu=True, parts=True), w2, fc2.bias, residual=x)
+
     def forward(self, positions, x, residual=None):
+        if self._by_parts(x):
+            return self._forward_parts(x), None
         if self.do_layer_norm_before:
             x = x + self.self_attn(positions, self.self_attn_layer_norm(x))
             x = x + self.fc2(F.relu(self.fc1(self.final_layer_norm(x))))

@@ -127,6 +127,9 @@ _SIGNATURES = {
                                                     c_int, c_int, c_int, c_void_p]),
     "mv_packed_weight_elems": (c_size_t, [c_int, c_int]),
     "mv_block_linear": (c_int, [c_void_p, c_int, c_void_p]),
+    "mv_split_f32_bytes": (c_size_t, [c_int, c_int]),
+    "mv_split_f32": (c_int, [c_void_p, c_void_p]),
+    "mv_linear_f32": (c_int, [c_void_p, c_void_p]),
     "mv_pack_weight": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "mv_linear_mid_m": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int,
                                 c_int, c_int, c_int, c_void_p]),
@@ -1007,6 +1010,82 @@ def block_linear(x, weight, blocks):
         a.first_input[i], a.first_output[i], a.outputs[i] = at, to, outputs
     _check(_lib.mv_block_linear(ctypes.byref(a), _dt(x), _stream()), "mv_block_linear")
     return out
+
+
+# ---------------------------------------------------------------- K21
+MV_SPLIT_F32_MAX = 4
+
+
+class MvSplitF32Args(ctypes.Structure):
+    """include/mvhip.h: MvSplitF32Args."""
+    _fields_ = [("src", c_void_p * MV_SPLIT_F32_MAX), ("dst", c_void_p * MV_SPLIT_F32_MAX), ("stride", c_int64 * MV_SPLIT_F32_MAX),
+                ("rows", c_int * MV_SPLIT_F32_MAX), ("k", c_int * MV_SPLIT_F32_MAX), ("norm_w", c_void_p), ("norm_b", c_void_p), ("eps", c_float),
+                ("count", c_int)]
+
+
+MvLinearF32Args = _struct(
+    "MvLinearF32Args", x__w__bias__residual__out=c_void_p, residual_stride__out_stride=c_int64, rows__n__k__relu__parts_out__tile=c_int)
+
+
+class F32Parts(NamedTuple):
+    """A matrix [rows, k] of fp32 numbers, each as three of bf16 (mv_split_f32)."""
+    data: torch.Tensor
+    rows: int
+    k: int
+
+
+def linear_f32_ok(x, *others) -> bool:
+    """May a projection of ``x`` [T, K] with these weights [N, K] and vectors [N] (None: not there) go by parts?  Plain numbers on the current device, of
+    which nobody asks for gradients, tangents or a trace."""
+    if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.float32) or x.device.index != torch.cuda.current_device() or torch.is_autocast_enabled("cuda"):
+        return False
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    for t in (x, *others):
+        if t is None:
+            continue
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+        if t.dtype != torch.float32 or t.device != x.device or t.data_ptr() % 16 or (torch.is_grad_enabled() and t.requires_grad):
+            return False
+        if t is x:
+            if t.shape[1] % 32 or t.stride(1) != 1 or t.stride(0) % 4 or t.stride(0) < t.shape[1]:
+                return False
+        elif not t.is_contiguous() or t.shape[0] % 4 or (t.dim() == 2 and t.shape[1] % 32) or t.dim() > 2:
+            return False
+    return True
+
+
+def split_f32(*matrices, norm=None):
+    """Each fp32 matrix [rows, k] in parts; ``norm``: a LayerNorm that the first one goes through."""
+    a, out = MvSplitF32Args(count=len(matrices)), []
+    if norm is not None:
+        a.norm_w, a.norm_b, a.eps = norm.weight.data_ptr(), _ptr(norm.bias), norm.eps
+    for i, m in enumerate(matrices):
+        rows, k = m.shape
+        out.append(F32Parts(torch.empty(_lib.mv_split_f32_bytes(rows, k), dtype=torch.uint8, device=m.device), rows, k))
+        a.src[i], a.dst[i], a.stride[i], a.rows[i], a.k[i] = m.data_ptr(), out[-1].data.data_ptr(), m.stride(0), rows, k
+    _check(_lib.mv_split_f32(ctypes.byref(a), _stream()), "mv_split_f32")
+    return out
+
+
+def linear_f32(x, w, bias=None, residual=None, relu=False, parts=False, tile=0):
+    """max(x W^T + bias, 0) if ``relu`` else x W^T + bias, + residual [rows, n]; x and w in parts -> [rows, n], or its parts.  ``tile``: 1 / 2: tiles of
+    128 x 128 / 64 x 64, 0: by the sizes."""
+    if x.k != w.k:
+        raise MvHipError(f"inputs of {x.k} and {w.k}")
+    rows, n = x.rows, w.rows
+    if bias is not None and (bias.dtype != torch.float32 or bias.shape != (n,) or not bias.is_contiguous()):
+        raise MvHipError(f"bias: {n} fp32 numbers required")
+    if residual is not None and (residual.dtype != torch.float32 or residual.shape != (rows, n) or residual.stride(1) != 1):
+        raise MvHipError(f"residual: [{rows}, {n}] fp32 numbers required")
+    data = torch.empty(_lib.mv_split_f32_bytes(rows, n), dtype=torch.uint8, device=x.data.device) if parts else \
+        torch.empty((rows, n), dtype=torch.float32, device=x.data.device)
+    a = MvLinearF32Args(x=x.data.data_ptr(), w=w.data.data_ptr(), bias=_ptr(bias), residual=_ptr(residual), out=data.data_ptr(),
+                        residual_stride=0 if residual is None else residual.stride(0), out_stride=n, rows=rows, n=n, k=x.k, relu=int(relu),
+                        parts_out=int(parts), tile=tile)
+    _check(_lib.mv_linear_f32(ctypes.byref(a), _stream()), "mv_linear_f32")
+    return F32Parts(data, rows, n) if parts else data
 
 
 # ---------------------------------------------------------------- K11

@@ -1,5 +1,5 @@
 """Tensor-parallel linear layers (mirror of minivllm/models/layers/linear.py:36-319).
-Prefill GEMMs stay on hipBLASLt through ``F.linear``.  Decode steps go to the hand-written kernels:
+Prefill GEMMs stay on hipBLASLt through ``F.linear``, but those of fp32 (csrc/linear_f32.hip).  Decode steps go to the hand-written kernels:
   * up to ``SMALL_M_MAX`` tokens every projection is a pure HBM stream of its weights
     (csrc/linear_small_m.hip; on the fragment-ordered copy below when there is one — whole-line loads —
     else on the row-major weights);
@@ -72,6 +72,12 @@ try:
         _TUNED = json.load(_f).get("plans", {})
 except (OSError, ValueError):
     _TUNED = {}
+
+
+# fp32 projections by parts of bf16 (csrc/linear_f32.hip) from so many tiles of 64 x 64 on, which have to fill the chip twice, and so many rows, which
+# have to pay for the weight's parts.  Parts and product / library: 492 tiles 1.02 .. 1.09, 504 1.07, 512 1.06 .. 1.11, 576 0.97, 624 0.72 .. 0.87, 672 0.81 ..
+# 0.86, 900 0.87; 50272 outputs of 300 rows 1.07, of 512 0.84, 12288 of 300 1.00, of 512 0.98
+F32_TILES_MIN, F32_ROWS_MIN = 600, 512
 
 
 class PartialSum:
@@ -159,7 +165,15 @@ def linear(x, weight, bias=None, packed=None, kind: str = "col"):
                 return PartialSum(hip_ops.linear_mid_m_partial(x, packed, n, splits, cfg), x.dtype)
             if cfg:
                 return hip_ops.linear_mid_m(x, packed, n, bias, cfg)
+    if x.dtype == torch.float32 and x.dim() == 2 and x.shape[0] >= F32_ROWS_MIN and f32_tiles(x.shape[0], weight.shape[0]) >= F32_TILES_MIN \
+            and x.shape[1] == weight.shape[1] and hip_ops.linear_f32_ok(x, weight, bias):
+        return hip_ops.linear_f32(*hip_ops.split_f32(x, weight), bias)
     return F.linear(x, weight, bias)
+
+
+def f32_tiles(rows: int, n: int) -> int:
+    """Tiles of 64 x 64 outputs."""
+    return -(-rows // 64) * -(-n // 64)
 
 
 def gelu_linear(x, lin):
