@@ -501,13 +501,18 @@ __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
 }
 
 // Very many rows: 128 x 256 per workgroup of four waves side by side, two workgroups to a CU, so that one multiplies while the other starts or ends.
-// Bound by the matrix cores, if their operands are there in time: three stages of 32 inputs, of which two are under way, and the operands of a stage
-// are read one by one between the products of the stage before.  Results leave through LDS, 128 bytes of a row (gated: 64) to a store.
+// Bound by the matrix cores and their power, if the operands are there in time: three stages of 32 inputs, of which two are under way, and the operands of a stage
+// are read one by one between the products of the stage before, as are the next transfers asked for.  A stage takes 1224 cycles where its products are 1024 (two
+// workgroups) and those with their transfers alone 1084, at 1.65 of 2.4 GHz.  Rows come 64 inputs at a time, in whole lines of memory, every other stage.
+// Results leave through LDS, 128 bytes of a row (gated: 64) to a store.
 // Workgroups are dealt to the XCDs in turn, and each XCD gets a run of an eighth of the work (eight tiles of rows and all their outputs at a time, the
 // rows first): its L2 holds what its workgroups share, and none has more than the others.
 // 36004 pairs of 32 experts, 2048 -> 2 x 768 gated and 768 -> 2048: 343 + 198 us (one workgroup of 256 x 256 to a CU, two stages of 64 inputs, four
-// tiles to an XCD in turn) -> 260 + 157.
+// tiles to an XCD in turn) -> 260 + 157 (rows by half lines, transfers at the start of a stage, tiles looked for one trip to memory behind the other; the layer
+// with all that is beside them 483) -> the layer 460.
 constexpr int kWideRows = 128, kWideStages = 3;
+// place of a row's piece among its eight, and the piece at a place: the lanes of a read (four each of different rows) are at different banks
+__device__ __forceinline__ int wide_piece(int row, int piece) { return piece ^ (row >> 1 & 7); }
 template <typename Tag, bool GATED, int ACT>
 __device__ __forceinline__ float wide_result(float x, float up, MvGateAct act) {
   if constexpr (!GATED) return x;
@@ -518,56 +523,74 @@ __device__ __forceinline__ float wide_result(float x, float up, MvGateAct act) {
 template <typename Tag, bool GATED>
 __global__ void __launch_bounds__(256, 2) moe_wide_kernel(MoeLinear p, int nx, int max_tiles) {
   typedef typename elem<Tag>::T T;
-  constexpr int TILES = 16, WM = 8, WN = 4, STAGE = (WM + TILES) * 1024, PER = 6;
-  extern __shared__ __attribute__((aligned(16))) char smem[];   // stages of rows [WM] | weights [TILES] fragments
+  constexpr int TILES = 16, WM = 8, WN = 4, WSTAGE = TILES * 1024, XSTAGE = WM * 2048;
+  extern __shared__ __attribute__((aligned(16))) char smem[];   // three stages of weights, two of rows (64 inputs)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  // the halves of a tile of 256 rows that are there
-  const unsigned long long below = (1ull << lane) - 1;
-  unsigned long long upper, lower;
-  auto halves = [&](int i0) {
-    const int i = min(i0 + lane, max_tiles - 1);
-    const bool there = i0 + lane < max_tiles && p.tiles[3 * i] >= 0;
-    upper = __ballot(there), lower = __ballot(there && p.tiles[3 * i + 2] > kWideRows);
-    return __popcll(upper) + __popcll(lower);
+  // the halves of a tile of 256 rows that are there: tiles 64 c + lane, all asked for at once (more of them: once more for the one that is looked for)
+  constexpr int AHEAD = 8;
+  int info[AHEAD][3];
+  auto look = [&](int i0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) info[c][q] = p.tiles[3 * min(i0 + 64 * c + lane, max_tiles - 1) + q];
   };
-  int total = 0;
-  for (int i0 = 0; i0 < max_tiles; i0 += 64) total += halves(i0);
+  auto upper_of = [&](int c, int i0) { return __ballot(i0 + 64 * c + lane < max_tiles && info[c][0] >= 0); };
+  auto lower_of = [&](int c, int i0) { return __ballot(i0 + 64 * c + lane < max_tiles && info[c][0] >= 0 && info[c][2] > kWideRows); };
+  int total = 0, held = 0;
+  for (int i0 = 0; i0 < max_tiles; i0 += 64 * AHEAD) {
+    look(held = i0);
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c) total += __popcll(upper_of(c, i0)) + __popcll(lower_of(c, i0));
+  }
   const int per = (total * nx + 7) / 8, turn = blockIdx.x >> 3, index = (blockIdx.x & 7) * per + turn;
   if (turn >= per || index >= total * nx) return;
   const int group = index / (8 * nx), in = index - group * 8 * nx, high = min(8, total - group * 8), tx = in / high;
-  int nth = group * 8 + in % high, i0 = 0;
-  for (int n = halves(0); nth >= n; n = halves(i0)) nth -= n, i0 += 64;
-  const int ahead = __popcll(upper & below) + __popcll(lower & below);
-  const bool second = (lower >> lane & 1) && nth == ahead + 1;
-  const unsigned long long mine = __ballot((upper >> lane & 1) && (nth == ahead || second));
-  const int32_t *tile = p.tiles + 3 * (i0 + __ffsll(mine) - 1);
-  const int skip = __ballot(second) ? kWideRows : 0, e = tile[0], m0 = tile[1] + skip, live = tile[2] - skip;
+  int nth = group * 8 + in % high, e = -1, m0 = 0, live = 0;
+  for (int i0 = 0; e < 0; i0 += 64 * AHEAD) {
+    if (i0 != held) look(held = i0);
+#pragma unroll
+    for (int c = 0; c < AHEAD; ++c) {
+      const unsigned long long upper = upper_of(c, i0), lower = lower_of(c, i0);
+      const int n = __popcll(upper) + __popcll(lower);
+      if (nth >= 0 && nth < n) {
+        const unsigned long long below = (1ull << lane) - 1;
+        const int ahead = __popcll(upper & below) + __popcll(lower & below);
+        const bool second = (lower >> lane & 1) && nth == ahead + 1;
+        const int mine = __ffsll(__ballot((upper >> lane & 1) && (nth == ahead || second))) - 1, skip = __ballot(second) ? kWideRows : 0;
+        e = __builtin_amdgcn_readlane(info[c][0], mine), m0 = __builtin_amdgcn_readlane(info[c][1], mine) + skip;
+        live = __builtin_amdgcn_readlane(info[c][2], mine) - skip;
+      }
+      nth -= n;
+    }
+  }
   const int ntiles = p.n / 16, steps = p.k / 32, nt0 = tx * (GATED ? TILES / 2 : TILES);
-  // this wave's fragments of a stage: two of the rows, four of the weights
-  const T *xs[2], *ws[4];
+  // this wave's transfers: eight rows x 64 inputs (whole lines of memory), of which there are four to a wave every other stage; four fragments of weights
+  const T *xs[4], *ws[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = 4 * i + wave, wt = min(nt0 + (GATED ? j >> 1 : j), ntiles - 1) + (GATED && (j & 1) ? ntiles : 0);
     ws[i] = (const T *)p.w + e * p.w_expert + (int64_t)wt * steps * 512;
-    if (i < 2) {
-      const int place = m0 + min(j * 16 + (lane >> 2), live - 1);
-      xs[i] = (const T *)p.x + (int64_t)(p.tokens ? p.tokens[place] : place) * p.x_stride + row_chunk(lane) * 8;
-    }
+    const int row = j * 8 + (lane >> 3), place = m0 + min(row, live - 1);
+    xs[i] = (const T *)p.x + (int64_t)(p.tokens ? p.tokens[place] : place) * p.x_stride + (wide_piece(row & 15, lane & 7)) * 8;
   }
   const int lane8 = lane * 8;
   auto transfer = [&](const T *from, char *to) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)from, (__attribute__((address_space(3))) void *)to, 16, 0, 0);
   };
-  auto fetch = [&](int t, int slot) {
-    char *to = smem + slot * STAGE + wave * 1024;
+  auto fetch_w = [&](int i, int t, int slot) __attribute__((always_inline)) { transfer(ws[i] + (int64_t)t * 512 + lane8, smem + slot * WSTAGE + (4 * i + wave) * 1024); };
+  auto fetch_x = [&](int i, int u) __attribute__((always_inline)) { transfer(xs[i] + (int64_t)u * 64, smem + kWideStages * WSTAGE + (u & 1) * XSTAGE + (4 * i + wave) * 1024); };
+  // stages 0 .. 2 of the weights, 0 .. 3 of the rows, in the order in which they are needed
+  for (int t = 0; t < min(kWideStages, steps); ++t) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) transfer(xs[i] + (int64_t)t * 32, to + i * 4096);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) transfer(ws[i] + (int64_t)t * 512 + lane8, to + WM * 1024 + i * 4096);
-  };
-  for (int t = 0; t < min(kWideStages, steps); ++t) fetch(t, t);
+    for (int i = 0; i < 4; ++i) {
+      if (t != 1) fetch_x(i, t >> 1);
+      fetch_w(i, t, t);
+    }
+  }
   f32x4 acc[WN][WM] = {};
-  const uint32_t rows = lds_address(smem) + row_place(r16, g) * 16, weights = lds_address(smem) + lane * 16 + (WM + wave * WN) * 1024;
+  const uint32_t rows = lds_address(smem) + kWideStages * WSTAGE + r16 * 128, weights = lds_address(smem) + lane * 16 + wave * WN * 1024;
+  const int piece_of[2] = {wide_piece(r16, g) * 16, wide_piece(r16, 4 + g) * 16};
   u32x4 a[2][WN], b[2][WM];
   auto landed = [&](auto H) __attribute__((always_inline)) {
     constexpr int h = decltype(H)::value;
@@ -577,29 +600,35 @@ __global__ void __launch_bounds__(256, 2) moe_wide_kernel(MoeLinear p, int nx, i
   int slot = 0;
   auto step = [&](auto H, int t) __attribute__((always_inline)) {
     constexpr int h = decltype(H)::value;
-    // stage t + 1 is there, and every wave has stage t in registers, whose place the stage three ahead takes
-    if (t + kWideStages - 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * (kWideStages - 2)) : "memory");
+    // stage t + 1 is there, and every wave has stage t in registers, whose place the stage three ahead takes (rows: that of stages t - 1 and t, at odd t)
+    if (t + kWideStages - 1 < steps) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(h == 0 ? 8 : 4) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
-    if (t + kWideStages < steps) fetch(t + kWideStages, slot);
+    const bool ahead = t + kWideStages < steps;
+    const int free = slot;
     slot = slot == kWideStages - 1 ? 0 : slot + 1;
-    const uint32_t xa = rows + slot * STAGE, wa = weights + slot * STAGE;   // (behind the last stage: an old one, for nobody)
+    // (behind the last stage: an old one, for nobody)
+    const uint32_t xa = rows + (h ? ((t + 1) >> 1 & 1) : (t >> 1 & 1)) * XSTAGE + piece_of[1 - h], wa = weights + slot * WSTAGE;
     static_for<WM>([&](auto I) {
       constexpr int i = decltype(I)::value;
       if constexpr (i < WN) lds_read128<i * 1024>(a[1 - h][i], wa);
-      lds_read128<i * 1024>(b[1 - h][i], xa);
+      lds_read128<i * 2048>(b[1 - h][i], xa);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < WN; ++j) acc[j][i] = mfma16x16x32<Tag>(a[h][j], b[h][i], acc[j][i]);
+      if (ahead) {
+        if constexpr (i >= 4) fetch_w(i - 4, t + kWideStages, free);
+        else if constexpr (h == 1) fetch_x(i, (t + kWideStages) >> 1);
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
     landed(std::integral_constant<int, 1 - h>{});
   };
-  if (steps >= kWideStages) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER * (kWideStages - 1)) : "memory");
+  if (steps >= kWideStages) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   lds_barrier();
   static_for<WN>([&](auto I) { lds_read128<decltype(I)::value * 1024>(a[0][decltype(I)::value], weights); });
-  static_for<WM>([&](auto I) { lds_read128<decltype(I)::value * 1024>(b[0][decltype(I)::value], rows); });
+  static_for<WM>([&](auto I) { lds_read128<decltype(I)::value * 2048>(b[0][decltype(I)::value], rows + piece_of[0]); });
   landed(std::integral_constant<int, 0>{});
   for (int t = 0; t < steps; t += 2) {   // (an even number of them)
     step(std::integral_constant<int, 0>{}, t);
@@ -696,7 +725,7 @@ int launch_linear(const MoeLinear &p, int tile_m, int max_tiles, hipStream_t st)
     const int nx = (nt * (GATED ? 2 : 1) + 15) / 16;
     if (int rc = mv_allow_lds<moe_wide_kernel<Tag, GATED>>()) return rc;
     hipLaunchKernelGGL((moe_wide_kernel<Tag, GATED>), dim3((unsigned)(((int64_t)max_tiles * 2 * nx + 7) / 8 * 8)), dim3(256),
-                       kWideStages * 24 * 1024, st, p, nx, max_tiles);
+                       80 * 1024, st, p, nx, max_tiles);
   } else {
     return MV_E_SHAPE;
   }

@@ -36,3 +36,17 @@ def test_halves_are_as_few_rows(H, counts, k, n, dtype, act, scaled):
     eps = torch.finfo(dtype).eps
     assert ((out[0] - out[1]).abs() <= 4 * eps * out[0].abs() + 2**-11).all()
     assert torch.isfinite(out[1]).all()
+
+
+@pytest.mark.parametrize("counts", [[1] * 700 + [300], [0] * 600 + [257] * 3 + [0] * 100 + [5], [130] * 515])
+def test_more_tiles_than_are_held(H, counts):
+    """Tiles that a workgroup looks for among more than 512: each place's result is its expert's."""
+    experts, rows, k, n = len(counts), sum(counts), 64, 32
+    ids = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts)).int().to(DEV)[:, None]
+    x = torch.ones(rows, k, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(experts, n, k, dtype=torch.bfloat16, device=DEV)
+    w[:, :, 0], w[:, :, 1] = (torch.arange(experts, device=DEV) // 16)[:, None].bfloat16(), (torch.arange(experts, device=DEV) % 16 / 16)[:, None].bfloat16()
+    groups = H.moe_group(ids, experts, 256)
+    got = H.moe_linear(x, H.pack_weight(w.view(-1, k)), n, groups, None, gather=True, experts=experts)
+    want = (ids.float() / 16).bfloat16().expand(rows, n)      # (exact sums, rounded once)
+    assert torch.equal(got[groups.place.long()], want)
