@@ -17,38 +17,10 @@
 // 1300 rows of 768 -> 3072 53 / 46; 8000 of 2048 -> 12288 2772 / 1715.
 #include <algorithm>
 
-#include "latent.h"
+#include "parts.h"
 
 namespace {
 
-// Eight numbers as three times eight of bf16 whose sums they are: each part is what rounding has left of the parts before.  The first part of a number
-// that bf16 rounds to infinity is cut off instead; one that is not finite has no second and third part.
-__device__ __forceinline__ void split3(float (&f)[8], u32x4 (&part)[3]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t v = pack_pair<bf16_tag>(f[2 * i], f[2 * i + 1]);
-    float lo = u2f(v << 16), hi = u2f(v & 0xffff0000u);
-    float rl = f[2 * i] - lo, rh = f[2 * i + 1] - hi;
-    if (!(fabsf(lo) < INFINITY) || !(fabsf(hi) < INFINITY)) {
-      auto cut = [](float x, float part, float &rest) {
-        if (fabsf(part) < INFINITY) return f2u(part);
-        const uint32_t top = f2u(x) & 0xffff0000u;
-        if (fabsf(x) < INFINITY) {
-          rest = x - u2f(top);
-          return top;
-        }
-        rest = 0.f;
-        return x != x ? top | 0x400000u : top;
-      };
-      const uint32_t a = cut(f[2 * i], lo, rl), b = cut(f[2 * i + 1], hi, rh);
-      v = a >> 16 | b;
-    }
-    part[0][i] = v;
-    v = pack_pair<bf16_tag>(rl, rh);
-    part[1][i] = v;
-    part[2][i] = pack_pair<bf16_tag>(rl - u2f(v << 16), rh - u2f(v & 0xffff0000u));
-  }
-}
 // Parts lie as the products read them: [16 rows][32 inputs][part][quarter of the inputs, row][8]
 __device__ __forceinline__ int64_t part_place(int64_t row, int piece, int k) { return ((row >> 4) * (k >> 5) + (piece >> 2)) * 192 + (piece & 3) * 16 + (row & 15); }
 
@@ -99,7 +71,7 @@ __global__ void __launch_bounds__(256) split_f32_kernel(Split q) {
       }
     float f[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
     u32x4 part[3];
-    split3(f, part);
+    split3<true>(f, part);
     u32x4 *to = (u32x4 *)p.dst[m] + part_place(row0 + (lane >> 2), i >> 3, k);
 #pragma unroll
     for (int s = 0; s < 3; ++s) to[64 * s] = part[s];
@@ -210,7 +182,7 @@ __global__ void __launch_bounds__(256, 2) linear_f32_kernel(MvLinearF32Args p, i
         f32x4 a = finish(*(const f32x4 *)from, live, n), b = finish(*(const f32x4 *)(from + 4), live, n + 4);
         float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
         u32x4 part[3];
-        split3(f, part);
+        split3<true>(f, part);
         u32x4 *to = (u32x4 *)p.out + part_place(row, n >> 3, p.n);
 #pragma unroll
         for (int s = 0; s < 3; ++s) to[64 * s] = part[s];

@@ -14,10 +14,11 @@
 //   head dim 128: 20 tokens 0.84 / 0.85, 50 0.99 / 1.05, 300 1.20 / 1.59, 1000 1.37 / 2.26     (chains of 32: 1.05, 1.28, 1.73, 2.25)
 // What the tree costs and gives, attention of a layer (us): 6131 tokens in 8 prompts, 12 heads of 64: vector kernel 801, chains of 16 products 137, this
 // 148 (62 TFLOP/s of visible pairs; 4 x 2048: 91); 16 x 1024, 16 heads of 128: 958 -> 771 (89), where the longer chains and rows of K and V
-// side by side left 69 registers in memory; now 4 (paged or masked: 12; head dim 64: 1, 6).
+// side by side left 69 registers in memory; now 4 (paged or masked: 12; head dim 64: 6).  Whole prompts of head dim 64 have a kernel of their own by now (below).
 // The vector kernel (prefill_simple.hip: a wave per query and head, every query reads its keys again) stays for head dim 256, and where queries see few
 // keys or are few themselves: vector_is_quicker below.
 // Reference: minivllm/models/layers/attention.py:467-504,554-597.
+#include "parts.h"
 #include "prefill_row.h"
 
 namespace {
@@ -311,6 +312,256 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
   }
 }
 
+// ---- whole prompts, keys side by side, head dim 64: the same tiles by parts of bf16 (parts.h), a product the six of its parts' products that matter.
+// 32 queries to a wave, K and V brought into parts on their way into LDS, for 128 queries at a time, or for 64, whose waves take 32 keys each of 64 in turn and meet
+// at the end, where there are not enough of the larger ones.  S^T = K Q^T puts four keys of a query in a lane, and P, as it lies in the accumulators, is the
+// operand of O^T += V^T P^T, whose V is read transposed in that order of keys.  Of a score's products and of a tile of values the smallest are added up first, and 32 keys'
+// values apart from the rest, so that one sum in 32 keys rounds at its size.  What is not finite goes to the vector kernel's rows.
+// Bound by vector arithmetic and products that do not overlap enough (58 + 40 % of the CUs' cycles): 200 instructions for the softmax and P's parts of 32 x 32, 120 for those
+// of K and V, beside 96 products.  us, the fp32 products' kernel / 64 queries / 128: 12 heads, 8 prompts of 511 .. 1021 tokens 141 / 90 / 83 (and the distance
+// from 64 bits 1.31e-7, 1.08, 1.10); one of 1000 64 / 44 / 63; 4 of 2048 283 / 177 / 159; 80 of 50 26 / 22 / 25.  Tried: v_dot2_f32_bf16 for the rests 86 (128 queries), two tiles of values
+// at a time 82, values' products straight into the sums 82 and 2.0e-7, priority for the products 82.
+typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
+// the largest bits of third parts: those of a number that is not finite, or that bf16 rounds to infinity, are no less than 0x7f80
+__device__ __forceinline__ void look(const u32x4 &third, u16x2 &odd) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) odd = __builtin_elementwise_max(odd, __builtin_bit_cast(u16x2, third[i] & 0x7fff7fffu));
+}
+__device__ __forceinline__ u32x2 read_tr(const char *p) {
+  typedef __attribute__((ext_vector_type(4))) short s16x4;
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p));
+}
+__device__ __forceinline__ f32x4 mfma(const u32x4 &a, const u32x4 &b, const f32x4 &c) { return mfma16x16x32<bf16_tag>(a, b, c); }
+
+template <int D, int GROUPS>   // (head dim 128: 55 registers in memory; 8 prompts of 511 .. 1021 tokens 255 -> 201 us, one of 1000 111 -> 157)
+__global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) {
+  constexpr int TURNS = 4 / GROUPS, BM = 32 * GROUPS, BN = 4096 / D, SUBS = BN / 32 / TURNS, KS = D / 32, DT = D / 16, CH = D / 8;   // (32 keys: a sub)
+  constexpr int PART = BN * D * 2;
+  static_assert(SUBS >= 1);
+  __shared__ __attribute__((aligned(16))) char kl[3 * PART], vl[3 * PART];
+  __shared__ int again;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4, group = wave % GROUPS, turn = wave / GROUPS;
+  const int head = blockIdx.x, seq = blockIdx.y, hkv = head / (p.n_heads / p.n_kv_heads);
+  const int q0 = p.cu_q[seq], sq = p.cu_q[seq + 1] - q0, k0 = p.cu_k[seq], sk = p.cu_k[seq + 1] - k0;
+  const int qb = ((int)gridDim.z - 1 - (int)blockIdx.z) * BM;   // the longest rows first
+  if (qb >= sq) return;
+  if (tid == 0) again = 0;
+  const int shift = sk - sq, last = min(qb + BM, sq) - 1, end = min(sk, last + shift + 1), steps = end > 0 ? (end + BN - 1) / BN : 0;
+  const int wave_lo = min(qb + group * 32, sq - 1) + shift, wave_hi = min(qb + group * 32 + 31, sq - 1) + shift;
+  // places of a row's pieces of eight, in orders that spread the rows that are read together over the banks
+  auto k_place = [](int row, int c) { return (row * CH + (c ^ (D == 64 ? row >> 1 & 7 : row & 15))) * 16; };
+  auto v_place = [](int row, int c) { return (row * CH + (c ^ (D == 64 ? row & 6 : (row & 7) << 1))) * 16; };
+
+  f32x4 raw[2][2][2];   // rows of K, V on their way
+  auto fetch = [&](int step) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int at = tid + n * 256, row = min(step * BN + at / CH, sk - 1), c = at % CH * 8;   // (rows behind the end: the last one again, masked)
+      const float *k = (const float *)p.k + (int64_t)(k0 + row) * p.k_stride + (int64_t)hkv * D + c, *v = (const float *)p.v + (int64_t)(k0 + row) * p.v_stride + (int64_t)hkv * D + c;
+      raw[0][n][0] = *(const f32x4 *)k, raw[0][n][1] = *(const f32x4 *)(k + 4);
+      raw[1][n][0] = *(const f32x4 *)v, raw[1][n][1] = *(const f32x4 *)(v + 4);
+    }
+  };
+  u16x2 odd = {0, 0};
+  auto put = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const int at = tid + n * 256, row = at / CH, c = at % CH;
+        const f32x4 &a = raw[w][n][0], &b = raw[w][n][1];
+        float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        u32x4 part[3];
+        split3<false>(f, part);
+        look(part[2], odd);
+#pragma unroll
+        for (int s = 0; s < 3; ++s) *(u32x4 *)((w ? vl : kl) + s * PART + (w ? v_place(row, c) : k_place(row, c))) = part[s];
+      }
+  };
+  if (steps > 0) fetch(0);
+  u32x4 q[2][KS][3];   // dims 32 s + 8 g .. of query 16 i + r16
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const float *from = (const float *)p.q + (int64_t)(q0 + min(qb + group * 32 + i * 16 + r16, sq - 1)) * p.q_stride + (int64_t)head * D + s * 32 + g * 8;
+      const f32x4 a = *(const f32x4 *)from, b = *(const f32x4 *)(from + 4);
+      float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      split3<false>(f, q[i][s]);
+      look(q[i][s][2], odd);
+    }
+  const float scale_log2 = p.scale * 1.4426950408889634f;
+  const bool late = scale_log2 > 0.f;   // scores are multiplied by `mul` where their exponent is formed, without a rounding between
+  const float mul = late ? scale_log2 : 1.f;
+  float m[2] = {-1e30f, -1e30f}, l[2] = {0.f, 0.f};
+  if (p.mask.sink)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) sink_start(((const float *)p.mask.sink)[head], g == 0 && turn == 0, m[i], l[i]);
+  f32x4 o[2][DT] = {};   // dims 16 t + 4 g .. of query 16 i + r16
+  for (int step = 0; step < steps; ++step) {
+    __syncthreads();   // every wave is done with the keys before
+    put();
+    if (step + 1 < steps) fetch(step + 1);
+    __syncthreads();
+#pragma unroll
+    for (int sub = 0; sub < SUBS; ++sub) {
+      const int in = (TURNS == 1 ? sub : turn) * 32, key0 = step * BN + in;
+      if (key0 > wave_hi || key0 >= sk) continue;   // (of the wave)
+      // scores, keys by queries: the smallest products first, so that only the last of a row's KS sums round at its size
+      f32x4 s[2][2] = {};
+      const char *kt = kl;
+#pragma unroll
+      for (int c = 0; c < KS; ++c) {
+        u32x4 k[2][3];
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) k[j][b] = *(const u32x4 *)(kt + b * PART + k_place(in + 16 * j + r16, 4 * c + g));
+#pragma unroll
+        for (int b = 2; b >= 1; --b)
+#pragma unroll
+          for (int a = 0; a <= b; ++a)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+              for (int i = 0; i < 2; ++i) s[j][i] = mfma(k[j][a], q[i][c][b - a], s[j][i]);
+      }
+#pragma unroll
+      for (int c = 0; c < KS; ++c) {
+        u32x4 k[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) k[j] = *(const u32x4 *)(kt + k_place(in + 16 * j + r16, 4 * c + g));
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) s[j][i] = mfma(k[j], q[i][c][0], s[j][i]);
+      }
+      if (!late)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) s[j][i] *= scale_log2;
+      if (key0 + 31 > wave_lo || key0 + 32 > sk) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int upto = min(min(qb + group * 32 + i * 16 + r16, sq - 1) + shift, sk - 1) - key0 - 4 * g;
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[j][i][e] = 16 * j + e <= upto ? s[j][i][e] : -INFINITY;
+        }
+      }
+      u32x4 w[2][3];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float mx = fmaxf(fmaxf(fmaxf(s[0][i][0], s[0][i][1]), fmaxf(s[0][i][2], s[0][i][3])), fmaxf(fmaxf(s[1][i][0], s[1][i][1]), fmaxf(s[1][i][2], s[1][i][3])));
+        float a, b;
+        swap16(mx, a, b);
+        swap32(fmaxf(a, b), a, b);
+        mx = fmaxf(m[i], fmaxf(a, b) * mul);
+        if (__any(mx > m[i])) {
+          const float alpha = __builtin_amdgcn_exp2f(m[i] - mx);
+          l[i] *= alpha;
+#pragma unroll
+          for (int t = 0; t < DT; ++t) o[i][t] *= alpha;
+          m[i] = mx;
+        }
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = __builtin_amdgcn_exp2f(fmaf(s[e >> 2][i][e & 3], mul, -m[i]));
+        l[i] += ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+        split3<false>(f, w[i]);
+      }
+      // values: a tile's products of these keys apart, the smallest first, one sum into the rest's
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        u32x4 v[3];
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+          const int row = in + 4 * g + (r16 >> 2), c = 2 * t + ((r16 & 3) >> 1);
+          const u32x2 lo = read_tr(vl + b * PART + v_place(row, c) + (r16 & 1) * 8), hi = read_tr(vl + b * PART + v_place(row + 16, c) + (r16 & 1) * 8);
+          v[b] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+        }
+        f32x4 sum[2] = {};
+#pragma unroll
+        for (int b = 2; b >= 0; --b)
+#pragma unroll
+          for (int a = 0; a <= b; ++a)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) sum[i] = mfma(v[a], w[i][b - a], sum[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) o[i][t] += sum[i];
+      }
+    }
+  }
+  // what the turns have of the same queries together; numbers that are not finite anywhere: these rows again, key by key
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float a, b;
+    swap16(l[i], a, b);
+    swap32(a + b, a, b);
+    l[i] = a + b;
+  }
+  bool bad = odd[0] >= 0x7f80 || odd[1] >= 0x7f80;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    bad |= !(l[i] < INFINITY);
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad |= !(fabsf(o[i][t][e]) < INFINITY);
+  }
+  __syncthreads();
+  if (__any(bad) && lane == 0) again = 1;
+  if constexpr (TURNS > 1) {
+    float *part = (float *)kl + group * 64 * (2 * DT * 4 + 4) + lane;
+    static_assert(GROUPS * 64 * (8 * DT + 4) * 4 <= 3 * PART);
+    if (turn > 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        part[64 * i] = m[i], part[64 * (2 + i)] = l[i];
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part[64 * (4 + (i * DT + t) * 4 + e)] = o[i][t][e];
+      }
+    }
+    __syncthreads();
+    if (turn == 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float m1 = part[64 * i], mx = fmaxf(m[i], m1), f0 = __builtin_amdgcn_exp2f(m[i] - mx), f1 = __builtin_amdgcn_exp2f(m1 - mx);
+        l[i] = l[i] * f0 + part[64 * (2 + i)] * f1;
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[i][t][e] = o[i][t][e] * f0 + part[64 * (4 + (i * DT + t) * 4 + e)] * f1;
+      }
+    }
+  } else {
+    __syncthreads();
+  }
+  if (again) {
+    for (int t = qb + wave; t <= last; t += 4) prefill_row<f32_tag, D>(p, seq, q0 + t, head);
+    return;
+  }
+  if (turn > 0) return;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int at = qb + group * 32 + i * 16 + r16;
+    if (at >= sq) continue;
+    const int64_t token = q0 + at;
+    float *op = (float *)p.out + token * p.out_stride + (int64_t)head * D + 4 * g;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      f32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = l[i] > 0.f ? o[i][t][e] / l[i] * attn_factor<f32_tag>(p.mask, token, head * D + 16 * t + 4 * g + e) : 0.f;
+      *(f32x4 *)(op + 16 * t) = w;
+    }
+  }
+}
+
 // Both kernels' times in ns, as they grew over 1700 shapes (1 .. 400 queries of 1 .. 2000 keys, 4 .. 32 heads, 1 .. 256 sequences): the vector kernel takes
 // 3 us, the walk to the sequence, and 0.11 us a key (twice that at head dim 128) or its reads of K and V, whichever is more; a tile of 64 queries 9 us for
 // the first 64 keys and 4 for each further 64, or what its turns on the chip take.  The other kernel is quicker by more than 5 % in 5 % of them, by 45 % at most.
@@ -338,7 +589,13 @@ int mv_prefill_f32_launch(const PrefillParams &p, bool always, hipStream_t strea
   const bool general = p.block_tables || p.chunk > 0 || p.mask.window > 0 || p.mask.softcap > 0.f;
   const dim3 block(WAVES * 64);
   if (p.head_dim == 64 && general) hipLaunchKernelGGL((prefill_f32_kernel<64, true>), grid, block, 0, stream, p);
-  else if (p.head_dim == 64) hipLaunchKernelGGL((prefill_f32_kernel<64, false>), grid, block, 0, stream, p);
+  else if (p.head_dim == 64) {
+    // 128 queries a workgroup where they fill the chip one and a half times (two a CU).  64 / 128 queries, over 130 shapes: 0.67 .. 1.0 of the time up to 600 workgroups of 128,
+    // 0.88 .. 1.05 up to 768, 0.91 .. 1.09 up to 1100, 1.0 .. 1.2 over that
+    const dim3 wide(p.n_heads, p.n_seqs, (p.max_seqlen_q + 127) / 128);
+    if ((int64_t)wide.x * wide.y * wide.z >= 768) hipLaunchKernelGGL((prefill_parts_kernel<64, 4>), wide, block, 0, stream, p);
+    else hipLaunchKernelGGL((prefill_parts_kernel<64, 2>), grid, block, 0, stream, p);
+  }
   else if (p.head_dim == 128 && general) hipLaunchKernelGGL((prefill_f32_kernel<128, true>), grid, block, 0, stream, p);
   else if (p.head_dim == 128) hipLaunchKernelGGL((prefill_f32_kernel<128, false>), grid, block, 0, stream, p);
   else return MV_E_SHAPE;

@@ -82,6 +82,33 @@ def test_whole_prompts_at_the_edges_of_tiles(H, monkeypatch, lens, d):
     _check(H, monkeypatch, [(n, n) for n in lens], 6, 2, d, sum(lens))
 
 
+def test_many_prompts_at_the_edges_of_tiles(H, monkeypatch):
+    """Enough of them for workgroups of 128 queries (those of 64: above)."""
+    _check(H, monkeypatch, [(n, n) for n in [31, 32, 33, 63, 64, 65, 1, 95, 96, 97, 127, 128, 129, 255, 256, 257]], 32, 8, 64, 11)
+    _check(H, monkeypatch, [(n, n) for n in [5, 128, 90] * 9], 32, 32, 64, 12, sink=True, gate=True)
+
+
+@pytest.mark.parametrize("kw", [dict(sink=True), dict(gate=True), dict(sink=True, gate=True)], ids=str)
+def test_sinks_and_gates_of_whole_prompts(H, monkeypatch, kw):
+    _check(H, monkeypatch, [(150, 150), (20, 20), (65, 65)], 4, 2, 64, 13, **kw)
+
+
+@pytest.mark.parametrize("heads", [2, 400])      # workgroups of 64 queries, of 128
+@pytest.mark.parametrize("what, at, value", [(0, 30, float("inf")), (0, 99, float("nan")), (1, 45, float("inf")), (1, 45, -float("inf")), (1, 0, float("nan")), (1, 64, 3.4e38),
+                                             (0, 3, 3.4e38), (2, 70, 3.4e38), (2, 70, -float("inf"))], ids=str)
+def test_numbers_that_have_no_parts(H, heads, what, at, value):
+    """Infinities, NaN and numbers that bf16 rounds to infinity in q, k or v: as the vector kernel makes of them (its rows are what they go to)."""
+    n = 200
+    rows = [torch.randn(n, heads, 64, generator=torch.Generator().manual_seed(i)).to(DEV) for i in range(3)]
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    call = lambda flags: H.prefill_varlen(*rows, cu, cu, n, n, 0.125, flags=flags)
+    before = call(H.MV_PREFILL_TILES)
+    rows[what][at, 1, 5] = value
+    got, want = call(H.MV_PREFILL_TILES), call(H.MV_PREFILL_SIMPLE)
+    torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-5, equal_nan=True)
+    assert torch.equal(got[:, 0], before[:, 0])      # (the other heads' are not touched)
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("kw", [dict(window=1), dict(window=40, keep=3), dict(window=33, keep=70), dict(chunk=32), dict(chunk=50), dict(cap=2.0),
                                 dict(sink=True), dict(gate=True), dict(window=64, keep=5, cap=3.0, sink=True, gate=True)], ids=str)
