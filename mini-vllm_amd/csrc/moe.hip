@@ -509,7 +509,7 @@ __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
 // rows first): its L2 holds what its workgroups share, and none has more than the others.
 // 36004 pairs of 32 experts, 2048 -> 2 x 768 gated and 768 -> 2048: 343 + 198 us (one workgroup of 256 x 256 to a CU, two stages of 64 inputs, four
 // tiles to an XCD in turn) -> 260 + 157 (rows by half lines, transfers at the start of a stage, tiles looked for one trip to memory behind the other; the layer
-// with all that is beside them 483) -> the layer 460.
+// with all that is beside them 483) -> the layer 449 (460 where 512 tiles are always asked for: the search 2.7 us of a workgroup's 65 -> 1.6).
 constexpr int kWideRows = 128, kWideStages = 3;
 // place of a row's piece among its eight, and the piece at a place: the lanes of a read (four each of different rows) are at different banks
 __device__ __forceinline__ int wide_piece(int row, int piece) { return piece ^ (row >> 1 & 7); }
@@ -526,14 +526,16 @@ __global__ void __launch_bounds__(256, 2) moe_wide_kernel(MoeLinear p, int nx, i
   constexpr int TILES = 16, WM = 8, WN = 4, WSTAGE = TILES * 1024, XSTAGE = WM * 2048;
   extern __shared__ __attribute__((aligned(16))) char smem[];   // three stages of weights, two of rows (64 inputs)
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4;
-  // the halves of a tile of 256 rows that are there: tiles 64 c + lane, all asked for at once (more of them: once more for the one that is looked for)
+  // the halves of a tile of 256 rows that are there: tiles 64 c + lane, all that there may be asked for at once (more than 512: once more for
+  // the one that is looked for)
   constexpr int AHEAD = 8;
   int info[AHEAD][3];
   auto look = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < AHEAD; ++c)
+      if (c == 0 || i0 + 64 * c < max_tiles)
 #pragma unroll
-      for (int q = 0; q < 3; ++q) info[c][q] = p.tiles[3 * min(i0 + 64 * c + lane, max_tiles - 1) + q];
+        for (int q = 0; q < 3; ++q) info[c][q] = p.tiles[3 * min(i0 + 64 * c + lane, max_tiles - 1) + q];
   };
   auto upper_of = [&](int c, int i0) { return __ballot(i0 + 64 * c + lane < max_tiles && info[c][0] >= 0); };
   auto lower_of = [&](int c, int i0) { return __ballot(i0 + 64 * c + lane < max_tiles && info[c][0] >= 0 && info[c][2] > kWideRows); };
@@ -541,7 +543,8 @@ __global__ void __launch_bounds__(256, 2) moe_wide_kernel(MoeLinear p, int nx, i
   for (int i0 = 0; i0 < max_tiles; i0 += 64 * AHEAD) {
     look(held = i0);
 #pragma unroll
-    for (int c = 0; c < AHEAD; ++c) total += __popcll(upper_of(c, i0)) + __popcll(lower_of(c, i0));
+    for (int c = 0; c < AHEAD; ++c)
+      if (c == 0 || i0 + 64 * c < max_tiles) total += __popcll(upper_of(c, i0)) + __popcll(lower_of(c, i0));
   }
   const int per = (total * nx + 7) / 8, turn = blockIdx.x >> 3, index = (blockIdx.x & 7) * per + turn;
   if (turn >= per || index >= total * nx) return;
@@ -551,9 +554,10 @@ __global__ void __launch_bounds__(256, 2) moe_wide_kernel(MoeLinear p, int nx, i
     if (i0 != held) look(held = i0);
 #pragma unroll
     for (int c = 0; c < AHEAD; ++c) {
+      if (nth < 0) break;
       const unsigned long long upper = upper_of(c, i0), lower = lower_of(c, i0);
       const int n = __popcll(upper) + __popcll(lower);
-      if (nth >= 0 && nth < n) {
+      if (nth < n) {
         const unsigned long long below = (1ull << lane) - 1;
         const int ahead = __popcll(upper & below) + __popcll(lower & below);
         const bool second = (lower >> lane & 1) && nth == ahead + 1;
