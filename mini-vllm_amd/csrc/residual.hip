@@ -37,14 +37,17 @@ struct ResidualParams {
 };
 
 template <typename Tag>
-__device__ __forceinline__ void load_row_vec(const typename elem<Tag>::T *p, float (&f)[elem<Tag>::VEC]) {
-  const u32x4 raw = *reinterpret_cast<const u32x4 *>(p);
+__device__ __forceinline__ void unpack_row_vec(u32x4 raw, float (&f)[elem<Tag>::VEC]) {
   if constexpr (elem<Tag>::VEC == 8) {
     unpack8<Tag>(raw, f);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) f[i] = u2f(raw[i]);
   }
+}
+template <typename Tag>
+__device__ __forceinline__ void load_row_vec(const typename elem<Tag>::T *p, float (&f)[elem<Tag>::VEC]) {
+  unpack_row_vec<Tag>(*reinterpret_cast<const u32x4 *>(p), f);
 }
 template <typename Tag>
 __device__ __forceinline__ void store_row_vec(typename elem<Tag>::T *p, const float (&f)[elem<Tag>::VEC]) {
@@ -135,6 +138,7 @@ __device__ __forceinline__ float norm_factors(float (&z)[MAXV][VEC], int cols_tr
   return 1.0f / sqrtf(ss / (float)cols_true + eps);
 }
 
+constexpr int kMoeAhead = 4;   // choices of a token asked for at a time
 // MAXV = vectors per thread
 template <typename Tag, int MAXV, bool LN>
 __global__ void __launch_bounds__(1024) residual_update_kernel(ResidualParams p) {
@@ -181,13 +185,26 @@ __global__ void __launch_bounds__(1024) residual_update_kernel(ResidualParams p)
 #pragma unroll
         for (int j = 0; j < VEC; ++j) e[i][j] += t[j];
       }
-      for (int k = 0; k < p.moe_top; ++k) {
-        const int from = p.moe_rows[(int64_t)row * p.moe_top + k];
-        const float mw = p.moe_w[(int64_t)row * p.moe_top + k];
-        float t[VEC];
-        if (from >= 0) load_row_vec<Tag>((const T *)p.moe_out + (int64_t)from * p.cols + c, t);
+      for (int k0 = 0; k0 < p.moe_top; k0 += kMoeAhead) {   // (places and weights of some choices, then their rows: two trips to memory)
+        int from[kMoeAhead];
+        float mw[kMoeAhead];
+        u32x4 raw[kMoeAhead];
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) y[i][j] = fmaf(mw, from >= 0 ? t[j] : x[i][j], y[i][j]);
+        for (int k = 0; k < kMoeAhead; ++k) {
+          const int64_t at = (int64_t)row * p.moe_top + min(k0 + k, p.moe_top - 1);
+          from[k] = p.moe_rows[at], mw[k] = p.moe_w[at];
+        }
+#pragma unroll
+        for (int k = 0; k < kMoeAhead; ++k)
+          if (k0 + k < p.moe_top && from[k] >= 0) raw[k] = *(const u32x4 *)((const T *)p.moe_out + (int64_t)from[k] * p.cols + c);
+#pragma unroll
+        for (int k = 0; k < kMoeAhead; ++k)
+          if (k0 + k < p.moe_top) {
+            float t[VEC];
+            unpack_row_vec<Tag>(raw[k], t);
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) y[i][j] = fmaf(mw[k], from[k] >= 0 ? t[j] : x[i][j], y[i][j]);
+          }
       }
       if (p.vec) load_row_vec<Tag>((const T *)p.vec + c, vv[i]);
       if (p.norm_w) load_row_vec<Tag>((const T *)p.norm_w + c, wn[i]);
