@@ -130,11 +130,87 @@ __device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c,
   }
 }
 
+// The same of four tokens, 16 lanes each, where a wave has that many: output 16 j + l in register j of lane l; at most 64 outputs and 8 groups.  Bits as of
+// `choose`: the sums run in its order, a tie goes to the lowest output.  9001 tokens, 34 outputs: this end of a workgroup 6.0 us, four tokens at once 2.3
+// (a wave that has one token only: 1.7, at once with three others 2.1).
+template <typename Tag>
+__device__ __forceinline__ void choose_four(const RouteParams &p, const float *s, int64_t token, bool there, const float (&correction)[4]) {
+  const int lane = threadIdx.x & 63, l = lane & 15, R = p.outputs, size = R / p.groups;
+  const bool sigmoid = p.flags & MV_ROUTE_SIGMOID;
+  bool is[4];
+  float v[4], choice[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) is[j] = j * 16 + l < R, v[j] = is[j] ? s[j * 16 + l] : -INFINITY;
+  if (sigmoid) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = 1.0f / (1.0f + expf(-v[j]));
+  } else {
+    const float mx = row16_max(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+    float sum[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = is[j] ? expf(v[j] - mx) : 0.f, sum[j] = row16_sum(v[j]);
+    const float all = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = v[j] / all;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) choice[j] = p.correction ? v[j] + correction[j] : v[j];
+  // the lowest index, among those that may be chosen, of the largest value (a row of NaN: the first of them)
+  auto best_of = [&](const float *x, auto N, unsigned long long free) {
+    constexpr int n = decltype(N)::value;
+    float m = -INFINITY, at = -64.f;
+#pragma unroll
+    for (int j = 0; j < n; ++j) m = fmaxf(m, free >> (j * 16 + l) & 1 ? x[j] : -INFINITY);
+    m = row16_max(m);
+#pragma unroll
+    for (int j = n - 1; j >= 0; --j)
+      if ((free >> (j * 16 + l) & 1) && x[j] == m) at = -(float)(j * 16 + l);
+    const int i = (int)-row16_max(at);
+    return i < 64 ? i : __builtin_ctzll(free);
+  };
+  unsigned long long free = R == 64 ? ~0ull : (1ull << R) - 1;
+  if (p.keep < p.groups) {
+    float best = -INFINITY;   // lane = group
+    for (int g = 0; g < p.groups; ++g) {
+      float m = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) m = fmaxf(m, is[j] && j * 16 + l >= g * size && j * 16 + l < (g + 1) * size ? choice[j] : -INFINITY);
+      m = row16_max(m);
+      if (l == g) best = m;
+    }
+    unsigned long long left = (1ull << p.groups) - 1;
+    free = 0;
+    for (int k = 0; k < p.keep; ++k) {
+      const int g = best_of(&best, std::integral_constant<int, 1>{}, left);
+      left &= ~(1ull << g);
+      free |= (size == 64 ? ~0ull : (1ull << size) - 1) << (g * size);
+    }
+  }
+  int mine[4] = {};   // choice 16 j + l
+  float weight[4] = {}, total = 0.f;
+  for (int k = 0; k < p.top; ++k) {
+    const int at = best_of(choice, std::integral_constant<int, 4>{}, free), j = at >> 4;
+    free &= ~(1ull << at);
+    const float chosen = __shfl(j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3], (lane & 48) + (at & 15), 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i * 16 + l == k) mine[i] = at, weight[i] = chosen;
+    total += chosen;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (there && i * 16 + l < p.top) {
+      p.ids[token * p.top + i * 16 + l] = mine[i];
+      p.weights[token * p.top + i * 16 + l] = (p.flags & MV_ROUTE_RAW ? weight[i] : weight[i] / (total + 1e-20f)) * p.scale;
+    }
+}
+
 // A workgroup: TT tiles of 16 tokens.  Latencies: the inputs are split over the waves, every operand of U steps is asked for before the first is
 // used (16 waves: all of 2048 inputs at once), and the choice of a token with up to 64 outputs stays in one wave's registers.  Few tokens: 16 waves
 // share a tile, so that a wave chooses for one token; many: eight waves (mv_moe_route).  34 outputs of 2048 inputs, alone: 24 tokens 18.8 -> 11.0 us; one
 // launch behind the other, eight waves with a step's loads at a time -> now: 24 tokens 14.7 -> 9.7, 9001 24 -> 16; 128 outputs of 512 inputs: one token
-// 12.7 -> 12.8, 24 20.5 -> 15.4, 20000 53 -> 51; fp32, 34 outputs of 2048 inputs, 4400 tokens: 392 -> 131.
+// 12.7 -> 12.8, 24 20.5 -> 15.4, 20000 53 -> 51; fp32, 34 outputs of 2048 inputs, 4400 tokens: 392 -> 131.  Now 9001 tokens with the choices of four tokens
+// at once, one launch between events, 29.3 -> 24.4: 8.5 of 20 us are the products (their inputs by half lines), 282 workgroups on 256 CUs.
 template <typename Tag, int WAVES, int TT>
 __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
   typedef typename elem<Tag>::T T;
@@ -143,7 +219,11 @@ __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m0 = blockIdx.x * TOKENS, R = p.outputs;
   float *sc = lds, *ch = sc + TOKENS * R;
   const T *x = (const T *)p.x, *w = (const T *)p.w;
-  const float correction = p.correction ? elem<Tag>::ld(((const T *)p.correction)[min(lane, R - 1)]) : 0.f;   // (asked for ahead of the products)
+  constexpr bool FOUR = WAVES < TOKENS;
+  float corrections[4] = {};   // (asked for ahead of the products)
+  if (p.correction)
+#pragma unroll
+    for (int j = 0; j < (FOUR ? 4 : 1); ++j) corrections[j] = elem<Tag>::ld(((const T *)p.correction)[min(FOUR ? j * 16 + (lane & 15) : lane, R - 1)]);
   if constexpr (__is_same(Tag, f32_tag)) {
     const int l = tid & 15;
     for (int i = tid >> 4; i < TOKENS * R; i += WAVES * 4) {
@@ -222,7 +302,11 @@ __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
     }
   }
   __syncthreads();
-  for (int t = wave; t < TOKENS && m0 + t < p.rows; t += WAVES) choose<Tag>(p, sc + t * R, ch + t * R, m0 + t, correction);   // (no barrier in it)
+  if (FOUR && R <= 64 && p.groups <= 8) {
+    for (int t = wave * 4 + (lane >> 4); t < TOKENS; t += WAVES * 4) choose_four<Tag>(p, sc + t * R, m0 + t, m0 + t < p.rows, corrections);
+    return;
+  }
+  for (int t = wave; t < TOKENS && m0 + t < p.rows; t += WAVES) choose<Tag>(p, sc + t * R, ch + t * R, m0 + t, corrections[0]);   // (no barrier in it)
 }
 
 // ---- grouping.  Workgroup (e, part): the pairs of expert e, which start behind those of the experts before it.  Each wave walks a run of all

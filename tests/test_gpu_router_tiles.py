@@ -62,3 +62,18 @@ def test_equal_and_undefined_scores(H, rows, outputs, groups):
     ids, _ = H.moe_route(x, w, None, 8, groups, groups)
     assert ids.min() >= 0 and ids.max() < outputs
     assert torch.equal(ids[::3], torch.arange(8, device=DEV, dtype=torch.int32).expand(len(ids[::3]), 8))
+
+
+@pytest.mark.parametrize("outputs, top, groups, keep", [(1, 1, 1, 1), (16, 16, 1, 1), (34, 4, 2, 1), (49, 20, 7, 6), (64, 33, 8, 5)])
+@pytest.mark.parametrize("dtype, sigmoid", [(torch.bfloat16, False), (torch.float16, True), (torch.float32, False)])
+def test_four_tokens_choose_as_one(H, outputs, top, groups, keep, dtype, sigmoid):
+    """Many tokens choose four at once, few one by one: with exact logits the bits are the same, NaN among them or not."""
+    g = torch.Generator().manual_seed(outputs)
+    x = torch.randint(-1, 2, (4099, 64), generator=g).to(DEV, dtype)
+    x[5::7] = float("nan")
+    w = (torch.randint(-4, 5, (outputs, 64), generator=g) / 8).to(DEV, dtype)
+    corr = torch.randn(outputs, generator=g).to(DEV, dtype)
+    ids, weights = H.moe_route(x, w, corr, top, groups, keep, 1.5, sigmoid=sigmoid)
+    for rows in (slice(0, 37), slice(4060, 4099)):
+        few, few_weights = H.moe_route(x[rows], w, corr, top, groups, keep, 1.5, sigmoid=sigmoid)
+        assert torch.equal(few, ids[rows]) and torch.equal(few_weights.view(torch.int32), weights[rows].view(torch.int32))
