@@ -38,44 +38,72 @@ __global__ void __launch_bounds__(256) split_f32_kernel(Split q) {
     if (i < p.count && (int)blockIdx.x >= q.first[i]) m = i;
   const int k = p.k[m], rows = p.rows[m], spans = (k + kSpan - 1) / kSpan, at = blockIdx.x - q.first[m], row0 = at / spans * 16, k0 = at % spans * kSpan;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  auto row_of = [&](int r) { return (const float *)p.src[m] + (int64_t)min(row0 + r, rows - 1) * p.stride[m]; };   // (rows behind the end repeat the last one)
-  const bool norm = m == 0 && p.norm_w;
-  __shared__ float mean_of[16], scale_of[16];
-  if (norm) {   // 16 lanes a row, its sums twice: of the numbers, of the squares of what they are off the mean
-    const float *src = row_of(tid >> 4);
-    float sum = 0.f, square = 0.f;
-    for (int i = (tid & 15) * 4; i < k; i += 64) {
-      const f32x4 v = *(const f32x4 *)(src + i);
-      sum += (v[0] + v[1]) + (v[2] + v[3]);
-    }
-    const float mean = lanes_sum<16>(sum) / (float)k;
-    for (int i = (tid & 15) * 4; i < k; i += 64) {
-      const f32x4 v = *(const f32x4 *)(src + i) - mean;
-      square += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-    }
-    square = lanes_sum<16>(square);
-    if ((tid & 15) == 0) mean_of[tid >> 4] = mean, scale_of[tid >> 4] = 1.f / sqrtf(square / (float)k + p.eps);
-    __syncthreads();
-  }
-  const float *src = row_of(lane >> 2);
-  const float mean = norm ? mean_of[lane >> 2] : 0.f, scale = norm ? scale_of[lane >> 2] : 1.f;
-  for (int t = wave; t < min(kSpan, k - k0) / 32; t += 4) {   // a wave takes 16 rows x 32 inputs, four lanes a row
-    const int i = k0 + t * 32 + (lane & 3) * 8;
-    f32x4 v[2] = {*(const f32x4 *)(src + i), *(const f32x4 *)(src + i + 4)};
-    if (norm)
+  // A wave takes 16 rows x 32 inputs at a time, four lanes a row, and holds all that it takes of the span; rows behind the end repeat the last one.
+  constexpr int TAKES = kSpan / 128;
+  const float *src = (const float *)p.src[m] + (int64_t)min(row0 + (lane >> 2), rows - 1) * p.stride[m] + (lane & 3) * 8;
+  f32x4 v[TAKES][2];
+  auto load = [&](int from) {   // takes of the span at `from` that are there
+    const int takes = (min(kSpan, k - from) / 32 - wave + 3) / 4;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const f32x4 w = *(const f32x4 *)((const float *)p.norm_w + i + 4 * h), b = p.norm_b ? *(const f32x4 *)((const float *)p.norm_b + i + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int n = 0; n < 4; ++n) v[h][n] = fmaf((v[h][n] - mean) * scale, w[n], b[n]);
+    for (int t = 0; t < TAKES; ++t)
+      if (t < takes) {
+        const float *at = src + from + (t * 4 + wave) * 32;
+        v[t][0] = *(const f32x4 *)at, v[t][1] = *(const f32x4 *)(at + 4);
       }
-    float f[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
-    u32x4 part[3];
-    split3<true>(f, part);
-    u32x4 *to = (u32x4 *)p.dst[m] + part_place(row0 + (lane >> 2), i >> 3, k);
+    return takes;
+  };
+  const bool norm = m == 0 && p.norm_w;
+  float mean = 0.f, scale = 1.f;
+  int takes;
+  if (norm) {   // a row's sums, over its four lanes and the waves: of the numbers, of the squares of what they are off the mean
+    __shared__ float sums[2][4][16];
+    auto sum_of = [&](float x, int which) {
+      x = lanes_sum<4>(x);
+      if ((lane & 3) == 0) sums[which][wave][lane >> 2] = x;
+      __syncthreads();
+      return (sums[which][0][lane >> 2] + sums[which][1][lane >> 2]) + (sums[which][2][lane >> 2] + sums[which][3][lane >> 2]);
+    };
+    float sum = 0.f, square = 0.f;
+    for (int i = 1; i <= spans; ++i) {   // (the own span last, which stays)
+      takes = load((k0 / kSpan + i) % spans * kSpan);
 #pragma unroll
-    for (int s = 0; s < 3; ++s) to[64 * s] = part[s];
+      for (int t = 0; t < TAKES; ++t)
+        if (t < takes) {
+          const f32x4 both = v[t][0] + v[t][1];
+          sum += (both[0] + both[1]) + (both[2] + both[3]);
+        }
+    }
+    mean = sum_of(sum, 0) / (float)k;
+    for (int i = 0; i < spans; ++i) {
+      if (i) takes = load((k0 / kSpan + i) % spans * kSpan);
+#pragma unroll
+      for (int t = 0; t < TAKES; ++t)
+        if (t < takes) {
+          const f32x4 a = v[t][0] - mean, b = v[t][1] - mean, both = a * a + b * b;
+          square += (both[0] + both[1]) + (both[2] + both[3]);
+        }
+    }
+    scale = 1.f / sqrtf(sum_of(square, 1) / (float)k + p.eps);
   }
+  if (!norm || spans > 1) takes = load(k0);
+#pragma unroll
+  for (int t = 0; t < TAKES; ++t)
+    if (t < takes) {
+      const int i = k0 + (t * 4 + wave) * 32 + (lane & 3) * 8;
+      if (norm)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 w = *(const f32x4 *)((const float *)p.norm_w + i + 4 * h), b = p.norm_b ? *(const f32x4 *)((const float *)p.norm_b + i + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int n = 0; n < 4; ++n) v[t][h][n] = fmaf((v[t][h][n] - mean) * scale, w[n], b[n]);
+        }
+      float f[8] = {v[t][0][0], v[t][0][1], v[t][0][2], v[t][0][3], v[t][1][0], v[t][1][1], v[t][1][2], v[t][1][3]};
+      u32x4 part[3];
+      split3<true>(f, part);
+      u32x4 *to = (u32x4 *)p.dst[m] + part_place(row0 + (lane >> 2), i >> 3, k);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) to[64 * s] = part[s];
+    }
 }
 
 constexpr int kSlots = 5;   // (of 16 KiB: two workgroups fill a CU)
