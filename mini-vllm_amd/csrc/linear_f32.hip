@@ -12,9 +12,10 @@
 // Bound by power: at 128 x 128 outputs a workgroup, two a CU, the matrix cores are busy 85 % of the time, at 1.6 GHz of 2.4 (operands of zeros: 2.3).  Hence
 // 16 x 16 x 32 instructions: in registers alone they reach 2010 TFLOP/s at 2.0 GHz where 32 x 32 x 16 reach 1770 at 1.76 (of zeros both 2450), here
 // 168 us -> 149.  LDS holds five stages of one part of 32 inputs; transfers are asked for between products (all at the start of a stage: 183 us, as waves
-// stand still until theirs are taken).  Tiles of 64 x 64, four a CU, where there are not enough of the larger ones.
-// us, library / this, with parts made of both operands: 6470 rows of 768 -> 2304 202 / 126, 768 -> 768 85 / 58, 768 -> 3072 279 / 163, 3072 -> 768 231 / 195;
-// 1300 rows of 768 -> 3072 53 / 46; 8000 of 2048 -> 12288 2772 / 1715.
+// stand still until theirs are taken).  Tiles of 64 x 64, six a CU with three stages each (parts written: five, four), where there are not enough of the larger ones
+// (four with five stages: 768 inputs to 768 outputs, 6470 rows 48 us where this takes 44, 3072 to 768 174, 158; tiles of 64 x 128, three a CU 47, 162).
+// us, library / this, with parts made of both operands: 6470 rows of 768 -> 2304 203 / 128, 768 -> 768 88 / 54, 768 -> 3072 280 / 166, 3072 -> 768 233 / 184;
+// 1300 rows of 768 -> 3072 56 / 47; 8000 of 2048 -> 12288 2772 / 1715.
 #include <algorithm>
 
 #include "parts.h"
@@ -106,10 +107,11 @@ __global__ void __launch_bounds__(256) split_f32_kernel(Split q) {
     }
 }
 
-constexpr int kSlots = 5;   // (of 16 KiB: two workgroups fill a CU)
-template <int XT, int WT, bool PARTS>   // 32 XT rows x 32 WT outputs of 2 x 2 waves
-__global__ void __launch_bounds__(256, 2) linear_f32_kernel(MvLinearF32Args p, int mt, int nt) {
-  constexpr int PIECES = 2 * (XT + WT), PER = PIECES / 4, STAGE = PIECES * 1024;   // fragments of 1 KiB; of a wave
+// 32 XT rows x 32 WT outputs of 2 x 2 waves; workgroups of a CU; stages in LDS
+template <int XT, int WT, int BESIDE, int SLOTS, bool PARTS>
+__global__ void __launch_bounds__(256, BESIDE) linear_f32_kernel(MvLinearF32Args p, int mt, int nt) {
+  constexpr int PIECES = 2 * (XT + WT), PER = PIECES / 4, STAGE = PIECES * 1024, kSlots = SLOTS;   // PIECES: fragments of 1 KiB; PER: of a wave
+  static_assert(PIECES % 4 == 0 && PER <= WT);
   extern __shared__ __attribute__((aligned(16))) char smem[];   // stages of one part of 32 inputs: rows [2 XT] | weights [2 WT]
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g = lane >> 4, wm = wave & 1, wn = wave >> 1;
   const int id = blockIdx.x, more = gridDim.x & 7, at = (id & 7) * (gridDim.x >> 3) + min(id & 7, more) + (id >> 3);
@@ -231,12 +233,13 @@ __global__ void __launch_bounds__(256, 2) linear_f32_kernel(MvLinearF32Args p, i
   }
 }
 
-template <int XT, int WT, bool PARTS>
+template <int XT, int WT, int BESIDE, int SLOTS, bool PARTS>
 int launch(const MvLinearF32Args &p, hipStream_t st) {
   const int64_t mt = ((int64_t)p.rows + 32 * XT - 1) / (32 * XT), nt = ((int64_t)p.n + 32 * WT - 1) / (32 * WT);
   if (mt * nt > 0x7fffffff) return MV_E_SHAPE;
-  if (int rc = mv_allow_lds<linear_f32_kernel<XT, WT, PARTS>>()) return rc;
-  hipLaunchKernelGGL((linear_f32_kernel<XT, WT, PARTS>), dim3((unsigned)(mt * nt)), dim3(256), kSlots * (XT + WT) * 2048, st, p, (int)mt, (int)nt);
+  if (int rc = mv_allow_lds<linear_f32_kernel<XT, WT, BESIDE, SLOTS, PARTS>>()) return rc;
+  constexpr int lds = SLOTS * (XT + WT) * 2048;
+  hipLaunchKernelGGL((linear_f32_kernel<XT, WT, BESIDE, SLOTS, PARTS>), dim3((unsigned)(mt * nt)), dim3(256), lds, st, p, (int)mt, (int)nt);
   MV_LAUNCH_CHECK();
   return MV_OK;
 }
@@ -275,10 +278,11 @@ extern "C" int mv_linear_f32(const MvLinearF32Args *a, void *stream) {
       (!a->parts_out && (a->out_stride & 3)) || (a->residual && (a->residual_stride & 3)))
     return MV_E_ALIGN;
   hipStream_t st = (hipStream_t)stream;
-  // 512 tiles of 128 x 128 run at a time.  us, 64 x 64 / 128 x 128: 378 tiles 51 / 56, 384 52 / 56, 416 of 2048 inputs 142 / 141, 468 65 / 58, 504 66 / 60;
-  // a second round for few is lost: 528 529 / 584, 576 182 / 204, 594 79 / 86, 624 81 / 86; 640 621 / 596, 672 225 / 217, 720 95 / 89, 792 102 / 106, 960 122 / 114
+  // 512 tiles of 128 x 128 run at a time: those where their last round is well filled, or there are many.  us, 64 x 64 / 128 x 128, by tiles of 128 x 128:
+  // 384 52 / 60, 416 of 2048 inputs 144 / 147 and 146 / 142, 468 65 / 62, 504 66 / 64, 594 80 / 89, 624 82 / 90, 720 95 / 96, 792 103 / 113, 832 265 / 277, 918 118 / 116,
+  // 960 120 / 119, 1008 324 / 300, 1056 343 / 339 and 321 / 337, 1134 147 / 148, 1224 155 / 151, 1280 400 / 363, 1422 180 / 176, 2016 638 / 571
   const int64_t wide = (((int64_t)a->rows + 127) / 128) * (((int64_t)a->n + 127) / 128);
-  const bool large = a->tile == 1 || (a->tile == 0 && wide >= 400 && (wide <= 512 || wide >= 640));
-  if (large) return a->parts_out ? launch<4, 4, true>(*a, st) : launch<4, 4, false>(*a, st);
-  return a->parts_out ? launch<2, 2, true>(*a, st) : launch<2, 2, false>(*a, st);
+  const bool large = a->tile == 1 || (a->tile == 0 && (wide >= 1150 || wide * 100 >= (wide + 511) / 512 * 512 * 85));
+  if (large) return a->parts_out ? launch<4, 4, 2, 5, true>(*a, st) : launch<4, 4, 2, 5, false>(*a, st);
+  return a->parts_out ? launch<2, 2, 5, 4, true>(*a, st) : launch<2, 2, 6, 3, false>(*a, st);
 }
