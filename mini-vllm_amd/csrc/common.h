@@ -218,6 +218,21 @@ __device__ __forceinline__ float clamped_glu(float gate, float up, float limit, 
   return g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
 }
 
+// a / (1 + exp(-a)), `a` a number of the dtype, to be rounded to it.  bf16: a power of two whose exponent is exact (log2(e) in 16 bits and the rest of it),
+// a hardware exponential and reciprocal, 13 instructions where the division takes 30: for all 65536 numbers the same bits.  (The factor of both sides of the
+// quotient keeps its reciprocal a normal number; of the factors that do, this is one with which no number rounds the other way.)
+template <typename Tag>
+__device__ __forceinline__ float silu_of_dtype(float a) {
+  if constexpr (__is_same(Tag, bf16_tag)) {
+    constexpr double LOG2E = 1.4426950408889634, LN2 = 0.6931471805599453;
+    constexpr float HIGH = 0x1.7154p+0f, LOW = (float)(-(LOG2E - (double)HIGH) * LN2), FACTOR = 0.1875f;
+    const float e = __builtin_amdgcn_exp2f(-HIGH * a), rest = __builtin_amdgcn_fmed3f(LOW * a, -0.01f, 0.01f);   // (|a| < 2048, or e is 0 or infinite)
+    return (FACTOR * a) * __builtin_amdgcn_rcpf(fmaf(FACTOR, fmaf(e, rest, e), FACTOR));
+  } else {
+    return a / (1.0f + expf(-a));
+  }
+}
+
 // act(gate) * up on the fp32 accumulators of a gated projection.  gelu, clamped, relu: fp32 throughout.  silu: the rounding points
 // of the unfused pair (GEMM -> dtype, silu -> dtype, product in fp32; the caller rounds it)
 template <typename Tag>
@@ -226,8 +241,7 @@ __device__ __forceinline__ float gated_act(float gate, float up, const MvGateAct
   if (a.kind == MV_ACT_CLAMPED) return clamped_glu(gate, up, a.limit, a.alpha);
   if (a.kind == MV_ACT_RELU) return __fmul_rn(fmaxf(gate, 0.f), up);
   const float gt = elem<Tag>::ld(elem<Tag>::st(gate)), ut = elem<Tag>::ld(elem<Tag>::st(up));
-  float sl = gt / (1.0f + expf(-gt));                        // rmsnorm.hip: silu_and_mul_kernel
-  sl = elem<Tag>::ld(elem<Tag>::st(sl));
+  const float sl = elem<Tag>::ld(elem<Tag>::st(silu_of_dtype<Tag>(gt)));   // rmsnorm.hip: silu_and_mul_kernel
   return __fmul_rn(sl, ut);
 }
 

@@ -246,8 +246,7 @@ silu_and_mul_kernel(const typename elem<Tag>::T *__restrict__ x, int64_t x_strid
             } else if constexpr (ACT == MV_ACT_RELU) {
               y[j] = __fmul_rn(fmaxf(a[u][j], 0.f), b[u][j]);
             } else {
-              float s = a[u][j] / (1.0f + expf(-a[u][j]));
-              s = elem<Tag>::ld(elem<Tag>::st(s));
+              const float s = elem<Tag>::ld(elem<Tag>::st(silu_of_dtype<Tag>(a[u][j])));
               y[j] = __fmul_rn(s, b[u][j]);
             }
           }
