@@ -209,7 +209,7 @@ extern "C" int mv_add_rmsnorm_partial(const float *partial, int splits, void *re
 template <typename Tag, int ACT>
 __global__ void __launch_bounds__(256)
 silu_and_mul_kernel(const typename elem<Tag>::T *__restrict__ x, int64_t x_stride,
-                    typename elem<Tag>::T *__restrict__ out, int64_t out_stride, int rows, int cols, MvGateAct act) {
+                    typename elem<Tag>::T *__restrict__ out, int64_t out_stride, int rows, int cols, MvGateAct act, bool far) {
   constexpr int VEC = elem<Tag>::VEC;
   constexpr int U = 4;   // vectors per thread and trip: 2 U loads in flight before the first exp (prefill rows: 4.3 -> TB/s)
   const int nvec = cols / VEC;
@@ -250,7 +250,11 @@ silu_and_mul_kernel(const typename elem<Tag>::T *__restrict__ x, int64_t x_strid
               y[j] = __fmul_rn(s, b[u][j]);
             }
           }
-          store_vec<Tag>(orow + c * VEC, y);
+          u32x4 o;
+          if constexpr (VEC == 8) o = pack8<Tag>(y);
+          else o = u32x4{f2u(y[0]), f2u(y[1]), f2u(y[2]), f2u(y[3])};
+          if (far) __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(orow + c * VEC));
+          else *reinterpret_cast<u32x4 *>(orow + c * VEC) = o;
         }
       }
     }
@@ -269,14 +273,15 @@ static int act_and_mul(const void *x, int64_t x_stride, void *out, int64_t out_s
     constexpr int VEC = elem<Tag>::VEC;
     if (cols % VEC) return MV_E_SHAPE;
     if ((x_stride % VEC) || (out_stride % VEC)) return MV_E_ALIGN;
-    // x: workgroups along a row (4 vectors per thread and trip), y: rows; ~2048+ workgroups in flight, 65535 at most
+    // x: workgroups along a row (4 vectors per thread and trip), y: rows
     const int nvec = cols / VEC;
-    int bx = (nvec + 256 * 4 - 1) / (256 * 4);
-    if (bx < 1) bx = 1;
-    int by = rows < 65535 ? rows : 65535;
-    while ((int64_t)bx * by > 16384 && by > 1) by = (by + 1) / 2;
+    const int bx = (nvec + 256 * 4 - 1) / (256 * 4);
+    const int by = rows < 65535 ? rows : 65535;
+    // Results that the last cache (256 MB) has no room for go past it, from 300 MiB on.  us, bf16, with / past it: 12000 x 11008 (264 MB) 120 / 138, 8000 x 18944 (303 MB) 158 / 146,
+    // 20000 x 11008 (440 MB) 245 / 231, 25672 x 18944 (973 MB) 545 / 482.  A workgroup a row: that one 571, 535 with eight rows behind each other.
+    const bool far = (int64_t)rows * cols * (int64_t)sizeof(T) > (int64_t)300 << 20;
     hipLaunchKernelGGL((silu_and_mul_kernel<Tag, ACT>), dim3((unsigned)bx, (unsigned)by), dim3(256), 0,
-                       (hipStream_t)stream, (const T *)x, x_stride, (T *)out, out_stride, rows, cols, act);
+                       (hipStream_t)stream, (const T *)x, x_stride, (T *)out, out_stride, rows, cols, act, far);
   });
   MV_LAUNCH_CHECK();
   return MV_OK;

@@ -22,3 +22,15 @@ def test_silu_of_every_number(dtype):
     assert (off <= (0.5 * torch.finfo(dtype).eps * 2.0 ** torch.floor(torch.log2(want.abs().clamp_min(1e-300)))) * (1 + 2**-12) + 4 * tiny)[finite & (x > -88.7)].all()
     assert (up[finite & (x < -88.75)] == 0).all()
     assert y[x == torch.inf] == torch.inf and torch.isnan(y[torch.isnan(x)]).all() and torch.isnan(y[x == -torch.inf]).all()
+
+
+@pytest.mark.parametrize("rows, cols", [(153593, 1024), (65537, 2400), (19200, 8200)])
+def test_results_that_go_past_the_last_cache(rows, cols):
+    """More rows than a grid has, rows that the workgroups' vectors leave ragged, results around 300 MiB: each row is that of a few rows alone."""
+    from minivllm_amd import hip_ops as H
+
+    g = torch.Generator(device="cuda:0").manual_seed(cols)
+    x = torch.randn(rows, 2 * cols, device="cuda:0", generator=g, dtype=torch.bfloat16)
+    y = H.silu_and_mul(x)
+    for at in (0, 40000 if rows > 65536 else 7000, rows - 64):
+        assert torch.equal(y[at:at + 64], H.silu_and_mul(x[at:at + 64]))
