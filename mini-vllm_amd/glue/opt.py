@@ -68,12 +68,15 @@ class OPTDecoderLayer(nn.Module):
         self.fc1 = ColumnParallelLinear(d, config.ffn_dim, bias=config.enable_bias)
         self.fc2 = RowParallelLinear(config.ffn_dim, d, bias=config.enable_bias)
         self.final_layer_norm = nn.LayerNorm(d)
+        self.parts_rows = (-(-F32_LAYER_TILES_MIN // -(-d // 64)) - 1) * 64 + 1   # the fewest rows of F32_LAYER_TILES_MIN tiles
 
     def _by_parts(self, x) -> bool:
+        if x.shape[0] < self.parts_rows or x.dtype != torch.float32:   # (small steps are bound by the host: nothing else is looked at)
+            return False
         att = self.self_attn
         linears, norms = (att.qkv_proj, att.out_proj, self.fc1, self.fc2), (self.self_attn_layer_norm, self.final_layer_norm)
-        return (x.dtype == torch.float32 and self.do_layer_norm_before and f32_tiles(x.shape[0], x.shape[1]) >= F32_LAYER_TILES_MIN
-                and all(lin.tp_size == 1 for lin in linears) and not any(m._forward_hooks or m._forward_pre_hooks for m in (*linears, *norms, att))
+        return (self.do_layer_norm_before and f32_tiles(x.shape[0], x.shape[1]) >= F32_LAYER_TILES_MIN and all(lin.tp_size == 1 for lin in linears)
+                and not any(m._forward_hooks or m._forward_pre_hooks for m in (*linears, *norms, att))
                 and hip_ops.linear_f32_ok(x, *(t for m in (*linears, *norms) for t in (m.weight, m.bias))))
 
     def _forward_parts(self, x):
