@@ -836,7 +836,8 @@ typedef struct MvBlockLinearArgs {
 } MvBlockLinearArgs;
 int mv_block_linear(const MvBlockLinearArgs *args, int dtype, void *stream);
 
-/* ---- K21 — fp32 projections from operands in parts: each number as three of bf16 that add up to it, [16 rows][32 columns][part][8 columns of 4][row][8].
+/* ---- K21 — fp32 projections from operands in parts: each number as three of bf16 that add up to it (below 2^-109, where three do not: the upper
+ * and the lower half of its own bits and a NaN), [16 rows][32 columns][part][8 columns of 4][row][8].
  * mv_split_f32: up to MV_SPLIT_F32_MAX matrices [rows][k] of fp32, k a multiple of 32, rows `stride` apart (a multiple of 4); dst of
  * mv_split_f32_bytes(rows, k) bytes; norm_w (NULL: none), norm_b (may be NULL): a LayerNorm over the k columns of the first matrix, in front.
  * mv_linear_f32: out[rows][n] = x[rows][k] w[n][k]^T + bias[n] (may be NULL), no less than 0 if `relu`, + residual[rows][n] (may be NULL); fp32, or with

@@ -1,7 +1,9 @@
 // K21 — fp32 projections on the 16-bit matrix cores: out = max(x W^T + bias, 0) + residual, operands in parts.
 //
-// A number of fp32 is the sum of three of bf16 (24 bits of significand), and a product is the six of its parts' products that matter: what is left out
-// is 2^-24 of it at the most.  A product of parts is exact and sums are fp32, those of the first parts apart from the rest, so that the rest's
+// A number of fp32 from 2^-109 on is the sum of three of bf16 (24 bits of significand), and a product is the six of its parts' products that matter: what is
+// left out is 2^-24 of it at the most.  Smaller numbers that are not (bf16 ends at 2^-133) go as their own 32 bits beside a NaN (parts.h), and fragments with results that
+// are not finite are made once more from the numbers by fp32 matrix instructions: 6470 rows of 768 -> 3072, parts and product, us: 180 (library 301), one such number in
+// x, or a NaN, 303, an output all of whose weights are 218, an input whose weights all are 1106.  A product of parts is exact and sums are fp32, those of the first parts apart from the rest, so that the rest's
 // roundings do not count; a matrix instruction adds 32 products at once.  Distance from 64 bits, relative, unit normal inputs: 768 inputs 1.6e-7 (library: 5.0e-7,
 // few rows 2.5e-7), 3072 that are not negative 2.7e-7 (6.9e-7, 3.5e-7).  Six bf16 products take less time than one of fp32 (a sixteenth of the rate).
 //
@@ -170,23 +172,23 @@ __global__ void __launch_bounds__(256, BESIDE) linear_f32_kernel(MvLinearF32Args
   constexpr int COLS = WT * 16, ROW = COLS * 4 + 16;   // a wave's outputs; bytes of a row of them in LDS
   char *const tile = smem + wave * (32 * ROW);
   const int first = (ni * 2 + wn) * COLS;
-  // a number whose products are not finite: once more, from what the parts add up to
-  auto again = [&](int row, int n) {
-    const u32x4 *xr = (const u32x4 *)p.x + part_place(row, 0, p.k), *wr = (const u32x4 *)p.w + part_place(n, 0, p.k);
-    float sum = 0.f;
-    for (int k = 0; k < p.k; k += 8, xr += k & 24 ? 16 : 144, wr += k & 24 ? 16 : 144) {
-      float a[3][8], b[3][8];
+  // A fragment of 16 rows x 16 outputs some of whose products are not finite, once more by fp32 matrix instructions from the numbers themselves
+  auto again = [&](int i, int j) {
+    const char *xr = (const char *)p.x + (int64_t)min(mi * 2 * XT + wm * XT + i, last_x) * stages * 1024 + lane * 16;
+    const char *wr = (const char *)p.w + (int64_t)min(ni * 2 * WT + wn * WT + j, last_w) * stages * 1024 + lane * 16;
+    f32x4 sum[2] = {};
+    for (int s = 0; s < stages; s += 3, xr += 3072, wr += 3072) {
+      u32x4 xp[3], wp[3];
 #pragma unroll
-      for (int s = 0; s < 3; ++s) unpack8<bf16_tag>(xr[64 * s], a[s]), unpack8<bf16_tag>(wr[64 * s], b[s]);
+      for (int q = 0; q < 3; ++q) xp[q] = *(const u32x4 *)(xr + q * 1024), wp[q] = *(const u32x4 *)(wr + q * 1024);
+      float xn[8], wn[8];
+      joined8(xp, xn), joined8(wp, wn);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) sum = fmaf(a[0][i] + (a[1][i] + a[2][i]), b[0][i] + (b[1][i] + b[2][i]), sum);
+      for (int q = 0; q < 8; ++q) sum[q & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(wn[q], xn[q], sum[q & 1], 0, 0, 0);
     }
-    return sum;
+    return sum[0] + sum[1];
   };
-  auto finish = [&](f32x4 v, int row, int n) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (!(fabsf(v[q]) < INFINITY)) v[q] = again(row, n + q);
+  auto finish = [&](f32x4 v, int n) __attribute__((always_inline)) {
     if (p.bias) v += *(const f32x4 *)((const float *)p.bias + n);
     if (p.relu) {
 #pragma unroll
@@ -196,20 +198,37 @@ __global__ void __launch_bounds__(256, BESIDE) linear_f32_kernel(MvLinearF32Args
   };
 #pragma unroll
   for (int i = 0; i < XT; i += 2) {   // 32 rows at a time
+    uint32_t odd = 0;   // fragments that have a number that is not finite
 #pragma unroll
     for (int j = 0; j < WT; ++j)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) *(f32x4 *)(tile + (h * 16 + r16) * ROW + j * 64 + g * 16) = acc[j][i + h] + low[j][i + h];
+      for (int h = 0; h < 2; ++h) {
+        const f32x4 v = acc[j][i + h] + low[j][i + h];
+        *(f32x4 *)(tile + (h * 16 + r16) * ROW + j * 64 + g * 16) = v;
+        uint32_t largest = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) largest = max(largest, f2u(v[q]) & 0x7fffffffu);
+        if (__any(largest >= 0x7f800000u)) odd |= 1u << (2 * j + h);
+      }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    for (; odd; odd &= odd - 1) {
+      const int at = __builtin_ctz(odd), h = at & 1, j = at >> 1;
+      const f32x4 sum = again(i + h, j);
+      f32x4 *const of = (f32x4 *)(tile + (h * 16 + r16) * ROW + j * 64 + g * 16);
+      f32x4 v = *of;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[q] = fabsf(v[q]) < INFINITY ? v[q] : sum[q];
+      *of = v;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
     const int row0 = (mi * 2 + wm) * XT * 16 + i * 16;
     if constexpr (PARTS) {
 #pragma unroll
       for (int r = 0; r < COLS / 16; ++r) {   // 16 rows x 32 outputs
         const int in_tile = r / (COLS / 32) * 16 + r16, row = row0 + in_tile, at = r % (COLS / 32) * 32 + g * 8, n = first + at;
         const float *from = (const float *)(tile + in_tile * ROW) + at;
-        if (row - r16 >= p.rows || n >= p.n) continue;
-        const int live = min(row, p.rows - 1);   // (rows behind the end, up to a whole tile, repeat what is there: nobody's results depend on them)
-        f32x4 a = finish(*(const f32x4 *)from, live, n), b = finish(*(const f32x4 *)(from + 4), live, n + 4);
+        if (row - r16 >= p.rows || n >= p.n) continue;   // (rows behind the end, up to a whole tile, are written too: nobody's results depend on them)
+        f32x4 a = finish(*(const f32x4 *)from, n), b = finish(*(const f32x4 *)(from + 4), n + 4);
         float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
         u32x4 part[3];
         split3<true>(f, part);
@@ -224,7 +243,7 @@ __global__ void __launch_bounds__(256, BESIDE) linear_f32_kernel(MvLinearF32Args
       for (int r = 0; r < 32 * LINE / 64; ++r) {
         const int in_tile = r * (64 / LINE) + lane / LINE, row = row0 + in_tile;
         if (row >= p.rows || n >= p.n) continue;
-        f32x4 v = finish(*(const f32x4 *)(tile + in_tile * ROW + lane % LINE * 16), row, n);
+        f32x4 v = finish(*(const f32x4 *)(tile + in_tile * ROW + lane % LINE * 16), n);
         if (p.residual) v += *(const f32x4 *)((const float *)p.residual + (int64_t)row * p.residual_stride + n);
         *(f32x4 *)((float *)p.out + (int64_t)row * p.out_stride + n) = v;
       }

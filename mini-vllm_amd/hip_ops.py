@@ -1028,7 +1028,7 @@ MvLinearF32Args = _struct(
 
 
 class F32Parts(NamedTuple):
-    """A matrix [rows, k] of fp32 numbers, each as three of bf16 (mv_split_f32)."""
+    """A matrix [rows, k] of fp32 numbers, each in three of bf16 (mv_split_f32)."""
     data: torch.Tensor
     rows: int
     k: int

@@ -36,6 +36,56 @@ def test_parts_add_up(rows, k):
     assert (_sum_of_parts(a) - want).abs().max() <= 2e-6
 
 
+def _numbers(p):
+    """What the parts stand for: their sum, or where the third is NaN the bits of the first and second."""
+    q = p.data.view(torch.int16).view(-1, p.k // 32, 3, 4, 16, 8).permute(0, 4, 1, 3, 5, 2).reshape(-1, p.k, 3)[:p.rows].contiguous()
+    bits = (q[..., 0].int() << 16) | (q[..., 1].int() & 0xffff)
+    parts = q.view(torch.bfloat16)
+    return torch.where(parts[..., 2].isnan(), bits.view(torch.float32).double(), parts.double().sum(-1))
+
+
+def test_small_numbers_keep_their_bits():
+    """Down to the smallest of fp32, also where bf16 has no number for the last of their bits."""
+    from minivllm_amd import hip_ops as H
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = _randn(g, 48, 1056) * 2.0 ** torch.arange(-150, -102, device=DEV).double()[:, None]
+    x = x.float()
+    x[:, 7] = 1.0
+    x[20, 8:40], x[21, 8:40] = 0.0, torch.finfo(torch.float32).tiny
+    assert torch.equal(_numbers(H.split_f32(x)[0]), x.double())
+
+
+def _chain_bound(x, w, y):
+    # a chain of sums of four products, each rounded at its size; below 2^-126 each product and sum at 2^-149
+    k = x.shape[1]
+    return 2.0 ** -24 * ((x.double().abs() @ w.double().abs().T) * (k / 4 + 2) + 4 * y.abs()) + 2.0 ** -149 * (1.5 * k + 4)
+
+
+@pytest.mark.parametrize("tile", [1, 2])
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("e", [-108, -112, -118, -124, -130])
+def test_products_of_small_numbers(e, which, tile):
+    """Rows (weights) below the numbers that three of bf16 add up to, all of them or some beside larger ones that meet zeros."""
+    from minivllm_amd import hip_ops as H
+
+    g = torch.Generator(device=DEV).manual_seed(-e)
+    a, b = _randn(g, 152, 160), _randn(g, 140, 160)
+    a[:70] *= 2.0 ** e
+    a[70:90, ::2] *= 2.0 ** e
+    b[:, 1::2] *= torch.where(torch.arange(140, device=DEV) < 70, 0.0, 1.0)[:, None]
+    x, w = (a, b) if which == 0 else (b, a)
+    got, want = H.linear_f32(*H.split_f32(x, w), tile=tile), x.double() @ w.double().T
+    assert ((got - want).abs() <= _chain_bound(x, w, want)).all()
+    tiny, library = (got[:70], F.linear(x, w)[:70]) if which == 0 else (got[:, :70], F.linear(x, w)[:, :70])
+    want = want[:70] if which == 0 else want[:, :70]
+    off = lambda y: ((y.double() - want).norm() / want.norm()).item()
+    assert off(tiny) <= off(library)
+    # as they leave for another projection
+    parts = H.linear_f32(*H.split_f32(x, w[:128].contiguous()), tile=tile, parts=True)
+    assert torch.equal(_numbers(parts), H.linear_f32(*H.split_f32(x, w[:128].contiguous()), tile=tile).double())
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2])
 @pytest.mark.parametrize("rows, n, k", [(1, 4, 32), (16, 32, 64), (63, 60, 96), (64, 64, 160), (127, 128, 768), (129, 132, 768), (700, 1000, 256), (300, 96, 3072)])
 def test_products(rows, n, k, tile):

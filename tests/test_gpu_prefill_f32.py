@@ -109,6 +109,27 @@ def test_numbers_that_have_no_parts(H, heads, what, at, value):
     assert torch.equal(got[:, 0], before[:, 0])      # (the other heads' are not touched)
 
 
+@pytest.mark.parametrize("heads", [2, 400])      # workgroups of 64 queries, of 128
+@pytest.mark.parametrize("eq, ek, ev, gap", [(0, 0, -118, 0), (0, 0, -124, 0), (118, -121, 0, 0), (-121, 118, 0, 0), (90, -120, 0, 0), (0, 0, -100, 110), (0, 0, 100, 124), (0, 0, 40, 120)], ids=str)
+def test_small_numbers_keep_their_bits(H, heads, eq, ek, ev, gap):
+    """q, k, v or probabilities below the numbers that three of bf16 add up to: as exact as ordinary ones.  ``gap``: key 0, whose values are zeros, is
+    so many powers of two ahead of the others."""
+    n = 200
+    q, k, v = (torch.randn(n, heads, 64, generator=torch.Generator().manual_seed(i)) for i in range(3))
+    if gap:
+        q[..., 0], k[:, :, 0], k[0], v[0] = 8 * gap * 0.6931471805599453, 0.0, 0.0, 0.0
+        k[0, :, 0] = 1.0
+    q, k, v = (x * 2.0 ** e for x, e in ((q, eq), (k, ek), (v, ev)))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    got = H.prefill_varlen(*(x.to(DEV) for x in (q, k, v)), cu, cu, n, n, 0.125, flags=H.MV_PREFILL_TILES).cpu().double()
+    some = slice(0, heads, max(1, heads // 4))
+    want = _attend(q[:, some], k[:, some], v[:, some], 0.125, _mask(n, n))
+    # sums of at most 200 products of 24 bits, by the size of a row's outputs; an exponent of `gap` has an error of some 2^-24 of it
+    # (five roundings); numbers below 2^-126 are rounded at 2^-149
+    bound = (1e-5 + gap * 5 * 2.0 ** -24) * want.abs().amax(-1, keepdim=True) + 2.0 ** -146
+    assert ((got[:, some] - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("kw", [dict(window=1), dict(window=40, keep=3), dict(window=33, keep=70), dict(chunk=32), dict(chunk=50), dict(cap=2.0),
                                 dict(sink=True), dict(gate=True), dict(window=64, keep=5, cap=3.0, sink=True, gate=True)], ids=str)
