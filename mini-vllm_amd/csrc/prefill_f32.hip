@@ -331,6 +331,10 @@ __device__ __forceinline__ u32x2 read_tr(const char *p) {
   typedef __attribute__((ext_vector_type(4))) short s16x4;
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p));
 }
+// Below 2^-109 three of bf16 do not add up to a number of fp32.  Values and probabilities are taken times 2^16, so that none is without its last bits.  Queries times
+// 2^32: what K loses is then 2^-38 of a score's unit for any query that is not too large for its parts itself (2^96; values: 2^112), and those take the other way.
+// Costs 2 %: 8 prompts of 511 .. 1021 tokens 81.1 -> 83.0 us, 4 of 2048 164 -> 169.
+constexpr float kQueries = 0x1p32f, kValues = 0x1p16f;
 __device__ __forceinline__ f32x4 mfma(const u32x4 &a, const u32x4 &b, const f32x4 &c) { return mfma16x16x32<bf16_tag>(a, b, c); }
 
 template <int D, int GROUPS>   // (head dim 128: 55 registers in memory; 8 prompts of 511 .. 1021 tokens 255 -> 201 us, one of 1000 111 -> 157)
@@ -370,7 +374,8 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
       for (int n = 0; n < 2; ++n) {
         const int at = tid + n * 256, row = at / CH, c = at % CH;
         const f32x4 &a = raw[w][n][0], &b = raw[w][n][1];
-        float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        const float by = w ? kValues : 1.f;
+        float f[8] = {a[0] * by, a[1] * by, a[2] * by, a[3] * by, b[0] * by, b[1] * by, b[2] * by, b[3] * by};
         u32x4 part[3];
         split3<false>(f, part);
         look(part[2], odd);
@@ -385,12 +390,12 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const float *from = (const float *)p.q + (int64_t)(q0 + min(qb + group * 32 + i * 16 + r16, sq - 1)) * p.q_stride + (int64_t)head * D + s * 32 + g * 8;
-      const f32x4 a = *(const f32x4 *)from, b = *(const f32x4 *)(from + 4);
+      const f32x4 a = *(const f32x4 *)from * kQueries, b = *(const f32x4 *)(from + 4) * kQueries;
       float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
       split3<false>(f, q[i][s]);
       look(q[i][s][2], odd);
     }
-  const float scale_log2 = p.scale * 1.4426950408889634f;
+  const float scale_log2 = p.scale * 1.4426950408889634f / kQueries;
   const bool late = scale_log2 > 0.f;   // scores are multiplied by `mul` where their exponent is formed, without a rounding between
   const float mul = late ? scale_log2 : 1.f;
   float m[2] = {-1e30f, -1e30f}, l[2] = {0.f, 0.f};
@@ -470,6 +475,8 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
 #pragma unroll
         for (int e = 0; e < 8; ++e) f[e] = __builtin_amdgcn_exp2f(fmaf(s[e >> 2][i][e & 3], mul, -m[i]));
         l[i] += ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] *= kValues;
         split3<false>(f, w[i]);
       }
       // values: a tile's products of these keys apart, the smallest first, one sum into the rest's
@@ -556,7 +563,7 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
     for (int t = 0; t < DT; ++t) {
       f32x4 w;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = l[i] > 0.f ? o[i][t][e] / l[i] * attn_factor<f32_tag>(p.mask, token, head * D + 16 * t + 4 * g + e) : 0.f;
+      for (int e = 0; e < 4; ++e) w[e] = l[i] > 0.f ? o[i][t][e] / l[i] * (1.f / (kValues * kValues)) * attn_factor<f32_tag>(p.mask, token, head * D + 16 * t + 4 * g + e) : 0.f;
       *(f32x4 *)(op + 16 * t) = w;
     }
   }
