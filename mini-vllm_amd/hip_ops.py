@@ -1058,6 +1058,17 @@ def linear_f32_ok(x, *others) -> bool:
 
 def split_f32(*matrices, norm=None):
     """Each fp32 matrix [rows, k] in parts; ``norm``: a LayerNorm that the first one goes through."""
+    if not 1 <= len(matrices) <= MV_SPLIT_F32_MAX:
+        raise MvHipError(f"1 to {MV_SPLIT_F32_MAX} matrices (got {len(matrices)})")
+    for m in matrices:
+        if m.dtype != torch.float32 or m.dim() != 2 or m.stride(1) != 1:
+            raise MvHipError("matrices of fp32 numbers required, a row's side by side")
+    if norm is not None:
+        for v in (norm.weight, norm.bias) if norm.bias is not None else (norm.weight,):
+            if v is None or v.dtype != torch.float32 or v.shape != (matrices[0].shape[1],) or not v.is_contiguous():
+                raise MvHipError(f"norm: {matrices[0].shape[1]} fp32 numbers required")
+        _need_cuda(norm.weight, norm.bias)
+    _need_cuda(*matrices)
     a, out = MvSplitF32Args(count=len(matrices)), []
     if norm is not None:
         a.norm_w, a.norm_b, a.eps = norm.weight.data_ptr(), _ptr(norm.bias), norm.eps
@@ -1079,6 +1090,10 @@ def linear_f32(x, w, bias=None, residual=None, relu=False, parts=False, tile=0):
         raise MvHipError(f"bias: {n} fp32 numbers required")
     if residual is not None and (residual.dtype != torch.float32 or residual.shape != (rows, n) or residual.stride(1) != 1):
         raise MvHipError(f"residual: [{rows}, {n}] fp32 numbers required")
+    for m in (x, w):
+        if m.data.dtype != torch.uint8 or not m.data.is_contiguous() or m.data.numel() < _lib.mv_split_f32_bytes(m.rows, m.k):
+            raise MvHipError(f"parts of a matrix [{m.rows}, {m.k}] required (split_f32)")
+    _need_cuda(x.data, w.data, bias, residual)
     data = torch.empty(_lib.mv_split_f32_bytes(rows, n), dtype=torch.uint8, device=x.data.device) if parts else \
         torch.empty((rows, n), dtype=torch.float32, device=x.data.device)
     a = MvLinearF32Args(x=x.data.data_ptr(), w=w.data.data_ptr(), bias=_ptr(bias), residual=_ptr(residual), out=data.data_ptr(),
