@@ -9,6 +9,7 @@ from typing import Any
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules import module as _modules
 
 from .. import hip_ops
 from ..layers import (Attention, ColumnParallelLinear, ParallelLMHead, QKVParallelLinear, RowParallelLinear,
@@ -74,10 +75,17 @@ class OPTDecoderLayer(nn.Module):
         if x.shape[0] < self.parts_rows or x.dtype != torch.float32:   # (small steps are bound by the host: nothing else is looked at)
             return False
         att = self.self_attn
+        if not self.do_layer_norm_before or f32_tiles(x.shape[0], x.shape[1]) < F32_LAYER_TILES_MIN or type(att) is not OPTAttention:
+            return False
+        # modules that are not called: nobody may have put another in their place, or wait for a call
         linears, norms = (att.qkv_proj, att.out_proj, self.fc1, self.fc2), (self.self_attn_layer_norm, self.final_layer_norm)
-        return (self.do_layer_norm_before and f32_tiles(x.shape[0], x.shape[1]) >= F32_LAYER_TILES_MIN and all(lin.tp_size == 1 for lin in linears)
-                and not any(m._forward_hooks or m._forward_pre_hooks for m in (*linears, *norms, att))
-                and hip_ops.linear_f32_ok(x, *(t for m in (*linears, *norms) for t in (m.weight, m.bias))))
+        if tuple(map(type, linears)) != (QKVParallelLinear, RowParallelLinear, ColumnParallelLinear, RowParallelLinear) \
+                or any(type(norm) is not nn.LayerNorm or norm.weight is None or norm.normalized_shape != (x.shape[1],) for norm in norms):
+            return False
+        if _modules._global_forward_hooks or _modules._global_forward_pre_hooks \
+                or any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (*linears, *norms, att)):
+            return False
+        return all(lin.tp_size == 1 for lin in linears) and hip_ops.linear_f32_ok(x, *(t for m in (*linears, *norms) for t in (m.weight, m.bias)))
 
     def _forward_parts(self, x):
         att, fc1, fc2 = self.self_attn, self.fc1, self.fc2

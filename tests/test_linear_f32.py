@@ -39,6 +39,64 @@ def test_linear_refuses():
         H.linear_f32(x, w)
 
 
+def _layer(monkeypatch, d=64, ffn=128):
+    from types import SimpleNamespace
+
+    from minivllm_amd.glue import opt
+
+    monkeypatch.setattr(H, "linear_f32_ok", lambda *a: True)      # (which asks for a GPU)
+    return opt.OPTDecoderLayer(SimpleNamespace(hidden_size=d, num_attention_heads=d // 64, enable_bias=True, do_layer_norm_before=True, ffn_dim=ffn)).requires_grad_(False)
+
+
+def _other_modules(layer):
+    from torch import nn
+
+    from minivllm_amd.layers import ColumnParallelLinear
+
+    class Scaled(ColumnParallelLinear):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    class Norm(nn.LayerNorm):
+        pass
+
+    att = type("Other", (type(layer.self_attn),), {})(64, 1)
+    return [("fc1", nn.Sequential(layer.fc1)), ("fc1", nn.Linear(64, 128)), ("fc1", Scaled(64, 128, True)), ("fc2", nn.Linear(128, 64)), ("self_attn", att),
+            ("self_attn_layer_norm", Norm(64)), ("final_layer_norm", nn.Identity()), ("final_layer_norm", nn.LayerNorm(64, elementwise_affine=False)),
+            ("final_layer_norm", nn.LayerNorm((20000, 64)))]
+
+
+@pytest.mark.parametrize("at", range(9))
+def test_opt_layer_with_other_modules(monkeypatch, at):
+    """An adapter or a norm in the place of a layer's own is called as a module."""
+    layer, x = _layer(monkeypatch), torch.zeros(20000, 64)
+    assert layer._by_parts(x)
+    name, other = _other_modules(layer)[at]
+    setattr(layer, name, other)
+    assert not layer._by_parts(x)
+
+
+def test_opt_layer_that_is_watched(monkeypatch):
+    """So is one that has a hook, or a forward of its own."""
+    from torch import nn
+
+    layer, x = _layer(monkeypatch), torch.zeros(20000, 64)
+    att = layer.self_attn
+    for m in (att, att.qkv_proj, att.out_proj, layer.fc1, layer.fc2, layer.self_attn_layer_norm, layer.final_layer_norm):
+        for hook in (m.register_forward_hook, m.register_forward_pre_hook):
+            handle = hook(lambda *a: None)
+            assert not layer._by_parts(x)
+            handle.remove()
+        m.forward = m.forward
+        assert not layer._by_parts(x)
+        del m.forward
+    for hook in (nn.modules.module.register_module_forward_hook, nn.modules.module.register_module_forward_pre_hook):
+        handle = hook(lambda *a: None)
+        assert not layer._by_parts(x)
+        handle.remove()
+    assert layer._by_parts(x)
+
+
 @pytest.mark.gpu
 def test_linear_refuses_vectors_elsewhere():
     x, w = H.split_f32(torch.zeros(20, 64, device="cuda:0"), torch.zeros(48, 64, device="cuda:0"))
