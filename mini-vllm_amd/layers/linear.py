@@ -165,8 +165,8 @@ def linear(x, weight, bias=None, packed=None, kind: str = "col"):
                 return PartialSum(hip_ops.linear_mid_m_partial(x, packed, n, splits, cfg), x.dtype)
             if cfg:
                 return hip_ops.linear_mid_m(x, packed, n, bias, cfg)
-    if x.dim() == 2 and x.shape[0] >= F32_ROWS_MIN and x.dtype == torch.float32 and f32_tiles(x.shape[0], weight.shape[0]) >= F32_TILES_MIN \
-            and x.shape[1] == weight.shape[1] and hip_ops.linear_f32_ok(x, weight, bias):
+    if x.dim() == 2 and x.shape[0] >= F32_ROWS_MIN and x.dtype == torch.float32 and weight.dim() == 2 and f32_tiles(x.shape[0], weight.shape[0]) >= F32_TILES_MIN \
+            and x.shape[1] == weight.shape[1] and (bias is None or bias.shape == weight.shape[:1]) and hip_ops.linear_f32_ok(x, weight, bias):
         return hip_ops.linear_f32(*hip_ops.split_f32(x, weight), bias)
     return F.linear(x, weight, bias)
 

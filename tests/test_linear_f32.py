@@ -97,6 +97,27 @@ def test_opt_layer_that_is_watched(monkeypatch):
     assert layer._by_parts(x)
 
 
+def test_forms_that_have_no_parts(monkeypatch):
+    """Weights and biases in the other forms that ``F.linear`` takes go to it."""
+    import torch.nn.functional as F
+
+    from minivllm_amd.layers.linear import linear
+
+    def refuse(*a):
+        raise AssertionError("by parts")
+
+    monkeypatch.setattr(H, "linear_f32_ok", lambda *a: True)
+    monkeypatch.setattr(H, "split_f32", refuse)
+    x, w = torch.randn(512, 4800), torch.randn(4800, 32)
+    assert torch.equal(linear(x, w[:, 0].contiguous()), F.linear(x, w[:, 0].contiguous()))
+    x = x[:, :32].contiguous()
+    for bias in (torch.tensor(2.0), torch.randn(1), torch.randn(1, 4800), torch.randn(512, 4800)):
+        assert torch.equal(linear(x, w, bias), F.linear(x, w, bias))
+    for bias in (None, torch.randn(4800)):
+        with pytest.raises(AssertionError, match="by parts"):
+            linear(x, w, bias)
+
+
 @pytest.mark.gpu
 def test_linear_refuses_vectors_elsewhere():
     x, w = H.split_f32(torch.zeros(20, 64, device="cuda:0"), torch.zeros(48, 64, device="cuda:0"))
