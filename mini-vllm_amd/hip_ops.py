@@ -13,6 +13,7 @@ from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_uint64, c_void
 from typing import NamedTuple
 
 import torch
+from torch.utils._device import DeviceContext as _DeviceMode
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libmvhip.so")
@@ -1036,17 +1037,20 @@ class F32Parts(NamedTuple):
 
 def linear_f32_ok(x, *others) -> bool:
     """May a projection of ``x`` [T, K] with these weights [N, K] and vectors [N] (None: not there) go by parts?  Plain numbers on the current device, of
-    which nobody asks for gradients, tangents or a trace."""
+    which nobody asks for gradients, tangents or a trace (a default device is a mode too, but one that only makes new tensors)."""
+    if torch.compiler.is_compiling():
+        return False
     if not (x.is_cuda and x.dim() == 2 and x.dtype == torch.float32) or x.device.index != torch.cuda.current_device() or torch.is_autocast_enabled("cuda"):
         return False
-    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0:
+    if torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() or torch.autograd.forward_ad._current_level >= 0 \
+            or any(type(mode) is not _DeviceMode for mode in torch.overrides._get_current_function_mode_stack()):
         return False
     for t in (x, *others):
         if t is None:
             continue
         if type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t):
             return False
-        if t.dtype != torch.float32 or t.device != x.device or t.data_ptr() % 16 or (torch.is_grad_enabled() and t.requires_grad):
+        if t.dtype != torch.float32 or t.device != x.device or t.data_ptr() % 16 or t.is_neg() or (torch.is_grad_enabled() and t.requires_grad):
             return False
         if t is x:
             if t.shape[1] % 32 or t.stride(1) != 1 or t.stride(0) % 4 or t.stride(0) < t.shape[1]:

@@ -119,6 +119,30 @@ def test_forms_that_have_no_parts(monkeypatch):
 
 
 @pytest.mark.gpu
+def test_who_is_asked_for():
+    """A mode that sees functions sees the library's, a compiled program holds it whole; a default device changes nothing."""
+    from torch.overrides import TorchFunctionMode
+
+    from minivllm_amd.layers.linear import linear
+
+    x, w = torch.randn(1300, 96, device="cuda:0"), torch.randn(2048, 96, device="cuda:0")
+    by_parts, seen = H.linear_f32(*H.split_f32(x, w)), []
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Watch():
+        y = linear(x, w)
+    assert torch.nn.functional.linear in seen and torch.equal(y, torch.nn.functional.linear(x, w))
+    with torch.device("cuda:0"):
+        assert torch.equal(linear(x, w), by_parts)
+    assert torch.equal(torch.compile(linear, backend="eager", fullgraph=True)(x, w), y)
+    assert torch.equal(linear(torch._neg_view(x), w), torch.nn.functional.linear(-x, w))
+
+
+@pytest.mark.gpu
 def test_linear_refuses_vectors_elsewhere():
     x, w = H.split_f32(torch.zeros(20, 64, device="cuda:0"), torch.zeros(48, 64, device="cuda:0"))
     for kw in (dict(bias=torch.zeros(48)), dict(residual=torch.zeros(20, 48))):
