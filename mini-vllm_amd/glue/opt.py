@@ -20,8 +20,11 @@ from ..parallel_state import get_tensor_parallel_world_size
 __all__ = ["OPTForCausalLM"]
 
 # fp32 layers go by parts of bf16 as a whole (norms, ReLU and residual sums within the projections' launches) from so many tiles of 64 x 64 hidden features
-# on.  us, 768 features, projections and what is between them, as modules / as a whole: 1000 rows (192 tiles) 154 / 170, 1300 (252) 188 / 183, 1600 (300) 230 / 215
-F32_LAYER_TILES_MIN = 264
+# and so many rows on, which have to pay for the weights' parts whatever the width.  us, projections and what is between them, as modules / as a whole:
+# 768 features: 1025 rows (204 tiles) 173 / 174, 1300 (252) 181 / 184, 1345 (264) 194 / 203, 1408 (264) 205 / 203, 1600 (300) 215 / 205, 1664 247 / 210; 1024: 769 (208) 200 / 222,
+# 1088 (272) 261 / 260, 1345 316 / 282; 2048: 513 (288) 474 / 562, 769 600 / 617, 1025 813 / 772; 4096: 257 (320) 933 / 1432, 513 1660 / 1733, 769 2238 / 2208,
+# 1025 2811 / 2795; 5120: 257 1640 / 1967, 1025 4532 / 4464; 7168: 129 (336) 1567 / 2979, 513 5278 / 5267, 1025 7296 / 7398
+F32_LAYER_TILES_MIN, F32_LAYER_ROWS_MIN = 264, 1024
 
 
 class OPTLearnedPositionalEmbedding(nn.Embedding):
@@ -69,7 +72,7 @@ class OPTDecoderLayer(nn.Module):
         self.fc1 = ColumnParallelLinear(d, config.ffn_dim, bias=config.enable_bias)
         self.fc2 = RowParallelLinear(config.ffn_dim, d, bias=config.enable_bias)
         self.final_layer_norm = nn.LayerNorm(d)
-        self.parts_rows = (-(-F32_LAYER_TILES_MIN // -(-d // 64)) - 1) * 64 + 1   # the fewest rows of F32_LAYER_TILES_MIN tiles
+        self.parts_rows = max(F32_LAYER_ROWS_MIN, (-(-F32_LAYER_TILES_MIN // -(-d // 64)) - 1) * 64 + 1)   # the fewest rows
 
     def _by_parts(self, x) -> bool:
         if x.shape[0] < self.parts_rows or x.dtype != torch.float32:   # (small steps are bound by the host: nothing else is looked at)

@@ -48,6 +48,14 @@ def _layer(monkeypatch, d=64, ffn=128):
     return opt.OPTDecoderLayer(SimpleNamespace(hidden_size=d, num_attention_heads=d // 64, enable_bias=True, do_layer_norm_before=True, ffn_dim=ffn)).requires_grad_(False)
 
 
+@pytest.mark.parametrize("d, rows", [(128, 8385), (768, 1345), (1024, 1025), (2048, 1024), (4096, 1024), (9216, 1024)])
+def test_rows_that_pay_for_a_layers_weights(monkeypatch, d, rows):
+    """However wide a layer is, few rows do not pay for the parts of its weights."""
+    with torch.device("meta"):
+        layer, x = _layer(monkeypatch, d, 4 * d), torch.zeros(rows, d)
+    assert layer._by_parts(x) and not layer._by_parts(x[:rows - 1])
+
+
 def _other_modules(layer):
     from torch import nn
 
