@@ -206,10 +206,11 @@ extern "C" int mv_add_rmsnorm_partial(const float *partial, int splits, void *re
 // relu in its place (fp32 inside, one rounding).
 // The reference rounds silu(x1) to the activation dtype before the multiply;
 // the same two rounding points are kept here.
-template <typename Tag, int ACT>
+// FAR (of the kernel: behind a branch between two stores of one place the compiler makes one plain store of both): results go past the last cache.
+template <typename Tag, int ACT, bool FAR>
 __global__ void __launch_bounds__(256)
 silu_and_mul_kernel(const typename elem<Tag>::T *__restrict__ x, int64_t x_stride,
-                    typename elem<Tag>::T *__restrict__ out, int64_t out_stride, int rows, int cols, MvGateAct act, bool far) {
+                    typename elem<Tag>::T *__restrict__ out, int64_t out_stride, int rows, int cols, MvGateAct act) {
   constexpr int VEC = elem<Tag>::VEC;
   constexpr int U = 4;   // vectors per thread and trip: 2 U loads in flight before the first exp (prefill rows: 4.3 -> TB/s)
   const int nvec = cols / VEC;
@@ -253,7 +254,7 @@ silu_and_mul_kernel(const typename elem<Tag>::T *__restrict__ x, int64_t x_strid
           u32x4 o;
           if constexpr (VEC == 8) o = pack8<Tag>(y);
           else o = u32x4{f2u(y[0]), f2u(y[1]), f2u(y[2]), f2u(y[3])};
-          if (far) __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(orow + c * VEC));
+          if constexpr (FAR) __builtin_nontemporal_store(o, reinterpret_cast<u32x4 *>(orow + c * VEC));
           else *reinterpret_cast<u32x4 *>(orow + c * VEC) = o;
         }
       }
@@ -277,11 +278,15 @@ static int act_and_mul(const void *x, int64_t x_stride, void *out, int64_t out_s
     const int nvec = cols / VEC;
     const int bx = (nvec + 256 * 4 - 1) / (256 * 4);
     const int by = rows < 65535 ? rows : 65535;
-    // Results that the last cache (256 MB) has no room for go past it, from 300 MiB on.  us, bf16, with / past it: 12000 x 11008 (264 MB) 120 / 138, 8000 x 18944 (303 MB) 158 / 146,
-    // 20000 x 11008 (440 MB) 245 / 231, 25672 x 18944 (973 MB) 545 / 482.  A workgroup a row: that one 571, 535 with eight rows behind each other.
-    const bool far = (int64_t)rows * cols * (int64_t)sizeof(T) > (int64_t)300 << 20;
-    hipLaunchKernelGGL((silu_and_mul_kernel<Tag, ACT>), dim3((unsigned)bx, (unsigned)by), dim3(256), 0,
-                       (hipStream_t)stream, (const T *)x, x_stride, (T *)out, out_stride, rows, cols, act, far);
+    // Results of 16 bits that the last cache (256 MiB) has no room for go past it.  us, bf16, through / past the cache, alone and with a copy of the result behind it:
+    // 18944 columns, 264 MB 119 / 124, 234 / 229, 303 MB 156 / 143, 270 / 262, 973 MB 541 / 482, 903 / 876; 11008, 264 MB 120 / 135, 236 / 239, 295 MB 151 / 152, 266 / 265,
+    // 303 MB 161 / 156, 273 / 273, 973 MB 543 / 511, 911 / 908; 2432, 275 MB 120 / 122, 241 / 229, 303 MB 151 / 135, 265 / 251.  fp32 gains 3 % alone, and loses as much with
+    // a reader behind it (18944, 303 MB 162 / 158, 275 / 283, 600 MB 327 / 317, 552 / 556).
+    const dim3 grid((unsigned)bx, (unsigned)by);
+    if (VEC == 8 && (int64_t)rows * cols * (int64_t)sizeof(T) >= 300000000)
+      hipLaunchKernelGGL((silu_and_mul_kernel<Tag, ACT, VEC == 8>), grid, dim3(256), 0, (hipStream_t)stream, (const T *)x, x_stride, (T *)out, out_stride, rows, cols, act);
+    else
+      hipLaunchKernelGGL((silu_and_mul_kernel<Tag, ACT, false>), grid, dim3(256), 0, (hipStream_t)stream, (const T *)x, x_stride, (T *)out, out_stride, rows, cols, act);
   });
   MV_LAUNCH_CHECK();
   return MV_OK;

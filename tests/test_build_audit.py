@@ -77,3 +77,20 @@ def test_64_row_prefill_kernel_owns_its_accumulator_file(asm):
         touched = [ln.strip() for ln in out_of_asm if re.search(r"accvgpr| a\[\d|, a\d", ln)]
         assert not touched, (name, touched[:4])
         assert _facts(body)["ScratchSize"] == 0 and "scratch_" not in body, name
+
+
+def test_results_past_the_last_cache_are_stored_so(tmp_path):
+    """The gated activation's kernel for large results stores non-temporally, the other one does not (csrc/rmsnorm.hip)."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not installed")
+    out = tmp_path / "rmsnorm.s"
+    subprocess.run([HIPCC, "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    "--cuda-device-only", "-S", "-o", str(out), os.path.join(ROOT, "mini-vllm_amd", "csrc", "rmsnorm.hip")], check=True, stderr=subprocess.DEVNULL)
+    text = out.read_text()
+    far = {}
+    for m in re.finditer(r"^(_Z\w*silu_and_mul_kernelI(\w+?)Li\dE(?:Lb(\d)E)?E\w*):\s*; @", text, re.M):
+        stores = [ln for ln in text[m.end():text.index("; ScratchSize", m.end())].split("\n") if "global_store" in ln]
+        past = [ln for ln in stores if re.search(r"\bnt\b", ln)]
+        assert stores and len(past) in (0, len(stores)), m.group(1)
+        far.setdefault((m.group(2), m.group(3)), []).append(bool(past))
+    assert far == {("8bf16_tag", "1"): [True] * 4, ("7f16_tag", "1"): [True] * 4, ("8bf16_tag", "0"): [False] * 4, ("7f16_tag", "0"): [False] * 4, ("7f32_tag", "0"): [False] * 4}

@@ -34,3 +34,17 @@ def test_results_that_go_past_the_last_cache(rows, cols):
     y = H.silu_and_mul(x)
     for at in (0, 40000 if rows > 65536 else 7000, rows - 64):
         assert torch.equal(y[at:at + 64], H.silu_and_mul(x[at:at + 64]))
+
+
+@pytest.mark.parametrize("rows", [7918, 7919])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_both_sides_of_the_last_caches_line(dtype, act, rows):
+    """Results of 299.997 and 300.035 MB (rows that lie apart, of which a few are asked for again)."""
+    from minivllm_amd import hip_ops as H
+
+    g = torch.Generator(device="cuda:0").manual_seed(rows)
+    x = torch.randn(rows, 2 * 18944 + 8, device="cuda:0", generator=g, dtype=dtype)[:, :2 * 18944]
+    y = H.act_and_mul(x, act)
+    for at in (0, 4000, rows - 16):
+        assert torch.equal(y[at:at + 16], H.act_and_mul(x[at:at + 16], act))
