@@ -341,7 +341,7 @@ template <int D, int GROUPS>   // (head dim 128: 55 registers in memory; 8 promp
 __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) {
   constexpr int TURNS = 4 / GROUPS, BM = 32 * GROUPS, BN = 4096 / D, SUBS = BN / 32 / TURNS, KS = D / 32, DT = D / 16, CH = D / 8;   // (32 keys: a sub)
   constexpr int PART = BN * D * 2;
-  static_assert(SUBS >= 1);
+  static_assert(SUBS >= 1 && D == 64);
   __shared__ __attribute__((aligned(16))) char kl[3 * PART], vl[3 * PART];
   __shared__ int again;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4, group = wave % GROUPS, turn = wave / GROUPS;
@@ -353,8 +353,8 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
   const int shift = sk - sq, last = min(qb + BM, sq) - 1, end = min(sk, last + shift + 1), steps = end > 0 ? (end + BN - 1) / BN : 0;
   const int wave_lo = min(qb + group * 32, sq - 1) + shift, wave_hi = min(qb + group * 32 + 31, sq - 1) + shift;
   // places of a row's pieces of eight, in orders that spread the rows that are read together over the banks
-  auto k_place = [](int row, int c) { return (row * CH + (c ^ (D == 64 ? row >> 1 & 7 : row & 15))) * 16; };
-  auto v_place = [](int row, int c) { return (row * CH + (c ^ (D == 64 ? row & 6 : (row & 7) << 1))) * 16; };
+  auto k_place = [](int row, int c) { return (row * CH + (c ^ (row >> 1 & 7))) * 16; };
+  auto v_place = [](int row, int c) { return (row * CH + (c ^ (row & 6))) * 16; };
 
   f32x4 raw[2][2][2];   // rows of K, V on their way
   auto fetch = [&](int step) __attribute__((always_inline)) {
@@ -569,12 +569,17 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
   }
 }
 
-// Both kernels' times in ns, as they grew over 1700 shapes (1 .. 400 queries of 1 .. 2000 keys, 4 .. 32 heads, 1 .. 256 sequences): the vector kernel takes
-// 3 us, the walk to the sequence, and 0.11 us a key (twice that at head dim 128) or its reads of K and V, whichever is more; a tile of 64 queries 9 us for
-// the first 64 keys and 4 for each further 64, or what its turns on the chip take.  The other kernel is quicker by more than 5 % in 5 % of them, by 45 % at most.
-// Vector kernel / this, us: one prompt of 8 tokens, 12 heads of 64 (128) 4 / 9 (4 / 15); 64 of 8 tokens 14 / 14 (16 / 31), of 16 24 / 14 (28 / 32);
-// one of 64 tokens 10 / 9 (17 / 15); 256 single queries of 400 paged keys, 32 heads of 64 (128) 193 / 953 (349 / 2270).
+// Both kernels' times in ns.  The vector kernel takes 3 us, the walk to the sequence, and 0.11 us a key (twice that at head dim 128) or its reads of K and V,
+// whichever is more.
+// fp32 products (head dim 128, pages, masks), as they grew over 1700 shapes (1 .. 400 queries of 1 .. 2000 keys, 4 .. 32 heads, 1 .. 256 sequences): a tile of 64
+// queries 9 us for the first 64 keys and 4 for each further 64, or what its turns on the chip take.  The other kernel is quicker by more than 5 % in 5 % of them, by 45 % at most.
+// Vector kernel / this, us: one prompt of 8 tokens, 12 heads of 128 4 / 15; 64 of 8 tokens 16 / 31, of 16 28 / 32; one of 64 tokens 17 / 15;
+// 256 single queries of 400 paged keys, 32 heads of 64 (128) 193 / 953 (349 / 2270).
+// Parts (whole prompts of head dim 64), over 3340 shapes (1 .. 1000 tokens, 4 .. 32 heads, 1 .. 128 prompts): 8.5 us for the first 64 keys and 1.7 for each further 64, or its turns.
+// The other one is quicker by more than 5 % in 1 %, by 33 % at most (with the fp32 products' figures 5 %, 53 %).  Vector kernel / this, us, 12 heads: one prompt of 8 tokens
+// 4.2 / 7.6, 48 8.4 / 8.6, 65 10.5 / 9.6, 87 12.7 / 10.7; 8 of 32 tokens 8.2 / 8.5, of 40 9.8 / 8.7; 64 of 8 tokens, 32 heads 27 / 28.
 // From 320 keys on, where the vector kernel is further from 64 bits, it has to take half as long or less.
+bool general(const PrefillParams &p) { return p.block_tables || p.chunk > 0 || p.mask.window > 0 || p.mask.softcap > 0.f; }
 bool vector_is_quicker(const PrefillParams &p) {
   const int64_t seen = p.max_seqlen_k, wide = p.head_dim / 64, beside = min(p.max_seqlen_q, BM) + BN - 2;   // keys that only other queries of a tile see
   const int64_t limit = p.chunk > 0 ? p.chunk : p.mask.window > 0 ? (int64_t)p.mask.window + p.mask.keep_first : seen;
@@ -582,8 +587,9 @@ bool vector_is_quicker(const PrefillParams &p) {
   const int64_t rows = (int64_t)p.n_heads * p.n_seqs * p.max_seqlen_q, groups = (int64_t)p.n_heads * p.n_seqs * ((p.max_seqlen_q + BM - 1) / BM);
   const int64_t read = rows * keys * wide / 25 / (p.n_heads >= 4 * p.n_kv_heads ? 2 : 1);
   const int64_t vector = 3000 + 70 * p.n_seqs + max(22 * wide * keys * (p.block_tables ? 6 : 5), read) + rows * p.n_seqs * 14 / 1000;
-  const int64_t tiles = max(4700 + 4000 * pieces, groups * (7 + 12 * pieces)) * (wide > 1 ? 7 : 4) / 4 *
-                        (p.block_tables ? 14 : limit < seen || p.mask.softcap > 0.f ? 12 : 10) / 10;
+  const int64_t tiles = wide == 1 && !general(p) ? max(6800 + 1700 * pieces, groups * (10 + 7 * pieces))
+                                                 : max(4700 + 4000 * pieces, groups * (7 + 12 * pieces)) * (wide > 1 ? 7 : 4) / 4 *
+                                                       (p.block_tables ? 14 : limit < seen || p.mask.softcap > 0.f ? 12 : 10) / 10;
   return vector * (keys > 320 ? 2 : 1) <= tiles;
 }
 
@@ -593,9 +599,8 @@ int mv_prefill_f32_launch(const PrefillParams &p, bool always, hipStream_t strea
   if (p.head_dim > 128 || (!always && vector_is_quicker(p))) return MV_E_SHAPE;
   const dim3 grid(p.n_heads, p.n_seqs, (p.max_seqlen_q + BM - 1) / BM);
   if (grid.y > 65535 || grid.z > 65535) return MV_E_SHAPE;
-  const bool general = p.block_tables || p.chunk > 0 || p.mask.window > 0 || p.mask.softcap > 0.f;
   const dim3 block(WAVES * 64);
-  if (p.head_dim == 64 && general) hipLaunchKernelGGL((prefill_f32_kernel<64, true>), grid, block, 0, stream, p);
+  if (p.head_dim == 64 && general(p)) hipLaunchKernelGGL((prefill_f32_kernel<64, true>), grid, block, 0, stream, p);
   else if (p.head_dim == 64) {
     // 128 queries a workgroup where they fill the chip one and a half times (two a CU).  64 / 128 queries, over 130 shapes: 0.67 .. 1.0 of the time up to 600 workgroups of 128,
     // 0.88 .. 1.05 up to 768, 0.91 .. 1.09 up to 1100, 1.0 .. 1.2 over that
@@ -603,7 +608,7 @@ int mv_prefill_f32_launch(const PrefillParams &p, bool always, hipStream_t strea
     if ((int64_t)wide.x * wide.y * wide.z >= 768) hipLaunchKernelGGL((prefill_parts_kernel<64, 4>), wide, block, 0, stream, p);
     else hipLaunchKernelGGL((prefill_parts_kernel<64, 2>), grid, block, 0, stream, p);
   }
-  else if (p.head_dim == 128 && general) hipLaunchKernelGGL((prefill_f32_kernel<128, true>), grid, block, 0, stream, p);
+  else if (p.head_dim == 128 && general(p)) hipLaunchKernelGGL((prefill_f32_kernel<128, true>), grid, block, 0, stream, p);
   else if (p.head_dim == 128) hipLaunchKernelGGL((prefill_f32_kernel<128, false>), grid, block, 0, stream, p);
   else return MV_E_SHAPE;
   MV_LAUNCH_CHECK();

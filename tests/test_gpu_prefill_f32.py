@@ -88,6 +88,17 @@ def test_many_prompts_at_the_edges_of_tiles(H, monkeypatch):
     _check(H, monkeypatch, [(n, n) for n in [5, 128, 90] * 9], 32, 32, 64, 12, sink=True, gate=True)
 
 
+@pytest.mark.parametrize("tokens, prompts, heads, d, tiles", [(8, 1, 12, 64, False), (40, 1, 12, 64, False), (65, 1, 12, 64, True), (80, 1, 12, 64, True), (65, 2, 32, 64, True),
+                                                              (69, 4, 12, 64, True), (8, 64, 32, 64, False), (40, 1, 12, 128, False), (128, 1, 12, 128, True)])
+def test_which_kernel_is_taken(H, tokens, prompts, heads, d, tiles):
+    """The quicker one by the rule: few tokens key by key, a second tile of 64 keys by tiles."""
+    q, k, v = (torch.randn(tokens * prompts, heads, d, generator=torch.Generator().manual_seed(i)).to(DEV) for i in range(3))
+    cu = torch.arange(0, tokens * prompts + 1, tokens, dtype=torch.int32, device=DEV)
+    call = lambda flags: H.prefill_varlen(q, k, v, cu, cu, tokens, tokens, d ** -0.5, flags=flags)
+    by_tiles, by_keys = call(H.MV_PREFILL_TILES), call(H.MV_PREFILL_SIMPLE)
+    assert not torch.equal(by_tiles, by_keys) and torch.equal(call(0), by_tiles if tiles else by_keys)
+
+
 @pytest.mark.parametrize("kw", [dict(sink=True), dict(gate=True), dict(sink=True, gate=True)], ids=str)
 def test_sinks_and_gates_of_whole_prompts(H, monkeypatch, kw):
     _check(H, monkeypatch, [(150, 150), (20, 20), (65, 65)], 4, 2, 64, 13, **kw)
