@@ -50,3 +50,32 @@ def test_more_tiles_than_are_held(H, counts):
     got = H.moe_linear(x, H.pack_weight(w.view(-1, k)), n, groups, None, gather=True, experts=experts)
     want = (ids.float() / 16).bfloat16().expand(rows, n)      # (exact sums, rounded once)
     assert torch.equal(got[groups.place.long()], want)
+
+
+@pytest.mark.parametrize("k", [64, 256])
+@pytest.mark.parametrize("counts", [[1] * 700 + [300], [0] * 600 + [257] * 3 + [0] * 100 + [5], [130] * 515])
+def test_tiles_beyond_those_held(H, counts, k):
+    """The same with the expert's number, the token's and a digit from each stage of 32 inputs in the outputs, all of them exact, tokens in any order: a
+    neighbour's tile, the other half of one's own, another row or stage is another result."""
+    experts, rows, n = len(counts), sum(counts), 32
+    e = torch.arange(experts, device=DEV)
+    g = torch.Generator().manual_seed(rows)
+    ids = torch.repeat_interleave(torch.arange(experts), torch.tensor(counts))[torch.randperm(rows, generator=g)].to(DEV)
+    t = torch.arange(rows, device=DEV)
+    x, w = torch.zeros(rows, k, device=DEV), torch.zeros(experts, n, k, device=DEV)
+    x[:, 0], w[:, 0, 0], w[:, 1, 0] = 1.0, (e // 32).float(), (e % 32).float()
+    for digit in range(3):
+        x[:, 1 + digit], w[:, 2 + digit, 1 + digit] = (t >> 8 * digit & 255).float(), 1.0
+    w[:, 5, 1], w[:, 5, 0] = 1.0 / 256, (e % 256).float() / 256         # (the expert and the token in one sum: 9 bits, rounded once)
+    for stage in range(k // 32):
+        x[:, 32 * stage + 5 + stage], w[:, 8 + stage, 32 * stage + 5 + stage] = ((t * 7 + stage) % 251).float(), 1.0
+    groups = H.moe_group(ids.int()[:, None].contiguous(), experts, 256)
+    got = H.moe_linear(x.bfloat16(), H.pack_weight(w.bfloat16().view(-1, k)), n, groups, None, gather=True, experts=experts)[groups.place.long()]
+    want = torch.zeros(rows, n, device=DEV)
+    want[:, 0], want[:, 1] = (ids // 32).float(), (ids % 32).float()
+    for digit in range(3):
+        want[:, 2 + digit] = (t >> 8 * digit & 255).float()
+    want[:, 5] = ((t & 255) + ids % 256).float() / 256
+    for stage in range(k // 32):
+        want[:, 8 + stage] = ((t * 7 + stage) % 251).float()
+    assert torch.equal(got, want.bfloat16())

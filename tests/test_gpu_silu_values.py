@@ -24,6 +24,25 @@ def test_silu_of_every_number(dtype):
     assert y[x == torch.inf] == torch.inf and torch.isnan(y[torch.isnan(x)]).all() and torch.isnan(y[x == -torch.inf]).all()
 
 
+def test_silu_of_bf16_has_the_divisions_bits():
+    """Every bf16 gate above fp32's last exponential: x / (1 + exp(-x)) of 64 bits, rounded once, to the bit, as fp32's division gives it too; below, a zero."""
+    from minivllm_amd import hip_ops as H
+
+    a = torch.arange(-32768, 32768, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(64, 1024)
+    y = H.silu_and_mul(torch.cat((a, torch.ones_like(a)), 1).to("cuda:0")).cpu()
+    x = a.double()
+    exact = x / (1 + torch.exp(-x))
+    ulp = 2.0 ** (torch.floor(torch.log2(exact.abs().clamp_min(1e-300))).clamp_min(-126) - 7)
+    want = (torch.round(exact / ulp) * ulp).to(torch.bfloat16)      # (half to even; a number of bf16 already)
+    there = torch.isfinite(x) & (x > -88.75)
+    assert torch.equal(y.view(torch.int16)[there], want.view(torch.int16)[there])
+    below = y[torch.isfinite(x) & (x < -88.75)]
+    assert (below == 0).all() and below.signbit().all()
+    wide = a.to("cuda:0").float()
+    division = (wide / (1 + torch.exp(-wide))).bfloat16().cpu()
+    assert torch.equal(y.view(torch.int16)[torch.isfinite(x)], division.view(torch.int16)[torch.isfinite(x)])
+
+
 @pytest.mark.parametrize("rows, cols", [(153593, 1024), (65537, 2400), (19200, 8200)])
 def test_results_that_go_past_the_last_cache(rows, cols):
     """More rows than a grid has, rows that the workgroups' vectors leave ragged, results around 300 MiB: each row is that of a few rows alone."""
