@@ -322,19 +322,20 @@ __global__ void __launch_bounds__(WAVES * 64, D == 64 ? 3 : 2) prefill_f32_kerne
 // from 64 bits 1.31e-7, 1.08, 1.10); one of 1000 64 / 44 / 63; 4 of 2048 283 / 177 / 159; 80 of 50 26 / 22 / 25.  Tried: v_dot2_f32_bf16 for the rests 86 (128 queries), two tiles of values
 // at a time 82, values' products straight into the sums 82 and 2.0e-7, priority for the products 82.
 typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
-// the largest bits of third parts: those of a number that is not finite, or that bf16 rounds to infinity, are no less than 0x7f80
-__device__ __forceinline__ void look(const u32x4 &third, u16x2 &odd) {
+// the largest bits of first parts, those of numbers that are too large and of what is not finite among them
+constexpr uint32_t kTooLarge = (127 + 104) << 7;
+__device__ __forceinline__ void look(const u32x4 &first, u16x2 &odd) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) odd = __builtin_elementwise_max(odd, __builtin_bit_cast(u16x2, third[i] & 0x7fff7fffu));
+  for (int i = 0; i < 4; ++i) odd = __builtin_elementwise_max(odd, __builtin_bit_cast(u16x2, first[i] & 0x7fff7fffu));
 }
 __device__ __forceinline__ u32x2 read_tr(const char *p) {
   typedef __attribute__((ext_vector_type(4))) short s16x4;
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4 *)p));
 }
-// Below 2^-109 three of bf16 do not add up to a number of fp32.  Values and probabilities are taken times 2^16, so that none is without its last bits.  Queries times
-// 2^32: what K loses is then 2^-38 of a score's unit for any query that is not too large for its parts itself (2^96; values: 2^112), and those take the other way.
+// Below 2^-109 three of bf16 do not add up to a number of fp32.  Values and probabilities are taken times 2^16, so that none is without its last bits.  What queries and
+// keys lose, 2^-134 at the most, is 2^-24 of a score's unit beside the largest that are taken (2^104; values: 2^88), and larger ones go the other way.
 // Costs 2 %: 8 prompts of 511 .. 1021 tokens 81.1 -> 83.0 us, 4 of 2048 164 -> 169.
-constexpr float kQueries = 0x1p32f, kValues = 0x1p16f;
+constexpr float kValues = 0x1p16f;
 __device__ __forceinline__ f32x4 mfma(const u32x4 &a, const u32x4 &b, const f32x4 &c) { return mfma16x16x32<bf16_tag>(a, b, c); }
 
 template <int D, int GROUPS>   // (head dim 128: 55 registers in memory; 8 prompts of 511 .. 1021 tokens 255 -> 201 us, one of 1000 111 -> 157)
@@ -378,7 +379,7 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
         float f[8] = {a[0] * by, a[1] * by, a[2] * by, a[3] * by, b[0] * by, b[1] * by, b[2] * by, b[3] * by};
         u32x4 part[3];
         split3<false>(f, part);
-        look(part[2], odd);
+        look(part[0], odd);
 #pragma unroll
         for (int s = 0; s < 3; ++s) *(u32x4 *)((w ? vl : kl) + s * PART + (w ? v_place(row, c) : k_place(row, c))) = part[s];
       }
@@ -390,12 +391,12 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const float *from = (const float *)p.q + (int64_t)(q0 + min(qb + group * 32 + i * 16 + r16, sq - 1)) * p.q_stride + (int64_t)head * D + s * 32 + g * 8;
-      const f32x4 a = *(const f32x4 *)from * kQueries, b = *(const f32x4 *)(from + 4) * kQueries;
+      const f32x4 a = *(const f32x4 *)from, b = *(const f32x4 *)(from + 4);
       float f[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
       split3<false>(f, q[i][s]);
-      look(q[i][s][2], odd);
+      look(q[i][s][0], odd);
     }
-  const float scale_log2 = p.scale * 1.4426950408889634f / kQueries;
+  const float scale_log2 = p.scale * 1.4426950408889634f;
   const bool late = scale_log2 > 0.f;   // scores are multiplied by `mul` where their exponent is formed, without a rounding between
   const float mul = late ? scale_log2 : 1.f;
   float m[2] = {-1e30f, -1e30f}, l[2] = {0.f, 0.f};
@@ -509,7 +510,7 @@ __global__ void __launch_bounds__(256, 2) prefill_parts_kernel(PrefillParams p) 
     swap32(a + b, a, b);
     l[i] = a + b;
   }
-  bool bad = odd[0] >= 0x7f80 || odd[1] >= 0x7f80;
+  bool bad = odd[0] >= kTooLarge || odd[1] >= kTooLarge;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     bad |= !(l[i] < INFINITY);
