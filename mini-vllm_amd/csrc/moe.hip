@@ -587,7 +587,8 @@ __global__ void __launch_bounds__(256, 2) moe_tile_kernel(MoeLinear p) {
 // Very many rows: 128 x 256 per workgroup of four waves side by side, two workgroups to a CU, so that one multiplies while the other starts or ends.
 // Bound by the matrix cores and their power, if the operands are there in time: three stages of 32 inputs, of which two are under way, and the operands of a stage
 // are read one by one between the products of the stage before, as are the next transfers asked for.  A stage takes 1224 cycles where its products are 1024 (two
-// workgroups) and those with their transfers alone 1084, at 1.65 of 2.4 GHz.  Rows come 64 inputs at a time, in whole lines of memory, every other stage.
+// workgroups) and those with their transfers alone 1084, at 1.65 of 2.4 GHz.  And by rounds: 9001 tokens of
+// 4 choices are 1728 gated and 2304 plain workgroups (2048 -> 2 x 768, 768 -> 2048) on 512 places, 3.4 and 4.5 rounds.  Rows come 64 inputs at a time, in whole lines of memory, every other stage.
 // Results leave through LDS, 128 bytes of a row (gated: 64) to a store.
 // Workgroups are dealt to the XCDs in turn, and each XCD gets a run of an eighth of the work (eight tiles of rows and all their outputs at a time, the
 // rows first): its L2 holds what its workgroups share, and none has more than the others.

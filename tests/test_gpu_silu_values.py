@@ -45,7 +45,7 @@ def test_silu_of_bf16_has_the_divisions_bits():
 
 @pytest.mark.parametrize("rows, cols", [(153593, 1024), (65537, 2400), (19200, 8200)])
 def test_results_that_go_past_the_last_cache(rows, cols):
-    """More rows than a grid has, rows that the workgroups' vectors leave ragged, results around 300 MiB: each row is that of a few rows alone."""
+    """More rows than a grid has, rows that the workgroups' vectors leave ragged, results of more than 300 MB: each row is that of a few rows alone."""
     from minivllm_amd import hip_ops as H
 
     g = torch.Generator(device="cuda:0").manual_seed(cols)
