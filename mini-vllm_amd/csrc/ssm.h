@@ -14,3 +14,7 @@ __device__ __forceinline__ float softplus_f32(float z) { return fmaxf(z, 0.f) + 
 // chunked form (16-bit); MV_E_SHAPE when it does not apply.  Without the workspace sequences are not cut into segments
 size_t mv_ssm_chunk_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n);
 int mv_ssm_chunk_launch(const MvSsmArgs &a, void *workspace, size_t ws_bytes, int total_q, int dtype, hipStream_t stream);
+bool mv_ssm_chunk_cuts(int n_seqs, int total_q, int max_q, int heads, int p, int n);   // into segments
+// the same for heads of 64 columns that share b and c
+size_t mv_ssm_heads_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n);
+int mv_ssm_heads_launch(const MvSsmArgs &a, void *workspace, size_t ws_bytes, int total_q, int dtype, hipStream_t stream);

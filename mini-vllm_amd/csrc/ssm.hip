@@ -353,8 +353,10 @@ extern "C" int mv_causal_conv(const MvSsmArgs *a, int dtype, void *stream) {
 }
 
 extern "C" size_t mv_ssm_prefill_workspace_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int dtype) {
-  if (n_seqs <= 0 || total_q <= 0 || max_q <= 0 || heads <= 0 || p <= 0 || (p & 15) || n <= 0 || dtype == MV_F32) return 0;
-  return mv_ssm_chunk_workspace(n_seqs, total_q, max_q, heads, p, n);
+  const bool shared = dtype & MV_SSM_SHARED;
+  if (n_seqs <= 0 || total_q <= 0 || max_q <= 0 || heads <= 0 || p <= 0 || (p & 15) || n <= 0 || (dtype & ~MV_SSM_SHARED) == MV_F32) return 0;
+  const size_t need = mv_ssm_chunk_workspace(n_seqs, total_q, max_q, heads, p, n), more = shared ? mv_ssm_heads_workspace(n_seqs, total_q, max_q, heads, p, n) : 0;
+  return more > need ? more : need;
 }
 
 extern "C" int mv_ssm_prefill_ws(const MvSsmArgs *a, void *workspace, size_t ws_bytes, int total_q, int dtype, int flags, void *stream) {

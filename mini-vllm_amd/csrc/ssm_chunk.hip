@@ -396,6 +396,8 @@ int launch(const MvSsmArgs &a, int seg, void *workspace, int total_q, hipStream_
 
 }  // namespace
 
+bool mv_ssm_chunk_cuts(int n_seqs, int total_q, int max_q, int heads, int p, int n) { return pick_segment(n_seqs, total_q, max_q, heads, p, n) != 0; }
+
 // states and decays of the segments, and the states that sequences come with
 size_t mv_ssm_chunk_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n) {
   const int seg = pick_segment(n_seqs, total_q, max_q, heads, p, n);
@@ -406,6 +408,8 @@ size_t mv_ssm_chunk_workspace(int n_seqs, int total_q, int max_q, int heads, int
 }
 
 int mv_ssm_chunk_launch(const MvSsmArgs &a, void *workspace, size_t ws_bytes, int total_q, int dtype, hipStream_t stream) {
+  const int rc = mv_ssm_heads_launch(a, workspace, ws_bytes, total_q, dtype, stream);
+  if (rc != MV_E_SHAPE) return rc;
   const size_t need = workspace ? mv_ssm_chunk_workspace(a.n_seqs, total_q, a.max_q, a.heads, a.p, a.n) : 0;
   const int seg = need && ws_bytes >= need ? pick_segment(a.n_seqs, total_q, a.max_q, a.heads, a.p, a.n) : 0;
 #define MV_SN(N_) \

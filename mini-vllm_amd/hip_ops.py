@@ -1498,6 +1498,7 @@ def latent_prefill(q, k, v, rot, cu_q, cu_k, max_q: int, max_k: int, positions, 
 
 # ---------------------------------------------------------------- K15
 MV_SSM_SCAN = 1
+MV_SSM_SHARED = 1 << 8
 
 
 def _ssm_args(shape, x, state_slots, out, conv_w=None, conv_b=None, conv_state=None, ssm_state=None, dt=None, dt_bias=None,
@@ -1556,7 +1557,8 @@ def ssm_prefill(x, dt, dt_bias, a_log, d, shape, ssm_state, state_slots, cu_q, c
     a.cu_q, a.cu_k, a.max_q = cu_q.data_ptr(), cu_k.data_ptr(), int(max_q)
     rows = x.shape[0]
     # (five chunks of 64 tokens and fewer are never cut)
-    n = 0 if flags & MV_SSM_SCAN or a.max_q <= 320 else int(_lib.mv_ssm_prefill_workspace_bytes(a.n_seqs, rows, a.max_q, a.heads, a.p, a.n, _dt(x)))
+    shared = 0 if a.heads // a.groups % 4 else MV_SSM_SHARED
+    n = 0 if flags & MV_SSM_SCAN or a.max_q <= 320 else int(_lib.mv_ssm_prefill_workspace_bytes(a.n_seqs, rows, a.max_q, a.heads, a.p, a.n, _dt(x) | shared))
     ws = torch.empty((n,), dtype=torch.uint8, device=x.device) if n else None
     _check(_lib.mv_ssm_prefill_ws(ctypes.byref(a), _ptr(ws), n, rows, _dt(x), int(flags), _stream()), "mv_ssm_prefill")
     return out
