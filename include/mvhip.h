@@ -776,6 +776,22 @@ typedef struct MvMoeLinearArgs {
   int max_tiles, tile_m, n, k;
 } MvMoeLinearArgs;
 int mv_moe_linear(const MvMoeLinearArgs *args, int dtype, void *stream);
+/* Router, grouping and both products of rows of x [rows][x_stride] in one call: weights [rows][top] and place [pairs] as from mv_moe_route and mv_moe_group,
+ * out [pairs][width] by place.  gate_up [experts][2][ff][k], down [experts][width][ff] as mv_moe_linear takes them; router [outputs][router_k], router_k <= k;
+ * weigh_inputs: the weights multiply the first product's inputs.  workspace: mv_moe_mlp_workspace_bytes(), aligned to 16.  tile_m: with MV_MOE_QUARTERS as
+ * mv_moe_linear takes it */
+typedef struct {
+  const void *x, *router, *correction, *gate_up, *down;
+  const MvGateAct *act;
+  float *weights;
+  int32_t *place;
+  void *out, *workspace;
+  int64_t x_stride, ws_bytes;
+  int rows, k, router_k, outputs, top, groups, keep, route_flags, experts, tile_m, ff, width, weigh_inputs;
+  float scale;
+} MvMoeMlpArgs;
+size_t mv_moe_mlp_workspace_bytes(int rows, int top, int experts, int tile_m, int ff, int dtype);
+int mv_moe_mlp(const MvMoeMlpArgs *args, int dtype, void *stream);
 
 /* ---- K18 — one edge of several residual streams (hyper-connections), kept in fp32: x [rows][streams][cols].  Per row:
  *     x'_j = sum_i mix[i][j] x_i + out_w[j] y      (embed given instead: x'_j = embed[ids[row]] for every j)

@@ -898,3 +898,53 @@ extern "C" int mv_moe_linear(const MvMoeLinearArgs *a, int dtype, void *stream) 
   if (dtype == MV_BF16) return a->act ? launch_linear<bf16_tag, true>(p, a->tile_m, a->max_tiles, st) : launch_linear<bf16_tag, false>(p, a->tile_m, a->max_tiles, st);
   return a->act ? launch_linear<f16_tag, true>(p, a->tile_m, a->max_tiles, st) : launch_linear<f16_tag, false>(p, a->tile_m, a->max_tiles, st);
 }
+
+namespace {
+// scratch memory of mv_moe_mlp: where its parts begin, in bytes
+struct MlpParts {
+  int64_t tokens, tiles, weights, z, end, max_tiles;
+};
+MlpParts mlp_parts(int rows, int top, int experts, int tile_m, int ff, int dtype) {
+  const auto up = [](int64_t v) { return (v + 255) & ~(int64_t)255; };
+  const int64_t pairs = (int64_t)rows * top, each = up(pairs * 4);
+  MlpParts m;
+  m.max_tiles = pairs / (tile_m & 0xffff) + experts;
+  m.tokens = each, m.tiles = 2 * each, m.weights = m.tiles + up(m.max_tiles * 12), m.z = m.weights + each;
+  m.end = m.z + pairs * ff * (dtype == MV_F32 ? 4 : 2);
+  return m;
+}
+}  // namespace
+
+extern "C" size_t mv_moe_mlp_workspace_bytes(int rows, int top, int experts, int tile_m, int ff, int dtype) {
+  if (rows <= 0 || top <= 0 || experts <= 0 || (tile_m & 0xffff) <= 0 || ff <= 0) return 0;
+  return (size_t)mlp_parts(rows, top, experts, tile_m, ff, dtype).end;
+}
+
+extern "C" int mv_moe_mlp(const MvMoeMlpArgs *a, int dtype, void *stream) {
+  if (!a) return MV_E_NULLPTR;
+  if (a->rows == 0) return MV_OK;
+  if (!a->workspace || !a->weights || !a->place || !a->out || !a->act) return MV_E_NULLPTR;
+  if (dtype != MV_BF16 && dtype != MV_F16 && dtype != MV_F32) return MV_E_DTYPE;
+  if (a->rows < 0 || a->top <= 0 || (int64_t)a->rows * a->top > INT32_MAX || a->experts <= 0 || (a->tile_m & 0xffff) <= 0 || a->ff <= 0 ||
+      a->router_k > a->k || a->outputs < a->experts)
+    return MV_E_SHAPE;
+  const MlpParts m = mlp_parts(a->rows, a->top, a->experts, a->tile_m, a->ff, dtype);
+  if (!mv_aligned16(a->workspace)) return MV_E_ALIGN;
+  if (a->ws_bytes < m.end || m.max_tiles > INT32_MAX) return MV_E_SHAPE;
+  char *ws = (char *)a->workspace;
+  int32_t *ids = (int32_t *)ws, *tokens = (int32_t *)(ws + m.tokens), *tiles = (int32_t *)(ws + m.tiles);
+  float *by_place = a->weigh_inputs ? (float *)(ws + m.weights) : nullptr;
+  const int pairs = a->rows * a->top, max_tiles = (int)m.max_tiles;
+  if (int rc = mv_moe_route(a->x, a->x_stride, a->router, a->correction, ids, a->weights, a->rows, a->router_k, a->outputs, a->top, a->groups, a->keep, a->scale,
+                            a->route_flags, dtype, stream))
+    return rc;
+  if (int rc = mv_moe_group(ids, pairs, a->top, a->experts, a->tile_m & 0xffff, max_tiles, a->place, tokens, tiles, by_place ? a->weights : nullptr, by_place, stream))
+    return rc;
+  MvMoeLinearArgs p{};
+  p.x = a->x, p.w = a->gate_up, p.out = ws + m.z, p.tokens = tokens, p.tiles = tiles, p.act = a->act, p.in_scale = by_place;
+  p.x_stride = a->x_stride, p.out_stride = a->ff, p.max_tiles = max_tiles, p.tile_m = a->tile_m, p.n = a->ff, p.k = a->k;
+  if (int rc = mv_moe_linear(&p, dtype, stream)) return rc;
+  p.x = ws + m.z, p.w = a->down, p.out = a->out, p.tokens = nullptr, p.act = nullptr, p.in_scale = nullptr;
+  p.x_stride = a->ff, p.out_stride = a->width, p.n = a->width, p.k = a->ff;
+  return mv_moe_linear(&p, dtype, stream);
+}

@@ -108,6 +108,8 @@ _SIGNATURES = {
     "mv_gru_prefill": (c_int, [c_void_p, c_int, c_void_p]),
     "mv_gru_step": (c_int, [c_void_p, c_int, c_void_p]),
     "mv_moe_linear": (c_int, [c_void_p, c_int, c_void_p]),
+    "mv_moe_mlp_workspace_bytes": (c_size_t, [c_int] * 6),
+    "mv_moe_mlp": (c_int, [c_void_p, c_int, c_void_p]),
     "mv_gated_act_small_m": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_void_p, c_int64, c_int, c_int, c_int, c_void_p,
                                      c_int, c_int, c_void_p]),
     "mv_gated_act_mid_m": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p, c_int, c_int,
@@ -255,6 +257,9 @@ MvMoeLinearArgs = _struct(
     "MvMoeLinearArgs", x__w__out__tokens__tiles__act__in_scale=c_void_p, x_stride__out_stride=c_int64, max_tiles__tile_m__n__k=c_int)
 
 
+MvMoeMlpArgs = _struct(
+    "MvMoeMlpArgs", x__router__correction__gate_up__down__act__weights__place__out__workspace=c_void_p, x_stride__ws_bytes=c_int64,
+    rows__k__router_k__outputs__top__groups__keep__route_flags__experts__tile_m__ff__width__weigh_inputs=c_int, scale=c_float)
 MvStreamArgs = _struct(
     "MvStreamArgs", x__x_out__y__mix__out_w__embed__ids__in_w__norm_w__shift__out__moe_out__moe_rows__moe_w__prev__positions__state_slots__cu_q=c_void_p,
     y_stride__out_stride__vocab__slots=c_int64, streams__y_splits__moe_top__n_seqs=c_int, eps=c_float, reserved=c_int)
@@ -365,7 +370,8 @@ def _ptr(t):
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # (torch.cuda.current_stream() makes an object around this number, 2.5 us of a call's 10; the tensors of a call have made the device known by now)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need_cuda(*ts):
@@ -1778,6 +1784,31 @@ def moe_linear(x, w, n: int, groups: ExpertGroups, act: GateAct | None = None, g
                         tile_m=groups.tile_m | (MV_MOE_QUARTERS if quarters else 0), n=n, k=k)
     _check(_lib.mv_moe_linear(ctypes.byref(a), _dt(x), _stream()), "mv_moe_linear")
     return out
+
+
+def moe_mlp(x, router, correction, gate_up, down, experts: int, ff: int, width: int, top: int, tile_m: int, act: GateAct, groups: int = 1, keep: int = 1,
+            scale: float = 1.0, sigmoid: bool = False, raw: bool = False, weigh_inputs: bool = False, quarters: bool = False):
+    """``moe_route``, ``moe_group`` and both ``moe_linear`` as one call -> (rows by place [pairs, width], place, weights [T, top])."""
+    _need_cuda(x, router, correction, gate_up, down)
+    _rows_ok("x", x, router.shape[1], gate_up.dtype)
+    rows, k, dtype = x.shape[0], x.shape[1], x.dtype
+    if router.dtype != dtype or not router.is_contiguous() or (correction is not None and (correction.dtype != dtype
+                                                                                          or correction.numel() != router.shape[0])):
+        raise MvHipError(f"router weight [outputs, K] and correction [outputs] of {dtype} required")
+    if (not gate_up.is_contiguous() or gate_up.numel() != experts * ff * k * 2 or not down.is_contiguous() or down.numel() != experts * width * ff
+            or down.dtype != dtype):
+        raise MvHipError(f"weights of {experts} experts, {k} -> 2 x {ff} and {ff} -> {width}, of {dtype} required")
+    dt, device, tile_m = _dt(x), x.device, tile_m | (MV_MOE_QUARTERS if quarters else 0)
+    need = _lib.mv_moe_mlp_workspace_bytes(rows, top, experts, tile_m, ff, dt)
+    ws = torch.empty((need,), dtype=torch.uint8, device=device)
+    weights = torch.empty((rows, top), dtype=torch.float32, device=device)
+    place = torch.empty((rows * top,), dtype=torch.int32, device=device)
+    out = torch.empty((rows * top, width), dtype=dtype, device=device)
+    a = MvMoeMlpArgs(x.data_ptr(), router.data_ptr(), _ptr(correction), gate_up.data_ptr(), down.data_ptr(), ctypes.addressof(act), weights.data_ptr(),
+                     place.data_ptr(), out.data_ptr(), ws.data_ptr(), x.stride(0), need, rows, k, router.shape[1], router.shape[0], top, groups, keep,
+                     (MV_ROUTE_SIGMOID if sigmoid else 0) | (MV_ROUTE_RAW if raw else 0), experts, tile_m, ff, width, int(weigh_inputs), float(scale))
+    _check(_lib.mv_moe_mlp(ctypes.byref(a), dt, _stream()), "mv_moe_mlp")
+    return out, place, weights
 
 
 # ---------------------------------------------------------------- K18

@@ -89,12 +89,17 @@ class GatedDeltaRule(nn.Module):
             a, gate = z[:, at["a"]:at["a"] + s.heads], z[:, at["g"]:at["g"] + s.heads * s.p]
         slots = ctx.state_slots
         nd = ctx.decode_rows if ctx.is_prefill else t
+        # (a slice is a microsecond or two of the host's: none where it would be the whole)
         if nd:
-            hip_ops.delta_step(s, x[:nd], beta[:nd], a[:nd], self.dt_bias, self.A_log, self.conv, self.conv_state, self.state, slots[:nd],
-                               ctx.context_lens[:nd], gate[:nd], self.norm, self.gate, self.out_scale, out=out[:nd])
+            first = (lambda v: v) if nd == t else (lambda v: v[:nd])
+            hip_ops.delta_step(s, first(x), first(beta), first(a), self.dt_bias, self.A_log, self.conv, self.conv_state, self.state,
+                               slots if slots.shape[0] == nd else slots[:nd], ctx.context_lens if ctx.context_lens.shape[0] == nd else ctx.context_lens[:nd],
+                               first(gate), self.norm, self.gate, self.out_scale, out=first(out))
         if nd < t:
             cu_q, cu_k, max_q = ((ctx.rest_cum_seqlens_q, ctx.rest_cum_seqlens_k, ctx.rest_max_seqlen_q) if nd else
                                  (ctx.cum_seqlens_q, ctx.cum_seqlens_k, ctx.max_seqlen_q))
-            xc = hip_ops.causal_conv(x[nd:], self.conv, None, s.conv, self.conv_state, slots[nd:], cu_q, cu_k, max_q)
-            hip_ops.delta_prefill(s, xc, beta[nd:], a[nd:], self.dt_bias, self.A_log, self.state, slots[nd:], cu_q, cu_k, max_q, out=out[nd:],
-                                  gate=gate[nd:], norm_w=self.norm, gate_kind=self.gate, out_scale=self.out_scale)
+            rest = (lambda v: v[nd:]) if nd else (lambda v: v)
+            slots = rest(slots)
+            xc = hip_ops.causal_conv(rest(x), self.conv, None, s.conv, self.conv_state, slots, cu_q, cu_k, max_q)
+            hip_ops.delta_prefill(s, xc, rest(beta), rest(a), self.dt_bias, self.A_log, self.state, slots, cu_q, cu_k, max_q, out=rest(out),
+                                  gate=rest(gate), norm_w=self.norm, gate_kind=self.gate, out_scale=self.out_scale)

@@ -101,19 +101,13 @@ class ExpertMLP(nn.Module):
         wide = rows * math.ceil(2 * self.f / 256) >= WIDE_GROUPS[0] and rows * math.ceil(self.w / 256) >= WIDE_GROUPS[1]
         return 256 if wide else 64
 
-    def route(self, h):
-        """-> (weights [T, top], the pairs sorted by expert)."""
-        ids, weights = hip_ops.moe_route(h, self.router, self.correction, self.top, self.groups, self.keep, self.scale, self.sigmoid,
-                                         self.raw_weights)
-        return weights, hip_ops.moe_group(ids, self.experts, self.tile_rows(h.shape[0]), weights if self.weigh_inputs else None)
-
     def forward(self, h):
         """-> (shared expert's output or None, the routed experts' part for ``hip_ops.residual_update``)."""
-        weights, g = self.route(h)
-        quarters = g.tile_m == 64 and h.shape[0] * self.top <= QUARTERS * self.experts
-        z = hip_ops.moe_linear(h, self.gate_up, self.f, g, self.act, gather=True, experts=self.experts, in_scale=g.weights, quarters=quarters)
-        y = hip_ops.moe_linear(z, self.down, self.w, g, experts=self.experts, quarters=quarters)
+        tile = self.tile_rows(h.shape[0])
+        y, place, weights = hip_ops.moe_mlp(h, self.router, self.correction, self.gate_up, self.down, self.experts, self.f, self.w, self.top, tile, self.act,
+                                            self.groups, self.keep, self.scale, self.sigmoid, self.raw_weights, self.weigh_inputs,
+                                            tile == 64 and h.shape[0] * self.top <= QUARTERS * self.experts)
         shared = None
         if self.shared_gate_up is not None:
             shared = self.shared_down(gated_linear(h, self.shared_gate_up, "silu"), partial_ok=True)
-        return shared, (y, g.place, None if self.weigh_inputs else weights)
+        return shared, (y, place, None if self.weigh_inputs else weights)
