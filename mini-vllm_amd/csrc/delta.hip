@@ -349,7 +349,8 @@ extern "C" size_t mv_delta_prefill_segments_bytes(int n_seqs, int total_q, int m
   return dtype == MV_F32 || (dtype == MV_BF16 && !channel_decay) ? 0 : mv_delta_segments_workspace(n_seqs, total_q, max_q, heads, p, n);
 }
 
-extern "C" int mv_delta_prefill(const MvDeltaArgs *a, int dtype, int flags, void *stream) {
+// raw: the channels ahead of the convolution, which the first launch does along the way (mv_delta_scalar_takes_conv), or NULL
+static int prefill(const MvDeltaArgs *a, const void *raw, int64_t raw_stride, int dtype, int flags, void *stream) {
   if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
   if (int e = check_delta(a, dtype)) return e;
   if (!a->cu_q || !a->cu_k) return MV_E_NULLPTR;
@@ -366,14 +367,34 @@ extern "C" int mv_delta_prefill(const MvDeltaArgs *a, int dtype, int flags, void
   };
   if (dtype != MV_F32 && !(flags & MV_DELTA_SCAN)) {
     bool normed = flags & MV_DELTA_NORM_WALK;
-    const int rc = mv_delta_chunk_launch(*a, dtype, norm ? &normed : nullptr, (hipStream_t)stream);
-    if (rc != MV_E_SHAPE) return behind(rc, normed);
+    const int rc = mv_delta_chunk_launch(*a, raw, raw_stride, dtype, norm ? &normed : nullptr, (hipStream_t)stream);
+    if (rc != MV_E_SHAPE || raw) return behind(rc, normed);
   }
   const size_t lds = (size_t)(3 * kScanRows * a->n + kScanRows * 17) * 4;
   const dim3 grid(a->p / 16, a->heads, a->n_seqs);
   MV_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((delta_scan_kernel<Tag>), grid, dim3(256), lds, (hipStream_t)stream, *a));
   MV_LAUNCH_CHECK();
   return behind(MV_OK, false);
+}
+
+extern "C" int mv_delta_prefill(const MvDeltaArgs *a, int dtype, int flags, void *stream) { return prefill(a, nullptr, 0, dtype, flags, stream); }
+
+extern "C" int mv_delta_prefill_conv(const MvDeltaArgs *a, void *xc, int dtype, int flags, void *stream) {
+  if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
+  if (!a || !xc) return MV_E_NULLPTR;
+  MvSsmArgs c{};
+  c.x = a->x, c.x_stride = a->x_stride, c.conv_w = a->conv_w, c.conv_state = a->conv_state, c.state_slots = a->state_slots, c.cu_q = a->cu_q, c.cu_k = a->cu_k;
+  c.out = xc, c.out_stride = a->channels, c.slots = a->conv_state ? a->slots : 0, c.n_seqs = a->n_seqs, c.max_q = a->max_q, c.channels = a->channels, c.taps = a->taps;
+  c.heads = a->heads, c.groups = a->groups, c.p = a->p, c.n = a->n, c.b_off = a->k_off, c.c_off = a->q_off;
+  MvDeltaArgs d = *a;
+  d.x = xc, d.x_stride = a->channels;
+  if (int e = mv_check_conv(&c, dtype)) return e;
+  if (int e = check_delta(&d, dtype)) return e;
+  if (dtype == MV_BF16 && !a->channel_decay && !(flags & MV_DELTA_SCAN) && a->workspace && (a->conv_state || a->taps == 1 || !a->slots) &&
+      mv_delta_chunk_workspace(a->n_seqs, a->total_q, a->heads, a->p, a->n) && mv_delta_scalar_takes_conv(*a))
+    return prefill(&d, a->x, a->x_stride, dtype, flags, stream);
+  if (int rc = mv_causal_conv(&c, dtype, stream)) return rc;
+  return prefill(&d, nullptr, 0, dtype, flags, stream);
 }
 
 extern "C" int mv_delta_step(const MvDeltaArgs *a, int dtype, void *stream) {

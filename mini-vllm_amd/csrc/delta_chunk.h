@@ -36,6 +36,8 @@ __device__ __forceinline__ float softplus_fast(float z) {
 struct DeltaPrep {
   MvDeltaArgs a;
   char *ws;
+  const void *raw;      // channels ahead of the convolution, or NULL: a.x is there already
+  int64_t raw_stride;
 };
 
 // chunk slot -> sequence (its slots start at cu_q / L + its number)

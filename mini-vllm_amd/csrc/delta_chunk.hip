@@ -877,14 +877,14 @@ size_t mv_delta_segments_workspace(int n_seqs, int total_q, int max_q, int heads
   return ((slots + n_seqs) * p + slots + slots * n) * (size_t)heads * n * 4;
 }
 
-int mv_delta_chunk_launch(const MvDeltaArgs &a, int dtype, bool *normed, hipStream_t stream) {
+int mv_delta_chunk_launch(const MvDeltaArgs &a, const void *raw, int64_t raw_stride, int dtype, bool *normed, hipStream_t stream) {
   const size_t need = mv_delta_chunk_workspace(a.n_seqs, a.total_q, a.heads, a.p, a.n);
   if (!need || !a.workspace) return MV_E_SHAPE;   // larger states: token by token
   if ((size_t)a.ws_bytes < need || !mv_aligned16(a.workspace)) return MV_E_WORKSPACE;
   if (!mv_aligned16(a.x) || (a.x_stride & 7) || (a.k_off & 7) || (a.q_off & 7) || a.total_q > 64 * 1000000) return MV_E_ALIGN;
   if (a.channel_decay && (!mv_aligned16(a.a) || (a.a_stride & 7) || !mv_aligned16(a.dt_bias))) return MV_E_ALIGN;
-  const DeltaPrep q{a, (char *)a.workspace};
-  if (!a.channel_decay && dtype == MV_BF16) return mv_delta_scalar_launch(a, normed, stream);
+  const DeltaPrep q{a, (char *)a.workspace, nullptr, 0};
+  if (!a.channel_decay && dtype == MV_BF16) return mv_delta_scalar_launch(a, raw, raw_stride, normed, stream);
   if (normed) *normed = false;
   const size_t more = mv_delta_segments_workspace(a.n_seqs, a.total_q, a.max_q, a.heads, a.p, a.n);
   const int seg = more && (size_t)a.ws_bytes >= need + more ? pick_segment(a.n_seqs, a.total_q, a.max_q, a.heads, a.p, a.n) : 0;

@@ -23,8 +23,13 @@ __device__ __forceinline__ int row_place(int row, int chunk) { return row * 4 + 
 
 // Workgroup = HEADS heads of four waves each that share k and q of a chunk: the products k k^T and q k^T are theirs in common, decays, solution and results
 // their own.  Bound by the latency of its phases, which 16 to 20 waves a CU cover in part: everything is asked for from memory at the start.
-template <int NK, int HEADS>
-__global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(DeltaPrep q) {
+// CONV (q.raw: projected channels; a group's heads are this workgroup's): the causal convolution and silu of causal_conv_kernel (the same sums) ahead of it, four
+// channels and eight tokens a thread and turn, into a.x, where the walk reads it, and k and q into LDS at once: a launch and a way of k and q through memory less.  Four
+// channels, not eight: 80 registers leave three workgroups a CU, whose convolutions run beside the others' chains.  16 heads over 8 of 128 x 128, 16 sequences of up
+// to 1490 tokens: 64 + 55 us as two launches, 120 with eight channels, 111 now (416 MB, 3.7 TB/s; a copy 4.7); the layer 248 -> 242.  Few tokens are the host's and a
+// launch's: 70 tokens of one sequence 57 -> 33.
+template <int NK, int HEADS, bool CONV>
+__global__ void __launch_bounds__(256 * HEADS, CONV ? 6 : 4) delta_scalar_prepare_kernel(DeltaPrep q) {
   typedef uint16_t T;
   typedef elem<B16>::T E;
   constexpr int N = NK * 32, KS = N + 8, W = 4 * HEADS;   // LDS row stride
@@ -47,12 +52,14 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
   // the same sum in either form); a head's first wave its betas and log2 decays, a lane a token
   {
     const int t = (tid & 255) >> 2, part = tid & 3;
-    const T *row = x + (int64_t)min(t, nt - 1) * p.x_stride + grp * N + part * 8;
     u32x4 a[NK], b[HEADS > 1 ? 1 : NK];
+    if constexpr (!CONV) {
+      const T *row = x + (int64_t)min(t, nt - 1) * p.x_stride + grp * N + part * 8;
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      a[i] = *(const u32x4 *)(row + (of ? p.q_off : p.k_off) + 32 * i);
-      if constexpr (HEADS == 1) b[i] = *(const u32x4 *)(row + p.q_off + 32 * i);
+      for (int i = 0; i < NK; ++i) {
+        a[i] = *(const u32x4 *)(row + (of ? p.q_off : p.k_off) + 32 * i);
+        if constexpr (HEADS == 1) b[i] = *(const u32x4 *)(row + p.q_off + 32 * i);
+      }
     }
     const bool leads = (wave & 3) == 0;
     float beta = 0.f, decay = 0.f, bias = 0.f, rate = 0.f;
@@ -60,6 +67,81 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
       const int64_t at = q0 + t0 + min(lane, nt - 1);
       beta = elem<B16>::ld(((const E *)p.beta)[at * p.beta_stride + head]), decay = elem<B16>::ld(((const E *)p.a)[at * p.a_stride + head]);
       rate = elem<B16>::ld(((const E *)p.a_log)[head]), bias = elem<B16>::ld(((const E *)p.dt_bias)[head]);
+    }
+    if constexpr (CONV) {
+      constexpr int TAPS = 4, ROWS = 8;
+      const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq], back = p.taps - 1, first = blockIdx.y * HEADS * p.p;
+      const bool keep = slot >= 0 && slot < p.slots;
+      const int64_t half = p.slots * back * p.channels;
+      const T *conv_w = (const T *)p.conv_w, *from = (const T *)q.raw + (int64_t)q0 * q.raw_stride;
+      const T *old_state = (const T *)p.conv_state + (before & 1) * half + (int64_t)(keep ? slot : 0) * back * p.channels;
+      T *xc = (T *)p.x + (int64_t)q0 * p.x_stride;
+      const int pieces = (2 * N + HEADS * p.p) / 4;   // of a token: k, q, the heads' v
+      const auto unpack4 = [](const u32x2 &v, float (&f)[4]) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) f[2 * i] = u2f(v[i] << 16), f[2 * i + 1] = u2f(v[i] & 0xffff0000u);
+      };
+      for (int item = tid; item < pieces * (L / ROWS); item += 256 * HEADS) {
+        const int piece = item % pieces, tr = item / pieces * ROWS, which = piece / (N / 4);   // 0: k, 1: q
+        const int c = which == 0 ? p.k_off + grp * N + piece * 4 : which == 1 ? p.q_off + grp * N + (piece - N / 4) * 4 : first + (piece - N / 2) * 4;
+        auto input = [&](int t) {   // input `t` of the step (t < 0: of the steps before it)
+          if (t >= 0) return *(const u32x2 *)(from + (int64_t)min(t, len - 1) * q.raw_stride + c);
+          if (before > 0 && keep && back + t >= 0) return *(const u32x2 *)(old_state + (int64_t)(back + t) * p.channels + c);
+          return u32x2{0u, 0u};
+        };
+        float w[TAPS][4], win[TAPS][4];
+        if (tr >= nt && which > 1) continue;
+        u32x2 raw[TAPS - 1], rows[ROWS];
+#pragma unroll
+        for (int i = 0; i < TAPS - 1; ++i) raw[i] = input(t0 + tr + i - (TAPS - 1));
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u) rows[u] = input(t0 + tr + u);
+#pragma unroll
+        for (int i = 0; i < TAPS; ++i) {
+          const int tap = i - (TAPS - p.taps);   // (weights stand at the current token's end)
+          u32x2 v = {0u, 0u};
+          if (tap >= 0) v = *(const u32x2 *)(conv_w + (int64_t)tap * p.channels + c);
+          unpack4(v, w[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < TAPS - 1; ++i) unpack4(raw[i], win[i + 1]);   // shifted down below
+        if (t0 + tr == 0 && keep && back > 0) {   // the only thread that reads the old state here writes the new one, behind its reads
+          u32x2 last[TAPS - 1];
+#pragma unroll
+          for (int j = 0; j < TAPS - 1; ++j)
+            if (j < back) last[j] = input(len - back + j);
+          T *ns = (T *)p.conv_state + ((before + len) & 1) * half + (int64_t)slot * back * p.channels + c;
+#pragma unroll
+          for (int j = 0; j < TAPS - 1; ++j)
+            if (j < back) *(u32x2 *)(ns + (int64_t)j * p.channels) = last[j];
+        }
+#pragma unroll
+        for (int u = 0; u < ROWS; ++u) {
+#pragma unroll
+          for (int i = 0; i < TAPS - 1; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) win[i][j] = win[i + 1][j];
+          unpack4(rows[u], win[TAPS - 1]);
+          f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < TAPS; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = fmaf(win[i][j], w[i][j], o[j]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[j] = silu_of<B16>(o[j]);
+          u32x2 done = pack_quad<B16>(o);
+          if (tr + u < nt) *(u32x2 *)(xc + (int64_t)(t0 + tr + u) * p.x_stride + c) = done;
+          else done = u32x2{0u, 0u};
+          if (which == 0) *(u32x2 *)(ks + (tr + u) * KS + piece * 4) = done;
+          if (which == 1) *(u32x2 *)(qs + (tr + u) * KS + (piece - N / 4) * 4) = done;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < NK; ++i) {
+        a[i] = *(const u32x4 *)((of ? qs : ks) + t * KS + part * 8 + 32 * i);
+        if constexpr (HEADS == 1) b[i] = *(const u32x4 *)(qs + t * KS + part * 8 + 32 * i);
+      }
     }
     auto length = [&](u32x4 *raw, T *to, float scale) {
       float sum = 0.f;
@@ -70,7 +152,7 @@ __global__ void __launch_bounds__(256 * HEADS, 4) delta_scalar_prepare_kernel(De
         unpack8<B16>(raw[i], f);
 #pragma unroll
         for (int j = 0; j < 8; ++j) sum = fmaf(f[j], f[j], sum);
-        *(u32x4 *)(to + t * KS + part * 8 + 32 * i) = raw[i];
+        if constexpr (!CONV) *(u32x4 *)(to + t * KS + part * 8 + 32 * i) = raw[i];
       }
       return scale / sqrtf(lanes_sum<4>(sum) + p.unit_eps);
     };
@@ -505,8 +587,11 @@ template <int NK>
 int launch(const DeltaPrep &q, bool *normed, hipStream_t stream) {
   const MvDeltaArgs &a = q.a;
   const unsigned slots = (unsigned)chunk_slots(a.n_seqs, a.total_q);
-  if (a.heads / a.groups % 2 == 0) hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 2>), dim3(slots, a.heads / 2), dim3(512), 0, stream, q);
-  else hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 1>), dim3(slots, a.heads), dim3(256), 0, stream, q);
+  const int of_group = a.heads / a.groups;
+  if (q.raw && of_group == 2) hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 2, true>), dim3(slots, a.heads / 2), dim3(512), 0, stream, q);
+  else if (q.raw) hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 1, true>), dim3(slots, a.heads), dim3(256), 0, stream, q);
+  else if (of_group % 2 == 0) hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 2, false>), dim3(slots, a.heads / 2), dim3(512), 0, stream, q);
+  else hipLaunchKernelGGL((delta_scalar_prepare_kernel<NK, 1, false>), dim3(slots, a.heads), dim3(256), 0, stream, q);
   MV_LAUNCH_CHECK();
   // Eight waves where workgroups of four would be more than the CUs, of which each holds one, and LDS holds their chunk (up to 128 channels: at
   // 160 four waves of one tile it is, 16 heads and 16 sequences of 1000 tokens 201 us, where four waves of two tiles took 211)
@@ -520,9 +605,15 @@ int launch(const DeltaPrep &q, bool *normed, hipStream_t stream) {
 
 }  // namespace
 
+// The convolution goes along where every channel is one workgroup's (which reads and writes what is kept of it) and a thread's window holds the taps
+bool mv_delta_scalar_takes_conv(const MvDeltaArgs &a) {
+  const int of_group = a.heads / a.groups;
+  return of_group <= 2 && a.taps >= 1 && a.taps <= 4 && a.k_off == a.heads * a.p && a.q_off == a.k_off + a.groups * a.n && a.channels == a.q_off + a.groups * a.n;
+}
+
 // (arguments checked by mv_delta_chunk_launch, whose workspace is larger)
-int mv_delta_scalar_launch(const MvDeltaArgs &a, bool *normed, hipStream_t stream) {
-  const DeltaPrep q{a, (char *)a.workspace};
+int mv_delta_scalar_launch(const MvDeltaArgs &a, const void *raw, int64_t raw_stride, bool *normed, hipStream_t stream) {
+  const DeltaPrep q{a, (char *)a.workspace, raw, raw_stride};
   switch (a.n / 32) {
     case 1: return launch<1>(q, normed, stream);
     case 2: return launch<2>(q, normed, stream);

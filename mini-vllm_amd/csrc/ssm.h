@@ -11,6 +11,8 @@ __device__ __forceinline__ float silu_of(float z) {
 }
 __device__ __forceinline__ float softplus_f32(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 
+int mv_check_conv(const MvSsmArgs *a, int dtype);   // what mv_causal_conv refuses
+
 // chunked form (16-bit); MV_E_SHAPE when it does not apply.  Without the workspace sequences are not cut into segments
 size_t mv_ssm_chunk_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n);
 int mv_ssm_chunk_launch(const MvSsmArgs &a, void *workspace, size_t ws_bytes, int total_q, int dtype, hipStream_t stream);

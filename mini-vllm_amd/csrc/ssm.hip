@@ -334,14 +334,18 @@ static int check_ssm(const MvSsmArgs *a, int dtype) {
   return MV_OK;
 }
 
-extern "C" int mv_causal_conv(const MvSsmArgs *a, int dtype, void *stream) {
-  if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
+int mv_check_conv(const MvSsmArgs *a, int dtype) {
   if (int e = check_ssm(a, dtype)) return e;
   if (!a->conv_w || !a->cu_q || !a->cu_k || (a->slots > 0 && a->taps > 1 && !a->conv_state)) return MV_E_NULLPTR;
   if (a->max_q < 0 || a->out_stride < a->channels) return MV_E_SHAPE;
   if (!mv_aligned16(a->conv_w) || (a->conv_b && !mv_aligned16(a->conv_b)) || (a->conv_state && !mv_aligned16(a->conv_state))) return MV_E_ALIGN;
+  return (a->max_q + kConvRows - 1) / kConvRows > 65535 ? MV_E_SHAPE : MV_OK;
+}
+
+extern "C" int mv_causal_conv(const MvSsmArgs *a, int dtype, void *stream) {
+  if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
+  if (int e = mv_check_conv(a, dtype)) return e;
   const int vec = dtype == MV_F32 ? 4 : 8, y = (a->max_q + kConvRows - 1) / kConvRows;
-  if (y > 65535) return MV_E_SHAPE;
   const dim3 grid((a->channels / vec + 63) / 64, y, a->n_seqs);
   MV_DISPATCH_DTYPE(dtype, {
     if (a->taps <= 2) hipLaunchKernelGGL((causal_conv_kernel<Tag, 2>), grid, dim3(64), 0, (hipStream_t)stream, *a);

@@ -96,6 +96,7 @@ _SIGNATURES = {
     "mv_delta_prefill_workspace_bytes": (c_size_t, [c_int] * 6),
     "mv_delta_prefill_segments_bytes": (c_size_t, [c_int] * 8),
     "mv_delta_prefill": (c_int, [c_void_p, c_int, c_int, c_void_p]),
+    "mv_delta_prefill_conv": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "mv_delta_step": (c_int, [c_void_p, c_int, c_void_p]),
     "mv_head_norm_gate": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_int,
                                   c_float, c_int, c_float, c_int, c_void_p]),
@@ -1653,10 +1654,20 @@ def _delta_args(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots, o
     return g
 
 
+def _delta_conv(g, s: DeltaShape, x, conv_w, conv_state) -> None:
+    if conv_w.dtype != x.dtype or conv_w.shape[1] != s.channels:
+        raise MvHipError(f"convolution weight [taps, {s.channels}] of {x.dtype} required")
+    g.conv_w, g.taps = conv_w.data_ptr(), conv_w.shape[0]
+    if g.slots and g.taps > 1:
+        if conv_state.dtype != x.dtype or tuple(conv_state.shape) != (2, g.slots, g.taps - 1, s.channels) or not conv_state.is_contiguous():
+            raise MvHipError(f"convolution state must be dense [2, {g.slots}, {g.taps - 1}, {s.channels}] of {x.dtype}")
+        g.conv_state = conv_state.data_ptr()
+
+
 def delta_prefill(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots, cu_q, cu_k, max_q: int, out=None, flags: int = 0,
-                  gate=None, norm_w=None, gate_kind: str = "silu", out_scale: float = 1.0):
+                  gate=None, norm_w=None, gate_kind: str = "silu", out_scale: float = 1.0, conv=None):
     """The gated delta rule over convolved channels [T, channels], raw beta [T, heads] and raw decays -> o [T, heads * p]; with ``gate``
-    [T, heads * p] and ``norm_w``: ``head_norm_gate`` of it."""
+    [T, heads * p] and ``norm_w``: ``head_norm_gate`` of it; with ``conv`` (weight, state): from projected channels, ``causal_conv`` of which comes first."""
     if out is None:
         out = torch.empty((x.shape[0], s.heads * s.p), dtype=x.dtype, device=x.device)
     g = _delta_args(s, x, beta, a, dt_bias, a_log, state, state_slots, out)
@@ -1664,8 +1675,10 @@ def delta_prefill(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots,
     n = 0 if flags & MV_DELTA_SCAN else int(_lib.mv_delta_prefill_workspace_bytes(g.n_seqs, g.total_q, s.heads, s.p, s.n, _dt(x)))
     if n and g.max_q > MV_DELTA_WHOLE:      # (0 otherwise: a call less)
         n += int(_lib.mv_delta_prefill_segments_bytes(g.n_seqs, g.total_q, g.max_q, s.heads, s.p, s.n, g.channel_decay, _dt(x)))
-    ws = torch.empty((n,), dtype=torch.uint8, device=x.device) if n else None
-    g.workspace, g.ws_bytes = _ptr(ws), n
+    xc = -(-x.shape[0] * s.channels * x.element_size() // 256) * 256 if conv is not None else 0
+    ws = torch.empty((xc + n,), dtype=torch.uint8, device=x.device) if xc + n else None
+    if n:
+        g.workspace, g.ws_bytes = ws.data_ptr() + xc, n
     if gate is not None:
         _need_cuda(gate, norm_w)
         _rows_ok("gate", gate, s.heads * s.p, x.dtype)
@@ -1673,7 +1686,12 @@ def delta_prefill(s: DeltaShape, x, beta, a, dt_bias, a_log, state, state_slots,
             raise MvHipError(f"norm weight of {s.p} {x.dtype} and as many rows of the gate and the output required")
         g.gate, g.gate_stride, g.norm_w, g.gate_kind, g.out_scale = gate.data_ptr(), gate.stride(0), norm_w.data_ptr(), GATES[gate_kind], float(out_scale)
         flags |= MV_DELTA_NORM
-    _check(_lib.mv_delta_prefill(ctypes.byref(g), _dt(x), int(flags), _stream()), "mv_delta_prefill")
+    if conv is not None:
+        _need_cuda(*conv)
+        _delta_conv(g, s, x, *conv)
+        _check(_lib.mv_delta_prefill_conv(ctypes.byref(g), _ptr(ws), _dt(x), int(flags), _stream()), "mv_delta_prefill")
+    else:
+        _check(_lib.mv_delta_prefill(ctypes.byref(g), _dt(x), int(flags), _stream()), "mv_delta_prefill")
     return out
 
 

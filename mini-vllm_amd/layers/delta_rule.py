@@ -100,6 +100,5 @@ class GatedDeltaRule(nn.Module):
                                  (ctx.cum_seqlens_q, ctx.cum_seqlens_k, ctx.max_seqlen_q))
             rest = (lambda v: v[nd:]) if nd else (lambda v: v)
             slots = rest(slots)
-            xc = hip_ops.causal_conv(rest(x), self.conv, None, s.conv, self.conv_state, slots, cu_q, cu_k, max_q)
-            hip_ops.delta_prefill(s, xc, rest(beta), rest(a), self.dt_bias, self.A_log, self.state, slots, cu_q, cu_k, max_q, out=rest(out),
-                                  gate=rest(gate), norm_w=self.norm, gate_kind=self.gate, out_scale=self.out_scale)
+            hip_ops.delta_prefill(s, rest(x), rest(beta), rest(a), self.dt_bias, self.A_log, self.state, slots, cu_q, cu_k, max_q, out=rest(out),
+                                  gate=rest(gate), norm_w=self.norm, gate_kind=self.gate, out_scale=self.out_scale, conv=(self.conv, self.conv_state))
