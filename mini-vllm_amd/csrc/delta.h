@@ -16,7 +16,7 @@ __device__ __forceinline__ float decay_log(float rate, float a, float bias) { re
 size_t mv_delta_chunk_workspace(int n_seqs, int total_q, int heads, int p, int n);
 size_t mv_delta_segments_workspace(int n_seqs, int total_q, int max_q, int heads, int p, int n);   // beside it, where sequences are cut
 // `normed` (NULL: not asked for): in: norm and gate in the walk whatever the rule on sizes says; out: they are already in the output
-// `raw` (bf16, one decay per head; mv_delta_scalar_takes_conv): the channels ahead of the convolution, which goes to a.x
+// `raw` (mv_delta_chunk_takes_conv): the channels ahead of the convolution, which goes to a.x if the walk reads it
 int mv_delta_chunk_launch(const MvDeltaArgs &a, const void *raw, int64_t raw_stride, int dtype, bool *normed, hipStream_t stream);
-bool mv_delta_scalar_takes_conv(const MvDeltaArgs &a);
+bool mv_delta_chunk_takes_conv(const MvDeltaArgs &a, int dtype);
 int mv_delta_scalar_launch(const MvDeltaArgs &a, const void *raw, int64_t raw_stride, bool *normed, hipStream_t stream);   // (from the above: bf16, one decay per head)

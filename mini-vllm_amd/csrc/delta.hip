@@ -349,7 +349,7 @@ extern "C" size_t mv_delta_prefill_segments_bytes(int n_seqs, int total_q, int m
   return dtype == MV_F32 || (dtype == MV_BF16 && !channel_decay) ? 0 : mv_delta_segments_workspace(n_seqs, total_q, max_q, heads, p, n);
 }
 
-// raw: the channels ahead of the convolution, which the first launch does along the way (mv_delta_scalar_takes_conv), or NULL
+// raw: the channels ahead of the convolution, which the first launch does along the way (mv_delta_chunk_takes_conv), or NULL
 static int prefill(const MvDeltaArgs *a, const void *raw, int64_t raw_stride, int dtype, int flags, void *stream) {
   if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
   if (int e = check_delta(a, dtype)) return e;
@@ -390,8 +390,8 @@ extern "C" int mv_delta_prefill_conv(const MvDeltaArgs *a, void *xc, int dtype, 
   d.x = xc, d.x_stride = a->channels;
   if (int e = mv_check_conv(&c, dtype)) return e;
   if (int e = check_delta(&d, dtype)) return e;
-  if (dtype == MV_BF16 && !a->channel_decay && !(flags & MV_DELTA_SCAN) && a->workspace && (a->conv_state || a->taps == 1 || !a->slots) &&
-      mv_delta_chunk_workspace(a->n_seqs, a->total_q, a->heads, a->p, a->n) && mv_delta_scalar_takes_conv(*a))
+  if (dtype != MV_F32 && !(flags & MV_DELTA_SCAN) && a->workspace && (a->conv_state || a->taps == 1 || !a->slots) &&
+      mv_delta_chunk_workspace(a->n_seqs, a->total_q, a->heads, a->p, a->n) && mv_delta_chunk_takes_conv(d, dtype))
     return prefill(&d, a->x, a->x_stride, dtype, flags, stream);
   if (int rc = mv_causal_conv(&c, dtype, stream)) return rc;
   return prefill(&d, nullptr, 0, dtype, flags, stream);

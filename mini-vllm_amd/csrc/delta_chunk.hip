@@ -41,7 +41,10 @@ struct Layout {
 // of its phases: everything is asked for from memory at the start, blocks of one row of A and B share that row's factors, K is made beside the
 // solution, and the solution is split into operands once.  3 sequences of 4011 tokens and less, 8 heads of 128 x 128 (1256 workgroups, two a CU):
 // 105 us with every block's factors, all of K and W by four waves, and operands of T by each item -> 83.
-template <typename Tag, int NK>
+// CONV (q.raw: projected channels, all of this head's alone): convolution and silu ahead of it (conv_chunk), k and q into their place in LDS, v by way of the decays' place
+// into registers.  Nobody else reads the convolved channels, so they leave the CU no more: a launch and 77 MB less.  The sequences above: 32 + 85 us as two launches, the
+// layer 250 -> 232.
+template <typename Tag, int NK, bool CONV>
 __global__ void __launch_bounds__(kPrepareWaves * 64, NK < 5 ? 4 : 2) delta_prepare_kernel(DeltaPrep q) {
   typedef typename elem<Tag>::T T;
   constexpr int N = NK * 32, W = kPrepareWaves, RS = N + 4, KS = N + 8;   // LDS row strides: fp32, 16-bit
@@ -67,7 +70,7 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, NK < 5 ? 4 : 2) delta_prep
   constexpr int KQ = (N + 63) / 64, AP = (L * N / 8 + W * 64 - 1) / (W * 64);   // pieces of 8 channels a thread
   const int tt = tid >> 3, part = tid & 7, columns = p.p / 16;
   u32x4 kraw[KQ], qraw[KQ], araw[AP], braw[AP];
-  {
+  if constexpr (!CONV) {
     const T *row = x + (int64_t)min(tt, nt - 1) * p.x_stride + grp * N;
 #pragma unroll
     for (int i = 0; i < KQ; ++i) {
@@ -95,7 +98,24 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, NK < 5 ? 4 : 2) delta_prep
 #pragma unroll
     for (int e = 0; e < 16; ++e) vraw[e] = v[(int64_t)min(16 * (e >> 2) + 4 * g + (e & 3), nt - 1) * p.x_stride];
   };
-  load_values(min(wave, columns - 1));
+  if constexpr (CONV) {
+    T *vs = (T *)smem;   // [L][VS], where the decays' sums come later
+    const int VS = p.p + 8;
+    conv_chunk<Tag, N, W * 64, true>(q, seq, q0, len, t0, nt, head, head * p.p, p.p, tid, [&](int which, int row, int at, int, u32x2 done) {
+      *(u32x2 *)(which == 0 ? ks + row * KS + at : which == 1 ? qs + row * KS + at : vs + row * VS + at) = done;
+    });
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) {
+      const int c = min(part * 8 + 64 * i, N - 8);
+      kraw[i] = *(const u32x4 *)(ks + tt * KS + c), qraw[i] = *(const u32x4 *)(qs + tt * KS + c);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) vraw[e] = vs[(16 * (e >> 2) + 4 * g + (e & 3)) * VS + min(wave, columns - 1) * 16 + r16];
+    __syncthreads();
+  } else {
+    load_values(min(wave, columns - 1));
+  }
 
   // ---- k, q (tokens behind the end: zeros) and their lengths
   {
@@ -110,8 +130,10 @@ __global__ void __launch_bounds__(kPrepareWaves * 64, NK < 5 ? 4 : 2) delta_prep
       unpack8<Tag>(qraw[i], fb);
 #pragma unroll
       for (int j = 0; j < 8; ++j) sk = fmaf(fa[j], fa[j], sk), sq = fmaf(fb[j], fb[j], sq);
-      *(u32x4 *)(ks + tt * KS + c) = kraw[i];
-      *(u32x4 *)(qs + tt * KS + c) = qraw[i];
+      if constexpr (!CONV) {
+        *(u32x4 *)(ks + tt * KS + c) = kraw[i];
+        *(u32x4 *)(qs + tt * KS + c) = qraw[i];
+      }
     }
 #pragma unroll
     for (int o = 1; o <= 4; o <<= 1) sk += __shfl_xor(sk, o, 64), sq += __shfl_xor(sq, o, 64);
@@ -823,9 +845,15 @@ int launch(const DeltaPrep &q, int seg, hipStream_t stream) {
   const MvDeltaArgs &a = q.a;
   constexpr int RS = NK * 32 + 4, KS = NK * 32 + 8;
   constexpr int QB = L * KS * 2 > L * (L + 4) * 4 ? L * KS * 2 : L * (L + 4) * 4;
-  if (int rc = mv_allow_lds<delta_prepare_kernel<Tag, NK>>()) return rc;
-  hipLaunchKernelGGL((delta_prepare_kernel<Tag, NK>), dim3((unsigned)chunk_slots(a.n_seqs, a.total_q), a.heads),
-                     dim3(kPrepareWaves * 64), L * RS * 4 + L * KS * 2 + QB + (3 + kPrepareWaves) * L * 4, stream, q);
+  const dim3 grid((unsigned)chunk_slots(a.n_seqs, a.total_q), a.heads), block(kPrepareWaves * 64);
+  constexpr int need = L * RS * 4 + L * KS * 2 + QB + (3 + kPrepareWaves) * L * 4;
+  if (q.raw) {
+    if (int rc = mv_allow_lds<delta_prepare_kernel<Tag, NK, true>>()) return rc;
+    hipLaunchKernelGGL((delta_prepare_kernel<Tag, NK, true>), grid, block, need, stream, q);
+  } else {
+    if (int rc = mv_allow_lds<delta_prepare_kernel<Tag, NK, false>>()) return rc;
+    hipLaunchKernelGGL((delta_prepare_kernel<Tag, NK, false>), grid, block, need, stream, q);
+  }
   MV_LAUNCH_CHECK();
   const int tiles = a.p / 16, wide = (tiles + 7) / 8, narrow = (tiles + 3) / 4;
   constexpr auto lds = [](int columns) { return (24 * NK + 16 * columns + 17) * 1024; };
@@ -862,6 +890,15 @@ int launch(const DeltaPrep &q, int seg, hipStream_t stream) {
 
 }  // namespace
 
+// The convolution goes along where every channel is one workgroup's (which reads and writes what is kept of it), a thread's window holds the taps and, with
+// a head's values prepared (not bf16 with one decay per head), a wave has one tile of them and LDS holds them in the decays' place
+bool mv_delta_chunk_takes_conv(const MvDeltaArgs &a, int dtype) {
+  const bool scalar = dtype == MV_BF16 && !a.channel_decay;
+  const int of_group = a.heads / a.groups;
+  return (scalar ? of_group <= 2 : of_group == 1 && a.p <= 16 * kPrepareWaves && a.p <= 2 * a.n) && a.taps >= 1 && a.taps <= 4 && a.k_off == a.heads * a.p &&
+         a.q_off == a.k_off + a.groups * a.n && a.channels == a.q_off + a.groups * a.n;
+}
+
 size_t mv_delta_chunk_workspace(int n_seqs, int total_q, int heads, int p, int n) {
   if (n_seqs <= 0 || total_q <= 0 || heads <= 0 || p <= 0 || n <= 0 || n > 160 || (n & 31)) return 0;
   return (size_t)chunk_slots(n_seqs, total_q) * heads * Layout(n / 32, p).total * 1024;
@@ -883,7 +920,7 @@ int mv_delta_chunk_launch(const MvDeltaArgs &a, const void *raw, int64_t raw_str
   if ((size_t)a.ws_bytes < need || !mv_aligned16(a.workspace)) return MV_E_WORKSPACE;
   if (!mv_aligned16(a.x) || (a.x_stride & 7) || (a.k_off & 7) || (a.q_off & 7) || a.total_q > 64 * 1000000) return MV_E_ALIGN;
   if (a.channel_decay && (!mv_aligned16(a.a) || (a.a_stride & 7) || !mv_aligned16(a.dt_bias))) return MV_E_ALIGN;
-  const DeltaPrep q{a, (char *)a.workspace, nullptr, 0};
+  const DeltaPrep q{a, (char *)a.workspace, raw, raw_stride};
   if (!a.channel_decay && dtype == MV_BF16) return mv_delta_scalar_launch(a, raw, raw_stride, normed, stream);
   if (normed) *normed = false;
   const size_t more = mv_delta_segments_workspace(a.n_seqs, a.total_q, a.max_q, a.heads, a.p, a.n);

@@ -69,73 +69,11 @@ __global__ void __launch_bounds__(256 * HEADS, CONV ? 6 : 4) delta_scalar_prepar
       rate = elem<B16>::ld(((const E *)p.a_log)[head]), bias = elem<B16>::ld(((const E *)p.dt_bias)[head]);
     }
     if constexpr (CONV) {
-      constexpr int TAPS = 4, ROWS = 8;
-      const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq], back = p.taps - 1, first = blockIdx.y * HEADS * p.p;
-      const bool keep = slot >= 0 && slot < p.slots;
-      const int64_t half = p.slots * back * p.channels;
-      const T *conv_w = (const T *)p.conv_w, *from = (const T *)q.raw + (int64_t)q0 * q.raw_stride;
-      const T *old_state = (const T *)p.conv_state + (before & 1) * half + (int64_t)(keep ? slot : 0) * back * p.channels;
-      T *xc = (T *)p.x + (int64_t)q0 * p.x_stride;
-      const int pieces = (2 * N + HEADS * p.p) / 4;   // of a token: k, q, the heads' v
-      const auto unpack4 = [](const u32x2 &v, float (&f)[4]) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) f[2 * i] = u2f(v[i] << 16), f[2 * i + 1] = u2f(v[i] & 0xffff0000u);
-      };
-      for (int item = tid; item < pieces * (L / ROWS); item += 256 * HEADS) {
-        const int piece = item % pieces, tr = item / pieces * ROWS, which = piece / (N / 4);   // 0: k, 1: q
-        const int c = which == 0 ? p.k_off + grp * N + piece * 4 : which == 1 ? p.q_off + grp * N + (piece - N / 4) * 4 : first + (piece - N / 2) * 4;
-        auto input = [&](int t) {   // input `t` of the step (t < 0: of the steps before it)
-          if (t >= 0) return *(const u32x2 *)(from + (int64_t)min(t, len - 1) * q.raw_stride + c);
-          if (before > 0 && keep && back + t >= 0) return *(const u32x2 *)(old_state + (int64_t)(back + t) * p.channels + c);
-          return u32x2{0u, 0u};
-        };
-        float w[TAPS][4], win[TAPS][4];
-        if (tr >= nt && which > 1) continue;
-        u32x2 raw[TAPS - 1], rows[ROWS];
-#pragma unroll
-        for (int i = 0; i < TAPS - 1; ++i) raw[i] = input(t0 + tr + i - (TAPS - 1));
-#pragma unroll
-        for (int u = 0; u < ROWS; ++u) rows[u] = input(t0 + tr + u);
-#pragma unroll
-        for (int i = 0; i < TAPS; ++i) {
-          const int tap = i - (TAPS - p.taps);   // (weights stand at the current token's end)
-          u32x2 v = {0u, 0u};
-          if (tap >= 0) v = *(const u32x2 *)(conv_w + (int64_t)tap * p.channels + c);
-          unpack4(v, w[i]);
-        }
-#pragma unroll
-        for (int i = 0; i < TAPS - 1; ++i) unpack4(raw[i], win[i + 1]);   // shifted down below
-        if (t0 + tr == 0 && keep && back > 0) {   // the only thread that reads the old state here writes the new one, behind its reads
-          u32x2 last[TAPS - 1];
-#pragma unroll
-          for (int j = 0; j < TAPS - 1; ++j)
-            if (j < back) last[j] = input(len - back + j);
-          T *ns = (T *)p.conv_state + ((before + len) & 1) * half + (int64_t)slot * back * p.channels + c;
-#pragma unroll
-          for (int j = 0; j < TAPS - 1; ++j)
-            if (j < back) *(u32x2 *)(ns + (int64_t)j * p.channels) = last[j];
-        }
-#pragma unroll
-        for (int u = 0; u < ROWS; ++u) {
-#pragma unroll
-          for (int i = 0; i < TAPS - 1; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) win[i][j] = win[i + 1][j];
-          unpack4(rows[u], win[TAPS - 1]);
-          f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int i = 0; i < TAPS; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) o[j] = fmaf(win[i][j], w[i][j], o[j]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) o[j] = silu_of<B16>(o[j]);
-          u32x2 done = pack_quad<B16>(o);
-          if (tr + u < nt) *(u32x2 *)(xc + (int64_t)(t0 + tr + u) * p.x_stride + c) = done;
-          else done = u32x2{0u, 0u};
-          if (which == 0) *(u32x2 *)(ks + (tr + u) * KS + piece * 4) = done;
-          if (which == 1) *(u32x2 *)(qs + (tr + u) * KS + (piece - N / 4) * 4) = done;
-        }
-      }
+      T *xc = (T *)p.x + (int64_t)(q0 + t0) * p.x_stride;
+      conv_chunk<B16, N, 256 * HEADS, false>(q, seq, q0, len, t0, nt, grp, blockIdx.y * HEADS * p.p, HEADS * p.p, tid, [&](int which, int row, int at, int c, u32x2 done) {
+        if (row < nt) *(u32x2 *)(xc + (int64_t)row * p.x_stride + c) = done;
+        if (which < 2) *(u32x2 *)((which ? qs : ks) + row * KS + at) = done;
+      });
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < NK; ++i) {
@@ -604,12 +542,6 @@ int launch(const DeltaPrep &q, bool *normed, hipStream_t stream) {
 }
 
 }  // namespace
-
-// The convolution goes along where every channel is one workgroup's (which reads and writes what is kept of it) and a thread's window holds the taps
-bool mv_delta_scalar_takes_conv(const MvDeltaArgs &a) {
-  const int of_group = a.heads / a.groups;
-  return of_group <= 2 && a.taps >= 1 && a.taps <= 4 && a.k_off == a.heads * a.p && a.q_off == a.k_off + a.groups * a.n && a.channels == a.q_off + a.groups * a.n;
-}
 
 // (arguments checked by mv_delta_chunk_launch, whose workspace is larger)
 int mv_delta_scalar_launch(const MvDeltaArgs &a, const void *raw, int64_t raw_stride, bool *normed, hipStream_t stream) {

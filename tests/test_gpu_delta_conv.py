@@ -1,4 +1,4 @@
-"""The gated delta rule's prompts from projected channels (the convolution along with the preparation of a chunk, csrc/delta_scalar.hip, or ahead of it), against the
+"""The gated delta rule's prompts from projected channels (the convolution along with the preparation of a chunk, csrc/delta_chunk.h, or ahead of it), against the
 convolution and the rule in calls of their own: the same bits, the kept inputs among them."""
 import pytest
 import torch
@@ -9,9 +9,12 @@ DEV = "cuda:0"
 SPANS = [(1, 0), (2, 5), (1, 1), (3, 2), (63, 5), (64, 0), (65, 64), (128, 7), (129, 0), (200, 1), (0, 3), (16, 900)]
 
 
-# with two heads to a group, one, four (which goes the other way), gaps between the channels, a decay per channel, one and two taps; the last sequence has no slot
+# with two heads to a group, one, four (which goes the other way), gaps between the channels, a decay per channel (values that fit the
+# decays' place in LDS and a wave's tile each, just or not), one and two taps; the last sequence has no slot
 @pytest.mark.parametrize("heads, groups, p, n, gap, channel", [(8, 4, 128, 128, 0, False), (3, 3, 64, 32, 0, False), (4, 2, 48, 96, 0, False), (8, 2, 64, 64, 0, False),
-                                                               (4, 2, 64, 64, 32, False), (2, 2, 64, 64, 0, True), (2, 1, 16, 160, 0, False)])
+                                                               (4, 2, 64, 64, 32, False), (2, 2, 64, 64, 0, True), (2, 1, 16, 160, 0, False),
+                                                               (2, 2, 128, 128, 0, True), (3, 3, 80, 32, 0, True), (2, 2, 144, 96, 0, True), (2, 2, 48, 160, 0, True),
+                                                               (4, 2, 32, 64, 0, True)])
 @pytest.mark.parametrize("taps", [4, 2, 1, 6])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_with_the_convolution(heads, groups, p, n, gap, channel, taps, dtype):
