@@ -10,15 +10,15 @@ namespace {
 template <typename Tag>
 __device__ __forceinline__ float param(const void *p, int i) { return elem<Tag>::ld(((const typename elem<Tag>::T *)p)[i]); }
 
-// ---- convolution: 8 (fp32: 4) channels per thread, kConvRows tokens per workgroup, a sliding window of inputs in registers
+// ---- convolution: 8 (fp32: 4) channels per thread, kConvRows tokens per workgroup (few workgroups: kConvAhead), a sliding window of inputs in registers
 constexpr int kConvRows = 32, kConvAhead = 8, kMaxTaps = 8;
 
-template <typename Tag, int TAPS>
+template <typename Tag, int TAPS, int ROWS>
 __global__ void __launch_bounds__(64) causal_conv_kernel(MvSsmArgs p) {
   typedef typename elem<Tag>::T T;
   constexpr int VEC = elem<Tag>::VEC;
   const int c = ((int)blockIdx.x * 64 + threadIdx.x) * VEC, s = blockIdx.z;
-  const int q0 = p.cu_q[s], len = p.cu_q[s + 1] - q0, t0 = blockIdx.y * kConvRows;
+  const int q0 = p.cu_q[s], len = p.cu_q[s + 1] - q0, t0 = blockIdx.y * ROWS;
   if (t0 >= len || c >= p.channels) return;
   const int before = p.cu_k[s + 1] - p.cu_k[s] - len, slot = p.state_slots[s], back = p.taps - 1;
   const bool keep = slot >= 0 && slot < p.slots;
@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(64) causal_conv_kernel(MvSsmArgs p) {
     for (int j = 0; j < kMaxTaps - 1; ++j)
       if (j < back) store_vec_row<Tag>(ns + (int64_t)j * p.channels, last[j]);
   }
-  const int t1 = min(len, t0 + kConvRows);
+  const int t1 = min(len, t0 + ROWS);
   for (int tb = t0; tb < t1; tb += kConvAhead) {
     u32x4 raw[kConvAhead];
 #pragma unroll
@@ -342,18 +342,28 @@ int mv_check_conv(const MvSsmArgs *a, int dtype) {
   return (a->max_q + kConvRows - 1) / kConvRows > 65535 ? MV_E_SHAPE : MV_OK;
 }
 
-extern "C" int mv_causal_conv(const MvSsmArgs *a, int dtype, void *stream) {
-  if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
-  if (int e = mv_check_conv(a, dtype)) return e;
-  const int vec = dtype == MV_F32 ? 4 : 8, y = (a->max_q + kConvRows - 1) / kConvRows;
-  const dim3 grid((a->channels / vec + 63) / 64, y, a->n_seqs);
+template <int ROWS>
+static int launch_conv(const MvSsmArgs &a, int x, int dtype, hipStream_t st) {
+  const dim3 grid(x, (a.max_q + ROWS - 1) / ROWS, a.n_seqs);
   MV_DISPATCH_DTYPE(dtype, {
-    if (a->taps <= 2) hipLaunchKernelGGL((causal_conv_kernel<Tag, 2>), grid, dim3(64), 0, (hipStream_t)stream, *a);
-    else if (a->taps <= 4) hipLaunchKernelGGL((causal_conv_kernel<Tag, 4>), grid, dim3(64), 0, (hipStream_t)stream, *a);
-    else hipLaunchKernelGGL((causal_conv_kernel<Tag, kMaxTaps>), grid, dim3(64), 0, (hipStream_t)stream, *a);
+    if (a.taps <= 2) hipLaunchKernelGGL((causal_conv_kernel<Tag, 2, ROWS>), grid, dim3(64), 0, st, a);
+    else if (a.taps <= 4) hipLaunchKernelGGL((causal_conv_kernel<Tag, 4, ROWS>), grid, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((causal_conv_kernel<Tag, kMaxTaps, ROWS>), grid, dim3(64), 0, st, a);
   });
   MV_LAUNCH_CHECK();
   return MV_OK;
+}
+
+extern "C" int mv_causal_conv(const MvSsmArgs *a, int dtype, void *stream) {
+  if (a && (a->n_seqs == 0 || a->max_q == 0)) return MV_OK;
+  if (int e = mv_check_conv(a, dtype)) return e;
+  // Few workgroups: eight tokens each, whose loads are one trip to memory, where 32 are four one behind the other; many, whose trips overlap: 32, which read the
+  // tokens ahead of theirs less often.  us with 8 and 32 by workgroups of 32 tokens: 18: 5.2 and 11.9, 162: 5.8 and 11.4, 330: 7.9 and 12.4, 594: 11.2 and 14.7,
+  // 1000: 14.7 and 16.4, 1620: 21.5 and 22.8, 1800: 23.8 and 23.1, 4392: the layer around it 225.3 and 222.9.
+  constexpr int64_t kFewConvs = 1700;
+  const int x = (a->channels / (dtype == MV_F32 ? 4 : 8) + 63) / 64;
+  if ((int64_t)x * ((a->max_q + kConvRows - 1) / kConvRows) * a->n_seqs <= kFewConvs) return launch_conv<kConvAhead>(*a, x, dtype, (hipStream_t)stream);
+  return launch_conv<kConvRows>(*a, x, dtype, (hipStream_t)stream);
 }
 
 extern "C" size_t mv_ssm_prefill_workspace_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int dtype) {
