@@ -3,7 +3,7 @@
 // (reference: minivllm/models/qwen_base.py:173-190 flat path,
 //  layers/layernorm.py:81-93, layers/rotary_embedding.py:77-81,166-193,
 //  layers/attention_backend.py:196-266).
-// One workgroup per token.  A head row (D elements) is spread over
+// One workgroup per token, of one, two or four waves.  A head row (D elements) is spread over
 // LPT = D/VEC adjacent lanes, 16 bytes each; the rotation partner
 // (dims i and i + D/2) lives LPT/2 lanes away and is fetched with one DPP
 // row rotate (bf16/f16, D=128) or a wave shuffle.
@@ -31,97 +31,122 @@ struct RopeParams {
 template <int LPT>
 __device__ __forceinline__ float lpt_sum(float x) {
   // butterfly over the LPT lanes of one head row; every lane gets the total
+  if constexpr (LPT <= 16) return lanes_sum<LPT>(x);   // (the same sums, without the LDS pipe)
   for (int off = 1; off < LPT; off <<= 1) x += __shfl_xor(x, off, 64);
   return x;
 }
 
-template <typename Tag, int D>
-__global__ void __launch_bounds__(256) rope_qk_store_kernel(RopeParams p) {
+// Rows of a token, 16 bytes a lane.  A thread reads its cosines and sines once, 64 bytes for 16 of each row, so that they are more of what passes through
+// the L1 than the rows themselves where a thread has two or three rows: with many tokens a token is one wave (two), which asks for four of its rows at a time; with few,
+// whose time is one token's latency, four waves, a row each at a time.
+template <typename Tag, int D, int THREADS>
+__global__ void __launch_bounds__(THREADS) rope_qk_store_kernel(RopeParams p) {
   typedef typename elem<Tag>::T T;
   constexpr int VEC = elem<Tag>::VEC;
   constexpr int LPT = D / VEC;
   const int tok = blockIdx.x;
   const int sub = threadIdx.x % LPT;
-  const int rows_per_iter = blockDim.x / LPT;
+  constexpr int rows_per_iter = THREADS / LPT;
   const int H = p.n_heads, HKV = p.n_kv_heads;
   const bool has_cache = p.k_cache != nullptr && p.slot_mapping != nullptr;
   int64_t slot = has_cache ? (int64_t)p.slot_mapping[tok] : -1;
   if (slot >= p.num_slots) slot = -1;
-  const int total_rows = H + HKV + (slot >= 0 ? HKV : 0);
-
+  const int total_rows = H + HKV + (has_cache ? HKV : 0);
   const int64_t pos = p.positions[tok];
+  constexpr int AHEAD = THREADS < 256 ? 4 : 1;
+  const auto source = [&](int r) {
+    return r < H          ? (const T *)p.q + (int64_t)tok * p.q_stride + r * D
+           : r < H + HKV ? (const T *)p.k + (int64_t)tok * p.k_stride + (r - H) * D
+                         : (const T *)p.v + (int64_t)tok * p.v_stride + (r - H - HKV) * D;
+  };
+  const int first = threadIdx.x / LPT;
+  u32x4 raws[AHEAD];
+  const auto ask = [&](int r0) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) raws[u] = *reinterpret_cast<const u32x4 *>(source(min(r0 + u * rows_per_iter, total_rows - 1)) + sub * VEC);
+  };
+  ask(first);
   const bool pos_ok = pos >= 0 && pos < p.max_pos;
   float cs[VEC], sn[VEC];
   rot_factors<D, VEC>(p.cos, p.sin, pos, pos_ok, sub, p.pairs, p.interleaved != 0, cs, sn);
 
-  for (int r = threadIdx.x / LPT; r < total_rows; r += rows_per_iter) {
-    if (r >= H + HKV) {  // raw V row -> cache
-      const int hv = r - H - HKV;
-      const T *src = (const T *)p.v + (int64_t)tok * p.v_stride + hv * D + sub * VEC;
-      T *dst = (T *)p.v_cache + (slot * HKV + hv) * D + sub * VEC;
-      *reinterpret_cast<u32x4 *>(dst) = *reinterpret_cast<const u32x4 *>(src);
-      continue;
-    }
-    const bool is_q = r < H;
-    const int hh = is_q ? r : r - H;
-    const T *src = is_q ? (const T *)p.q + (int64_t)tok * p.q_stride + hh * D
-                        : (const T *)p.k + (int64_t)tok * p.k_stride + hh * D;
-    const T *nw = is_q ? (const T *)p.q_norm_w : (const T *)p.k_norm_w;
-    float x[VEC];
-    {
-      const u32x4 raw = *reinterpret_cast<const u32x4 *>(src + sub * VEC);
-      if constexpr (VEC == 8) unpack8<Tag>(raw, x);
+  for (int r0 = first; r0 - first < total_rows; r0 += AHEAD * rows_per_iter) {
+    if (r0 != first) ask(r0);
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int r = r0 + u * rows_per_iter;
+      if (r >= total_rows) continue;   // (the lanes of a row together)
+      if (r >= H + HKV) {  // raw V row -> cache
+        if (slot >= 0) *reinterpret_cast<u32x4 *>((T *)p.v_cache + (slot * HKV + r - H - HKV) * D + sub * VEC) = raws[u];
+        continue;
+      }
+      const bool is_q = r < H;
+      const int hh = is_q ? r : r - H;
+      const T *nw = is_q ? (const T *)p.q_norm_w : (const T *)p.k_norm_w;
+      float x[VEC];
+      if constexpr (VEC == 8) unpack8<Tag>(raws[u], x);
       else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) x[j] = u2f(raw[j]);
+        for (int j = 0; j < 4; ++j) x[j] = u2f(raws[u][j]);
       }
-    }
-    float rs = 1.0f;
-    if (nw != nullptr || p.unit) {   // (a rotation keeps the length)
-      float ss = 0.f;
+      float rs = 1.0f;
+      if (nw != nullptr || p.unit) {   // (a rotation keeps the length)
+        float ss = 0.f;
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) ss = fmaf(x[j], x[j], ss);
-      ss = lpt_sum<LPT>(ss);
-      rs = 1.0f / sqrtf(ss / (float)p.norm_dim + p.eps);
-    }
-    if (nw != nullptr) {  // per-head RMSNorm, result rounded to dtype like the reference
-      float w[VEC];
-      const u32x4 wraw = *reinterpret_cast<const u32x4 *>(nw + sub * VEC);
-      if constexpr (VEC == 8) unpack8<Tag>(wraw, w);
+        for (int j = 0; j < VEC; ++j) ss = fmaf(x[j], x[j], ss);
+        ss = lpt_sum<LPT>(ss);
+        rs = 1.0f / sqrtf(ss / (float)p.norm_dim + p.eps);
+      }
+      if (nw != nullptr) {  // per-head RMSNorm, result rounded to dtype like the reference
+        float w[VEC];
+        const u32x4 wraw = *reinterpret_cast<const u32x4 *>(nw + sub * VEC);
+        if constexpr (VEC == 8) unpack8<Tag>(wraw, w);
+        else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) w[j] = u2f(wraw[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+          x[j] = elem<Tag>::ld(elem<Tag>::st(__fmul_rn(__fmul_rn(x[j], rs), w[j])));
+      }
+      float y[VEC];
+      rot_apply<D, VEC>(x, cs, sn, sub, p.interleaved != 0, y);
+      if (p.unit) {
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) y[j] = __fmul_rn(y[j], rs);
+      }
+      u32x4 packed;
+      if constexpr (VEC == 8) packed = pack8<Tag>(y);
       else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = u2f(wraw[j]);
+        for (int j = 0; j < 4; ++j) packed[j] = f2u(y[j]);
       }
-#pragma unroll
-      for (int j = 0; j < VEC; ++j)
-        x[j] = elem<Tag>::ld(elem<Tag>::st(__fmul_rn(__fmul_rn(x[j], rs), w[j])));
-    }
-    float y[VEC];
-    rot_apply<D, VEC>(x, cs, sn, sub, p.interleaved != 0, y);
-    if (p.unit) {
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) y[j] = __fmul_rn(y[j], rs);
-    }
-    u32x4 packed;
-    if constexpr (VEC == 8) packed = pack8<Tag>(y);
-    else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) packed[j] = f2u(y[j]);
-    }
-    if (is_q) {
-      T *dst = (T *)p.q_out + ((int64_t)tok * H + hh) * D + sub * VEC;
-      *reinterpret_cast<u32x4 *>(dst) = packed;
-    } else {
-      if (p.k_out != nullptr) {
-        T *dst = (T *)p.k_out + ((int64_t)tok * HKV + hh) * D + sub * VEC;
-        *reinterpret_cast<u32x4 *>(dst) = packed;
-      }
-      if (slot >= 0) {
-        T *dst = (T *)p.k_cache + (slot * HKV + hh) * D + sub * VEC;
-        *reinterpret_cast<u32x4 *>(dst) = packed;
+      if (is_q) {
+        *reinterpret_cast<u32x4 *>((T *)p.q_out + ((int64_t)tok * H + hh) * D + sub * VEC) = packed;
+      } else {
+        if (p.k_out != nullptr) *reinterpret_cast<u32x4 *>((T *)p.k_out + ((int64_t)tok * HKV + hh) * D + sub * VEC) = packed;
+        if (slot >= 0) *reinterpret_cast<u32x4 *>((T *)p.k_cache + (slot * HKV + hh) * D + sub * VEC) = packed;
       }
     }
   }
+}
+
+// us by waves of a token, 4 / 2 / 1; bf16, 16 + 8 heads of 128 with norms: 300 tokens 6.4 / 6.4 / 7.5, 600 8.1 / 7.3 / 8.1, 1000 9.8 / 8.7 / 9.1, 1366 12.5 / 11.1 / 10.5,
+// 5000 29.6 / 24.0 / 20.9, 25200 143 / 96 / 92; 28 + 4 of 128, 25200: 130 / 102 / 97; 16 + 8 of 64: 81 / 59 / 50; 8 + 4 of 256, 1366: 17.8 / 14.1 / 13.0.  fp32 rows
+// are as quick either way (16 + 8 of 128, 5000: 33.8 / 34.4 / 33.1) and slower below (1000: 10.7 / 11.7 / 16.2).
+template <typename Tag, int D>
+static void launch_rope(const RopeParams &p, int n_tok, hipStream_t st) {
+  if constexpr (elem<Tag>::VEC == 8) {
+    if (n_tok > 1024) {
+      hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 64>), dim3(n_tok), dim3(64), 0, st, p);
+      return;
+    }
+    if (n_tok > 512) {
+      hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 128>), dim3(n_tok), dim3(128), 0, st, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 256>), dim3(n_tok), dim3(256), 0, st, p);
 }
 
 extern "C" int mv_rope_qk_store_ex(const void *q, const void *k, const void *v, int64_t q_stride_tok,
@@ -166,11 +191,11 @@ extern "C" int mv_rope_qk_store_ex(const void *q, const void *k, const void *v, 
   p.pairs = p.interleaved ? opts->rot_pairs : head_dim / 2;
   hipStream_t st = (hipStream_t)stream;
   if (head_dim == 256) {
-    MV_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((rope_qk_store_kernel<Tag, 256>), dim3(n_tok), dim3(256), 0, st, p));
+    MV_DISPATCH_DTYPE(dtype, (launch_rope<Tag, 256>(p, n_tok, st)));
   } else if (head_dim == 128) {
-    MV_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((rope_qk_store_kernel<Tag, 128>), dim3(n_tok), dim3(256), 0, st, p));
+    MV_DISPATCH_DTYPE(dtype, (launch_rope<Tag, 128>(p, n_tok, st)));
   } else {
-    MV_DISPATCH_DTYPE(dtype, hipLaunchKernelGGL((rope_qk_store_kernel<Tag, 64>), dim3(n_tok), dim3(256), 0, st, p));
+    MV_DISPATCH_DTYPE(dtype, (launch_rope<Tag, 64>(p, n_tok, st)));
   }
   MV_LAUNCH_CHECK();
   return MV_OK;
