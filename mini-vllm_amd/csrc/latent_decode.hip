@@ -225,40 +225,40 @@ __global__ void __launch_bounds__(256, 2) latent_decode_kernel(DecodeParams p) {
   }
 }
 
-// one (sequence, head) per workgroup: 4 columns per thread, the parts dealt to blockDim.x / (kv_cols / 4) groups of threads
-template <typename Tag>
-__global__ void __launch_bounds__(256) latent_merge_kernel(const float *part, const float *part_ml, void *out, int splits, int kv_cols) {
+// 128 columns of a (sequence, head) per wave, four a lane; either half of the wave every other part, ROWS of them (as many as `splits` needs), which are asked for
+// at once and ahead of their weights: two trips to memory are one.  16 heads of 512 columns, with a workgroup a head and four parts a thread on their way at a time
+// -> now: 8 sequences, 30 parts 7.7 -> 5.2 us (the step 23.0 -> 21.2); 64 sequences, four parts 4.7 -> 4.2 (42.0 -> 41.3).  The same bits at 512 columns.
+template <typename Tag, int ROWS>
+__global__ void __launch_bounds__(64) latent_merge_kernel(const float *part, const float *part_ml, void *out, int splits, int kv_cols) {
   typedef typename elem<Tag>::T T;
-  __shared__ float w[kMaxSplits];
-  __shared__ f32x4 sums[256];
   const int64_t row = blockIdx.x;
-  const int tid = threadIdx.x, per = kv_cols / 4, groups = 256 / per, c = tid % per, first = tid / per;
-  float total;
-  {
-    const float *ml = part_ml + row * splits * 2;
-    const int lane = tid & 63;      // (kMaxSplits = one wave)
-    const float m = lane < splits ? ml[2 * lane] : -1e30f, l = lane < splits ? ml[2 * lane + 1] : 0.f;
-    const float top = wave_max(l > 0.f ? m : -1e30f);   // (all lanes take part)
-    const float e = l > 0.f ? __builtin_amdgcn_exp2f(m - top) : 0.f;
-    total = wave_sum(l * e);
-    if (tid < splits) w[tid] = e;
-  }
-  __syncthreads();
+  const int lane = threadIdx.x, half = lane >> 5, c = blockIdx.y * 128 + (lane & 31) * 4;
+  const float *p = part + row * splits * kv_cols + min(c, kv_cols - 4);
+  f32x4 v[ROWS];
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) v[u] = *(const f32x4 *)(p + (int64_t)min(2 * u + half, splits - 1) * kv_cols);
+  const float *ml = part_ml + row * splits * 2;   // (kMaxSplits = one wave)
+  const float m = lane < splits ? ml[2 * lane] : -1e30f, l = lane < splits ? ml[2 * lane + 1] : 0.f;
+  const float top = wave_max(l > 0.f ? m : -1e30f);
+  const float e = l > 0.f ? __builtin_amdgcn_exp2f(m - top) : 0.f;   // (0 of a part that is not there)
+  const float total = wave_sum(l * e);
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
-  if (first < groups) {
-    const float *p = part + row * splits * kv_cols + 4 * c;
-#pragma unroll 4
-    for (int s = first; s < splits; s += groups) {
-      const f32x4 v = *(const f32x4 *)(p + (int64_t)s * kv_cols);
-      o += w[s] > 0.f ? v * w[s] : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    const float w = __shfl(e, 2 * u + half, 64);
+    o += w > 0.f ? v[u] * w : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  sums[tid] = o;
-  __syncthreads();
-  if (tid < per) {
-    for (int i = 1; i < groups; ++i) o += sums[i * per + tid];
-    *(u32x2 *)((T *)out + row * kv_cols + 4 * c) = pack_quad<Tag>(o * (total > 0.f ? 1.0f / total : 0.f));
-  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) o[i] += __shfl_xor(o[i], 32, 64);
+  if (half == 0 && c < kv_cols) *(u32x2 *)((T *)out + row * kv_cols + c) = pack_quad<Tag>(o * (total > 0.f ? 1.0f / total : 0.f));
+}
+
+template <typename Tag>
+void launch_merge(const DecodeParams &p, int rows, hipStream_t st) {
+  const dim3 grid(rows, (p.kv_cols + 127) / 128);
+  if (p.splits <= 4) hipLaunchKernelGGL((latent_merge_kernel<Tag, 2>), grid, dim3(64), 0, st, p.part, p.part_ml, p.out, p.splits, p.kv_cols);
+  else if (p.splits <= 16) hipLaunchKernelGGL((latent_merge_kernel<Tag, 8>), grid, dim3(64), 0, st, p.part, p.part_ml, p.out, p.splits, p.kv_cols);
+  else hipLaunchKernelGGL((latent_merge_kernel<Tag, kMaxSplits / 2>), grid, dim3(64), 0, st, p.part, p.part_ml, p.out, p.splits, p.kv_cols);
 }
 
 int head_groups(int heads) { return heads > 16 ? 2 : 1; }
@@ -326,11 +326,8 @@ int mv_latent_decode_mfma_launch(const void *q, const void *plane, const int32_t
   if (dtype == MV_BF16) rc = hg == 2 ? launch<bf16_tag, 2>(p, grid, lds, stream) : launch<bf16_tag, 1>(p, grid, lds, stream);
   else rc = hg == 2 ? launch<f16_tag, 2>(p, grid, lds, stream) : launch<f16_tag, 1>(p, grid, lds, stream);
   if (rc != MV_OK || splits == 1) return rc;
-  const int rows = batch * heads;
-  if (dtype == MV_BF16)
-    hipLaunchKernelGGL((latent_merge_kernel<bf16_tag>), dim3(rows), dim3(256), 0, stream, p.part, p.part_ml, out, splits, kv_cols);
-  else
-    hipLaunchKernelGGL((latent_merge_kernel<f16_tag>), dim3(rows), dim3(256), 0, stream, p.part, p.part_ml, out, splits, kv_cols);
+  if (dtype == MV_BF16) launch_merge<bf16_tag>(p, batch * heads, stream);
+  else launch_merge<f16_tag>(p, batch * heads, stream);
   MV_LAUNCH_CHECK();
   return MV_OK;
 }
