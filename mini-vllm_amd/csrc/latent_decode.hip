@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(256, 2) latent_decode_kernel(DecodeParams p) {
 
 // 128 columns of a (sequence, head) per wave, four a lane; either half of the wave every other part, ROWS of them (as many as `splits` needs), which are asked for
 // at once and ahead of their weights: two trips to memory are one.  16 heads of 512 columns, with a workgroup a head and four parts a thread on their way at a time
-// -> now: 8 sequences, 30 parts 7.7 -> 5.2 us (the step 23.0 -> 21.2); 64 sequences, four parts 4.7 -> 4.2 (42.0 -> 41.3).  The same bits at 512 columns.
+// -> now: 8 sequences, 30 parts 7.7 -> 5.2 us (the step 23.0 -> 21.2); 64 sequences, four parts 4.7 and 4.2 .. 4.9 (42.0 -> 41.3).  The same bits at 512 columns.
 template <typename Tag, int ROWS>
 __global__ void __launch_bounds__(64) latent_merge_kernel(const float *part, const float *part_ml, void *out, int splits, int kv_cols) {
   typedef typename elem<Tag>::T T;
