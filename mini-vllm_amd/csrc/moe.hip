@@ -20,6 +20,14 @@ struct RouteParams {
   float scale;
 };
 constexpr int kRouteTiles = 4;   // tiles of 16 outputs at a time
+// grouping by the router's own (only) workgroup
+typedef __attribute__((ext_vector_type(4))) int s32x4;
+struct RouteGroups {
+  int32_t *place, *tokens, *tiles;
+  float *by_place;   // or NULL
+  int experts, tile_m, max_tiles;
+};
+constexpr int kRouteRows = 16, kRoutePairs = 256, kRouteExperts = 512;
 
 // largest value of the wave and the lowest index that has it
 __device__ __forceinline__ void wave_argmax(float &v, int &i) {
@@ -40,7 +48,7 @@ __device__ __forceinline__ int wave_best(float v, unsigned long long free) {
 
 // the scores of a token's R outputs, in s (logits) and c (scratch): choice and weights, by one wave; `correction`: of output `lane`
 template <typename Tag>
-__device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c, int64_t token, float correction) {
+__device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c, int64_t token, float correction, int *ids_too = nullptr, float *weights_too = nullptr) {
   typedef typename elem<Tag>::T T;
   const int lane = threadIdx.x & 63, R = p.outputs, size = R / p.groups;
   const bool sigmoid = p.flags & MV_ROUTE_SIGMOID;
@@ -125,8 +133,10 @@ __device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c,
     }
   }
   if (lane < p.top) {
+    const float w = (p.flags & MV_ROUTE_RAW ? weight : weight / (total + 1e-20f)) * p.scale;
     p.ids[token * p.top + lane] = mine;
-    p.weights[token * p.top + lane] = (p.flags & MV_ROUTE_RAW ? weight : weight / (total + 1e-20f)) * p.scale;
+    p.weights[token * p.top + lane] = w;
+    if (ids_too) ids_too[token * p.top + lane] = mine, weights_too[token * p.top + lane] = w;
   }
 }
 
@@ -205,15 +215,51 @@ __device__ __forceinline__ void choose_four(const RouteParams &p, const float *s
     }
 }
 
+// What moe_group_kernel makes of the choices, `pairs` of them in LDS (a multiple of four readable, -1 behind the last), by one workgroup of 16 waves: a pair to a
+// thread of the first four, an expert to one of the last eight.
+__device__ __forceinline__ void group_few(const RouteGroups &q, const int *ids, const float *weights, int pairs, int top) {
+  const int tid = threadIdx.x;
+  const bool pair = tid < pairs;
+  const int e = pair ? ids[tid] : tid - 512;
+  if (!pair && (e < 0 || e >= q.experts)) return;
+  if (pair && e >= q.experts) {
+    q.place[tid] = -1;
+    return;
+  }
+  int less = 0, equal = 0, ahead = 0;
+  for (int j = 0; j < pairs; j += 4) {
+    const s32x4 v = *(const s32x4 *)(ids + j);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      less += v[u] >= 0 && v[u] < e, equal += v[u] == e, ahead += v[u] == e && j + u < tid;
+    }
+  }
+  if (pair) {
+    const int place = less + ahead;
+    q.place[tid] = place, q.tokens[place] = tid / top;
+    if (q.by_place) q.by_place[place] = weights[tid];
+    return;
+  }
+  const int t0 = less / q.tile_m + e, t1 = e + 1 < q.experts ? (less + equal) / q.tile_m + e + 1 : q.max_tiles;
+  for (int t = t0; t < t1; ++t) {
+    const int first = (t - t0) * q.tile_m;
+    q.tiles[3 * t] = first < equal ? e : -1, q.tiles[3 * t + 1] = less + first, q.tiles[3 * t + 2] = min(q.tile_m, equal - first);
+  }
+}
+
 // A workgroup: TT tiles of 16 tokens.  Latencies: the inputs are split over the waves, every operand of U steps is asked for before the first is
 // used (16 waves: all of 2048 inputs at once), and the choice of a token with up to 64 outputs stays in one wave's registers.  Few tokens: 16 waves
 // share a tile, so that a wave chooses for one token; many: eight waves (mv_moe_route).  34 outputs of 2048 inputs, alone: 24 tokens 18.8 -> 11.0 us; one
 // launch behind the other, eight waves with a step's loads at a time -> now: 24 tokens 14.7 -> 9.7, 9001 24 -> 16; 128 outputs of 512 inputs: one token
 // 12.7 -> 12.8, 24 20.5 -> 15.4, 20000 53 -> 51; fp32, 34 outputs of 2048 inputs, 4400 tokens: 392 -> 131.  Now 9001 tokens with the choices of four tokens
 // at once, one launch between events, 29.3 -> 24.4: 8.5 of 20 us are the products (their inputs by half lines), 282 workgroups on 256 CUs.
-template <typename Tag, int WAVES, int TT>
-__global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
+// GROUP (one workgroup has all tokens): the choices stay in LDS for the grouping behind them, a launch and a trip to memory less.  Both products with what is around them, 32
+// experts: 12 tokens of 4 choices (2048 -> 768) 67.2 -> 65.7 us, 4 of 8 (1024 -> 384; the host's) 48.5 -> 44.5, 16 of 8 49.3 -> 45.2.  Up to one tile: two tiles in one
+// workgroup in place of two workgroups cost more than the launch (24 of 4 70.2 -> 74.0, 32 of 8 84 -> 95).
+template <typename Tag, int WAVES, int TT, bool GROUP>
+__global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p, RouteGroups q) {
   typedef typename elem<Tag>::T T;
+  static_assert(!GROUP || (WAVES == 16 && TT == 1 && !__is_same(Tag, f32_tag)), "sixteen waves group, in the place of the partial tiles");
   constexpr int TOKENS = 16 * TT, U = WAVES == 16 ? 4 : 2;
   extern __shared__ float lds[];   // logits [TOKENS][outputs] | scratch [TOKENS][outputs] | (16-bit) partial tiles
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m0 = blockIdx.x * TOKENS, R = p.outputs;
@@ -301,12 +347,22 @@ __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p) {
       __syncthreads();
     }
   }
+  int *ids_too = GROUP ? (int *)(ch + TOKENS * R) : nullptr;
+  float *weights_too = GROUP ? (float *)(ids_too + kRoutePairs + 4) : nullptr;
   __syncthreads();
+  if constexpr (GROUP) {
+    const int pairs = p.rows * p.top;
+    if (tid < 4) ids_too[pairs + tid] = -1;
+  }
   if (FOUR && R <= 64 && p.groups <= 8) {
     for (int t = wave * 4 + (lane >> 4); t < TOKENS; t += WAVES * 4) choose_four<Tag>(p, sc + t * R, m0 + t, m0 + t < p.rows, corrections);
     return;
   }
-  for (int t = wave; t < TOKENS && m0 + t < p.rows; t += WAVES) choose<Tag>(p, sc + t * R, ch + t * R, m0 + t, corrections[0]);   // (no barrier in it)
+  for (int t = wave; t < TOKENS && m0 + t < p.rows; t += WAVES) choose<Tag>(p, sc + t * R, ch + t * R, m0 + t, corrections[0], ids_too, weights_too);   // (no barrier in it)
+  if constexpr (GROUP) {
+    __syncthreads();
+    group_few(q, ids_too, weights_too, p.rows * p.top, p.top);
+  }
 }
 
 // ---- grouping.  Workgroup (e, part): the pairs of expert e, which start behind those of the experts before it.  Each wave walks a run of all
@@ -822,18 +878,19 @@ int launch_linear(const MoeLinear &p, int tile_m, int max_tiles, hipStream_t st)
   return MV_OK;
 }
 
-template <typename Tag, int WAVES, int TT>
-int launch_route(const RouteParams &p, hipStream_t st) {
+template <typename Tag, int WAVES, int TT, bool GROUP = false>
+int launch_route(const RouteParams &p, hipStream_t st, const RouteGroups &q = {}) {
   const size_t lds = (size_t)2 * 16 * TT * p.outputs * 4 + (__is_same(Tag, f32_tag) ? 0 : WAVES * kRouteTiles * TT * 1024);
-  if (int rc = mv_allow_lds<moe_route_kernel<Tag, WAVES, TT>>()) return rc;
-  hipLaunchKernelGGL((moe_route_kernel<Tag, WAVES, TT>), dim3((p.rows + 16 * TT - 1) / (16 * TT)), dim3(WAVES * 64), lds, st, p);
+  if (int rc = mv_allow_lds<moe_route_kernel<Tag, WAVES, TT, GROUP>>()) return rc;
+  hipLaunchKernelGGL((moe_route_kernel<Tag, WAVES, TT, GROUP>), dim3((p.rows + 16 * TT - 1) / (16 * TT)), dim3(WAVES * 64), lds, st, p, q);
   return MV_OK;
 }
 
 }  // namespace
 
-extern "C" int mv_moe_route(const void *x, int64_t x_stride, const void *w, const void *correction, int32_t *ids, float *weights,
-                            int rows, int k, int outputs, int top, int groups, int keep, float scale, int flags, int dtype, void *stream) {
+// `group` (or NULL): grouping along, where one workgroup has all tokens; *grouped says whether
+static int route(const void *x, int64_t x_stride, const void *w, const void *correction, int32_t *ids, float *weights, int rows, int k, int outputs, int top, int groups,
+                 int keep, float scale, int flags, int dtype, void *stream, const RouteGroups *group, bool *grouped) {
   if (rows == 0) return MV_OK;
   if (!x || !w || !ids || !weights) return MV_E_NULLPTR;
   if (flags & ~(MV_ROUTE_SIGMOID | MV_ROUTE_RAW)) return MV_E_RANGE;
@@ -851,6 +908,12 @@ extern "C" int mv_moe_route(const void *x, int64_t x_stride, const void *w, cons
     const hipStream_t st = (hipStream_t)stream;
     const bool full = k > 2048 && (rows <= 8192 || (k >= 4096 && (rows - 1) % 8192 >= 4096));
     int rc;
+    if constexpr (!__is_same(Tag, f32_tag)) {
+      if (group && rows <= kRouteRows && rows * top <= kRoutePairs && group->experts <= kRouteExperts && outputs <= 64 && groups <= 8) {
+        *grouped = true;
+        return launch_route<Tag, 16, 1, true>(p, st, *group);
+      }
+    }
     if (rows <= 16 * 256) rc = launch_route<Tag, 16, 1>(p, st);
     else if (dtype != MV_F32 && (outputs <= 64 ? k >= 2048 : outputs <= 256 && full)) rc = launch_route<Tag, 8, 2>(p, st);
     else rc = launch_route<Tag, 8, 1>(p, st);
@@ -858,6 +921,11 @@ extern "C" int mv_moe_route(const void *x, int64_t x_stride, const void *w, cons
   });
   MV_LAUNCH_CHECK();
   return MV_OK;
+}
+
+extern "C" int mv_moe_route(const void *x, int64_t x_stride, const void *w, const void *correction, int32_t *ids, float *weights,
+                            int rows, int k, int outputs, int top, int groups, int keep, float scale, int flags, int dtype, void *stream) {
+  return route(x, x_stride, w, correction, ids, weights, rows, k, outputs, top, groups, keep, scale, flags, dtype, stream, nullptr, nullptr);
 }
 
 extern "C" int mv_moe_group(const int32_t *ids, int pairs, int top, int experts, int tile_m, int max_tiles, int32_t *rows,
@@ -935,11 +1003,15 @@ extern "C" int mv_moe_mlp(const MvMoeMlpArgs *a, int dtype, void *stream) {
   int32_t *ids = (int32_t *)ws, *tokens = (int32_t *)(ws + m.tokens), *tiles = (int32_t *)(ws + m.tiles);
   float *by_place = a->weigh_inputs ? (float *)(ws + m.weights) : nullptr;
   const int pairs = a->rows * a->top, max_tiles = (int)m.max_tiles;
-  if (int rc = mv_moe_route(a->x, a->x_stride, a->router, a->correction, ids, a->weights, a->rows, a->router_k, a->outputs, a->top, a->groups, a->keep, a->scale,
-                            a->route_flags, dtype, stream))
+  // (few tokens are grouped by the router's workgroup)
+  const RouteGroups few{a->place, tokens, tiles, by_place, a->experts, a->tile_m & 0xffff, max_tiles};
+  bool grouped = false;
+  if (int rc = route(a->x, a->x_stride, a->router, a->correction, ids, a->weights, a->rows, a->router_k, a->outputs, a->top, a->groups, a->keep, a->scale,
+                     a->route_flags, dtype, stream, &few, &grouped))
     return rc;
-  if (int rc = mv_moe_group(ids, pairs, a->top, a->experts, a->tile_m & 0xffff, max_tiles, a->place, tokens, tiles, by_place ? a->weights : nullptr, by_place, stream))
-    return rc;
+  if (!grouped)
+    if (int rc = mv_moe_group(ids, pairs, a->top, a->experts, a->tile_m & 0xffff, max_tiles, a->place, tokens, tiles, by_place ? a->weights : nullptr, by_place, stream))
+      return rc;
   MvMoeLinearArgs p{};
   p.x = a->x, p.w = a->gate_up, p.out = ws + m.z, p.tokens = tokens, p.tiles = tiles, p.act = a->act, p.in_scale = by_place;
   p.x_stride = a->x_stride, p.out_stride = a->ff, p.max_tiles = max_tiles, p.tile_m = a->tile_m, p.n = a->ff, p.k = a->k;

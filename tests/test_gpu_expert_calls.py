@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("rows, tile", [(1, 16), (24, 32), (77, 64), (700, 256)])
+@pytest.mark.parametrize("rows, tile", [(1, 16), (16, 16), (17, 16), (24, 32), (32, 16), (33, 16), (77, 64), (700, 256)])      # (up to 16 rows the router groups)
 @pytest.mark.parametrize("weigh", [False, True])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_one_call_is_four(rows, tile, weigh, dtype):
