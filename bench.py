@@ -651,6 +651,17 @@ def _mfma_busy_quote():
     return None, None
 
 
+def moe_mlp_by_parts(x, router, correction, gate_up, down, experts, ff, width, top, tile_m, act, groups=1, keep=1, scale=1.0, sigmoid=False, raw=False,
+                     weigh_inputs=False, quarters=False):
+    """``hip_ops.moe_mlp`` as the four calls that it is one of (the same launches from 17 tokens on), so that a probe sees each product."""
+    from minivllm_amd import hip_ops
+
+    ids, weights = hip_ops.moe_route(x, router, correction, top, groups, keep, scale, sigmoid, raw)
+    g = hip_ops.moe_group(ids, experts, tile_m, weights if weigh_inputs else None)
+    z = hip_ops.moe_linear(x, gate_up, ff, g, act, gather=True, experts=experts, in_scale=g.weights, quarters=quarters)
+    return hip_ops.moe_linear(z, down, width, g, experts=experts, quarters=quarters), g.place, weights
+
+
 def prefill_records(engine, model, gpus=1, cases=PREFILL_CASES, reps=5):
     """Prefill tokens/s of the whole model step (config-4 prompt shapes): n prompts x len fresh
     random tokens through ``execute_batch(prefill=True)`` -- input build, H2D, every layer, LM head on the last
@@ -679,10 +690,11 @@ def prefill_records(engine, model, gpus=1, cases=PREFILL_CASES, reps=5):
             probing = rep == reps + 1
             entries = {entry: "prefill", "ssm_prefill": "ssm", "delta_prefill": "delta", "moe_linear": "experts", "gru_prefill": "gru",
                        "stream_update": "edges", "residual_update": "edges", "gelu_erf": "act", "act_and_mul": "act"}
-            reals = {e: getattr(hip_ops, e) for e in entries}
+            reals = {e: getattr(hip_ops, e) for e in (*entries, "moe_mlp")}
             if probing:
                 for e, key in entries.items():
                     setattr(attn_mod.hip_ops, e, probe.wrap(key, reals[e]))
+                attn_mod.hip_ops.moe_mlp = moe_mlp_by_parts
             try:
                 torch.cuda.synchronize()
                 t0 = time.perf_counter()
@@ -723,14 +735,14 @@ def prefill_records(engine, model, gpus=1, cases=PREFILL_CASES, reps=5):
         if gru_modules(ex):
             m0, us = gru_modules(ex)[0], statistics.median(probe.times_us("gru"))
             out[-1]["ssm_roofline"] = dict(_hbm(n * ln * m0.n * 4 * ex.dtype.itemsize, us), kernel="gru_chunk_kernel + gru_walk_kernel")
-            out[-1].update(_delta_and_expert_prefill(ex, n * ln, probe))
+            out[-1].update(_delta_and_expert_prefill(ex, n, n * ln, probe))
         elif recurrent_modules(ex) and hasattr(recurrent_modules(ex)[0], "state"):
-            out[-1].update(_delta_and_expert_prefill(ex, n * ln, probe))
+            out[-1].update(_delta_and_expert_prefill(ex, n, n * ln, probe))
         elif ex.state_modules:
             m0, t_ssm = ex.state_modules[0], sorted(probe.times_us("ssm"))
             us = t_ssm[len(t_ssm) // 2]
             byt = n * ln * (2 * m0.heads * m0.p + 2 * m0.groups * m0.n + m0.heads) * ex.dtype.itemsize
-            out[-1]["ssm_roofline"] = {"bound": "hbm", "kernel": "ssm_chunk_kernel", "bytes_per_launch": byt, "us_per_launch": round(us, 2),
+            out[-1]["ssm_roofline"] = {"bound": "hbm", "kernel": "ssm_chunk_kernel or ssm_heads_kernel", "bytes_per_launch": byt, "us_per_launch": round(us, 2),
                                        "achieved": round(byt / us / 1e3, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                        "frac": round(byt / us / 1e3 / HBM_PEAK_GBS, 4)}
     return out
@@ -762,21 +774,25 @@ def _edge_prefill(ex, tokens: int, probe) -> dict:
     return out
 
 
-def _delta_and_expert_prefill(ex, tokens: int, probe) -> dict:
-    """Rooflines of mv_delta_prefill (bytes of its inputs and outputs, the layers of each kind apart) and of the two expert products."""
+def _delta_and_expert_prefill(ex, prompts: int, tokens: int, probe) -> dict:
+    """Rooflines of mv_delta_prefill_conv (bytes of its inputs and outputs, the convolution's weights and kept inputs among them, the layers of each kind
+    apart) and of the two expert products."""
     out, mods = {}, recurrent_modules(ex)
     t = probe.times_us("delta")
     for key, kind in (("ssm_roofline", False), ("channel_decay_roofline", True)):
         mine = [(m, us) for m, us in zip(mods, t) if m.shape.channel_decay == kind]
         if mine:
             s, us = mine[0][0].shape, statistics.median(u for _, u in mine)
-            byt = tokens * (2 * s.heads * s.p + 2 * s.groups * s.n + s.heads * (1 + (s.n if kind else 1))) * ex.dtype.itemsize
-            names = "delta_prepare_kernel + delta_walk_kernel" if kind else "delta_scalar_prepare_kernel + delta_scalar_walk_kernel"
+            taps = mine[0][0].conv.shape[0]
+            byt = (tokens * (2 * s.heads * s.p + 2 * s.groups * s.n + s.heads * (1 + (s.n if kind else 1)))
+                   + s.channels * (taps + prompts * (taps - 1))) * ex.dtype.itemsize
+            names = ("causal convolution (of its own or in the next kernel) + "
+                     + ("delta_prepare_kernel + delta_walk_kernel" if kind else "delta_scalar_prepare_kernel + delta_scalar_walk_kernel"))
             out[key] = {"bound": "hbm", "kernel": names, "bytes_per_launch": byt,
                         "us_per_launch": round(us, 2), "achieved": round(byt / us / 1e3, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                         "frac": round(byt / us / 1e3 / HBM_PEAK_GBS, 4)}
     experts, t = expert_modules(ex), probe.times_us("experts")
-    if experts:
+    if experts and t:
         m0 = experts[0]
         pairs = tokens * m0.top * m0.experts / m0.router.shape[0]      # (identity experts have no product)
         for key, us, n in (("gate_up", t[0::2], 2), ("down", t[1::2], 1)):
@@ -1229,7 +1245,8 @@ def _delta_graph_roofline(ex, lens, slots) -> dict:
 
 
 def expert_graph_rooflines(engine, batch: int) -> dict | None:
-    """Routing and the two expert products of every layer with experts, on random rows: weight bytes of the experts that were chosen."""
+    """Routing and the two expert products of every layer with experts, on random rows: weight bytes of the experts that were chosen.  (Router and grouping as
+    two launches; a step of up to 16 rows has them in one.)"""
     from minivllm_amd import hip_ops
 
     ex = engine.model_runner.inference_executor

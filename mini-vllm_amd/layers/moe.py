@@ -101,6 +101,12 @@ class ExpertMLP(nn.Module):
         wide = rows * math.ceil(2 * self.f / 256) >= WIDE_GROUPS[0] and rows * math.ceil(self.w / 256) >= WIDE_GROUPS[1]
         return 256 if wide else 64
 
+    def route(self, h):
+        """-> (weights [T, top], the pairs sorted by expert), for callers that have use for the parts; ``forward`` makes both in its one call."""
+        ids, weights = hip_ops.moe_route(h, self.router, self.correction, self.top, self.groups, self.keep, self.scale, self.sigmoid,
+                                         self.raw_weights)
+        return weights, hip_ops.moe_group(ids, self.experts, self.tile_rows(h.shape[0]), weights if self.weigh_inputs else None)
+
     def forward(self, h):
         """-> (shared expert's output or None, the routed experts' part for ``hip_ops.residual_update``)."""
         tile = self.tile_rows(h.shape[0])

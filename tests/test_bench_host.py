@@ -189,3 +189,76 @@ def test_design_configurations_have_the_layer_sizes_of_their_peers():
     assert args.design == "mofarax" and bench.parse([]).design is None and bench.parse([]).model == "qwen3-1.7b"
     # a chunk mask cuts the work of a prompt into the chunks' triangles
     assert bench.prefill_flops(2, 64, [100], 30) == bench.prefill_flops(2, 64, [30, 30, 30, 10])
+
+
+def test_probes_drive_a_model_with_experts(monkeypatch):
+    """The records of ``--design``, with kernels by stand-ins that only have their shapes: the prefill probe sees both products of every layer with experts and the
+    delta rule's one call, the decode probe routes through the layer; a model whose experts are not asked for makes no record of them."""
+    import inspect
+
+    import torch
+    from minivllm_amd import hip_ops
+    from minivllm_amd.layers.delta_rule import GatedDeltaRule
+    from minivllm_amd.layers.moe import ExpertMLP
+
+    # the four calls take what the one does
+    assert ([(p.name, p.default) for p in inspect.signature(bench.moe_mlp_by_parts).parameters.values()]
+            == [(p.name, p.default) for p in inspect.signature(hip_ops.moe_mlp).parameters.values()])
+
+    class Event:
+        def record(self, stream=None):
+            pass
+
+        def elapsed_time(self, other):
+            return 0.5
+
+    def group(ids, experts, tile_m, weights=None):
+        pairs, by = ids.numel(), torch.zeros(ids.numel()) if weights is not None else None
+        tiles = torch.tensor([[e if (ids == e).any() else -1, 0, 0] for e in range(experts)], dtype=torch.int32)
+        return hip_ops.ExpertGroups(torch.arange(pairs, dtype=torch.int32), torch.zeros(pairs, dtype=torch.int32), tiles, tile_m, by)
+
+    def linear(x, w, n, groups, act=None, gather=False, experts=0, in_scale=None, quarters=False):
+        assert w.numel() == experts * n * x.shape[1] * (2 if act is not None else 1)
+        return torch.zeros(groups.tokens.numel(), n)
+
+    calls = []
+    whole = lambda x, *a: calls.append(a) or (torch.zeros(x.shape[0] * a[7], a[6]), None, torch.zeros(x.shape[0], a[7]))
+    for name, fake in (("moe_route", lambda x, w, c, top, *a: (torch.arange(x.shape[0] * top, dtype=torch.int32).view(-1, top) % 4, torch.zeros(x.shape[0], top))),
+                       ("moe_group", group), ("moe_linear", linear), ("moe_mlp", whole), ("prefill_varlen", lambda: None), ("delta_prefill", lambda: None)):
+        monkeypatch.setattr(hip_ops, name, fake)
+    monkeypatch.setattr(torch.cuda, "Event", lambda **kw: Event())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: None)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: None)
+    monkeypatch.setattr(bench, "_graph_time_us", lambda fn, launches, reps=5: (fn(), 5.0)[1])
+
+    mlps = [ExpertMLP(64, 4, 1, 2, 1, 1, 1.0, 64), ExpertMLP(64, 4, 0, 2, 1, 1, 1.0, 64, weigh_inputs=True)]
+    rule = GatedDeltaRule(2, 1, 32, 32, 4, 1e-6)
+
+    class Executor:
+        device, dtype, latents, state_modules, model = "cpu", torch.bfloat16, [], [rule], torch.nn.ModuleList([*mlps, rule])
+        asked = mlps
+
+        def execute_batch(self, seqs, prefill):
+            hip_ops.prefill_varlen()
+            hip_ops.delta_prefill()
+            for m in self.asked:
+                m(torch.zeros(3, m.w))
+
+    blocks = type("Blocks", (), {"allocate": lambda self, s: None, "deallocate": lambda self, s: None})()
+    engine = type("Engine", (), {})()
+    engine.scheduler = type("Scheduler", (), {"block_manager": blocks})()
+    engine.model_runner = type("Runner", (), {"inference_executor": Executor()})()
+
+    rec, = bench.prefill_records(engine, "qwen3-0.6b", cases=((2, 8),), reps=2)
+    assert len(calls) == 3 * len(mlps) and hip_ops.moe_mlp is whole      # the timed batches as they are; nothing left behind
+    for part, n in (("gate_up", 2), ("down", 1)):
+        r = rec[f"expert_{part}_roofline"]
+        assert r["us_per_launch"] == 500.0 and r["flops_per_launch"] == int(2 * (16 * 2 * 4 / 5) * n * 64 * 64)
+    s, r = rule.shape, rec["ssm_roofline"]
+    assert r["bytes_per_launch"] == 2 * (16 * (s.channels + 2 * 32 + 2 * 2) + s.channels * (4 + 2 * 3)) and "convolution" in r["kernel"]
+    Executor.asked = []
+    rec, = bench.prefill_records(engine, "qwen3-0.6b", cases=((2, 8),), reps=1)
+    assert "ssm_roofline" in rec and not any(k.startswith("expert") for k in rec)
+
+    rec = bench.expert_graph_rooflines(engine, 3)
+    assert rec["gate_up"]["bytes_per_launch"] == 2 * rec["down"]["bytes_per_launch"] == 2 * 4 * 64 * 64 * 2 and rec["route_and_group_us"] == 5.0
