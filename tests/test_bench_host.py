@@ -255,7 +255,7 @@ def test_probes_drive_a_model_with_experts(monkeypatch):
         r = rec[f"expert_{part}_roofline"]
         assert r["us_per_launch"] == 500.0 and r["flops_per_launch"] == int(2 * (16 * 2 * 4 / 5) * n * 64 * 64)
     s, r = rule.shape, rec["ssm_roofline"]
-    assert r["bytes_per_launch"] == 2 * (16 * (s.channels + 2 * 32 + 2 * 2) + s.channels * (4 + 2 * 3)) and "convolution" in r["kernel"]
+    assert r["bytes_per_launch"] == 2 * (16 * (4 * 32 + 2 * 32 + 2 * 2) + s.channels * (4 + 2 * 3)) and "convolution" in r["kernel"]
     Executor.asked = []
     rec, = bench.prefill_records(engine, "qwen3-0.6b", cases=((2, 8),), reps=1)
     assert "ssm_roofline" in rec and not any(k.startswith("expert") for k in rec)
