@@ -10,7 +10,8 @@ namespace {
 template <typename Tag>
 __device__ __forceinline__ float param(const void *p, int i) { return elem<Tag>::ld(((const typename elem<Tag>::T *)p)[i]); }
 
-// ---- convolution: 8 (fp32: 4) channels per thread, kConvRows tokens per workgroup (few workgroups: kConvAhead), a sliding window of inputs in registers
+// ---- convolution: 8 (fp32: 4) channels per thread, kConvRows tokens per workgroup (few workgroups: kConvAhead), a sliding window of inputs in registers.  The
+// window is the taps: in one of more, an infinite input times a weight that is not there would reach tokens that it does not belong to, by where workgroups begin
 constexpr int kConvRows = 32, kConvAhead = 8, kMaxTaps = 8;
 
 template <typename Tag, int TAPS, int ROWS>
@@ -20,7 +21,8 @@ __global__ void __launch_bounds__(64) causal_conv_kernel(MvSsmArgs p) {
   const int c = ((int)blockIdx.x * 64 + threadIdx.x) * VEC, s = blockIdx.z;
   const int q0 = p.cu_q[s], len = p.cu_q[s + 1] - q0, t0 = blockIdx.y * ROWS;
   if (t0 >= len || c >= p.channels) return;
-  const int before = p.cu_k[s + 1] - p.cu_k[s] - len, slot = p.state_slots[s], back = p.taps - 1;
+  constexpr int back = TAPS - 1;
+  const int before = p.cu_k[s + 1] - p.cu_k[s] - len, slot = p.state_slots[s];
   const bool keep = slot >= 0 && slot < p.slots;
   const int64_t half = p.slots * back * p.channels;
   T *state = (T *)p.conv_state;
@@ -33,30 +35,20 @@ __global__ void __launch_bounds__(64) causal_conv_kernel(MvSsmArgs p) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) f[j] = 0.f;
   };
-  // weights aligned at the current token: tap TAPS - 1 is its own
-  float w[TAPS][VEC], bias[VEC], win[TAPS][VEC];
-#pragma unroll
-  for (int i = 0; i < TAPS; ++i)
-#pragma unroll
-    for (int j = 0; j < VEC; ++j) w[i][j] = win[i][j] = 0.f;
+  float w[TAPS][VEC], bias[VEC], win[TAPS][VEC];   // tap TAPS - 1 is the current token's
 #pragma unroll
   for (int i = 0; i < TAPS; ++i) {
-    const int tap = i - (TAPS - p.taps);
-    if (tap >= 0) {
-      load_vec_row<Tag>((const T *)p.conv_w + (int64_t)tap * p.channels + c, w[i]);
-      if (i < TAPS - 1) input(t0 + i - (TAPS - 1), win[i + 1]);   // shifted down below
-    }
+    load_vec_row<Tag>((const T *)p.conv_w + (int64_t)i * p.channels + c, w[i]);
+    if (i < back) input(t0 + i - back, win[i + 1]);   // shifted down below
   }
 #pragma unroll
   for (int j = 0; j < VEC; ++j) bias[j] = 0.f;
   if (p.conv_b) load_vec_row<Tag>((const T *)p.conv_b + c, bias);
-  if (t0 == 0 && keep && back > 0) {   // the only workgroup that reads the old state writes the new one, behind its reads
-    float last[kMaxTaps - 1][VEC];
-    for (int j = 0; j < kMaxTaps - 1; ++j)
-      if (j < back) input(len - back + j, last[j]);
+  if (back > 0 && t0 == 0 && keep) {   // the only workgroup that reads the old state writes the new one, behind its reads
+    float last[TAPS][VEC];
+    for (int j = 0; j < back; ++j) input(len - back + j, last[j]);
     T *ns = state + ((before + len) & 1) * half + (int64_t)slot * back * p.channels + c;
-    for (int j = 0; j < kMaxTaps - 1; ++j)
-      if (j < back) store_vec_row<Tag>(ns + (int64_t)j * p.channels, last[j]);
+    for (int j = 0; j < back; ++j) store_vec_row<Tag>(ns + (int64_t)j * p.channels, last[j]);
   }
   const int t1 = min(len, t0 + ROWS);
   for (int tb = t0; tb < t1; tb += kConvAhead) {
@@ -67,14 +59,14 @@ __global__ void __launch_bounds__(64) causal_conv_kernel(MvSsmArgs p) {
     for (int u = 0; u < kConvAhead; ++u) {
       float o[VEC];
 #pragma unroll
-      for (int i = 0; i < TAPS - 1; ++i)
+      for (int i = 0; i < back; ++i)
 #pragma unroll
         for (int j = 0; j < VEC; ++j) win[i][j] = win[i + 1][j];
       if constexpr (VEC == 8) {
-        unpack8<Tag>(raw[u], win[TAPS - 1]);
+        unpack8<Tag>(raw[u], win[back]);
       } else {
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) win[TAPS - 1][j] = u2f(raw[u][j]);
+        for (int j = 0; j < VEC; ++j) win[back][j] = u2f(raw[u][j]);
       }
 #pragma unroll
       for (int j = 0; j < VEC; ++j) o[j] = bias[j];
@@ -345,11 +337,11 @@ int mv_check_conv(const MvSsmArgs *a, int dtype) {
 template <int ROWS>
 static int launch_conv(const MvSsmArgs &a, int x, int dtype, hipStream_t st) {
   const dim3 grid(x, (a.max_q + ROWS - 1) / ROWS, a.n_seqs);
-  MV_DISPATCH_DTYPE(dtype, {
-    if (a.taps <= 2) hipLaunchKernelGGL((causal_conv_kernel<Tag, 2, ROWS>), grid, dim3(64), 0, st, a);
-    else if (a.taps <= 4) hipLaunchKernelGGL((causal_conv_kernel<Tag, 4, ROWS>), grid, dim3(64), 0, st, a);
-    else hipLaunchKernelGGL((causal_conv_kernel<Tag, kMaxTaps, ROWS>), grid, dim3(64), 0, st, a);
-  });
+#define MV_TAPS(T_) \
+  case T_: hipLaunchKernelGGL((causal_conv_kernel<Tag, T_, ROWS>), grid, dim3(64), 0, st, a); break
+  static_assert(kMaxTaps == 8, "a case each");
+  MV_DISPATCH_DTYPE(dtype, switch (a.taps) { MV_TAPS(1); MV_TAPS(2); MV_TAPS(3); MV_TAPS(4); MV_TAPS(5); MV_TAPS(6); MV_TAPS(7); MV_TAPS(8); });
+#undef MV_TAPS
   MV_LAUNCH_CHECK();
   return MV_OK;
 }

@@ -30,3 +30,26 @@ def test_rows_of_a_workgroup(taps, dtype):
         got = H.causal_conv(x[i * total:(i + 1) * total], w, b, shape, part, ints(range(i * n, (i + 1) * n)), cu(tokens), cu(ends), max(tokens))
         assert torch.equal(got, out[i * total:(i + 1) * total])
         assert torch.equal(part[:, i * n:(i + 1) * n], all_kept[:, i * n:(i + 1) * n])
+
+
+@pytest.mark.parametrize("taps", range(1, 9))
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_infinite_inputs_reach_their_taps(taps, dtype):
+    """An infinity or NaN reaches the tokens that have a tap for it and no other, wherever a workgroup's tokens begin, in either form."""
+    from minivllm_amd import hip_ops as H
+
+    tokens, channels, struck = 99, 96, {0: float("inf"), 6: float("nan"), 31: float("-inf"), 61: float("nan"), 98: float("inf")}
+    g = torch.Generator(device=DEV).manual_seed(taps)
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    x, w = (torch.randn(n, channels, generator=g, device=DEV).to(dtype) for n in (tokens, taps))
+    for t, v in struck.items():
+        x[t] = v
+    for times in (1, 450):      # 4 workgroups of 32 tokens, 1800
+        cu = ints(range(0, tokens * times + 1, tokens))
+        kept = torch.zeros(2, times, taps - 1, channels, dtype=dtype, device=DEV)
+        out = H.causal_conv(x.repeat(times, 1), w, None, (2, 1, 16, 32, 32, 64), kept, ints(range(times)), cu, cu, tokens).view(times, tokens, channels)
+        reached = torch.zeros(tokens, dtype=torch.bool, device=DEV)
+        for t in struck:
+            reached[t:t + taps] = True
+        assert torch.isfinite(out[:, ~reached]).all()
+        assert all(not torch.isfinite(out[:, t]).any(0).all() for t in struck)
