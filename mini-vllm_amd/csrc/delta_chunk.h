@@ -50,15 +50,16 @@ __device__ __forceinline__ int chunk_sequence(const MvDeltaArgs &p, int slot) {
   }
   return seq;
 }
-// The causal convolution and silu of causal_conv_kernel (the same sums) for a chunk's channels of a group, THREADS threads, four channels and eight tokens a
-// thread and turn: k and q of group `grp` (N channels each), `values` of v from `first` on.  put(0: k, 1: q, 2: v; row; place among those channels; channel;
-// results, zeros behind the end): every row of k and q, with ALL of v too.  What is kept of the inputs is written along with a sequence's first rows.
+constexpr int kChunkTaps = 4;
+// The causal convolution of kChunkTaps taps and silu of causal_conv_kernel (the same sums) for a chunk's channels of a group, THREADS threads, four channels and
+// eight tokens a thread and turn: k and q of group `grp` (N channels each), `values` of v from `first` on.  put(0: k, 1: q, 2: v; row; place among those channels;
+// channel; results, zeros behind the end): every row of k and q, with ALL of v too.  What is kept of the inputs is written along with a sequence's first rows.
 template <typename Tag, int N, int THREADS, bool ALL, typename Put>
 __device__ __forceinline__ void conv_chunk(const DeltaPrep &q, int seq, int q0, int len, int t0, int nt, int grp, int first, int values, int tid, Put put) {
   typedef uint16_t T;
-  constexpr int TAPS = 4, ROWS = 8;
+  constexpr int TAPS = kChunkTaps, ROWS = 8, back = TAPS - 1;
   const MvDeltaArgs &p = q.a;
-  const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq], back = p.taps - 1;
+  const int before = p.cu_k[seq + 1] - p.cu_k[seq] - len, slot = p.state_slots[seq];
   const bool keep = slot >= 0 && slot < p.slots;
   const int64_t half = p.slots * back * p.channels;
   const T *conv_w = (const T *)p.conv_w, *from = (const T *)q.raw + (int64_t)q0 * q.raw_stride;
@@ -75,42 +76,35 @@ __device__ __forceinline__ void conv_chunk(const DeltaPrep &q, int seq, int q0, 
     const int c = which == 0 ? p.k_off + grp * N + at : which == 1 ? p.q_off + grp * N + at : first + at;
     auto input = [&](int t) {   // input `t` of the step (t < 0: of the steps before it)
       if (t >= 0) return *(const u32x2 *)(from + (int64_t)min(t, len - 1) * q.raw_stride + c);
-      if (before > 0 && keep && back + t >= 0) return *(const u32x2 *)(old_state + (int64_t)(back + t) * p.channels + c);
+      if (before > 0 && keep) return *(const u32x2 *)(old_state + (int64_t)(back + t) * p.channels + c);
       return u32x2{0u, 0u};
     };
     float w[TAPS][4], win[TAPS][4];
     if (!ALL && tr >= nt && which > 1) continue;
-    u32x2 raw[TAPS - 1], rows[ROWS];
+    u32x2 raw[back], rows[ROWS];
 #pragma unroll
-    for (int i = 0; i < TAPS - 1; ++i) raw[i] = input(t0 + tr + i - (TAPS - 1));
+    for (int i = 0; i < back; ++i) raw[i] = input(t0 + tr + i - back);
 #pragma unroll
     for (int u = 0; u < ROWS; ++u) rows[u] = input(t0 + tr + u);
 #pragma unroll
-    for (int i = 0; i < TAPS; ++i) {
-      const int tap = i - (TAPS - p.taps);   // (weights stand at the current token's end)
-      u32x2 v = {0u, 0u};
-      if (tap >= 0) v = *(const u32x2 *)(conv_w + (int64_t)tap * p.channels + c);
-      unpack4(v, w[i]);
-    }
+    for (int i = 0; i < TAPS; ++i) unpack4(*(const u32x2 *)(conv_w + (int64_t)i * p.channels + c), w[i]);
 #pragma unroll
-    for (int i = 0; i < TAPS - 1; ++i) unpack4(raw[i], win[i + 1]);   // shifted down below
-    if (t0 + tr == 0 && keep && back > 0) {   // the only thread that reads the old state here writes the new one, behind its reads
-      u32x2 last[TAPS - 1];
+    for (int i = 0; i < back; ++i) unpack4(raw[i], win[i + 1]);   // shifted down below
+    if (t0 + tr == 0 && keep) {   // the only thread that reads the old state here writes the new one, behind its reads
+      u32x2 last[back];
 #pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j)
-        if (j < back) last[j] = input(len - back + j);
+      for (int j = 0; j < back; ++j) last[j] = input(len - back + j);
       T *ns = (T *)p.conv_state + ((before + len) & 1) * half + (int64_t)slot * back * p.channels + c;
 #pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j)
-        if (j < back) *(u32x2 *)(ns + (int64_t)j * p.channels) = last[j];
+      for (int j = 0; j < back; ++j) *(u32x2 *)(ns + (int64_t)j * p.channels) = last[j];
     }
 #pragma unroll
     for (int u = 0; u < ROWS; ++u) {
 #pragma unroll
-      for (int i = 0; i < TAPS - 1; ++i)
+      for (int i = 0; i < back; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) win[i][j] = win[i + 1][j];
-      unpack4(rows[u], win[TAPS - 1]);
+      unpack4(rows[u], win[back]);
       float o[8] = {};   // (four of them: packed as causal_conv_kernel packs eight)
 #pragma unroll
       for (int i = 0; i < TAPS; ++i)

@@ -890,12 +890,13 @@ int launch(const DeltaPrep &q, int seg, hipStream_t stream) {
 
 }  // namespace
 
-// The convolution goes along where every channel is one workgroup's (which reads and writes what is kept of it), a thread's window holds the taps and, with
-// a head's values prepared (not bf16 with one decay per head), a wave has one tile of them and LDS holds them in the decays' place
+// The convolution goes along where every channel is one workgroup's (which reads and writes what is kept of it), a thread's window is the taps (in one of more, an
+// infinite input times a weight that is not there would reach tokens that it does not belong to) and, with a head's values prepared (not bf16 with one decay
+// per head), a wave has one tile of them and LDS holds them in the decays' place
 bool mv_delta_chunk_takes_conv(const MvDeltaArgs &a, int dtype) {
   const bool scalar = dtype == MV_BF16 && !a.channel_decay;
   const int of_group = a.heads / a.groups;
-  return (scalar ? of_group <= 2 : of_group == 1 && a.p <= 16 * kPrepareWaves && a.p <= 2 * a.n) && a.taps >= 1 && a.taps <= 4 && a.k_off == a.heads * a.p &&
+  return (scalar ? of_group <= 2 : of_group == 1 && a.p <= 16 * kPrepareWaves && a.p <= 2 * a.n) && a.taps == kChunkTaps && a.k_off == a.heads * a.p &&
          a.q_off == a.k_off + a.groups * a.n && a.channels == a.q_off + a.groups * a.n;
 }
 
