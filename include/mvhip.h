@@ -740,7 +740,8 @@ size_t mv_delta_prefill_workspace_bytes(int n_seqs, int total_q, int heads, int 
 enum { MV_DELTA_WHOLE = 512 };
 size_t mv_delta_prefill_segments_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int channel_decay, int dtype);
 int mv_delta_prefill(const MvDeltaArgs *args, int dtype, int flags, void *stream);
-/* the same from projected channels: mv_causal_conv (conv_w, taps, conv_state; no bias) into xc [total_q][channels], by a launch of its own or along the way */
+/* the same from projected channels: mv_causal_conv (conv_w, taps, conv_state, which `slots` counts too; no bias) comes first, by a launch of its own or along the
+ * way.  xc: scratch memory, [total_q][channels], of no meaning afterwards */
 int mv_delta_prefill_conv(const MvDeltaArgs *args, void *xc, int dtype, int flags, void *stream);
 /* one token per sequence, from projected channels: convolution, recurrence and mv_head_norm_gate in one launch; writes both states */
 int mv_delta_step(const MvDeltaArgs *args, int dtype, void *stream);

@@ -384,13 +384,13 @@ extern "C" int mv_delta_prefill_conv(const MvDeltaArgs *a, void *xc, int dtype, 
   if (!a || !xc) return MV_E_NULLPTR;
   MvSsmArgs c{};
   c.x = a->x, c.x_stride = a->x_stride, c.conv_w = a->conv_w, c.conv_state = a->conv_state, c.state_slots = a->state_slots, c.cu_q = a->cu_q, c.cu_k = a->cu_k;
-  c.out = xc, c.out_stride = a->channels, c.slots = a->conv_state ? a->slots : 0, c.n_seqs = a->n_seqs, c.max_q = a->max_q, c.channels = a->channels, c.taps = a->taps;
+  c.out = xc, c.out_stride = a->channels, c.slots = a->slots, c.n_seqs = a->n_seqs, c.max_q = a->max_q, c.channels = a->channels, c.taps = a->taps;
   c.heads = a->heads, c.groups = a->groups, c.p = a->p, c.n = a->n, c.b_off = a->k_off, c.c_off = a->q_off;
   MvDeltaArgs d = *a;
   d.x = xc, d.x_stride = a->channels;
   if (int e = mv_check_conv(&c, dtype)) return e;
   if (int e = check_delta(&d, dtype)) return e;
-  if (dtype != MV_F32 && !(flags & MV_DELTA_SCAN) && a->workspace && (a->conv_state || a->taps == 1 || !a->slots) &&
+  if (dtype != MV_F32 && !(flags & MV_DELTA_SCAN) && a->workspace &&
       mv_delta_chunk_workspace(a->n_seqs, a->total_q, a->heads, a->p, a->n) && mv_delta_chunk_takes_conv(d, dtype))
     return prefill(&d, a->x, a->x_stride, dtype, flags, stream);
   if (int rc = mv_causal_conv(&c, dtype, stream)) return rc;

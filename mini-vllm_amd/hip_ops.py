@@ -1658,8 +1658,10 @@ def _delta_conv(g, s: DeltaShape, x, conv_w, conv_state) -> None:
     if conv_w.dtype != x.dtype or conv_w.shape[1] != s.channels:
         raise MvHipError(f"convolution weight [taps, {s.channels}] of {x.dtype} required")
     g.conv_w, g.taps = conv_w.data_ptr(), conv_w.shape[0]
-    if g.slots and g.taps > 1:
-        if conv_state.dtype != x.dtype or tuple(conv_state.shape) != (2, g.slots, g.taps - 1, s.channels) or not conv_state.is_contiguous():
+    has = conv_state is not None and conv_state.numel() > 0
+    if has or (g.slots and g.taps > 1):      # (both states or none)
+        if (not has or conv_state.dtype != x.dtype or tuple(conv_state.shape) != (2, g.slots, g.taps - 1, s.channels)
+                or not conv_state.is_contiguous()):
             raise MvHipError(f"convolution state must be dense [2, {g.slots}, {g.taps - 1}, {s.channels}] of {x.dtype}")
         g.conv_state = conv_state.data_ptr()
 

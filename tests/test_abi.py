@@ -66,6 +66,31 @@ def test_struct_layouts_of_the_binding_match_the_library():
     assert hip_ops.lib().mv_decode_layers_persistent_workspace_bytes(1, 2048, 16, 8, 128, 6144, 64, 64) > 4096
 
 
+def test_delta_prompts_with_convolution_need_its_state():
+    """A pool of states without the kept inputs, or the other way round, is refused as mv_causal_conv refuses it, in the entry point and ahead of it."""
+    from minivllm_amd import hip_ops as H
+
+    at = torch.zeros(64, dtype=torch.uint8)
+    p = (at.data_ptr() + 15) & ~15      # (nothing is read)
+    s = H.DeltaShape(2, 2, 64, 64, 128, 256, 64, 0.125, False)
+
+    def call(**kw):
+        a = H.MvDeltaArgs(**dict(dict(x=p, beta=p, a=p, conv_w=p, dt_bias=p, a_log=p, state=p, state_slots=p, cu_q=p, cu_k=p, out=p, x_stride=s.channels, beta_stride=8,
+                                      a_stride=8, out_stride=128, slots=3, n_seqs=1, max_q=70, total_q=70, channels=s.channels, taps=4, heads=2, groups=2, p=64,
+                                      p_true=64, n=64, k_off=128, q_off=256), **kw))
+        return H.lib().mv_delta_prefill_conv(ctypes.byref(a), p, H.MV_BF16, 0, None)
+
+    assert call() == -1 and call(conv_state=p, state=None) == -1 and call(conv_state=p, taps=9) == -2 and call(conv_state=p + 8) == -5
+    x, w, kept = (torch.zeros(*n, dtype=torch.bfloat16) for n in ((5, s.channels), (4, s.channels), (2, 3, 3, s.channels)))
+    for slots, state in ((3, None), (3, kept[:, :, :2]), (3, kept.half()), (0, kept), (3, kept[:, :0])):
+        with pytest.raises(H.MvHipError, match="convolution state"):
+            H._delta_conv(H.MvDeltaArgs(slots=slots), s, x, w, state)
+    for slots, state, weight in ((3, kept, w), (0, None, w), (0, kept[:, :0], w), (3, None, w[:1]), (3, kept[:, :, :0], w[:1])):
+        g = H.MvDeltaArgs(slots=slots)
+        H._delta_conv(g, s, x, weight, state)
+        assert g.conv_state == (kept.data_ptr() if state is kept else None) and g.taps == weight.shape[0]
+
+
 def test_no_cpu_fallback():
     from minivllm_amd import hip_ops
 
