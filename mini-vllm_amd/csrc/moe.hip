@@ -904,22 +904,20 @@ static int route(const void *x, int64_t x_stride, const void *w, const void *cor
   // workgroup a CU, 16 waves 123, eight 91).  Two tiles, which read the weights once, where those are long: 34 outputs of 4096 inputs, 4400 tokens
   // 23 us, one tile 28.  More than 64 outputs leave two tiles one workgroup a CU, so its rounds over the chip have to be full: 128 outputs of 4096
   // inputs, 4400 tokens 73 us, 12000 145; one tile 87 and 122.  LDS has the scores of two tiles up to 256 outputs.
+  const bool along = group && dtype != MV_F32 && rows <= kRouteRows && rows * top <= kRoutePairs && group->experts <= kRouteExperts && outputs <= 64 && groups <= 8;
   MV_DISPATCH_DTYPE(dtype, {
     const hipStream_t st = (hipStream_t)stream;
     const bool full = k > 2048 && (rows <= 8192 || (k >= 4096 && (rows - 1) % 8192 >= 4096));
-    int rc;
-    if constexpr (!__is_same(Tag, f32_tag)) {
-      if (group && rows <= kRouteRows && rows * top <= kRoutePairs && group->experts <= kRouteExperts && outputs <= 64 && groups <= 8) {
-        *grouped = true;
-        return launch_route<Tag, 16, 1, true>(p, st, *group);
-      }
-    }
-    if (rows <= 16 * 256) rc = launch_route<Tag, 16, 1>(p, st);
+    int rc = MV_E_DTYPE;
+    if (along) {
+      if constexpr (!__is_same(Tag, f32_tag)) rc = launch_route<Tag, 16, 1, true>(p, st, *group);
+    } else if (rows <= 16 * 256) rc = launch_route<Tag, 16, 1>(p, st);
     else if (dtype != MV_F32 && (outputs <= 64 ? k >= 2048 : outputs <= 256 && full)) rc = launch_route<Tag, 8, 2>(p, st);
     else rc = launch_route<Tag, 8, 1>(p, st);
     if (rc) return rc;
   });
   MV_LAUNCH_CHECK();
+  if (along) *grouped = true;
   return MV_OK;
 }
 
