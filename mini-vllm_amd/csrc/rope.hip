@@ -9,6 +9,8 @@
 // row rotate (bf16/f16, D=128) or a wave shuffle.
 // Rounding points are the reference's: norm result -> dtype, rotation in
 // fp32 with separately rounded products -> dtype.
+#include <algorithm>
+
 #include "common.h"
 
 struct RopeParams {
@@ -131,22 +133,27 @@ __global__ void __launch_bounds__(THREADS) rope_qk_store_kernel(RopeParams p) {
   }
 }
 
-// us by waves of a token, 4 / 2 / 1; bf16, 16 + 8 heads of 128 with norms: 300 tokens 6.4 / 6.4 / 7.5, 600 8.1 / 7.3 / 8.1, 1000 9.8 / 8.7 / 9.1, 1366 12.5 / 11.1 / 10.5,
-// 5000 29.6 / 24.0 / 20.9, 25200 143 / 96 / 92; 28 + 4 of 128, 25200: 130 / 102 / 97; 16 + 8 of 64: 81 / 59 / 50; 8 + 4 of 256, 1366: 17.8 / 14.1 / 13.0.  fp32 rows
-// are as quick either way (16 + 8 of 128, 5000: 33.8 / 34.4 / 33.1) and slower below (1000: 10.7 / 11.7 / 16.2).
+// Waves of a token.  A wave has its rows one batch of four behind the other, a norm about doubles what a batch takes, and tokens beside each other on a SIMD cover that:
+// the more rows, the more tokens it takes until fewer waves are ahead.  bf16, us by 4 / 2 / 1 waves, with norms: 16 + 8 heads of 128 (rows of q, k and v: 32) 600 tokens
+// 8.3 / 7.6 / 8.3, 1200 11.0 / 9.7 / 10.3, 2048 16.0 / 13.5 / 12.9, 25200 143 / 96 / 92; 64 + 8 of 128 1000 14.9 / 15.4 / 17.9, 1400 18.9 / 20.9 / 22.1, 2800 28.5 / 27.9 /
+// 29.0, 5600 55.0 / 53.1 / 50.9; 32 + 8 of 256 1100 22.7 / 23.3 / 29.2, 5600 83.7 / 73.8 / 68.9; without: 28 + 4 of 128 513 6.6 / 6.5 / 7.2, 1025 9.2 / 8.5 / 8.5, 5000
+// 27.5 / 23.1 / 19.7; 4 + 1 of 128 513 5.6 / 4.6 / 4.3; 64 + 8 of 128 1000 12.0 / 12.0 / 13.7, 2000 20.7 / 18.9 / 18.1; 40 + 40 of 128 (120 rows) 520 11.2 / 11.7 / 15.8,
+// 2800 37.6 / 35.4 / 35.2, 8000 112.8 / 118.3 / 122.6; more than six batches of a single wave: 32 + 16 of 256 with norms 4000 72.6 / 72.6 / 76.5.  Over 36 shapes of 3 to 213
+// rows, 513 to 8000 tokens: 0.91 of the time by four waves in the mean, at worst 4 % above it (4.8 -> 5.0, 22.7 -> 23.5).  fp32 rows are as quick either way (16 + 8 of 128, 5000: 33.8 / 34.4 / 33.1) and slower below (1000: 10.7 / 11.7 / 16.2).
+static int waves_of_token(const RopeParams &p, int head_dim, int n_tok) {
+  const int rows = p.n_heads + (p.k_cache ? 2 : 1) * p.n_kv_heads, work = (p.q_norm_w || p.unit) ? 2 * rows : rows;
+  if (rows > 100 || n_tok <= 512) return 4;
+  return n_tok > 24 * work && rows * head_dim <= 6 * 4 * 512 ? 1 : n_tok > std::min(2048, 20 * work - 500) ? 2 : 4;
+}
+
 template <typename Tag, int D>
 static void launch_rope(const RopeParams &p, int n_tok, hipStream_t st) {
+  const int waves = elem<Tag>::VEC == 8 ? waves_of_token(p, D, n_tok) : 4;
   if constexpr (elem<Tag>::VEC == 8) {
-    if (n_tok > 1024) {
-      hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 64>), dim3(n_tok), dim3(64), 0, st, p);
-      return;
-    }
-    if (n_tok > 512) {
-      hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 128>), dim3(n_tok), dim3(128), 0, st, p);
-      return;
-    }
+    if (waves == 1) hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 64>), dim3(n_tok), dim3(64), 0, st, p);
+    if (waves == 2) hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 128>), dim3(n_tok), dim3(128), 0, st, p);
   }
-  hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 256>), dim3(n_tok), dim3(256), 0, st, p);
+  if (waves == 4) hipLaunchKernelGGL((rope_qk_store_kernel<Tag, D, 256>), dim3(n_tok), dim3(256), 0, st, p);
 }
 
 extern "C" int mv_rope_qk_store_ex(const void *q, const void *k, const void *v, int64_t q_stride_tok,

@@ -6,9 +6,9 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# rows of a token: fewer than a wave takes at a time, one more than a batch of them, many
+# rows of a token: fewer than a wave takes at a time, one more than a batch of them, many; tokens: by one, two and four waves
 @pytest.mark.parametrize("heads, kv, dim", [(1, 1, 64), (9, 1, 128), (28, 4, 128), (8, 4, 256)])
-@pytest.mark.parametrize("tokens", [513, 1024, 1025])
+@pytest.mark.parametrize("tokens", [513, 941, 1025, 1729])
 @pytest.mark.parametrize("form", ["norm", "plain", "unit", "pairs"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_waves_of_a_token(heads, kv, dim, tokens, form, dtype):

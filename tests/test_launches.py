@@ -1,0 +1,110 @@
+"""What entry points send to the GPU, on the host: the runtime's launch functions by stand-ins that count the launches, keep the last one's size and let one fail."""
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.skipif(not shutil.which("g++"), reason="no C++ compiler")
+
+STAND_INS = r"""
+extern "C" {
+static int launches, fails, last;
+static unsigned long long threads;
+void fail_at(int n) { launches = last = 0, fails = n; }
+int launched() { return launches; }
+int threads_x() { return (int)(threads & 0xffffffff); }
+int hipLaunchKernel(const void *, unsigned long long, unsigned, unsigned long long block, unsigned, void **, unsigned long, void *) {
+  threads = block;
+  if (++launches != fails) return 0;
+  return last = 719;   // (kept until it is asked for)
+}
+static struct { unsigned long long grid, block; unsigned grid_z, block_z; } pushed;
+int __hipPushCallConfiguration(unsigned long long grid, unsigned grid_z, unsigned long long block, unsigned block_z, unsigned long, void *) {
+  pushed = {grid, block, grid_z, block_z};
+  return 0;
+}
+int __hipPopCallConfiguration(unsigned *grid, unsigned *block, unsigned long *shared, void **stream) {
+  grid[0] = (unsigned)pushed.grid, grid[1] = (unsigned)(pushed.grid >> 32), grid[2] = pushed.grid_z;
+  block[0] = (unsigned)pushed.block, block[1] = (unsigned)(pushed.block >> 32), block[2] = pushed.block_z;
+  *shared = 0, *stream = 0;
+  return 0;
+}
+int hipFuncSetAttribute(const void *, int, int) { return 0; }
+int hipGetLastError() { const int e = last; last = 0; return e; }
+}
+"""
+
+START = r"""
+import ctypes, sys
+stand_ins = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+dtype, p = int(sys.argv[3]), 4096      # (an address that the host does not look at)
+"""
+
+EXPERTS = START + r"""
+class Act(ctypes.Structure):
+    _fields_ = [("fields", ctypes.c_int64 * 8)]
+class Args(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_void_p) for n in "x router correction gate_up down act weights place out workspace".split()]
+                + [(n, ctypes.c_int64) for n in "x_stride ws_bytes".split()]
+                + [(n, ctypes.c_int) for n in "rows k router_k outputs top groups keep route_flags experts tile_m ff width weigh_inputs".split()] + [("scale", ctypes.c_float)])
+act = Act()
+for rows in (16, 17):
+    a = Args(x=p, router=p, gate_up=p, down=p, act=ctypes.addressof(act), weights=p, place=p, out=p, workspace=p, x_stride=64, ws_bytes=1 << 20, rows=rows, k=64, router_k=64,
+             outputs=8, top=2, groups=1, keep=1, experts=8, tile_m=16, ff=64, width=64, scale=1.0)
+    stand_ins.fail_at(0)
+    print(lib.mv_moe_mlp(ctypes.byref(a), dtype, None), stand_ins.launched(), end=" ")
+    for n in range(1, stand_ins.launched() + 1):
+        stand_ins.fail_at(n)
+        print(lib.mv_moe_mlp(ctypes.byref(a), dtype, None), stand_ins.launched(), end=" ")
+"""
+
+ROTATION = START + r"""
+i, v, f = ctypes.c_int, ctypes.c_void_p, ctypes.c_float
+q = ctypes.c_int64
+for heads, kv, dim, norm, cache, tokens in eval(sys.argv[4]):
+    w, c = p if norm else None, p if cache else None
+    rc = lib.mv_rope_qk_store_ex(v(p), v(p), v(p), q(16384), q(16384), q(16384), v(p), v(p), v(p), q(64), v(w), v(w), f(1e-6), v(p), None if cache else v(p), v(c), v(c), v(c),
+                                 q(64), i(tokens), i(heads), i(kv), i(dim), i(dtype), None, None)
+    print(stand_ins.threads_x() if rc == 0 else rc, end=" ")
+"""
+
+
+@pytest.fixture(scope="module")
+def call(tmp_path_factory):
+    from minivllm_amd import hip_ops
+
+    folder = tmp_path_factory.mktemp("stand_ins")
+    (folder / "stand_ins.cpp").write_text(STAND_INS)
+    lib = str(folder / "stand_ins.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-o", lib, str(folder / "stand_ins.cpp")], check=True)
+
+    def run(program, dtype, *more):
+        return subprocess.run([sys.executable, "-c", program, lib, hip_ops.LIB_PATH, str(dtype), *more], check=True, capture_output=True, text=True, timeout=60).stdout.split()
+    return run
+
+
+def test_a_launch_that_fails_ends_the_experts(call):
+    """The launches behind it would work on what it left out: they are not sent."""
+    from minivllm_amd import hip_ops
+
+    # router with grouping and two products; router, grouping and two products
+    assert call(EXPERTS, hip_ops.MV_BF16) == "0 3 719 1 719 2 719 3".split() + "0 4 719 1 719 2 719 3 719 4".split()
+
+
+# heads, heads of keys and values, columns, norms, cache: tokens -> threads of a token: the lines by the rows that a wave would have one behind the other
+ROTATIONS = {(16, 8, 128, True, True): {512: 256, 780: 256, 781: 128, 1536: 128, 1537: 64}, (28, 4, 128, False, True): {512: 256, 513: 128, 864: 128, 865: 64},
+             (64, 8, 128, True, True): {1025: 256, 2048: 256, 2049: 128, 3840: 128, 3841: 64}, (64, 8, 64, False, True): {1100: 256, 1101: 128, 1920: 128, 1921: 64},
+             (4, 1, 128, True, True): {512: 256, 513: 64}, (1, 1, 64, False, False): {513: 64}, (40, 40, 128, False, True): {513: 256, 9000: 256},
+             (40, 40, 128, False, False): {1100: 256, 1101: 128, 1921: 64}, (32, 8, 256, True, True): {2304: 128, 2305: 64}, (32, 16, 256, True, True): {2049: 128, 9000: 128}}
+
+
+def test_waves_of_a_token(call):
+    from minivllm_amd import hip_ops
+
+    cases = [(*k, t) for k, v in ROTATIONS.items() for t in v]
+    want = [n for v in ROTATIONS.values() for n in v.values()]
+    for dtype in (hip_ops.MV_BF16, hip_ops.MV_F16):
+        assert list(map(int, call(ROTATION, dtype, repr(cases)))) == want
+    assert set(call(ROTATION, hip_ops.MV_F32, repr(cases))) == {"256"}
