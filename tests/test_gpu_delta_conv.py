@@ -13,7 +13,7 @@ SPANS = [(1, 0), (2, 5), (1, 1), (3, 2), (63, 5), (64, 0), (65, 64), (128, 7), (
 # decays' place in LDS and a wave's tile each, just or not), other numbers of taps, which go the other way too; the last sequence has no slot
 @pytest.mark.parametrize("heads, groups, p, n, gap, channel", [(8, 4, 128, 128, 0, False), (3, 3, 64, 32, 0, False), (4, 2, 48, 96, 0, False), (8, 2, 64, 64, 0, False),
                                                                (4, 2, 64, 64, 32, False), (2, 2, 64, 64, 0, True), (2, 1, 16, 160, 0, False),
-                                                               (2, 2, 128, 128, 0, True), (3, 3, 80, 32, 0, True), (2, 2, 144, 96, 0, True), (2, 2, 48, 160, 0, True),
+                                                               (2, 2, 128, 128, 0, True), (2, 2, 80, 32, 0, True), (2, 2, 144, 96, 0, True), (2, 2, 48, 160, 0, True),
                                                                (4, 2, 32, 64, 0, True)])
 @pytest.mark.parametrize("taps", [4, 2, 1, 6])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -26,8 +26,7 @@ def test_with_the_convolution(heads, groups, p, n, gap, channel, taps, dtype):
     total, slots = sum(t for t, _ in SPANS), len(SPANS) - 1
     k_off = heads * p + gap
     s = H.DeltaShape(heads, groups, p, n, k_off, k_off + groups * n, p, n ** -0.5, channel)
-    if s.channels % 32:
-        pytest.skip("no convolution of such rows")
+    assert s.channels % 32 == 0      # (other rows have no convolution)
     width = heads * (n if channel else 1)
     z = torch.nn.functional.pad(rand(total, s.channels), (8, 24)).to(dtype)[:, 8:8 + s.channels]      # rows that are apart
     beta, a, gate = (torch.nn.functional.pad(rand(total, c), (0, -c % 8)).to(dtype)[:, :c] for c in (heads, width, heads * p))
