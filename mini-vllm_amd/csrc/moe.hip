@@ -27,7 +27,7 @@ struct RouteGroups {
   float *by_place;   // or NULL
   int experts, tile_m, max_tiles;
 };
-constexpr int kRouteRows = 16, kRoutePairs = 256, kRouteExperts = 512;
+constexpr int kRouteRows = 16, kRoutePairs = 64, kRouteExperts = 512;
 
 // largest value of the wave and the lowest index that has it
 __device__ __forceinline__ void wave_argmax(float &v, int &i) {
@@ -216,7 +216,7 @@ __device__ __forceinline__ void choose_four(const RouteParams &p, const float *s
 }
 
 // What moe_group_kernel makes of the choices, `pairs` of them in LDS (a multiple of four readable, -1 behind the last), by one workgroup of 16 waves: a pair to a
-// thread of the first four, an expert to one of the last eight.
+// thread of the first wave, an expert to one of the last eight.
 __device__ __forceinline__ void group_few(const RouteGroups &q, const int *ids, const float *weights, int pairs, int top) {
   const int tid = threadIdx.x;
   const bool pair = tid < pairs;
@@ -254,8 +254,10 @@ __device__ __forceinline__ void group_few(const RouteGroups &q, const int *ids, 
 // 12.7 -> 12.8, 24 20.5 -> 15.4, 20000 53 -> 51; fp32, 34 outputs of 2048 inputs, 4400 tokens: 392 -> 131.  Now 9001 tokens with the choices of four tokens
 // at once, one launch between events, 29.3 -> 24.4: 8.5 of 20 us are the products (their inputs by half lines), 282 workgroups on 256 CUs.
 // GROUP (one workgroup has all tokens): the choices stay in LDS for the grouping behind them, a launch and a trip to memory less.  Both products with what is around them, 32
-// experts: 12 tokens of 4 choices (2048 -> 768) 67.2 -> 65.7 us, 4 of 8 (1024 -> 384; the host's) 48.5 -> 44.5, 16 of 8 49.3 -> 45.2.  Up to one tile: two tiles in one
-// workgroup in place of two workgroups cost more than the launch (24 of 4 70.2 -> 74.0, 32 of 8 84 -> 95).
+// experts: 12 tokens of 4 choices (2048 -> 768) 67.2 -> 65.7 us, 4 of 8 (1024 -> 384; the host's) 48.5 -> 44.5.  Up to one tile: two tiles in one
+// workgroup in place of two workgroups cost more than the launch (24 of 4 70.2 -> 74.0, 32 of 8 84 -> 95).  Up to 64 pairs: a thread looks at all of them, four at a time,
+// one behind the other.  Router, grouping and products in a graph, grouped by another launch and here, 16 experts of 512 -> 128: 1 token of 8 choices 18.1 -> 15.5 (1024 ->
+// 384), 64 pairs 15.1 and 15.1, 80 15.9 and 16.4, 128 16.6 and 19.7, 192 18.1 and 24.2; 32 of 2048 -> 768: 64 63.8 and 63.6, 128 69.4 and 72.2.
 template <typename Tag, int WAVES, int TT, bool GROUP>
 __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p, RouteGroups q) {
   typedef typename elem<Tag>::T T;

@@ -6,13 +6,15 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("rows, tile", [(1, 16), (16, 16), (17, 16), (24, 32), (32, 16), (33, 16), (77, 64), (700, 256)])      # (up to 16 rows the router groups)
+# (up to 16 rows and 64 pairs the router groups)
+@pytest.mark.parametrize("rows, top, tile", [(1, 3, 16), (16, 3, 16), (16, 4, 16), (8, 8, 16), (13, 5, 16), (16, 8, 16), (17, 3, 16), (24, 3, 32), (32, 3, 16), (33, 3, 16), (77, 3, 64),
+                                             (700, 3, 256)])
 @pytest.mark.parametrize("weigh", [False, True])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-def test_one_call_is_four(rows, tile, weigh, dtype):
+def test_one_call_is_four(rows, top, tile, weigh, dtype):
     from minivllm_amd import hip_ops as H
 
-    experts, extra, top, k, ff = 8, 0 if weigh else 2, 3, 256, 128
+    experts, extra, k, ff = 8, 0 if weigh else 2, 256, 128
     g = torch.Generator(device=DEV).manual_seed(rows)
     rand = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)
     form = (lambda w: w) if dtype == torch.float32 else (lambda w: H.pack_weight(w.view(-1, w.shape[-1])))

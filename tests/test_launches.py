@@ -1,4 +1,6 @@
 """What entry points send to the GPU, on the host: the runtime's launch functions by stand-ins that count the launches, keep the last one's size and let one fail."""
+import ctypes
+import json
 import shutil
 import subprocess
 import sys
@@ -10,12 +12,13 @@ pytestmark = pytest.mark.skipif(not shutil.which("g++"), reason="no C++ compiler
 STAND_INS = r"""
 extern "C" {
 static int launches, fails, last;
-static unsigned long long threads;
+static unsigned long long threads, blocks;
 void fail_at(int n) { launches = last = 0, fails = n; }
 int launched() { return launches; }
 int threads_x() { return (int)(threads & 0xffffffff); }
-int hipLaunchKernel(const void *, unsigned long long, unsigned, unsigned long long block, unsigned, void **, unsigned long, void *) {
-  threads = block;
+int blocks_y() { return (int)(blocks >> 32); }
+int hipLaunchKernel(const void *, unsigned long long grid, unsigned, unsigned long long block, unsigned, void **, unsigned long, void *) {
+  threads = block, blocks = grid;
   if (++launches != fails) return 0;
   return last = 719;   // (kept until it is asked for)
 }
@@ -60,6 +63,18 @@ for rows in (16, 17):
         print(lib.mv_moe_mlp(ctypes.byref(a), dtype, None), stand_ins.launched(), end=" ")
 """
 
+# one call per dict of sys.argv[6]: the fields of the arguments' struct (names and type codes in sys.argv[5]) that are not a pointer or 0 -> launches, y of the last one
+STRUCT = START + r"""
+import json
+fields = [(n, {"P": ctypes.c_void_p, "l": ctypes.c_int64, "q": ctypes.c_int64, "i": ctypes.c_int, "f": ctypes.c_float}[t]) for n, t in json.loads(sys.argv[5])]
+Args = type("Args", (ctypes.Structure,), {"_fields_": fields})
+for case in json.loads(sys.argv[6]):
+    a = Args(**{n: p for n, t in fields if t is ctypes.c_void_p}, **case)
+    stand_ins.fail_at(0)
+    rc = getattr(lib, sys.argv[4])(ctypes.byref(a), *eval(sys.argv[7]))
+    print(*((stand_ins.launched(), stand_ins.blocks_y()) if rc == 0 else (rc, rc)), end=" ")
+"""
+
 ROTATION = START + r"""
 i, v, f = ctypes.c_int, ctypes.c_void_p, ctypes.c_float
 q = ctypes.c_int64
@@ -85,6 +100,13 @@ def call(tmp_path_factory):
     return run
 
 
+def _launches(call, entry, struct, dtype, cases, more="dtype, None"):
+    """-> (launches, y of the last one) of each case."""
+    fields = json.dumps([(n, t._type_) for n, t in struct._fields_])
+    out = list(map(int, call(STRUCT, dtype, entry, fields, json.dumps(cases), more)))
+    return list(zip(out[::2], out[1::2]))
+
+
 def test_a_launch_that_fails_ends_the_experts(call):
     """The launches behind it would work on what it left out: they are not sent."""
     from minivllm_amd import hip_ops
@@ -108,3 +130,17 @@ def test_waves_of_a_token(call):
     for dtype in (hip_ops.MV_BF16, hip_ops.MV_F16):
         assert list(map(int, call(ROTATION, dtype, repr(cases)))) == want
     assert set(call(ROTATION, hip_ops.MV_F32, repr(cases))) == {"256"}
+
+
+def test_grouping_by_the_router(call):
+    """Up to 16 tokens and 64 pairs of 16 bits."""
+    from minivllm_amd import hip_ops as H
+
+    cases = {(1, 8): 3, (8, 8): 3, (16, 4): 3, (13, 5): 4, (9, 8): 4, (16, 8): 4, (17, 1): 4}
+    fields = [dict(x_stride=64, ws_bytes=1 << 20, rows=r, k=64, router_k=64, outputs=16, top=t, groups=1, keep=1, experts=16, tile_m=16, ff=64, width=64, scale=1.0)
+              for r, t in cases]
+    assert ctypes.sizeof(H.GateAct) <= 32
+    program = STRUCT.replace("for case in", "act = (ctypes.c_int64 * 4)()\nfor case in").replace("**case)", "**case)\n    a.act = ctypes.addressof(act)")
+    names = json.dumps([(n, t._type_) for n, t in H.MvMoeMlpArgs._fields_])
+    for dtype, want in ((H.MV_BF16, list(cases.values())), (H.MV_F16, list(cases.values())), (H.MV_F32, [4] * len(cases))):
+        assert list(map(int, call(program, dtype, "mv_moe_mlp", names, json.dumps(fields), "dtype, None")))[::2] == want
