@@ -146,6 +146,33 @@ def test_grouping_by_the_router(call):
         assert list(map(int, call(program, dtype, "mv_moe_mlp", names, json.dumps(fields), "dtype, None")))[::2] == want
 
 
+# (heads of a group, groups, p, n, sequences, tokens of all, of the longest) -> along with the preparation, bf16 and one decay per head.  Turns of a workgroup's threads: one; two;
+# three and four; a head a group of 1.5, three and four
+ALONG = {(2, 8, 64, 64, 1, 700, 700): True, (2, 8, 64, 32, 4, 15000, 4000): True, (2, 8, 64, 32, 16, 18000, 1490): False, (2, 8, 128, 128, 1, 256, 256): True,
+         (2, 8, 128, 128, 1, 257, 257): False, (2, 8, 128, 128, 3, 704, 280): False, (2, 8, 128, 128, 4, 704, 280): True, (2, 8, 128, 128, 16, 18000, 1490): True,
+         (2, 8, 256, 128, 1, 60, 60): False, (2, 8, 256, 128, 16, 18000, 1490): False, (1, 8, 64, 64, 1, 341, 341): True, (1, 8, 64, 64, 1, 383, 383): False,
+         (1, 8, 64, 64, 1, 448, 448): True, (1, 8, 128, 128, 16, 704, 60): False, (1, 8, 128, 128, 16, 1024, 171): True,
+         (1, 8, 256, 128, 16, 18000, 1490): False, (4, 2, 64, 64, 16, 18000, 1490): False}
+
+
+def test_convolution_along_with_the_preparation(call):
+    from minivllm_amd import hip_ops as H
+
+    def fields(per, groups, p, n, seqs, total, longest, taps=4, channel=0):
+        heads, channels = per * groups, groups * (per * p + 2 * n)
+        return dict(x_stride=channels, beta_stride=heads, a_stride=heads * (n if channel else 1), out_stride=heads * p, slots=seqs, ws_bytes=1 << 34, n_seqs=seqs, max_q=longest,
+                    total_q=total, channels=channels, taps=taps, heads=heads, groups=groups, p=p, p_true=p, n=n, k_off=heads * p, q_off=heads * p + groups * n,
+                    channel_decay=channel)
+    run = lambda cases, dtype: [n for n, _ in _launches(call, "mv_delta_prefill_conv", H.MvDeltaArgs, dtype, cases, "ctypes.c_void_p(p), dtype, 0, None")]
+    assert run([fields(*k) for k in ALONG], H.MV_BF16) == [2 if v else 3 for v in ALONG.values()]
+    # other taps, and more heads than two of a group, never; heads of 16 bits otherwise, and decays per channel: by their sizes alone, with or without it the same launches
+    assert run([fields(2, 8, 64, 64, 1, 100, 100, taps=t) for t in (1, 2, 3, 5)], H.MV_BF16) == [3] * 4
+    some = [(1, 4, 64, 64), (1, 4, 128, 64), (1, 4, 144, 96), (1, 4, 80, 32), (2, 4, 64, 64)]
+    for dtype in (H.MV_BF16, H.MV_F16):
+        got = run([fields(*k, 1, 100, 100, channel=1) for k in some], dtype)
+        assert [b - got[0] for b in got] == [0, 0, 1, 1, 1]
+
+
 def test_tokens_of_a_convolution(call):
     """Eight a workgroup up to 1700 workgroups of 32, with more than four taps up to 1000."""
     from minivllm_amd import hip_ops as H
