@@ -27,7 +27,7 @@ struct RouteGroups {
   float *by_place;   // or NULL
   int experts, tile_m, max_tiles;
 };
-constexpr int kRouteRows = 16, kRoutePairs = 64, kRouteExperts = 512;
+constexpr int kRouteRows = 16, kRouteItems = 256, kPairBits = 8;   // (items: pairs and experts, four lanes each)
 
 // largest value of the wave and the lowest index that has it
 __device__ __forceinline__ void wave_argmax(float &v, int &i) {
@@ -48,7 +48,7 @@ __device__ __forceinline__ int wave_best(float v, unsigned long long free) {
 
 // the scores of a token's R outputs, in s (logits) and c (scratch): choice and weights, by one wave; `correction`: of output `lane`
 template <typename Tag>
-__device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c, int64_t token, float correction, int *ids_too = nullptr, float *weights_too = nullptr) {
+__device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c, int64_t token, float correction, int *keys = nullptr, float *weights_too = nullptr) {
   typedef typename elem<Tag>::T T;
   const int lane = threadIdx.x & 63, R = p.outputs, size = R / p.groups;
   const bool sigmoid = p.flags & MV_ROUTE_SIGMOID;
@@ -136,7 +136,10 @@ __device__ __forceinline__ void choose(const RouteParams &p, float *s, float *c,
     const float w = (p.flags & MV_ROUTE_RAW ? weight : weight / (total + 1e-20f)) * p.scale;
     p.ids[token * p.top + lane] = mine;
     p.weights[token * p.top + lane] = w;
-    if (ids_too) ids_too[token * p.top + lane] = mine, weights_too[token * p.top + lane] = w;
+    if (keys) {
+      const int pair = (int)token * p.top + lane;
+      keys[pair] = mine << kPairBits | pair, weights_too[pair] = w;
+    }
   }
 }
 
@@ -215,35 +218,37 @@ __device__ __forceinline__ void choose_four(const RouteParams &p, const float *s
     }
 }
 
-// What moe_group_kernel makes of the choices, `pairs` of them in LDS (a multiple of four readable, -1 behind the last), by one workgroup of 16 waves: a pair to a
-// thread of the first wave, an expert to one of the last eight.
-__device__ __forceinline__ void group_few(const RouteGroups &q, const int *ids, const float *weights, int pairs, int top) {
-  const int tid = threadIdx.x;
-  const bool pair = tid < pairs;
-  const int e = pair ? ids[tid] : tid - 512;
-  if (!pair && (e < 0 || e >= q.experts)) return;
-  if (pair && e >= q.experts) {
-    q.place[tid] = -1;
-    return;
-  }
-  int less = 0, equal = 0, ahead = 0;
-  for (int j = 0; j < pairs; j += 4) {
-    const s32x4 v = *(const s32x4 *)(ids + j);
+// What moe_group_kernel makes of the choices, `pairs` of them in LDS as id << kPairBits | number (a multiple of 16 readable, the largest int behind the last), by one
+// workgroup of 16 waves: four lanes to a pair, or behind those to an expert, each counts a quarter of the choices that sort ahead of it.  (One lane each, and choices
+// of lower experts, of the same and of those the ones ahead counted apart: 128 pairs took 3 us more than the launch that it saves.)
+__device__ __forceinline__ void group_few(const RouteGroups &q, const int *keys, const float *weights, int pairs, int top) {
+  const int item = threadIdx.x >> 2, part = threadIdx.x & 3;
+  const bool pair = item < pairs;
+  const int own = pair ? keys[item] : 0, e = pair ? own >> kPairBits : item - pairs;
+  if (!pair && e >= q.experts) return;
+  const int from = pair ? own : e << kPairBits, to = from + (1 << kPairBits);
+  int ahead = 0, upto = 0;
+#pragma unroll 2
+  for (int j = 4 * part; j < pairs; j += 16) {
+    const s32x4 v = *(const s32x4 *)(keys + j);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      less += v[u] >= 0 && v[u] < e, equal += v[u] == e, ahead += v[u] == e && j + u < tid;
-    }
+    for (int u = 0; u < 4; ++u) ahead += v[u] < from, upto += v[u] < to;
   }
+#pragma unroll
+  for (int o = 1; o <= 2; o <<= 1) ahead += __shfl_xor(ahead, o, 64), upto += __shfl_xor(upto, o, 64);   // (the four of an item together)
   if (pair) {
-    const int place = less + ahead;
-    q.place[tid] = place, q.tokens[place] = tid / top;
-    if (q.by_place) q.by_place[place] = weights[tid];
+    if (part) return;
+    const bool has = e < q.experts;
+    q.place[item] = has ? ahead : -1;
+    if (!has) return;
+    q.tokens[ahead] = item / top;
+    if (q.by_place) q.by_place[ahead] = weights[item];
     return;
   }
-  const int t0 = less / q.tile_m + e, t1 = e + 1 < q.experts ? (less + equal) / q.tile_m + e + 1 : q.max_tiles;
-  for (int t = t0; t < t1; ++t) {
+  const int count = upto - ahead, t0 = ahead / q.tile_m + e, t1 = e + 1 < q.experts ? upto / q.tile_m + e + 1 : q.max_tiles;
+  for (int t = t0 + part; t < t1; t += 4) {
     const int first = (t - t0) * q.tile_m;
-    q.tiles[3 * t] = first < equal ? e : -1, q.tiles[3 * t + 1] = less + first, q.tiles[3 * t + 2] = min(q.tile_m, equal - first);
+    q.tiles[3 * t] = first < count ? e : -1, q.tiles[3 * t + 1] = ahead + first, q.tiles[3 * t + 2] = min(q.tile_m, count - first);
   }
 }
 
@@ -255,9 +260,8 @@ __device__ __forceinline__ void group_few(const RouteGroups &q, const int *ids, 
 // at once, one launch between events, 29.3 -> 24.4: 8.5 of 20 us are the products (their inputs by half lines), 282 workgroups on 256 CUs.
 // GROUP (one workgroup has all tokens): the choices stay in LDS for the grouping behind them, a launch and a trip to memory less.  Both products with what is around them, 32
 // experts: 12 tokens of 4 choices (2048 -> 768) 67.2 -> 65.7 us, 4 of 8 (1024 -> 384; the host's) 48.5 -> 44.5.  Up to one tile: two tiles in one
-// workgroup in place of two workgroups cost more than the launch (24 of 4 70.2 -> 74.0, 32 of 8 84 -> 95).  Up to 64 pairs: a thread looks at all of them, four at a time,
-// one behind the other.  Router, grouping and products in a graph, grouped by another launch and here, 16 experts of 512 -> 128: 1 token of 8 choices 18.1 -> 15.5 (1024 ->
-// 384), 64 pairs 15.1 and 15.1, 80 15.9 and 16.4, 128 16.6 and 19.7, 192 18.1 and 24.2; 32 of 2048 -> 768: 64 63.8 and 63.6, 128 69.4 and 72.2.
+// workgroup in place of two workgroups cost more than the launch (24 of 4 70.2 -> 74.0, 32 of 8 84 -> 95).  Router, grouping and products in a graph, grouped by another
+// launch and here, 16 experts of 512 -> 128: 64 pairs 15.2 and 12.4, 128 16.8 and 14.5, 192 18.3 and 16.6; of 2048 -> 768 256 (apart then) would be 56.5 and 56.5.
 template <typename Tag, int WAVES, int TT, bool GROUP>
 __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p, RouteGroups q) {
   typedef typename elem<Tag>::T T;
@@ -349,21 +353,20 @@ __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p, Ro
       __syncthreads();
     }
   }
-  int *ids_too = GROUP ? (int *)(ch + TOKENS * R) : nullptr;
-  float *weights_too = GROUP ? (float *)(ids_too + kRoutePairs + 4) : nullptr;
+  int *keys = GROUP ? (int *)(ch + TOKENS * R) : nullptr;
+  float *weights_too = GROUP ? (float *)(keys + kRouteItems + 16) : nullptr;
   __syncthreads();
   if constexpr (GROUP) {
-    const int pairs = p.rows * p.top;
-    if (tid < 4) ids_too[pairs + tid] = -1;
+    if (tid < 16) keys[p.rows * p.top + tid] = INT32_MAX;
   }
   if (FOUR && R <= 64 && p.groups <= 8) {
     for (int t = wave * 4 + (lane >> 4); t < TOKENS; t += WAVES * 4) choose_four<Tag>(p, sc + t * R, m0 + t, m0 + t < p.rows, corrections);
     return;
   }
-  for (int t = wave; t < TOKENS && m0 + t < p.rows; t += WAVES) choose<Tag>(p, sc + t * R, ch + t * R, m0 + t, corrections[0], ids_too, weights_too);   // (no barrier in it)
+  for (int t = wave; t < TOKENS && m0 + t < p.rows; t += WAVES) choose<Tag>(p, sc + t * R, ch + t * R, m0 + t, corrections[0], keys, weights_too);   // (no barrier in it)
   if constexpr (GROUP) {
     __syncthreads();
-    group_few(q, ids_too, weights_too, p.rows * p.top, p.top);
+    group_few(q, keys, weights_too, p.rows * p.top, p.top);
   }
 }
 
@@ -906,7 +909,7 @@ static int route(const void *x, int64_t x_stride, const void *w, const void *cor
   // workgroup a CU, 16 waves 123, eight 91).  Two tiles, which read the weights once, where those are long: 34 outputs of 4096 inputs, 4400 tokens
   // 23 us, one tile 28.  More than 64 outputs leave two tiles one workgroup a CU, so its rounds over the chip have to be full: 128 outputs of 4096
   // inputs, 4400 tokens 73 us, 12000 145; one tile 87 and 122.  LDS has the scores of two tiles up to 256 outputs.
-  const bool along = group && dtype != MV_F32 && rows <= kRouteRows && rows * top <= kRoutePairs && group->experts <= kRouteExperts && outputs <= 64 && groups <= 8;
+  const bool along = group && dtype != MV_F32 && rows <= kRouteRows && rows * top + group->experts <= kRouteItems && outputs <= 64 && groups <= 8;
   MV_DISPATCH_DTYPE(dtype, {
     const hipStream_t st = (hipStream_t)stream;
     const bool full = k > 2048 && (rows <= 8192 || (k >= 4096 && (rows - 1) % 8192 >= 4096));

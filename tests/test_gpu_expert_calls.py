@@ -6,8 +6,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-# (up to 16 rows and 64 pairs the router groups)
-@pytest.mark.parametrize("rows, top, tile", [(1, 3, 16), (16, 3, 16), (16, 4, 16), (8, 8, 16), (13, 5, 16), (16, 8, 16), (17, 3, 16), (24, 3, 32), (32, 3, 16), (33, 3, 16), (77, 3, 64),
+# (up to 16 rows the router groups, a quarter of the pairs to a lane)
+@pytest.mark.parametrize("rows, top, tile", [(1, 3, 16), (16, 3, 16), (16, 4, 16), (8, 8, 16), (13, 5, 16), (16, 8, 16), (5, 1, 16), (17, 3, 16), (24, 3, 32), (32, 3, 16), (33, 3, 16), (77, 3, 64),
                                              (700, 3, 256)])
 @pytest.mark.parametrize("weigh", [False, True])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
