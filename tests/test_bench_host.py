@@ -195,12 +195,15 @@ def test_probes_drive_a_model_with_experts(monkeypatch):
     """The records of ``--design``, with kernels by stand-ins that only have their shapes: the prefill probe sees both products of every layer with experts and the
     delta rule's one call, the decode probe routes through the layer; a model whose experts are not asked for makes no record of them."""
     import inspect
+    import itertools
 
     import torch
     from minivllm_amd import hip_ops
+    from minivllm_amd.engine.sequence import Sequence
     from minivllm_amd.layers.delta_rule import GatedDeltaRule
     from minivllm_amd.layers.moe import ExpertMLP
 
+    monkeypatch.setattr(Sequence, "counter", itertools.count())     # (numbers of its own: tests of two processes compare theirs)
     # the four calls take what the one does
     assert ([(p.name, p.default) for p in inspect.signature(bench.moe_mlp_by_parts).parameters.values()]
             == [(p.name, p.default) for p in inspect.signature(hip_ops.moe_mlp).parameters.values()])
