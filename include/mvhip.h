@@ -694,7 +694,8 @@ enum { MV_SSM_SCAN = 1 };
 int mv_ssm_prefill(const MvSsmArgs *args, int dtype, int flags, void *stream);
 /* the same with scratch memory of mv_ssm_prefill_workspace_bytes() bytes (0: none is of use): few long sequences are then worked on in
  * several places at once.  total_q = rows of x, at least cu_q[n_seqs]: the segments are counted from it.  Whole sequences, as above, with
- * no workspace, a smaller one, or total_q < max_q */
+ * no workspace, a smaller one, or total_q < max_q.  Where a sequence is cut goes by the whole call, n_seqs, total_q and max_q, and with MV_SSM_SHARED by the lengths
+ * of the sequences ahead of it too: its last bits (fp32 sums in another order) then differ with the others of a call.  The same in any call without a workspace */
 /* dtype | MV_SSM_SHARED: also enough for four heads with the same b and c (heads / groups a multiple of 4) to a workgroup, where that is faster */
 enum { MV_SSM_SHARED = 1 << 8 };
 size_t mv_ssm_prefill_workspace_bytes(int n_seqs, int total_q, int max_q, int heads, int p, int n, int dtype);

@@ -6,7 +6,8 @@
 // element below the diagonal tiles the weight is two products instead of an exponential.  1.4 us a chunk and head: of 13 100 cycles of a chunk of four heads, LDS reads
 // (744 KB, at the 115 bytes a cycle that they reach) are 6500, products 5800, vector instructions 6500; the two waves of a SIMD are in the same phase most of the
 // time, so that these take turns in part.  A workgroup takes a CU's LDS, so that sequences as workgroups would leave half of the chip idle: the chunks of all sequences
-// are dealt out evenly instead (Rows).  64 heads of 64 x 128, 4 sequences of up to 3900 tokens, convolution and norm included: 258 -> 222 us (states 55 -> 44, outputs 143
+// are dealt out evenly instead (Rows).  So a sequence is cut where those ahead of it say, and its last bits differ with its neighbours (results within a unit, kept
+// states within 2^-16 of their norm), also at sizes where a head a workgroup would take whole sequences, the same bits in any call: without scratch memory that still holds.  64 heads of 64 x 128, 4 sequences of up to 3900 tokens, convolution and norm included: 258 -> 222 us (states 55 -> 44, outputs 143
 // -> 97 under the profiler).  Tried: scores of a chunk made once for the four heads and weighted by each wave (LDS reads 464 KB, vector instructions by a fifth more), and a
 // third barrier for weights made once: as slow; both token tiles of a wave's scores at once, two steps ahead: 97 -> 103.
 #include <algorithm>

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from test_gpu_ssm_segments import H, _case  # noqa: F401
+from test_gpu_ssm_segments import DEV, H, _case  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +59,32 @@ def test_what_stays_with_a_head_a_workgroup(H, monkeypatch, spans, heads, groups
     state = case[6].clone()
     got = H.ssm_prefill(*case[:6], state, *case[7:])
     assert torch.equal(got, runs[0][0]) and torch.equal(state, runs[0][1])
+
+
+@pytest.mark.parametrize("spans, heads, groups, n", [(FOUR, 32, 2, 64), (RAGGED, 64, 1, 128)], ids=["four", "ragged"])
+@pytest.mark.parametrize("whole", [False, True])
+def test_a_sequence_alone_and_among_others(H, monkeypatch, spans, heads, groups, n, whole):  # noqa: F811
+    """The same bits without scratch memory; with it, where a sequence is cut goes by the others: fp32 sums in another order."""
+    case = _case(spans, heads, groups, 64, n, torch.bfloat16, H)
+    x, dt, bias, a_log, d, shape, state, slots, _, _, _ = case
+    if whole:
+        monkeypatch.setattr(H._lib, "mv_ssm_prefill_workspace_bytes", lambda *a: 0)
+    else:
+        assert _scratch(H, case)[1] > _scratch(H, case)[0]
+    left = state.clone()
+    out = H.ssm_prefill(*case[:6], left, *case[7:])
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    begin = 0
+    for (t, before), slot in zip(spans, slots.tolist()):
+        rows, begin = slice(begin, begin + t), begin + t
+        if t < 64:
+            continue
+        kept = state[:, max(slot, 0):max(slot, 0) + 1].contiguous()
+        alone = H.ssm_prefill(x[rows], dt[rows], bias, a_log, d, shape, kept, ints(min(slot, 0)), ints(0, t), ints(0, t + before), t)
+        side = (t + before) & 1
+        if whole:
+            assert torch.equal(out[rows], alone) and (slot < 0 or torch.equal(left[side, slot], kept[side, 0]))
+        else:
+            torch.testing.assert_close(out[rows].float(), alone.float(), rtol=2 ** -7, atol=2 ** -11 * alone.float().abs().max().item())
+            # (each within 2^-17 of token by token)
+            assert slot < 0 or ((left[side, slot] - kept[side, 0]).norm() / kept[side, 0].norm()).item() < 2 ** -16
