@@ -134,16 +134,20 @@ __global__ void __launch_bounds__(THREADS) rope_qk_store_kernel(RopeParams p) {
 }
 
 // Waves of a token.  A wave has its rows one batch of four behind the other, a norm about doubles what a batch takes, and tokens beside each other on a SIMD cover that:
-// the more rows, the more tokens it takes until fewer waves are ahead.  bf16, us by 4 / 2 / 1 waves, with norms: 16 + 8 heads of 128 (rows of q, k and v: 32) 600 tokens
-// 8.3 / 7.6 / 8.3, 1200 11.0 / 9.7 / 10.3, 2048 16.0 / 13.5 / 12.9, 25200 143 / 96 / 92; 64 + 8 of 128 1000 14.9 / 15.4 / 17.9, 1400 18.9 / 20.9 / 22.1, 2800 28.5 / 27.9 /
-// 29.0, 5600 55.0 / 53.1 / 50.9; 32 + 8 of 256 1100 22.7 / 23.3 / 29.2, 5600 83.7 / 73.8 / 68.9; without: 28 + 4 of 128 513 6.6 / 6.5 / 7.2, 1025 9.2 / 8.5 / 8.5, 5000
-// 27.5 / 23.1 / 19.7; 4 + 1 of 128 513 5.6 / 4.6 / 4.3; 64 + 8 of 128 1000 12.0 / 12.0 / 13.7, 2000 20.7 / 18.9 / 18.1; 40 + 40 of 128 (120 rows) 520 11.2 / 11.7 / 15.8,
-// 2800 37.6 / 35.4 / 35.2, 8000 112.8 / 118.3 / 122.6; more than six batches of a single wave: 32 + 16 of 256 with norms 4000 72.6 / 72.6 / 76.5.  Over 36 shapes of 3 to 213
-// rows, 513 to 8000 tokens: 0.91 of the time by four waves in the mean, at worst 4 % above it (4.8 -> 5.0, 22.7 -> 23.5).  fp32 rows are as quick either way (16 + 8 of 128, 5000: 33.8 / 34.4 / 33.1) and slower below (1000: 10.7 / 11.7 / 16.2).
+// the more rows, the more tokens it takes until fewer waves are ahead; up to 768 tokens there are at most three workgroups to a CU, of four waves or of two.  bf16, us by 4 / 2 / 1
+// waves, launches of a graph.  With norms: 16 + 8 heads of 128 (rows of q, k and v: 32) 513 tokens 6.5 / 6.1 / 7.2, 780 8.3 / 7.3 / 7.7, 1200 10.0 / 8.9 / 9.4, 1600 12.7 / 10.9 /
+// 10.4; 24 + 8 513 6.9 / 7.3 / 8.6; 40 + 8 (56 rows) 720 9.1 / 9.7 / 11.6, 780 10.5 / 9.9 / 11.8, 1024 11.3 / 10.6 / 12.6, 1450 14.8 / 15.5 / 16.1; 64 + 8 (80) 720 11.2 / 12.5 / 15.5, 900
+// 13.9 / 14.1 / 16.7, 1450 17.8 / 19.9 / 21.2, 2800 28.5 / 27.9 / 29.0; 16 + 4 of 256 (24) 513 10.8 / 10.3 / 13.3, 1450 19.5 / 17.4 / 17.6, 1900 23.5 / 20.2 / 19.4; 32 + 8 of 256 (48) 1100
+// 22.7 / 23.3 / 29.2, 1900 30.1 / 28.3 / 30.9, 3500 48.0 / 45.5 / 42.0.  Without: 28 + 4 of 128 (36) 513 6.0 / 5.8 / 6.6, 1024 8.2 / 7.4 / 7.4; 64 + 8 720 .. 760 9.3 / 9.4 / 11.7, 780 10.5 / 9.8 /
+// 11.9, 1450 15.8 / 14.8 / 14.8, 1900 18.9 / 17.8 / 16.6; 40 + 40 of 128 (120) 520 11.2 / 11.7 / 15.8, 2800 37.6 / 35.4 / 35.2, 8000 112.8 / 118.3 / 122.6; more than six batches of a
+// single wave: 32 + 16 of 256 with norms 4000 72.6 / 72.6 / 76.5.  Over 23 shapes of 18 to 96 rows, 513 to 5000 tokens (269 pairs): 0.93 of four waves' time in the mean, at worst
+// 6 % above the best.  fp32 rows are as quick either way (16 + 8 of 128, 5000: 33.8 / 34.4 / 33.1) and slower below (1000: 10.7 / 11.7 / 16.2).
 static int waves_of_token(const RopeParams &p, int head_dim, int n_tok) {
-  const int rows = p.n_heads + (p.k_cache ? 2 : 1) * p.n_kv_heads, work = (p.q_norm_w || p.unit) ? 2 * rows : rows;
+  const int rows = p.n_heads + (p.k_cache ? 2 : 1) * p.n_kv_heads, wide = head_dim == 256 ? rows * 3 / 2 : rows;
+  const bool norm = p.q_norm_w || p.unit;
   if (rows > 100 || n_tok <= 512) return 4;
-  return n_tok > 24 * work && rows * head_dim <= 6 * 4 * 512 ? 1 : n_tok > std::min(2048, 20 * work - 500) ? 2 : 4;
+  if (n_tok > (norm ? 44 * wide : std::min(25 * wide, 1400)) && rows * head_dim <= 6 * 4 * 512) return 1;
+  return n_tok > (norm && rows > 64 ? 2048 : rows > (norm ? 36 : 64) ? 768 : 512) ? 2 : 4;
 }
 
 template <typename Tag, int D>

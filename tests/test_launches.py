@@ -116,10 +116,11 @@ def test_a_launch_that_fails_ends_the_experts(call):
 
 
 # heads, heads of keys and values, columns, norms, cache: tokens -> threads of a token: the lines by the rows that a wave would have one behind the other
-ROTATIONS = {(16, 8, 128, True, True): {512: 256, 780: 256, 781: 128, 1536: 128, 1537: 64}, (28, 4, 128, False, True): {512: 256, 513: 128, 864: 128, 865: 64},
-             (64, 8, 128, True, True): {1025: 256, 2048: 256, 2049: 128, 3840: 128, 3841: 64}, (64, 8, 64, False, True): {1100: 256, 1101: 128, 1920: 128, 1921: 64},
-             (4, 1, 128, True, True): {512: 256, 513: 64}, (1, 1, 64, False, False): {513: 64}, (40, 40, 128, False, True): {513: 256, 9000: 256},
-             (40, 40, 128, False, False): {1100: 256, 1101: 128, 1921: 64}, (32, 8, 256, True, True): {2304: 128, 2305: 64}, (32, 16, 256, True, True): {2049: 128, 9000: 128}}
+ROTATIONS = {(16, 8, 128, True, True): {512: 256, 513: 128, 1408: 128, 1409: 64}, (28, 4, 128, False, True): {512: 256, 513: 128, 900: 128, 901: 64},
+             (24, 8, 128, True, True): {768: 256, 769: 128, 1760: 128, 1761: 64}, (64, 8, 128, True, True): {1025: 256, 2048: 256, 2049: 128, 3520: 128, 3521: 64},
+             (64, 8, 64, False, True): {768: 256, 769: 128, 1400: 128, 1401: 64}, (4, 1, 128, True, True): {512: 256, 513: 64}, (1, 1, 64, False, False): {513: 64},
+             (40, 40, 128, False, True): {513: 256, 9000: 256}, (40, 40, 128, False, False): {768: 256, 769: 128, 1401: 64},
+             (32, 8, 256, True, True): {768: 256, 769: 128, 3168: 128, 3169: 64}, (32, 16, 256, True, True): {769: 128, 9000: 128}}
 
 
 def test_waves_of_a_token(call):
