@@ -351,11 +351,12 @@ extern "C" int mv_causal_conv(const MvSsmArgs *a, int dtype, void *stream) {
   if (int e = mv_check_conv(a, dtype)) return e;
   // Few workgroups: eight tokens each, whose loads are one trip to memory, where 32 are four one behind the other; many, whose trips overlap: 32, which read the
   // tokens ahead of theirs less often.  us with 8 and 32 by workgroups of 32 tokens: 18: 5.2 and 11.9, 162: 5.8 and 11.4, 330: 7.9 and 12.4, 594: 11.2 and 14.7,
-  // 1000: 14.7 and 16.4, 1620: 21.5 and 22.8, 1800: 23.8 and 23.1, 4392: the layer around it 225.3 and 222.9.  With eight taps, which are seven
-  // tokens ahead: 576: 14.4 and 17.9, 720 (fp32): 14.5 and 18.5, 1020: 20.9 and 20.6 (fp32 21.1 and 19.6), 1125: 21.9 and 24.4, 1620: 28.1 and 25.8.
-  const int64_t few = a->taps > 4 ? 1000 : 1700;
+  // 1000: 14.7 and 16.4, 1620: 21.5 and 22.8, 1800: 23.8 and 23.1, 4392: the layer around it 225.3 and 222.9.  Any number of taps: 100 drawn shapes
+  // of 500 to 1700 workgroups 0.43 .. 0.94 of the time by 32 (five to eight taps of 1281, 1300, 1640 workgroups 0.91, 0.86, 0.88; one of eight taps elsewhere, of 1298, 1.2), 30 of
+  // 1700 to 4000 0.77 .. 1.11.
+  constexpr int64_t kFewConvs = 1700;
   const int x = (a->channels / (dtype == MV_F32 ? 4 : 8) + 63) / 64;
-  if ((int64_t)x * ((a->max_q + kConvRows - 1) / kConvRows) * a->n_seqs <= few) return launch_conv<kConvAhead>(*a, x, dtype, (hipStream_t)stream);
+  if ((int64_t)x * ((a->max_q + kConvRows - 1) / kConvRows) * a->n_seqs <= kFewConvs) return launch_conv<kConvAhead>(*a, x, dtype, (hipStream_t)stream);
   return launch_conv<kConvRows>(*a, x, dtype, (hipStream_t)stream);
 }
 
