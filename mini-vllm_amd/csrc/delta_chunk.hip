@@ -890,12 +890,13 @@ int launch(const DeltaPrep &q, int seg, hipStream_t stream) {
 
 // bf16, one decay per head: whether the convolution along with the preparation is the shorter way.  Its pieces (four channels, eight tokens) are one turn of a workgroup's
 // threads or several, each a trip to memory of its own, where the convolution's own launch has a piece to a thread; chunks beside each other on a CU cover that, and
-// short prompts of up to two turns are the host's, for whom it is a launch less (beyond, the GPU loses more than the host gains).  us along / apart by turns and workgroups; two heads of 128 x 128 (two turns), in a graph: 8 workgroups
-// 22.9 / 21.4, 68 32.6 / 31.1, 84 56.4 / 55.3, 136 39.2 / 39.7, 736 72.5 / 73.5; the layer around them: 1 x 64 tokens 34.1 / 36.2, 2 x 239 34.4 / 36.9, 1 x 281 36.2 and
-// 37.5 / 37.0 and 36.5, 2 x 400 43.1 / 41.6; of 64 x 64 (one turn): 6 22.0 / 22.9, 496 37.0 / 39.0; of 256 x 128 (three): 40 54.5 / 50.1, 1096 193.8 / 190.6.  One head of
-// 128 x 32 (1.5): 28 26.6 / 25.3, of 64 x 64 (1.5): 198 73.1 / 75.1, 2512 113.5 / 121.6; of 128 x 128 (three): 48 24.3 / 21.5, 200 30.9 / 29.1, 404 54.4 / 56.2, 992 73.1 / 79.2; four turns:
-// 296 80.6 / 78.5.  Two heads of 64 x 32 (one turn; why is not
-// known): 1656 174 / 176, 2512 137 / 134, 5024 265 / 254
+// short prompts of up to two turns are the host's, for whom it is a launch less (beyond, the GPU loses more than the host gains).  us along / apart by workgroups:
+//   two heads of 64 x 64 (one turn): 6 22.0 / 22.9, 496 37.0 / 39.0; of 64 x 32 (one turn; why is not known): 1656 174 / 176, 2512 137 / 134, 5024 265 / 254
+//   two heads of 128 x 128 (two turns), in a graph: 8 22.9 / 21.4, 68 32.6 / 31.1, 84 56.4 / 55.3, 136 39.2 / 39.7, 736 72.5 / 73.5; the layer around them: 1 x 64 tokens
+//   34.1 / 36.2, 2 x 239 34.4 / 36.9, 1 x 281 36.2 and 37.5 / 37.0 and 36.5, 2 x 400 43.1 / 41.6
+//   two heads of 256 x 128 (three): 40 54.5 / 50.1, 1096 193.8 / 190.6
+//   one head of 128 x 32 (1.5): 28 26.6 / 25.3; of 64 x 64 (1.5): 198 73.1 / 75.1, 2512 113.5 / 121.6; of 128 x 128 (three): 48 24.3 / 21.5, 200 30.9 / 29.1,
+//   404 54.4 / 56.2, 992 73.1 / 79.2; four turns: 296 80.6 / 78.5
 bool conv_along(const MvDeltaArgs &a) {
   const int of_group = a.heads / a.groups;
   const int64_t threads = 256 * of_group, pieces = (2 * a.n + of_group * a.p) / 4 * (L / 8), groups = chunk_slots(a.n_seqs, a.total_q) * a.groups;

@@ -1,15 +1,17 @@
 // K15 — the chunked recurrence of ssm_chunk.hip for heads of 64 columns that share b and c: four heads of a group to a workgroup, two waves each.
 //
 // There, a workgroup is a head, whose four waves of 16 columns each read all of b and c out of LDS: its vector instructions, its LDS reads and its products took
-// turns, 2.9 us a chunk and head of a CU.  Here a wave has 32 columns, so that LDS reads are half as many, b and c are staged once for four heads (two stages,
+// turns, 3.1 us a chunk and head of a CU.  Here a wave has 32 columns, so that LDS reads are half as many, b and c are staged once for four heads (two stages,
 // asked for a chunk ahead, without a trip through registers), and the vector unit makes the state's next parts while the matrix cores are at the ones before.  Per
-// element below the diagonal tiles the weight is two products instead of an exponential.  1.4 us a chunk and head: of 13 100 cycles of a chunk of four heads, LDS reads
-// (744 KB, at the 115 bytes a cycle that they reach) are 6500, products 5800, vector instructions 6500; the two waves of a SIMD are in the same phase most of the
-// time, so that these take turns in part.  A workgroup takes a CU's LDS, so that sequences as workgroups would leave half of the chip idle: the chunks of all sequences
-// are dealt out evenly instead (Rows).  So a sequence is cut where those ahead of it say, and its last bits differ with its neighbours (results within a unit, kept
-// states within 2^-16 of their norm), also at sizes where a head a workgroup would take whole sequences, the same bits in any call: without scratch memory that still holds.  64 heads of 64 x 128, 4 sequences of up to 3900 tokens, convolution and norm included: 258 -> 222 us (states 55 -> 44, outputs 143
-// -> 97 under the profiler).  Tried: scores of a chunk made once for the four heads and weighted by each wave (LDS reads 464 KB, vector instructions by a fifth more), and a
-// third barrier for weights made once: as slow; both token tiles of a wave's scores at once, two steps ahead: 97 -> 103.
+// element below the diagonal tiles the weight is two products instead of an exponential.  2.2 us a chunk and head of a CU: a row's 12 chunks of four heads take the
+// outputs' launch 99 .. 105 us, its start and end included, 16 500 cycles each (counters, at 2.0 GHz).  LDS reads (744 KB, at the 115 bytes a cycle that they reach) are 6500 of
+// them, products 5700 (the matrix cores are busy for 34 % of the launch), vector instructions 6500; the two waves of a SIMD are in the same phase most of the time, so that these
+// take turns in part.  A workgroup takes a CU's LDS, so that sequences as workgroups would leave half of the chip idle: the chunks of all sequences are dealt out evenly instead
+// (Rows).  So a sequence is cut where those ahead of it say, and its last bits differ with its neighbours (results within a unit, kept states within 2^-16 of their norm), also at
+// sizes where a head a workgroup would take whole sequences, the same bits in any call: without scratch memory that still holds.  64 heads of 64 x 128, 4 sequences of up to 3900
+// tokens, convolution and norm included: 258 -> 222 us (states 56 -> 45, outputs 145 -> 105 under the profiler).  Tried: scores of a chunk made once for the four heads and
+// weighted by each wave (LDS reads 464 KB, vector instructions by a fifth more), and a third barrier for weights made once: as slow; both token tiles of a wave's scores at once,
+// two steps ahead: 6 % slower.
 #include <algorithm>
 
 #include "ssm.h"
