@@ -261,7 +261,7 @@ __device__ __forceinline__ void group_few(const RouteGroups &q, const int *keys,
 // GROUP (one workgroup has all tokens): the choices stay in LDS for the grouping behind them, a launch and a trip to memory less.  Both products with what is around them, 32
 // experts: 12 tokens of 4 choices (2048 -> 768) 67.2 -> 65.7 us, 4 of 8 (1024 -> 384; the host's) 48.5 -> 44.5.  Up to one tile: two tiles in one
 // workgroup in place of two workgroups cost more than the launch (24 of 4 70.2 -> 74.0, 32 of 8 84 -> 95).  Router, grouping and products in a graph, grouped by another
-// launch and here, 16 experts of 512 -> 128: 64 pairs 15.2 and 12.4, 128 16.8 and 14.5, 192 18.3 and 16.6; of 2048 -> 768 256 (apart then) would be 56.5 and 56.5.
+// launch and here, 16 experts of 512 -> 128: 64 pairs 15.2 and 12.4, 128 16.8 and 14.5, 192 18.3 and 16.6; 256 of 2048 -> 768, which would be on the other side of the line, 56.5 either way.
 template <typename Tag, int WAVES, int TT, bool GROUP>
 __global__ void __launch_bounds__(WAVES * 64) moe_route_kernel(RouteParams p, RouteGroups q) {
   typedef typename elem<Tag>::T T;
